@@ -29,6 +29,7 @@ constexpr int kBlock = 256;   // synthetic-field generator
 constexpr int kResWaves = 8;  // rescale: 8 waves per block, 1 mode per lane per step, next step prefetched
 constexpr int kResUnroll = 1;
 constexpr int kResBlocksPerSlot = 16;
+constexpr int kResModesPerThread = 16;
 
 int *g_nan_flag = nullptr;    // device flag raised by the rescale on a NaN factor
 
@@ -41,25 +42,44 @@ int *nan_flag_ptr()
     return g_nan_flag;
 }
 
+// Blocks of the rescale sweep of a.rows rows, and each block's share of them.
+// Every block first builds its LDS tables, so a block gets at least
+// kResModesPerThread modes per thread before a resident slot is given a second
+// block, up to kResBlocksPerSlot of them: many short row ranges balance a long
+// sweep's tail across the channels (1024^3: 3.76 ms at one block per slot, 3.43
+// at eight, 3.35-3.40 at sixteen), few keep a short sweep from building tables
+// most of its time.  With the Green's function, us per sweep at sixteen per
+// slot whatever the size, and by this rule (8, 16, 32 modes per thread):
+// 128^3 86 -> 16, 16, 16; 256^3 135 -> 65, 63, 63; 384^3 255 -> 211, 197, 204;
+// 512^3 477 -> 479, 453, 456; 1024^3 3620 -> the same grid.
 template <bool GREEN>
-int res_grid(long long rows, size_t smem)
+int res_grid(kn_res::ResArgs &a, size_t smem)
 {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        KN_CHECK(hipGetDevice(&dev));
+    static thread_local size_t known_smem = ~(size_t)0;  // occupancy of the last LDS size asked for
+    static thread_local int known_dev = -1, slots = 0;
+    int dev = 0;
+    KN_CHECK(hipGetDevice(&dev));
+    if (smem != known_smem || dev != known_dev) {
+        int cus = 0, per_cu = 0;
         KN_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const void *k = (const void *)kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>;
+        if (smem > 64 * 1024) KN_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        KN_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>, 64 * kResWaves, smem));
+        slots = (per_cu > 0 ? per_cu : 1) * cus;
+        known_smem = smem;
+        known_dev = dev;
     }
-    int per_cu = 0;
-    const void *k = (const void *)kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>;
-    if (smem > 64 * 1024) KN_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    KN_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>,
-                                                          64 * kResWaves, smem));
-    // sixteen blocks per resident slot: smaller contiguous row ranges per block
-    // balance the sweep's tail across the channels (1024^3: 3.76 ms at one,
-    // 3.43 at eight; with non-temporal loads and stores 3.35-3.40 at sixteen)
-    const long long g = (long long)(per_cu > 0 ? per_cu : 1) * cus * kResBlocksPerSlot;
-    return (int)(rows < g ? rows : g);
+    const long long threads = (long long)slots * 64 * kResWaves, modes = a.rows * (a.dims / 2 + 1);
+    long long per = modes / (threads * kResModesPerThread);
+    per = per < 1 ? 1 : (per > kResBlocksPerSlot ? kResBlocksPerSlot : per);
+    long long g = per * slots;
+    const long long useful = (modes + 64 * kResWaves - 1) / (64 * kResWaves);  // a mode per thread
+    if (g > useful) g = useful;
+    if (g > a.rows) g = a.rows;
+    a.rq = a.rows / g;
+    a.rr = (int)(a.rows % g);
+    return (int)g;
 }
 
 // ---- synthetic Gaussian random field -----------------------------------
@@ -143,7 +163,8 @@ extern "C" int kn_rescale_device(fftw_complex *d_field, int dims, int startslab,
     a.ratio = d_ratio;
     a.nan_flag = nan_flag_ptr();
     a.gw = nullptr;
-    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll>), dim3(res_grid<false>(a.rows, smem)),
+    const int grid = res_grid<false>(a, smem);
+    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll>), dim3(grid),
                        dim3(64 * kResWaves), smem, (hipStream_t)stream, a);
     KN_CHECK(hipGetLastError());
     return 0;
@@ -202,7 +223,8 @@ extern "C" int kn_rescale_green_device(fftw_complex *d_field, int dims, int star
     a.ratio = d_ratio;
     a.nan_flag = nan_flag_ptr();
     a.gw = gw_d;
-    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, true>), dim3(res_grid<true>(a.rows, smem)),
+    const int grid = res_grid<true>(a, smem);
+    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, true>), dim3(grid),
                        dim3(64 * kResWaves), smem, (hipStream_t)stream, a);
     KN_CHECK(hipGetLastError());
     return 0;

@@ -19,6 +19,8 @@ struct ResArgs {
     double2 *F;
     int dims, startslab, nbins, nbuckets;
     long long rows;
+    long long rq;  // block b sweeps rq rows, one more for b < rr (rows = gridDim.x rq + rr)
+    int rr;
     double boxsize, norm;
     const double *logkk, *ratio;
     int *nan_flag;
@@ -121,13 +123,19 @@ __device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
     }
 }
 
-__device__ __forceinline__ Pos pos_of(long long off, long long row0, int rowlen, int dims)
+// Position of mode `off` of the rows from row0 on.
+__device__ __forceinline__ Pos pos_of(int off, long long row0, int rowlen, int dims)
 {
     Pos p;
+    p.z = off % rowlen;
     const long long rl = row0 + off / rowlen;
-    p.z = (int)(off % rowlen);
-    p.j = (int)(rl % dims);
-    p.i = (int)(rl / dims);
+    if (rl < 0x7fffffffLL) {  // rows of any grid that fits the card: 32-bit division
+        p.j = (int)((unsigned)rl % (unsigned)dims);
+        p.i = (int)((unsigned)rl / (unsigned)dims);
+    } else {
+        p.j = (int)(rl % dims);
+        p.i = (int)(rl / dims);
+    }
     return p;
 }
 
@@ -150,7 +158,9 @@ __device__ __forceinline__ double green_of(int k2, double gx, double gy, double 
 // The rescale sweep: each block a contiguous row range, lane l of the block
 // takes modes l, l + B, ... (coalesced), the next UNROLL modes loaded before
 // the current ones are rescaled and stored; loads and stores carry the
-// non-temporal hint (each mode is read and written once per sweep).
+// non-temporal hint (each mode is read and written once per sweep).  The
+// first modes are requested before the tables are built, so that their
+// latency and the tables' pass together.
 // GREEN: the same sweep also applies the Green's function (F s_nu, then times
 // G, the two roundings of the two passes it replaces) and zeroes the k = 0
 // mode; with nbins 0 it applies the Green's function alone.
@@ -158,6 +168,17 @@ template <int WAVES, int UNROLL, bool GREEN = false>
 __global__ __launch_bounds__(64 * WAVES) void k_rescale_rows_pf(ResArgs a)
 {
     constexpr int B = 64 * WAVES;
+    const int rowlen = a.dims / 2 + 1;
+    const long long b = blockIdx.x, r0 = b * a.rq + (b < a.rr ? b : a.rr), r1 = r0 + a.rq + (b < a.rr);
+    const long long m1 = r1 * rowlen;
+    const long long S = (long long)B * UNROLL;
+    long long m = r0 * rowlen + threadIdx.x;
+    double2 cur[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; u++) {
+        const long long mu = m + (long long)B * u;
+        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+    }
     Tab T;
     const double *gw = nullptr;
     if (!GREEN || a.nbins > 0) T = load_tab(a, B);
@@ -169,19 +190,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_rescale_rows_pf(ResArgs a)
         __syncthreads();
         gw = gw_l;
     }
-    const int rowlen = a.dims / 2 + 1;
-    const long long r0 = a.rows * blockIdx.x / gridDim.x, r1 = a.rows * (blockIdx.x + 1) / gridDim.x;
-    const long long m1 = r1 * rowlen;
-    const long long S = (long long)B * UNROLL;
     Pos p = pos_of(threadIdx.x, r0, rowlen, a.dims);
     bool saw_nan = false;
-    long long m = r0 * rowlen + threadIdx.x;
-    double2 cur[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; u++) {
-        const long long mu = m + (long long)B * u;
-        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
-    }
     for (; m < m1; m += S) {
         double2 nxt[UNROLL];
 #pragma unroll
