@@ -82,13 +82,19 @@ __device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
     }
 }
 
-__device__ __forceinline__ Pos pos_of(long long off, long long row0, int rowlen, int dims)
+// Position of mode `off` of the rows from row0 on.
+__device__ __forceinline__ Pos pos_of(int off, long long row0, int rowlen, int dims)
 {
     Pos p;
+    p.z = off % rowlen;
     const long long rl = row0 + off / rowlen;
-    p.z = (int)(off % rowlen);
-    p.j = (int)(rl % dims);
-    p.i = (int)(rl / dims);
+    if (rl < 0x7fffffffLL) {  // rows of any grid that fits the card: 32-bit division
+        p.j = (int)((unsigned)rl % (unsigned)dims);
+        p.i = (int)((unsigned)rl / (unsigned)dims);
+    } else {
+        p.j = (int)(rl % dims);
+        p.i = (int)(rl / dims);
+    }
     return p;
 }
 
@@ -103,16 +109,6 @@ __device__ __forceinline__ double mode_weight(double2 f, double iwxy, double iwz
     if (kz != 0 && kz != half) v *= 2.0;
     return v;
 }
-
-struct BinArgs {
-    const double2 *F;
-    int dims, startslab, nrbins;
-    long long rows;
-    const int *thr;
-    const double *iw;
-    float half_bpu;
-    double *partial;  // gridDim.x * nrbins
-};
 
 // A step of n modes along the flattened [slab][row][z] order, split so that
 // advancing a position costs two compares whatever n is.
@@ -129,6 +125,19 @@ __host__ __device__ inline Step step_of(long long n, int rowlen, int dims)
     s.di = (int)(r / dims);
     return s;
 }
+
+struct BinArgs {
+    const double2 *F;
+    int dims, startslab, nrbins;
+    long long rows;
+    long long rq;  // rows = gridDim.x rq + rr: every block rq rows, rr of them one more
+    unsigned rr;
+    const int *thr;
+    const double *iw;
+    float half_bpu;
+    double *partial;  // gridDim.x * nrbins
+    Step step;        // one pass of a block: 64 kSweepRun modes per wavefront
+};
 
 __device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int dims)
 {
@@ -155,13 +164,14 @@ enum TablePlace { kTablesLds = 0, kWindowGlobal = 1, kTablesGlobal = 2 };
 constexpr int kSweepWaves = 8;  // wavefronts per block
 constexpr int kSweepRun = 4;    // consecutive modes per lane (one staged chunk: 64 * kSweepRun modes per wave)
 
-// LDS bytes of the sweep: the staging buffers, then the tables the placement keeps there.
-__host__ __device__ constexpr size_t sweep_smem_bytes(int place, int dims, int nrbins)
+// LDS bytes of the sweep: the staging buffers, then the tables the placement
+// keeps there (own: one set of bin sums per wavefront).
+__host__ __device__ constexpr size_t sweep_smem_bytes(int place, int dims, int nrbins, bool own = false)
 {
     return sizeof(double2) * (size_t)kSweepWaves * 64 * kSweepRun +
            (place == kTablesGlobal
                 ? 0
-                : sizeof(double) * (size_t)nrbins + sizeof(int) * (size_t)(nrbins + 1 + ((nrbins + 1) & 1)) +
+                : sizeof(double) * (size_t)nrbins * (own ? kSweepWaves : 1) + sizeof(int) * (size_t)(nrbins + 1 + ((nrbins + 1) & 1)) +
                       (place == kTablesLds ? sizeof(double) * (size_t)dims : 0));
 }
 
@@ -186,16 +196,35 @@ __device__ __forceinline__ int stage_slot(int m)
 // of it: along a row |k|^2 grows with z, so after a run's first mode its bin
 // is found incrementally (the next threshold kept in a register, at most one
 // step before a full search), equal-bin runs are summed in registers and
-// flushed with one atomic add per run.  The block's wavefronts share one set
-// of bin sums, so the order of the adds between wavefronts (and the last bit
-// of a sum) can differ from run to run; the block writes its sums to its
-// partial row, which k_reduce_partials adds in a fixed order.
-template <int PLACE>
+// flushed with one atomic add per run.  With OWN every wavefront has its own
+// bin sums, added in a fixed order at the end, and the result is the same on
+// every run; without it the block's wavefronts share one set, so the order of
+// the adds between wavefronts (and the last bit of a sum) can differ from run
+// to run.  The block writes its sums to its partial row, and
+// k_reduce_partials adds the rows in a fixed order.
+template <int PLACE, bool OWN = false>
 __global__ __launch_bounds__(64 * kSweepWaves) void k_bin_sweep(BinArgs a)
 {
     constexpr int WAVES = kSweepWaves, RUN = kSweepRun;
     extern __shared__ double smem[];
     double2 *stage_all = (double2 *)smem;  // WAVES * 64 * RUN modes, 16-byte aligned
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rowlen = a.dims / 2 + 1, half = a.dims / 2;
+    // rows gridDim.x-ths by b rows / gridDim.x: ranges of both lengths in turn (all longer ones first: 1.45 ms
+    // against 1.42 at 1024^3, the blocks' addresses then being one stride apart); the host keeps gridDim.x <= 65535
+    const unsigned blk = blockIdx.x, e0 = blk * a.rr / gridDim.x, e1 = (blk + 1) * a.rr / gridDim.x;
+    const long long r0 = blk * a.rq + e0, r1 = r0 + a.rq + (e1 - e0);
+    const long long m0 = r0 * rowlen, m1 = r1 * rowlen;
+    constexpr int CH = 64 * RUN;
+    constexpr long long S = (long long)CH * WAVES;
+    long long c = m0 + (long long)wave * CH;
+    // the first chunk is requested before the tables are read, so that the two latencies overlap
+    double2 cur[RUN];
+#pragma unroll
+    for (int u = 0; u < RUN; u++) {
+        const long long mu = c + 64 * u + lane;
+        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+    }
     double *hist;
     const double *iw;
     const int *thr;
@@ -206,8 +235,9 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_bin_sweep(BinArgs a)
         for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES) hist[t] = 0.0;
     } else {
         hist = (double *)(stage_all + (size_t)WAVES * 64 * RUN);
-        int *thr_l = (int *)(hist + a.nrbins);
-        for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES) hist[t] = 0.0;
+        const int nhist = OWN ? WAVES * a.nrbins : a.nrbins;
+        int *thr_l = (int *)(hist + nhist);
+        for (int t = threadIdx.x; t < nhist; t += 64 * WAVES) hist[t] = 0.0;
         for (int t = threadIdx.x; t <= a.nrbins; t += 64 * WAVES) thr_l[t] = a.thr[t];
         thr = thr_l;
         if constexpr (PLACE == kTablesLds) {
@@ -219,22 +249,11 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_bin_sweep(BinArgs a)
         }
     }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double *const all = hist;
+    if constexpr (OWN) hist += wave * a.nrbins;
     double2 *stage = stage_all + (size_t)wave * 64 * RUN;
-    const int rowlen = a.dims / 2 + 1, half = a.dims / 2;
-    const long long r0 = a.rows * blockIdx.x / gridDim.x, r1 = a.rows * (blockIdx.x + 1) / gridDim.x;
-    const long long m0 = r0 * rowlen, m1 = r1 * rowlen;
-    constexpr int CH = 64 * RUN;
-    const long long S = (long long)CH * WAVES;
-    const Step sS = step_of(S, rowlen, a.dims);
-    long long c = m0 + (long long)wave * CH;
-    Pos p = pos_of((long long)wave * CH + (long long)lane * RUN, r0, rowlen, a.dims);
-    double2 cur[RUN];
-#pragma unroll
-    for (int u = 0; u < RUN; u++) {
-        const long long mu = c + 64 * u + lane;
-        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
-    }
+    const Step sS = a.step;
+    Pos p = pos_of(wave * CH + lane * RUN, r0, rowlen, a.dims);
     for (; c < m1; c += S) {
         double2 nxt[RUN];
 #pragma unroll
@@ -310,8 +329,13 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_bin_sweep(BinArgs a)
     }
     if constexpr (PLACE != kTablesGlobal) {
         __syncthreads();
-        for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES)
-            a.partial[(size_t)blockIdx.x * a.nrbins + t] = hist[t];
+        for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES) {
+            double v = all[t];
+            if constexpr (OWN)
+#pragma unroll
+                for (int w = 1; w < WAVES; w++) v += all[w * a.nrbins + t];
+            a.partial[(size_t)blockIdx.x * a.nrbins + t] = v;
+        }
     }
 }
 

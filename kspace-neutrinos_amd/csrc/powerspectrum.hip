@@ -43,7 +43,16 @@ using kn_bin::kval;
 constexpr int kBlock = 256;  // geometry pass
 constexpr int kWaves = kBlock / 64;
 constexpr int kSweepSlots = 2;  // bin sweep blocks per resident slot (1.41-1.44 ms at 1024^3 against 1.45 at three)
+constexpr int kSweepPasses = 8;  // passes a block gets before a slot takes a second block (sweep_grid)
 constexpr size_t kLdsMax = 160 * 1024;
+
+// How one geometry is swept: where the tables are, whether every wavefront has
+// its own bin sums, the blocks and their LDS.
+struct SweepPlan {
+    int place = 0, grid = 0;
+    bool own = false;
+    size_t smem = 0;
+};
 
 struct BinGeom {
     int dims, nrbins, startslab, nslab;
@@ -52,9 +61,8 @@ struct BinGeom {
     float half_bpu;   // 0.5 * binsperunit, for the fp32 estimate
     std::vector<long long> count;
     std::vector<double> keff_sum;
-    int grid, ggrid;        // power-pass and geometry-pass grids
-    int place;              // where the sweep keeps its tables (kn_bin::TablePlace)
-    size_t smem;            // the sweep's LDS bytes
+    SweepPlan plan;         // the power pass
+    int ggrid;              // geometry-pass grid
     double *d_partial;      // max(grid, ggrid) * nrbins
     unsigned *d_cpartial;   // ggrid * nrbins (geometry pass)
     double *d_sum;          // nrbins + 1 (last: |F0|^2)
@@ -136,37 +144,52 @@ __global__ __launch_bounds__(kBlock) void k_bin_geometry(int dims, int startslab
     }
 }
 
-// Fixed-order sum of per-block partial histograms: 64 bins per block across
-// lanes, 16 waves split the blocks, then a fixed-order combine in LDS.
-constexpr int kRedWaves = 16;
-__global__ __launch_bounds__(64 * kRedWaves) void k_reduce_partials(const double *__restrict__ partial, int nblk,
-                                                                     int nrbins, double *__restrict__ out)
+// Fixed-order sum of the per-block partial histograms into out[nrbins], and
+// |F0|^2 (powerspectrum.c:45-47; 0 on a rank without the zero mode) into
+// mass_out.  A block takes kRedBins bins (one 64-byte line of every partial
+// row); its kRedGroups threads per bin each add every kRedGroups-th row, with
+// kRedLoads loads in flight, and a fixed tree in LDS adds the threads' sums.
+// The reads are latency: with 64 bins per block and 96 rows per thread in
+// batches of eight, the 1536 rows of a 256^3 sweep took 12.3 us, and |F0|^2
+// another launch of 4-5.6 us.
+constexpr int kRedBins = 8, kRedGroups = 128, kRedLoads = 8;
+__global__ __launch_bounds__(kRedBins * kRedGroups) void k_reduce_partials(const double *__restrict__ partial, int nblk,
+                                                                           int nrbins, double *__restrict__ out,
+                                                                           const double2 *__restrict__ F,
+                                                                           int has_zero_mode,
+                                                                           double *__restrict__ mass_out)
 {
-    __shared__ double acc[kRedWaves][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int b = blockIdx.x * 64 + lane;
-    const int g0 = nblk * wave / kRedWaves, g1 = nblk * (wave + 1) / kRedWaves;
+    __shared__ double acc[kRedGroups][kRedBins];
+    const int l = threadIdx.x % kRedBins, grp = threadIdx.x / kRedBins;
+    const int b = blockIdx.x * kRedBins + l;
     double s = 0.0;
     if (b < nrbins) {
-        // eight loads in flight, added in block order
-        constexpr int U = 8;
-        int g = g0;
-        for (; g + U <= g1; g += U) {
-            double v[U];
+        for (int g = grp; g < nblk; g += kRedGroups * kRedLoads) {
+            double v[kRedLoads];
 #pragma unroll
-            for (int u = 0; u < U; u++) v[u] = partial[(size_t)(g + u) * nrbins + b];
+            for (int u = 0; u < kRedLoads; u++) {
+                const int r = g + u * kRedGroups;
+                v[u] = r < nblk ? partial[(size_t)r * nrbins + b] : 0.0;
+            }
 #pragma unroll
-            for (int u = 0; u < U; u++) s += v[u];
+            for (int u = 0; u < kRedLoads; u++) s += v[u];
         }
-        for (; g < g1; g++) s += partial[(size_t)g * nrbins + b];
     }
-    acc[wave][lane] = s;
-    __syncthreads();
-    if (wave == 0 && b < nrbins) {
-        double t = acc[0][lane];
-        for (int w = 1; w < kRedWaves; w++) t += acc[w][lane];
-        out[b] = t;
+    acc[grp][l] = s;
+    if (blockIdx.x == 0 && threadIdx.x == kRedBins * kRedGroups - 1) {
+        double m = 0.0;
+        if (has_zero_mode) {
+            const double2 f = F[0];
+            m = f.x * f.x + f.y * f.y;
+        }
+        *mass_out = m;
     }
+#pragma unroll
+    for (int d = kRedGroups / 2; d >= 1; d >>= 1) {
+        __syncthreads();
+        if (grp < d) acc[grp][l] += acc[grp + d][l];
+    }
+    if (grp == 0 && b < nrbins) out[b] = acc[0][l];
 }
 
 __global__ void k_reduce_counts(const unsigned *__restrict__ cpartial, const double *__restrict__ kpartial,
@@ -183,17 +206,6 @@ __global__ void k_reduce_counts(const unsigned *__restrict__ cpartial, const dou
     }
     count[b] = c;
     ksum[b] = s;
-}
-
-// |F0|^2 from the rank holding slab 0 (powerspectrum.c:45-47), else 0.
-__global__ void k_total_mass2(const double2 *__restrict__ F, int has_zero_mode, double *__restrict__ out)
-{
-    if (has_zero_mode) {
-        const double2 f = F[0];
-        *out = f.x * f.x + f.y * f.y;
-    } else {
-        *out = 0.0;
-    }
 }
 
 int num_cus()
@@ -220,6 +232,63 @@ int resident_blocks(K kernel, int threads, size_t smem)
     return n > 0 ? n : 1;
 }
 
+typedef void (*SweepKernel)(kn_bin::BinArgs);
+SweepKernel sweep_kernel(const SweepPlan &p)
+{
+    if (p.place == kn_bin::kTablesLds)
+        return p.own ? kn_bin::k_bin_sweep<kn_bin::kTablesLds, true> : kn_bin::k_bin_sweep<kn_bin::kTablesLds>;
+    if (p.place == kn_bin::kWindowGlobal)
+        return p.own ? kn_bin::k_bin_sweep<kn_bin::kWindowGlobal, true> : kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>;
+    return kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>;
+}
+
+// The tables' placement: the first whose LDS leaves room for two blocks per
+// CU, else the first that fits at all (kTablesGlobal always does).  Own bin
+// sums where they leave three blocks per CU their LDS (as many as the sweep's
+// registers allow).
+// Blocks: a pass is 64 kSweepRun modes per wavefront of a block.  A block with
+// less than one spends its time on its tables and its partial row, so a small
+// grid gets one block per pass (with own bin sums, now whatever their LDS:
+// no second block waits for it); then one block per resident slot; and two per
+// slot (a better balanced tail) only from kSweepPasses passes per block on.
+// A small grid with so many bins that own sums do not fit gets a block per
+// row: there, too, its sums are the same on every run.
+// us per call, sweep and reduction, at two per slot whatever the size, and by
+// this rule: 64^3 24.3 -> 10.1, 128^3 27.0 -> 14.4, 192^3 36.6 -> 22.0, 256^3
+// 49.2 -> 35.2, 512^3 199.6 -> 191, 1024^3 1429 -> 1419 (its grid unchanged).
+SweepPlan sweep_plan(long long rows, int dims, int nrbins)
+{
+    SweepPlan p;
+    p.place = kn_bin::kTablesGlobal;
+    for (size_t most : {kLdsMax, kLdsMax / 2})
+        for (int pl : {kn_bin::kWindowGlobal, kn_bin::kTablesLds})
+            if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= most) p.place = pl;
+    const long long pass = 64LL * kn_bin::kSweepRun * kn_bin::kSweepWaves;
+    const long long passes = (rows * (dims / 2 + 1) + pass - 1) / pass;
+    const size_t own = kn_bin::sweep_smem_bytes(p.place, dims, nrbins, true);
+    const bool few = passes < num_cus();  // no CU gets a second block
+    p.own = p.place != kn_bin::kTablesGlobal && own <= (few ? kLdsMax : kLdsMax / 3);
+    p.smem = p.own ? own : kn_bin::sweep_smem_bytes(p.place, dims, nrbins);
+    const long long slots = (long long)resident_blocks(sweep_kernel(p), 64 * kn_bin::kSweepWaves, p.smem) * num_cus();
+    long long g = passes < slots ? passes : slots;
+    if (passes >= kSweepPasses * kSweepSlots * slots || (few && !p.own)) g = kSweepSlots * slots;
+    if (g > 65535) g = 65535;  // the sweep's 32-bit row shares
+    p.grid = (int)(rows < g ? rows : g);
+    return p;
+}
+
+void launch_sweep(kn_bin::BinArgs &a, const SweepPlan &p, hipStream_t st, double *sum_out, double *mass_out)
+{
+    a.rq = a.rows / p.grid;
+    a.rr = (unsigned)(a.rows % p.grid);
+    a.step = kn_bin::step_of(64LL * kn_bin::kSweepRun * kn_bin::kSweepWaves, a.dims / 2 + 1, a.dims);
+    hipLaunchKernelGGL(sweep_kernel(p), dim3(p.grid), dim3(64 * kn_bin::kSweepWaves), p.smem, st, a);
+    KN_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(k_reduce_partials, dim3((a.nrbins + kRedBins - 1) / kRedBins), dim3(kRedBins * kRedGroups), 0,
+                       st, a.partial, p.grid, a.nrbins, sum_out, a.F, a.startslab == 0 ? 1 : 0, mass_out);
+    KN_CHECK(hipGetLastError());
+}
+
 BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
 {
     for (BinGeom *g : g_geoms)
@@ -239,32 +308,9 @@ BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
     kn_bin::build_invwindow(dims, iw);
     g->half_bpu = (float)(0.5 * (nrbins - 1) / log(sqrt(3) * dims / 2.0));
     const long long rows = (long long)nslab * dims;
-    // the first table placement whose LDS leaves room for two blocks per CU,
-    // else the first that fits at all (kTablesGlobal always does)
-    g->place = kn_bin::kTablesGlobal;
-    for (int pl : {kn_bin::kTablesLds, kn_bin::kWindowGlobal})
-        if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= kLdsMax / 2) {
-            g->place = pl;
-            break;
-        }
-    if (g->place == kn_bin::kTablesGlobal)
-        for (int pl : {kn_bin::kTablesLds, kn_bin::kWindowGlobal})
-            if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= kLdsMax) {
-                g->place = pl;
-                break;
-            }
-    g->smem = kn_bin::sweep_smem_bytes(g->place, dims, nrbins);
-    const int per_cu = g->place == kn_bin::kTablesLds
-                           ? resident_blocks(kn_bin::k_bin_sweep<kn_bin::kTablesLds>, 64 * kn_bin::kSweepWaves, g->smem)
-                       : g->place == kn_bin::kWindowGlobal
-                           ? resident_blocks(kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>, 64 * kn_bin::kSweepWaves,
-                                             g->smem)
-                           : resident_blocks(kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>, 64 * kn_bin::kSweepWaves,
-                                             g->smem);
-    const long long pgrid = (long long)per_cu * num_cus() * kSweepSlots;
-    g->grid = (int)(rows < pgrid ? rows : pgrid);
+    g->plan = sweep_plan(rows, dims, nrbins);
     g->ggrid = (int)(rows < 4LL * num_cus() ? rows : 4LL * num_cus());
-    const int pmax = g->grid > g->ggrid ? g->grid : g->ggrid;
+    const int pmax = g->plan.grid > g->ggrid ? g->plan.grid : g->ggrid;
     KN_CHECK(hipMalloc(&g->d_thr, sizeof(int) * (nrbins + 1)));
     KN_CHECK(hipMalloc(&g->d_iw, sizeof(double) * dims));
     KN_CHECK(hipMalloc(&g->d_partial, sizeof(double) * (size_t)pmax * nrbins));
@@ -320,19 +366,7 @@ void launch_power(BinGeom *g, const double2 *F, hipStream_t st, double *sum_out 
     a.iw = g->d_iw;
     a.half_bpu = g->half_bpu;
     a.partial = g->d_partial;
-    const dim3 grid(g->grid), block(64 * kn_bin::kSweepWaves);
-    if (g->place == kn_bin::kTablesLds)
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kTablesLds>, grid, block, g->smem, st, a);
-    else if (g->place == kn_bin::kWindowGlobal)
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>, grid, block, g->smem, st, a);
-    else
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>, grid, block, g->smem, st, a);
-    KN_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_reduce_partials, dim3((g->nrbins + 63) / 64), dim3(64 * kRedWaves), 0, st, g->d_partial,
-                       g->grid, g->nrbins, sum_out);
-    KN_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_total_mass2, dim3(1), dim3(1), 0, st, F, g->startslab == 0 ? 1 : 0, mass_out);
-    KN_CHECK(hipGetLastError());
+    launch_sweep(a, g->plan, st, sum_out, mass_out);
 }
 
 // Adjoint sweep of the binning: Fbar_m = s_m F_m with s_m = 2 c_m W_m^-4
@@ -372,7 +406,7 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_bin_adjoint(const double2 *_
     const long long r0 = rows * blockIdx.x / gridDim.x, r1 = rows * (blockIdx.x + 1) / gridDim.x;
     const long long m1 = r1 * rowlen;
     constexpr long long S = (long long)B * kAdjUnroll;
-    Pos p = kn_bin::pos_of(threadIdx.x, r0, rowlen, dims);
+    Pos p = kn_bin::pos_of((int)threadIdx.x, r0, rowlen, dims);
     long long m = r0 * rowlen + threadIdx.x;
     double2 cur[kAdjUnroll];
 #pragma unroll
@@ -444,6 +478,8 @@ constexpr int kScratchMaxDevices = 64;
 struct ScratchDev {
     unsigned char *ptr = nullptr;  // this device's copy of scratch (hipGetSymbolAddress)
     int dims = 0, nrbins = 0;      // the geometry whose tables the copy holds
+    SweepPlan plan;                // that geometry's plan for plan_rows rows (grid 0: none yet)
+    long long plan_rows = 0;
 };
 ScratchDev g_scratch[kScratchMaxDevices];
 
@@ -511,33 +547,16 @@ extern "C" int kn_bin_power_device_noalloc(const fftw_complex *d_field, int dims
         KN_CHECK(hipStreamSynchronize(st));  // the host tables may be rebuilt by the next call
         sd.dims = dims;
         sd.nrbins = nrbins;
+        sd.plan.grid = 0;
     }
-    // placement and grid as get_geom chooses them, the grid capped by the scratch
-    int place = kn_bin::kTablesGlobal;
-    for (int pl : {kn_bin::kTablesLds, kn_bin::kWindowGlobal})
-        if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= kLdsMax / 2) {
-            place = pl;
-            break;
-        }
-    if (place == kn_bin::kTablesGlobal)
-        for (int pl : {kn_bin::kTablesLds, kn_bin::kWindowGlobal})
-            if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= kLdsMax) {
-                place = pl;
-                break;
-            }
-    const size_t smem = kn_bin::sweep_smem_bytes(place, dims, nrbins);
-    const int per_cu = place == kn_bin::kTablesLds
-                           ? resident_blocks(kn_bin::k_bin_sweep<kn_bin::kTablesLds>, 64 * kn_bin::kSweepWaves, smem)
-                       : place == kn_bin::kWindowGlobal
-                           ? resident_blocks(kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>, 64 * kn_bin::kSweepWaves,
-                                             smem)
-                           : resident_blocks(kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>, 64 * kn_bin::kSweepWaves,
-                                             smem);
+    // the plan get_geom makes, the grid capped by the scratch
     const long long rows = (long long)nslab * dims;
-    long long grid = (long long)per_cu * num_cus() * kSweepSlots;
-    const long long fit = (long long)((kScratchBytes - off_part) / (sizeof(double) * (size_t)nrbins));
-    if (grid > fit) grid = fit;
-    if (grid > rows) grid = rows;
+    if (sd.plan.grid == 0 || sd.plan_rows != rows) {
+        sd.plan = sweep_plan(rows, dims, nrbins);
+        sd.plan_rows = rows;
+        const long long fit = (long long)((kScratchBytes - off_part) / (sizeof(double) * (size_t)nrbins));
+        if (sd.plan.grid > fit) sd.plan.grid = (int)fit;
+    }
     kn_bin::BinArgs a;
     a.F = (const double2 *)d_field;
     a.dims = dims;
@@ -548,19 +567,7 @@ extern "C" int kn_bin_power_device_noalloc(const fftw_complex *d_field, int dims
     a.iw = (const double *)(sd.ptr + off_iw);
     a.half_bpu = (float)(0.5 * (nrbins - 1) / log(sqrt(3) * dims / 2.0));
     a.partial = (double *)(sd.ptr + off_part);
-    const dim3 gr((unsigned)grid), block(64 * kn_bin::kSweepWaves);
-    if (place == kn_bin::kTablesLds)
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kTablesLds>, gr, block, smem, st, a);
-    else if (place == kn_bin::kWindowGlobal)
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>, gr, block, smem, st, a);
-    else
-        hipLaunchKernelGGL(kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>, gr, block, smem, st, a);
-    KN_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_reduce_partials, dim3((nrbins + 63) / 64), dim3(64 * kRedWaves), 0, st, a.partial,
-                       (int)grid, nrbins, d_power);
-    KN_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_total_mass2, dim3(1), dim3(1), 0, st, a.F, startslab == 0 ? 1 : 0, d_total_mass2);
-    KN_CHECK(hipGetLastError());
+    launch_sweep(a, sd.plan, st, d_power, d_total_mass2);
     return 0;
 }
 

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle_py as O
-from test_gpu_binning import _rand_grid
+from test_gpu_binning import _rand_grid, check_against_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,38 @@ def test_rescale_shares(kn, torch_cuda, N, start, nslab, green):
         W = O.green(W, BOX, asmth, start)
     assert rc == 0 and rc2 == 0
     np.testing.assert_allclose(d.cpu().numpy().view(np.float64), W.view(np.float64), rtol=1e-14, atol=0)
+
+
+@pytest.mark.parametrize("N,start,nslab,nb", [(4, 0, 4, 15), (5, 3, 1, 7), (33, 0, 33, 9), (96, 0, 96, 96), (192, 0, 192, 64),
+                                              (250, 100, 37, 64), (250, 0, 250, 1000), (64, 0, 64, 12000)])
+def test_bin_shares(kn, torch_cuda, N, start, nslab, nb):
+    """One block and one partial row, a pass per block, a block per resident slot; few and many bins for the reduction
+    (counts equal, sums to 1e-12 as the other tests of the sums: they are added in another order)."""
+    torch = torch_cuda
+    F = _rand_grid(N, 7, nslab)
+    if start == 0:
+        check_against_oracle(kn, torch, F, nb)
+        return
+    d, p = torch.from_numpy(F).cuda(), torch.full((nb + 1,), -1.0, dtype=torch.float64, device="cuda")
+    for fn in (kn.kn_bin_power_device, kn.kn_bin_power_device_noalloc):
+        print("bin shares", N, start, nslab, nb, flush=True)
+        assert fn(d.data_ptr(), N, nb, start, nslab, p.data_ptr(), p.data_ptr() + 8 * nb, None) == 0
+        got = p.cpu().numpy()
+        want = O.bin_sums(F, nb, start)[0]
+        np.testing.assert_allclose(got[:nb], want, rtol=1e-12, atol=0)
+        assert got[nb] == 0.0
+
+
+@pytest.mark.parametrize("N,nb", [(8, 10), (32, 1500), (36, 12000), (64, 64), (256, 128)])
+def test_bin_sums_repeat(kn, torch_cuda, N, nb):
+    """Own bin sums per wavefront (small grids, and few bins at any size), and small grids with a block per row for want of
+    LDS: the same bits on every run."""
+    torch = torch_cuda
+    print("bin repeat", N, nb, flush=True)
+    d = torch.from_numpy(_rand_grid(N, 9)).cuda()
+    out = []
+    for _ in range(4):
+        p = torch.zeros(nb + 1, dtype=torch.float64, device="cuda")
+        assert kn.kn_bin_power_device(d.data_ptr(), N, nb, 0, N, p.data_ptr(), p.data_ptr() + 8 * nb, None) == 0
+        out.append(p.cpu().numpy())
+    assert all(np.array_equal(out[0], o) for o in out[1:])
