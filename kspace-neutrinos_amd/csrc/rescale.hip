@@ -9,10 +9,10 @@
 //    smth = 1 + norm * (linear interpolation of ratio in logk);
 //    NaN smth is fatal (code 5); F *= smth.
 // MI355X design: one coalesced read+write sweep (32 B per mode, non-temporal
-// loads and stores).  The ratio table and a uniform bucket index over logk
-// live in LDS, so the segment search is a bucket lookup plus a short forward
-// probe instead of a binary search.  All arithmetic is FP64 and follows the
-// reference's expression order.
+// loads and stores).  The ratio table with its slopes, a table for the
+// logarithm and a uniform bucket index over logk live in LDS, so the segment
+// search is a bucket lookup plus a short forward probe instead of a binary
+// search.  All arithmetic is FP64.
 #include <math.h>
 #include <string.h>
 
@@ -26,10 +26,8 @@
 namespace {
 
 constexpr int kBlock = 256;   // synthetic-field generator
-constexpr int kResWaves = 8;  // rescale: 8 waves per block, 1 mode per lane per step, next step prefetched
-constexpr int kResUnroll = 1;
-constexpr int kResBlocksPerSlot = 16;
-constexpr int kResModesPerThread = 16;
+constexpr int kResWaves = 8;  // rescale: wavefronts per block, two blocks per CU
+constexpr int kResUnroll = 2; // modes per lane of a tile
 
 int *g_nan_flag = nullptr;    // device flag raised by the rescale on a NaN factor
 
@@ -42,44 +40,55 @@ int *nan_flag_ptr()
     return g_nan_flag;
 }
 
-// Blocks of the rescale sweep of a.rows rows, and each block's share of them.
-// Every block first builds its LDS tables, so a block gets at least
-// kResModesPerThread modes per thread before a resident slot is given a second
-// block, up to kResBlocksPerSlot of them: many short row ranges balance a long
-// sweep's tail across the channels (1024^3: 3.76 ms at one block per slot, 3.43
-// at eight, 3.35-3.40 at sixteen), few keep a short sweep from building tables
-// most of its time.  With the Green's function, us per sweep at sixteen per
-// slot whatever the size, and by this rule (8, 16, 32 modes per thread):
-// 128^3 86 -> 16, 16, 16; 256^3 135 -> 65, 63, 63; 384^3 255 -> 211, 197, 204;
-// 512^3 477 -> 479, 453, 456; 1024^3 3620 -> the same grid.
-template <bool GREEN>
-int res_grid(kn_res::ResArgs &a, size_t smem)
+int res_cus()
 {
-    static thread_local size_t known_smem = ~(size_t)0;  // occupancy of the last LDS size asked for
-    static thread_local int known_dev = -1, slots = 0;
-    int dev = 0;
-    KN_CHECK(hipGetDevice(&dev));
-    if (smem != known_smem || dev != known_dev) {
-        int cus = 0, per_cu = 0;
-        KN_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const void *k = (const void *)kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>;
-        if (smem > 64 * 1024) KN_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-        KN_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, GREEN>, 64 * kResWaves, smem));
-        slots = (per_cu > 0 ? per_cu : 1) * cus;
-        known_smem = smem;
-        known_dev = dev;
-    }
-    const long long threads = (long long)slots * 64 * kResWaves, modes = a.rows * (a.dims / 2 + 1);
-    long long per = modes / (threads * kResModesPerThread);
-    per = per < 1 ? 1 : (per > kResBlocksPerSlot ? kResBlocksPerSlot : per);
-    long long g = per * slots;
-    const long long useful = (modes + 64 * kResWaves - 1) / (64 * kResWaves);  // a mode per thread
-    if (g > useful) g = useful;
-    if (g > a.rows) g = a.rows;
-    a.rq = a.rows / g;
-    a.rr = (int)(a.rows % g);
-    return (int)g;
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        KN_CHECK(hipGetDevice(&dev));
+        KN_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+        return n;
+    }();
+    return cus;
+}
+
+// Buckets of a table of nbins: four per bin, one where those do not fit in LDS.
+int res_buckets(int nbins, int green_dims)
+{
+    return kn_res::smem_bytes(nbins, 4 * nbins, green_dims) <= 160 * 1024 ? 4 * nbins : nbins;
+}
+
+// A table of nbins (with green_dims Green's factors) is taken up to this many
+// bytes of log k, ratio and four buckets per bin: about 5100 bins.
+bool res_fits(int nbins, int green_dims)
+{
+    return sizeof(double) * (2 * (size_t)nbins + green_dims) + sizeof(int) * ((4 * (size_t)nbins + 2) & ~(size_t)1) <=
+           160 * 1024;
+}
+
+template <int U, bool GREEN, bool WIDE>
+void res_launch_as(kn_res::ResArgs &a, hipStream_t st)
+{
+    const size_t smem = kn_res::smem_bytes(a.nbins, a.nbuckets, GREEN ? a.dims : 0);
+    const void *k = (const void *)kn_res::k_rescale<kResWaves, U, GREEN, WIDE>;
+    if (smem > 64 * 1024) KN_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    const int rowlen = a.dims / 2 + 1, B = 64 * kResWaves;
+    const long long T = (long long)B * U, slots = (smem <= 80 * 1024 ? 2LL : 1LL) * res_cus();
+    a.modes = a.rows * rowlen;
+    long long g = (a.modes + T - 1) / T;
+    if (g > slots) g = slots;
+    a.in_tile = kn_res::step_of(B, rowlen, a.dims);
+    a.to_next = kn_res::step_of((g - 1) * T + B, rowlen, a.dims);
+    hipLaunchKernelGGL((kn_res::k_rescale<kResWaves, U, GREEN, WIDE>), dim3((int)g), dim3(B), smem, st, a);
+    KN_CHECK(hipGetLastError());
+}
+
+// Rows of 64 modes or more: the wide form; of fewer, a mode per lane and tile
+// (the largest such grid, 125^3, has two tiles for each resident block).
+template <bool GREEN>
+void res_launch(kn_res::ResArgs &a, hipStream_t st)
+{
+    if (a.dims / 2 + 1 >= 64) res_launch_as<kResUnroll, GREEN, true>(a, st);
+    else res_launch_as<1, GREEN, false>(a, st);
 }
 
 // ---- synthetic Gaussian random field -----------------------------------
@@ -147,26 +156,21 @@ extern "C" int kn_rescale_device(fftw_complex *d_field, int dims, int startslab,
                                  const double *d_logkk, const double *d_ratio, int nbins, double norm, void *stream)
 {
     if (nbins < 1 || dims < 2 || nslab < 1) return KN_ERR_ARG;
-    const int nbuckets = kn_res::kBucketsPerBin * nbins;
-    const size_t smem = kn_res::smem_bytes(nbins, nbuckets);
-    if (smem > 160 * 1024) return KN_ERR_ARG;
+    if (!res_fits(nbins, 0)) return KN_ERR_ARG;
     kn_res::ResArgs a;
     a.F = (double2 *)d_field;
     a.dims = dims;
     a.startslab = startslab;
     a.nbins = nbins;
-    a.nbuckets = nbuckets;
+    a.nbuckets = res_buckets(nbins, 0);
     a.rows = (long long)nslab * dims;
-    a.boxsize = boxsize;
+    a.log_kunit = log(2 * M_PI / boxsize);
     a.norm = norm;
     a.logkk = d_logkk;
     a.ratio = d_ratio;
     a.nan_flag = nan_flag_ptr();
     a.gw = nullptr;
-    const int grid = res_grid<false>(a, smem);
-    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll>), dim3(grid),
-                       dim3(64 * kResWaves), smem, (hipStream_t)stream, a);
-    KN_CHECK(hipGetLastError());
+    res_launch<false>(a, (hipStream_t)stream);
     return 0;
 }
 
@@ -181,9 +185,7 @@ extern "C" int kn_rescale_green_device(fftw_complex *d_field, int dims, int star
         kn_set_last_error("kn_rescale_green_device: bad arguments");
         return KN_ERR_ARG;
     }
-    const int nbuckets = kn_res::kBucketsPerBin * nbins;
-    const size_t smem = kn_res::smem_bytes(nbins, nbuckets, dims);
-    if (smem > 160 * 1024) {
+    if (!res_fits(nbins, dims)) {
         kn_set_last_error("kn_rescale_green_device: nbins=%d dims=%d exceed the LDS budget", nbins, dims);
         return KN_ERR_RANGE;
     }
@@ -215,18 +217,15 @@ extern "C" int kn_rescale_green_device(fftw_complex *d_field, int dims, int star
     a.dims = dims;
     a.startslab = startslab;
     a.nbins = nbins;
-    a.nbuckets = nbuckets;
+    a.nbuckets = res_buckets(nbins, dims);
     a.rows = (long long)nslab * dims;
-    a.boxsize = boxsize;
+    a.log_kunit = log(2 * M_PI / boxsize);
     a.norm = norm;
     a.logkk = d_logkk;
     a.ratio = d_ratio;
     a.nan_flag = nan_flag_ptr();
     a.gw = gw_d;
-    const int grid = res_grid<true>(a, smem);
-    hipLaunchKernelGGL((kn_res::k_rescale_rows_pf<kResWaves, kResUnroll, true>), dim3(grid),
-                       dim3(64 * kResWaves), smem, (hipStream_t)stream, a);
-    KN_CHECK(hipGetLastError());
+    res_launch<true>(a, (hipStream_t)stream);
     return 0;
 }
 

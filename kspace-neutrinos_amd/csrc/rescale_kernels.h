@@ -9,48 +9,66 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "kn_logtab.h"
 #include "kn_mem.h"
 
 namespace kn_res {
 
 __host__ __device__ inline int kval(int n, int dims) { return n <= dims / 2 ? n : n - dims; }
 
+// A step of n modes along the flattened [slab][row][z] order.
+struct Step {
+    int di, dj, dz;
+};
+
+inline Step step_of(long long n, int rowlen, int dims)
+{
+    const long long r = n / rowlen;
+    Step s;
+    s.dz = (int)(n % rowlen);
+    s.dj = (int)(r % dims);
+    s.di = (int)(r / dims);
+    return s;
+}
+
 struct ResArgs {
     double2 *F;
     int dims, startslab, nbins, nbuckets;
     long long rows;
-    long long rq;  // block b sweeps rq rows, one more for b < rr (rows = gridDim.x rq + rr)
-    int rr;
-    double boxsize, norm;
+    long long modes;           // of all rows
+    Step in_tile, to_next;     // from a lane's mode to its next one in the block's tile, and from its last one to the next tile's first
+    double log_kunit, norm;    // log(2 pi / BoxSize); the ratio's factor
     const double *logkk, *ratio;
     int *nan_flag;
     // Green's function of the PM potential (GREEN sweeps): per axis index t,
     // gw[t] = exp(-kt^2 asmth2) W(t)^-4 (dims doubles; kt the integer
     // wavenumber, W the CiC window, asmth2 = (2 pi r_s / BoxSize)^2)
-    const double *gw;
+    const double *__restrict__ gw;
 };
 
-constexpr int kBucketsPerBin = 4;
-
+// LDS of the sweep: the table's log k, ratio and slope, the logarithm's table,
+// the buckets, and the Green's factors of one axis.
 __host__ __device__ inline size_t smem_bytes(int nbins, int nbuckets, int green_dims = 0)
 {
-    return sizeof(double) * (2 * (size_t)nbins + (size_t)green_dims) +
+    return sizeof(double) * (3 * (size_t)nbins + 2 * KN_LOGTAB_N + (size_t)green_dims) +
            sizeof(int) * (size_t)(nbuckets + 1 + ((nbuckets + 1) & 1));
 }
 
 struct Tab {
-    const double *lk, *rt;
+    const double *lk, *rt, *sl;  // log k, ratio, and slope of the segment above each bin
+    const double2 *lg;           // kn_logtab
     const int *bucket;
     int nbins, nbuckets;
-    double x0, x1, inv_bw, lower_clamp, norm, log_kunit;
+    double x0, x1, inv_bw, norm, log_kunit;
 };
 
-// Ratio table and bucket index into LDS (all threads of the block).
+// Ratio table, slopes, logarithm table and bucket index into LDS (all threads of the block).
 __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 {
     extern __shared__ double sm[];
-    double *lk = sm, *rt = sm + a.nbins;
-    int *bucket = (int *)(rt + a.nbins);
+    double *lg = sm, *lk = lg + 2 * KN_LOGTAB_N, *rt = lk + a.nbins, *sl = rt + a.nbins;
+    int *bucket = (int *)(sl + a.nbins);
+    for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) lg[t] = kn_logtab[t];
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
         lk[t] = a.logkk[t];
         rt[t] = a.ratio[t];
@@ -59,15 +77,20 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     Tab T;
     T.lk = lk;
     T.rt = rt;
+    T.sl = sl;
+    T.lg = (const double2 *)lg;
     T.bucket = bucket;
     T.nbins = a.nbins;
     T.nbuckets = a.nbuckets;
     T.x0 = lk[0];
     T.x1 = lk[a.nbins - 1];
     T.inv_bw = a.nbins > 1 ? a.nbuckets / (T.x1 - T.x0) : 0.0;
-    T.lower_clamp = T.x0 - log(2.0);
     T.norm = a.norm;
-    T.log_kunit = log(2 * M_PI / a.boxsize);
+    T.log_kunit = a.log_kunit;
+    for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
+        const double h = t + 1 < a.nbins ? lk[t + 1] - lk[t] : 0.0;
+        sl[t] = h > 0.0 ? (rt[t + 1] - rt[t]) / h : 0.0;
+    }
     // bucket[q]: the GSL segment index (largest i <= n-2 with lk[i] <= x) at the bucket's left edge
     for (int q = threadIdx.x; q <= a.nbuckets; q += nthreads) {
         const double edge = T.x0 + q / T.inv_bw;
@@ -83,60 +106,76 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     return T;
 }
 
+// log(sqrt(k2)), k2 >= 1, by kn_logtab: k2 = 2^e m with m in the table's
+// interval j, log m = -log r_j + log1p(m r_j - 1) with six terms of the series
+// (|m r_j - 1| <= 2^-8: the seventh is below 2e-18).  Within 1.8e-15 for all
+// int k2, as half of a log(k2) rounded to double is.  18 operations where the
+// math library's log and its double-double steps are about 75.
+__device__ __forceinline__ double half_log(int k2, const double2 *lg)
+{
+    const unsigned long long v = __double_as_longlong((double)k2);
+    const int hi = (int)(v >> 32), e = (hi >> 20) - 1023;
+    const double m = __longlong_as_double((v & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
+    const double2 t = lg[(hi >> 13) & (KN_LOGTAB_N - 1)];
+    const double r = fma(m, t.x, -1.0), ef = (double)e;
+    double q = fma(r, -1.0 / 6.0, 1.0 / 5.0);
+    q = fma(r, q, -1.0 / 4.0);
+    q = fma(r, q, 1.0 / 3.0);
+    q = fma(r, q, -1.0 / 2.0);
+    const double p = fma(r * r, q, r);
+    return fma(ef, KN_HALF_LN2_HI, 0.5 * t.y) + fma(ef, KN_HALF_LN2_LO, 0.5 * p);
+}
+
 // 1 + get_dnudcdm_powerspec(log(|k|)) for k2 > 0, with |k| = sqrt(k2) 2 pi / BoxSize.
-// log|k| is evaluated as 0.5 log(k2) + log(2 pi / BoxSize): the same value as
-// the reference's log(sqrt(k2)*2*M_PI/BoxSize) to about one ulp, with one
-// transcendental per mode instead of sqrt, two divides and a log.
+// log|k| is evaluated as log(sqrt(k2)) + log(2 pi / BoxSize): the same value as
+// the reference's log(sqrt(k2)*2*M_PI/BoxSize) to about one ulp, without the
+// sqrt and the divisions.
 __device__ __forceinline__ double smth_of(int k2i, const Tab &T)
 {
-    double kk = 0.5 * log((double)k2i) + T.log_kunit;
-    if (kk < T.x0 && kk > T.lower_clamp) kk = T.x0;
-    if (kk < T.lower_clamp) kk = T.x0;
-    if (kk > T.x1) kk = T.x1;
-    double interp;
-    if (T.nbins == 1) {
-        interp = T.rt[0];
-    } else {
-        int q = (int)((kk - T.x0) * T.inv_bw);
-        q = q < 0 ? 0 : (q > T.nbuckets ? T.nbuckets : q);
-        int i = T.bucket[q];
-        while (i < T.nbins - 2 && T.lk[i + 1] <= kk) i++;
-        const double xl = T.lk[i], h = T.lk[i + 1] - xl;
-        interp = h > 0.0 ? T.rt[i] + (kk - xl) / h * (T.rt[i + 1] - T.rt[i]) : T.rt[i];
-    }
-    return 1 + T.norm * interp;
+    double kk = half_log(k2i, T.lg) + T.log_kunit;
+    kk = kk < T.x0 ? T.x0 : kk;
+    kk = kk > T.x1 ? T.x1 : kk;
+    int q = (int)((kk - T.x0) * T.inv_bw);
+    q = q < 0 ? 0 : (q > T.nbuckets ? T.nbuckets : q);
+    int i = T.bucket[q];
+    while (i < T.nbins - 2 && T.lk[i + 1] <= kk) i++;
+    return fma(T.norm, fma(kk - T.lk[i], T.sl[i], T.rt[i]), 1.0);
 }
 
 struct Pos {
-    int i, j, z;
+    int i, j, z;  // slab, row and z of a mode
 };
 
-__device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
-{
-    p.z += step;
-    while (p.z >= rowlen) {
-        p.z -= rowlen;
-        if (++p.j == dims) {
-            p.j = 0;
-            p.i++;
-        }
-    }
-}
-
-// Position of mode `off` of the rows from row0 on.
-__device__ __forceinline__ Pos pos_of(int off, long long row0, int rowlen, int dims)
+__device__ __forceinline__ Pos pos_of(long long m, int rowlen, int dims)
 {
     Pos p;
-    p.z = off % rowlen;
-    const long long rl = row0 + off / rowlen;
-    if (rl < 0x7fffffffLL) {  // rows of any grid that fits the card: 32-bit division
-        p.j = (int)((unsigned)rl % (unsigned)dims);
-        p.i = (int)((unsigned)rl / (unsigned)dims);
+    if (m < 0x7fffffffLL) {  // 32-bit divisions
+        const unsigned r = (unsigned)m / (unsigned)rowlen;
+        p.z = (int)((unsigned)m - r * (unsigned)rowlen);
+        p.j = (int)(r % (unsigned)dims);
+        p.i = (int)(r / (unsigned)dims);
     } else {
-        p.j = (int)(rl % dims);
-        p.i = (int)(rl / dims);
+        const long long r = m / rowlen;
+        p.z = (int)(m - r * rowlen);
+        p.j = (int)(r % dims);
+        p.i = (int)(r / dims);
     }
     return p;
+}
+
+__device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int dims)
+{
+    p.z += s.dz;
+    p.j += s.dj;
+    p.i += s.di;
+    if (p.z >= rowlen) {
+        p.z -= rowlen;
+        p.j++;
+    }
+    if (p.j >= dims) {
+        p.j -= dims;
+        p.i++;
+    }
 }
 
 // The PM Green's function with CiC deconvolution at k2 > 0, as the potential
@@ -147,86 +186,128 @@ __device__ __forceinline__ Pos pos_of(int off, long long row0, int rowlen, int d
 // over the axes, so with gw (ResArgs) it is -gw[x] gw[y] gw[z] / k2: no
 // exponential per mode, and 1/k2 from the hardware reciprocal refined by one
 // Newton step (a few units in the last place from the direct form).
-__device__ __forceinline__ double green_of(int k2, double gx, double gy, double gz)
+__device__ __forceinline__ double green_of(int k2, double gxy, double gz)
 {
     const double d = (double)k2;
     const double r = __builtin_amdgcn_rcp(d);
     const double inv = fma(r, fma(-d, r, 1.0), r);
-    return -((gx * gy) * gz) * inv;
+    return -(gxy * gz) * inv;
 }
 
-// The rescale sweep: each block a contiguous row range, lane l of the block
-// takes modes l, l + B, ... (coalesced), the next UNROLL modes loaded before
-// the current ones are rescaled and stored; loads and stores carry the
-// non-temporal hint (each mode is read and written once per sweep).  The
-// first modes are requested before the tables are built, so that their
-// latency and the tables' pass together.
+// The rescale sweep.  The grid is cut into tiles of 64 WAVES U consecutive
+// modes, block b taking tiles b, b + gridDim.x, ...: the blocks move over the
+// grid together, two of 8 wavefronts per CU, each lane U = 2 modes of a tile
+// (loads and stores 16 bytes per lane, consecutive across a wavefront, with the
+// non-temporal hint).  HBM bounds it: reading and writing reach the most this
+// way (an empty in-place sweep of 1024^3: 5.1-5.5 TB/s from contiguous ranges
+// per block, 5.5-6.0 from tiles in turn by 16 wavefronts per CU), but only with
+// few operations per mode.  So a wavefront's place is scalar (its 64 modes lie
+// in at most two rows, WIDE), log k comes from a table (half_log) and the
+// ratio's segment has its slope stored: 77 vector operations per mode against
+// 174, a third of the sweep's time.  ms per sweep, contiguous ranges with the
+// library's log against this form (Green's function in parentheses): 256^3
+// 0.062 -> 0.049 (0.063 -> 0.050), 512^3 0.436 -> 0.360 (0.452 -> 0.365), 768^3
+// 1.472 -> 1.250, 1024^3 3.330 -> 3.063 (3.451 -> 3.088), 5.62 TB/s.  At 1024^3
+// one, two, three and four blocks per CU take 3.38, 3.07, 3.18 and 3.60 ms, U =
+// 1, 3, 4 and 8 3.11, 3.39, 3.38 and 3.41.
 // GREEN: the same sweep also applies the Green's function (F s_nu, then times
 // G, the two roundings of the two passes it replaces) and zeroes the k = 0
 // mode; with nbins 0 it applies the Green's function alone.
-template <int WAVES, int UNROLL, bool GREEN = false>
-__global__ __launch_bounds__(64 * WAVES) void k_rescale_rows_pf(ResArgs a)
+// WIDE: rows of 64 modes or more (else every lane finds its own row).
+template <int WAVES, int U, bool GREEN, bool WIDE>
+__global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
 {
-    constexpr int B = 64 * WAVES;
-    const int rowlen = a.dims / 2 + 1;
-    const long long b = blockIdx.x, r0 = b * a.rq + (b < a.rr ? b : a.rr), r1 = r0 + a.rq + (b < a.rr);
-    const long long m1 = r1 * rowlen;
-    const long long S = (long long)B * UNROLL;
-    long long m = r0 * rowlen + threadIdx.x;
-    double2 cur[UNROLL];
+    constexpr int B = 64 * WAVES, T = B * U;
+    const int rowlen = a.dims / 2 + 1, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    long long m = (long long)blockIdx.x * T + 64 * wave;  // the wavefront's first mode
+    const long long n = a.modes, S = (long long)gridDim.x * T;
+    double2 cur[U];
 #pragma unroll
-    for (int u = 0; u < UNROLL; u++) {
-        const long long mu = m + (long long)B * u;
-        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+    for (int u = 0; u < U; u++) {
+        const long long mu = m + B * u + lane;
+        cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
     }
-    Tab T;
+    Tab Tb;
     const double *gw = nullptr;
-    if (!GREEN || a.nbins > 0) T = load_tab(a, B);
+    if (!GREEN || a.nbins > 0) Tb = load_tab(a, B);
     if constexpr (GREEN) {
         extern __shared__ double sm[];
-        int *after_buckets = (int *)(sm + 2 * (size_t)a.nbins) + a.nbuckets + 1 + ((a.nbuckets + 1) & 1);
-        double *gw_l = (double *)after_buckets;  // 8-byte aligned
+        double *gw_l = a.nbins > 0 ? (double *)((int *)(sm + 2 * KN_LOGTAB_N + 3 * (size_t)a.nbins) + a.nbuckets + 1 +
+                                                ((a.nbuckets + 1) & 1))
+                                   : sm;
         for (int t = threadIdx.x; t < a.dims; t += B) gw_l[t] = a.gw[t];
         __syncthreads();
         gw = gw_l;
     }
-    Pos p = pos_of(threadIdx.x, r0, rowlen, a.dims);
+    Pos p = pos_of(m, rowlen, a.dims);
     bool saw_nan = false;
-    for (; m < m1; m += S) {
-        double2 nxt[UNROLL];
+    for (; m < n; m += S) {
+        // the wavefront's rows: z of its first mode, kx^2 + ky^2 there and in the next row (GREEN: both rows' x and y)
+        int z0[U], kxy[U][2], gx[U][2], gy[U][2];
+        if constexpr (WIDE) {
 #pragma unroll
-        for (int u = 0; u < UNROLL; u++) {
-            const long long mu = m + S + (long long)B * u;
-            nxt[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+            for (int u = 0; u < U; u++) {
+                const int x0 = a.startslab + p.i;
+                int x1 = x0, j1 = p.j + 1;
+                if (j1 == a.dims) {
+                    j1 = 0;
+                    x1 = x0 + 1;
+                }
+                const int kx0 = kval(x0, a.dims), ky0 = kval(p.j, a.dims), kx1 = kval(x1, a.dims), ky1 = kval(j1, a.dims);
+                z0[u] = p.z;
+                kxy[u][0] = kx0 * kx0 + ky0 * ky0;
+                kxy[u][1] = kx1 * kx1 + ky1 * ky1;
+                gx[u][0] = x0, gx[u][1] = x1, gy[u][0] = p.j, gy[u][1] = j1;
+                advance(p, u + 1 < U ? a.in_tile : a.to_next, rowlen, a.dims);
+            }
         }
 #pragma unroll
-        for (int u = 0; u < UNROLL; u++) {
-            const long long mu = m + (long long)B * u;
-            const Pos q = p;
-            advance(p, B, rowlen, a.dims);
-            if (mu >= m1) continue;
-            const int kx = kval(a.startslab + q.i, a.dims), ky = kval(q.j, a.dims);
-            const int k2 = kx * kx + ky * ky + q.z * q.z;
+        for (int u = 0; u < U; u++) {
+            const long long mu = m + B * u + lane;
+            int z, k2;
+            int x = 0, y = 0;
+            if constexpr (WIDE) {
+                z = z0[u] + lane;
+                const bool next = z >= rowlen;
+                z -= next ? rowlen : 0;
+                k2 = (next ? kxy[u][1] : kxy[u][0]) + __mul24(z, z);
+                if constexpr (GREEN) {
+                    x = next ? gx[u][1] : gx[u][0];
+                    y = next ? gy[u][1] : gy[u][0];
+                }
+            } else {
+                const Pos q = pos_of(mu < n ? mu : 0, rowlen, a.dims);
+                const int kx = kval(a.startslab + q.i, a.dims), ky = kval(q.j, a.dims);
+                z = q.z;
+                k2 = kx * kx + ky * ky + z * z;
+                x = a.startslab + q.i;
+                y = q.j;
+            }
+            if (mu >= n) continue;
+            double2 f = cur[u];
             if (k2 <= 0) {
                 if (GREEN) kn_mem::st<true>(a.F + mu, make_double2(0.0, 0.0));
                 continue;
             }
-            double2 f = cur[u];
             if (!GREEN || a.nbins > 0) {
-                const double s = smth_of(k2, T);
+                const double s = smth_of(k2, Tb);
                 saw_nan |= isnan(s);
                 f.x *= s;
                 f.y *= s;
             }
             if constexpr (GREEN) {
-                const double g = green_of(k2, gw[a.startslab + q.i], gw[q.j], gw[q.z]);
+                const double g = green_of(k2, gw[x] * gw[y], gw[z]);
                 f.x *= g;
                 f.y *= g;
             }
             kn_mem::st<true>(a.F + mu, f);
         }
 #pragma unroll
-        for (int u = 0; u < UNROLL; u++) cur[u] = nxt[u];
+        for (int u = 0; u < U; u++) {
+            const long long mu = m + S + B * u + lane;
+            cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+        }
     }
     if (saw_nan) atomicOr(a.nan_flag, 1);
 }

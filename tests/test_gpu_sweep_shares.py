@@ -70,3 +70,47 @@ def test_bin_sums_repeat(kn, torch_cuda, N, nb):
         assert kn.kn_bin_power_device(d.data_ptr(), N, nb, 0, N, p.data_ptr(), p.data_ptr() + 8 * nb, None) == 0
         out.append(p.cpu().numpy())
     assert all(np.array_equal(out[0], o) for o in out[1:])
+
+
+@pytest.mark.parametrize("N", [6, 124, 125, 126, 250])
+def test_rescale_log_k(kn, torch_cuda, N):
+    """A ratio equal to log k turns each mode's factor into 1 + norm log k.  The bound: log k (below 12) within 1.8e-15 of
+    its logarithm's table and three roundings at 12 (0.9e-15 each), norm times that, over a factor of 1.9 or more."""
+    torch = torch_cuda
+    print("rescale log k", N, flush=True)
+    lk = np.array([math.log(2 * math.pi / BOX) - 1e-3, math.log(math.sqrt(3) * math.pi * N / BOX) + 1e-3])
+    tab, norm = torch.from_numpy(np.concatenate([lk, lk])).cuda(), 0.5
+    d = torch.ones((N, N, N // 2 + 1), dtype=torch.complex128, device="cuda")
+    assert kn.kn_rescale_device(d.data_ptr(), N, 0, N, BOX, tab.data_ptr(), tab.data_ptr() + 16, 2, norm, None) == 0
+    i = np.arange(N)
+    kv = np.where(i <= N // 2, i, i - N)
+    k2 = (kv[:, None, None] ** 2 + kv[None, :, None] ** 2 + np.arange(N // 2 + 1)[None, None, :] ** 2).astype(np.longdouble)
+    k2[0, 0, 0] = 1
+    s = 1 + np.longdouble(norm) * (np.log(k2) / 2 + np.log(2 * np.longdouble(math.pi) / BOX))
+    got = d.cpu().numpy().real
+    assert got[0, 0, 0] == 1.0
+    e = np.abs(got / s - 1)
+    e[0, 0, 0] = 0
+    print("  worst %.2e" % float(e.max()))
+    assert float(e.max()) < norm * 4.5e-15 / 1.9 + 2.3e-16
+
+
+@pytest.mark.parametrize("nb", [1, 2, 700, 4050, 5000])
+def test_rescale_table_sizes(kn, torch_cuda, nb):
+    """One bin to the largest tables (a bucket per bin in place of four from 4045 bins on), unevenly spaced; past the
+    limit the call is refused as ever."""
+    torch = torch_cuda
+    print("rescale table", nb, flush=True)
+    N, rng = 130, np.random.default_rng(nb)
+    F = _rand_grid(N, 11, 9)
+    lk = np.sort(rng.uniform(math.log(math.pi / BOX), math.log(2 * math.pi * N / BOX), nb)) if nb > 1 else np.array([-9.0])
+    rt = rng.uniform(-1, 1, nb)
+    d, tab = torch.from_numpy(F).cuda(), torch.from_numpy(np.concatenate([lk, rt])).cuda()
+    assert kn.kn_rescale_device(d.data_ptr(), N, 0, 9, BOX, tab.data_ptr(), tab.data_ptr() + 8 * nb, nb, 0.05, None) == 0
+    torch.cuda.synchronize()
+    rc, W = O.rescale(F, BOX, lk, rt, 0.05, 0)
+    assert rc == 0
+    # a segment of width h turns an error of 4e-15 in log k into one of norm |d ratio| 4e-15 / h in the factor
+    h = max(np.min(np.diff(lk)), 1e-9) if nb > 1 else 1.0
+    np.testing.assert_allclose(d.cpu().numpy().view(np.float64), W.view(np.float64), rtol=1e-14 + 0.05 * 2 * 4e-15 / h, atol=0)
+    assert kn.kn_rescale_device(d.data_ptr(), N, 0, 9, BOX, tab.data_ptr(), tab.data_ptr(), 5200, 0.05, None) == 3002
