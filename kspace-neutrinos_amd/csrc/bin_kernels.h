@@ -82,18 +82,20 @@ __device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
     }
 }
 
-// Position of mode `off` of the rows from row0 on.
-__device__ __forceinline__ Pos pos_of(int off, long long row0, int rowlen, int dims)
+// Position of mode m of the rank's slabs.
+__device__ __forceinline__ Pos pos_of(long long m, int rowlen, int dims)
 {
     Pos p;
-    p.z = off % rowlen;
-    const long long rl = row0 + off / rowlen;
-    if (rl < 0x7fffffffLL) {  // rows of any grid that fits the card: 32-bit division
-        p.j = (int)((unsigned)rl % (unsigned)dims);
-        p.i = (int)((unsigned)rl / (unsigned)dims);
+    if (m < 0x7fffffffLL) {  // 32-bit divisions
+        const unsigned r = (unsigned)m / (unsigned)rowlen;
+        p.z = (int)((unsigned)m - r * (unsigned)rowlen);
+        p.j = (int)(r % (unsigned)dims);
+        p.i = (int)(r / (unsigned)dims);
     } else {
-        p.j = (int)(rl % dims);
-        p.i = (int)(rl / dims);
+        const long long r = m / rowlen;
+        p.z = (int)(m - r * rowlen);
+        p.j = (int)(r % dims);
+        p.i = (int)(r / dims);
     }
     return p;
 }
@@ -129,14 +131,13 @@ __host__ __device__ inline Step step_of(long long n, int rowlen, int dims)
 struct BinArgs {
     const double2 *F;
     int dims, startslab, nrbins;
-    long long rows;
-    long long rq;  // rows = gridDim.x rq + rr: every block rq rows, rr of them one more
-    unsigned rr;
+    long long modes;        // of the rank's slabs
+    Step in_tile, to_next;  // from a lane's mode to its next one in the block's tile, and from its last one to the next tile's first
     const int *thr;
     const double *iw;
     float half_bpu;
     double *partial;  // gridDim.x * nrbins
-    Step step;        // one pass of a block: 64 kSweepRun modes per wavefront
+    int cshift;       // copies of the bin sums: 2^cshift
 };
 
 __device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int dims)
@@ -161,179 +162,139 @@ __device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int d
 // global atomics into the block's own partial row (any number of bins).
 enum TablePlace { kTablesLds = 0, kWindowGlobal = 1, kTablesGlobal = 2 };
 
-constexpr int kSweepWaves = 8;  // wavefronts per block
-constexpr int kSweepRun = 4;    // consecutive modes per lane (one staged chunk: 64 * kSweepRun modes per wave)
+constexpr int kSweepWaves = 8;      // wavefronts per block
+constexpr int kSweepUnroll = 2;     // modes per lane of a tile
 
-// LDS bytes of the sweep: the staging buffers, then the tables the placement
-// keeps there (own: one set of bin sums per wavefront).
-__host__ __device__ constexpr size_t sweep_smem_bytes(int place, int dims, int nrbins, bool own = false)
+// LDS bytes of the sweep with `sets` sets of bin sums.
+__host__ __device__ constexpr size_t sweep_smem_bytes(int place, int dims, int nrbins, int sets)
 {
-    return sizeof(double2) * (size_t)kSweepWaves * 64 * kSweepRun +
-           (place == kTablesGlobal
-                ? 0
-                : sizeof(double) * (size_t)nrbins * (own ? kSweepWaves : 1) + sizeof(int) * (size_t)(nrbins + 1 + ((nrbins + 1) & 1)) +
-                      (place == kTablesLds ? sizeof(double) * (size_t)dims : 0));
+    return place == kTablesGlobal ? 0
+                                  : sizeof(double) * (size_t)nrbins * sets +
+                                        sizeof(int) * (size_t)(nrbins + 1 + ((nrbins + 1) & 1)) +
+                                        (place == kTablesLds ? sizeof(double) * (size_t)dims : 0);
 }
 
-// Slot of mode m (0 <= m < 64 * kSweepRun) of a wavefront's staging buffer.
-// Lanes write consecutive modes (m = 64u + l) and read back runs (m = 4l + r).
-// A 16-byte access pass serves 8 or 16 lanes; for the reads the lanes of a
-// pass differ in lane bits l1..l3, so (l1 ^ l3, l2) is XOR-ed into the slot's
-// two low bits (one-to-one for both pass widths); the writes of a pass keep
-// distinct low bits since the XOR term is constant across each aligned group
-// of 8 lanes.  The slot stays inside m's aligned group of 4.
-__device__ __forceinline__ int stage_slot(int m)
-{
-    return m ^ ((((m >> 3) ^ (m >> 5)) & 1) | (((m >> 4) & 1) << 1));
-}
-
-// The bin sweep (powerspectrum.c:56-89).  Block b takes a contiguous range of
-// rows; wavefront w of the block takes chunks of 256 consecutive modes (w,
-// w + 8, ...).  Load u of a chunk is one 1 KB contiguous dwordx4 load across
-// the wave, non-temporal (each mode is read once per sweep); the next chunk's
-// loads are issued before the current one is binned.  The chunk passes
-// through the wave's LDS staging buffer so that lane l holds modes 4l .. 4l+3
-// of it: along a row |k|^2 grows with z, so after a run's first mode its bin
-// is found incrementally (the next threshold kept in a register, at most one
-// step before a full search), equal-bin runs are summed in registers and
-// flushed with one atomic add per run.  With OWN every wavefront has its own
-// bin sums, added in a fixed order at the end, and the result is the same on
-// every run; without it the block's wavefronts share one set, so the order of
+// The bin sweep (powerspectrum.c:56-89).  The grid is cut into tiles of 64
+// WAVES U consecutive modes, block b taking tiles b, b + gridDim.x, ...; loads
+// are 16 bytes per lane, consecutive across a wavefront, non-temporal (each
+// mode is read once per sweep).  A wavefront's place is scalar (WIDE: its 64
+// modes lie in at most two rows).  A mode's bin is an fp32 estimate,
+// within one of the right one, corrected by the integer thresholds of two
+// bins; its weighted power is added to the bin's sum in LDS.  Neighbouring
+// lanes often share a bin, and lanes that add to one address wait for each
+// other: 2^cshift copies of the sums, taken in turn by the lanes, part them.
+// With OWN every wavefront has its own copies and the result is the same on
+// every run; without it the block's wavefronts share them, so the order of
 // the adds between wavefronts (and the last bit of a sum) can differ from run
-// to run.  The block writes its sums to its partial row, and
-// k_reduce_partials adds the rows in a fixed order.
-template <int PLACE, bool OWN = false>
-__global__ __launch_bounds__(64 * kSweepWaves) void k_bin_sweep(BinArgs a)
+// to run.  The block adds the copies in a fixed order into its partial row,
+// and k_reduce_partials adds the rows in a fixed order.
+// A read at the most this card reaches takes 1.23 ms at 1024^3.  An earlier
+// form loaded runs of consecutive modes per lane (a transpose through LDS) to
+// merge equal bins before the adds: about 110 vector operations per mode
+// where this one has 52, and they, not memory, set its time (1.41 ms at 1024^3
+// with the reduction against 1.32).  At 1024^3 one, two and four copies take
+// 1548, 1315 and 1320 us; two, three and four blocks per CU 1391, 1315 and 1527.
+template <int PLACE, int WAVES, int U, bool OWN, bool WIDE>
+__global__ __launch_bounds__(64 * WAVES) void k_bin_sweep(BinArgs a)
 {
-    constexpr int WAVES = kSweepWaves, RUN = kSweepRun;
+    constexpr int B = 64 * WAVES, T = B * U;
+    const int cshift = PLACE == kTablesGlobal ? 0 : a.cshift, cbyte = cshift + 3;
     extern __shared__ double smem[];
-    double2 *stage_all = (double2 *)smem;  // WAVES * 64 * RUN modes, 16-byte aligned
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rowlen = a.dims / 2 + 1, half = a.dims / 2;
-    // rows gridDim.x-ths by b rows / gridDim.x: ranges of both lengths in turn (all longer ones first: 1.45 ms
-    // against 1.42 at 1024^3, the blocks' addresses then being one stride apart); the host keeps gridDim.x <= 65535
-    const unsigned blk = blockIdx.x, e0 = blk * a.rr / gridDim.x, e1 = (blk + 1) * a.rr / gridDim.x;
-    const long long r0 = blk * a.rq + e0, r1 = r0 + a.rq + (e1 - e0);
-    const long long m0 = r0 * rowlen, m1 = r1 * rowlen;
-    constexpr int CH = 64 * RUN;
-    constexpr long long S = (long long)CH * WAVES;
-    long long c = m0 + (long long)wave * CH;
-    // the first chunk is requested before the tables are read, so that the two latencies overlap
-    double2 cur[RUN];
+    const int rowlen = a.dims / 2 + 1, half = a.dims / 2, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    long long m = (long long)blockIdx.x * T + 64 * wave;  // the wavefront's first mode
+    const long long n = a.modes, S = (long long)gridDim.x * T;
+    double2 cur[U];
 #pragma unroll
-    for (int u = 0; u < RUN; u++) {
-        const long long mu = c + 64 * u + lane;
-        cur[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+    for (int u = 0; u < U; u++) {
+        const long long mu = m + B * u + lane;
+        cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
     }
-    double *hist;
-    const double *iw;
-    const int *thr;
+    double *hist = smem;
+    const double *iw = a.iw;
+    const int *thr = a.thr;
     if constexpr (PLACE == kTablesGlobal) {
         hist = a.partial + (size_t)blockIdx.x * a.nrbins;
-        iw = a.iw;
-        thr = a.thr;
-        for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES) hist[t] = 0.0;
+        for (int t = threadIdx.x; t < a.nrbins; t += B) hist[t] = 0.0;
     } else {
-        hist = (double *)(stage_all + (size_t)WAVES * 64 * RUN);
-        const int nhist = OWN ? WAVES * a.nrbins : a.nrbins;
+        const int nhist = ((OWN ? WAVES : 1) * a.nrbins) << cshift;
         int *thr_l = (int *)(hist + nhist);
-        for (int t = threadIdx.x; t < nhist; t += 64 * WAVES) hist[t] = 0.0;
-        for (int t = threadIdx.x; t <= a.nrbins; t += 64 * WAVES) thr_l[t] = a.thr[t];
+        for (int t = threadIdx.x; t < nhist; t += B) hist[t] = 0.0;
+        for (int t = threadIdx.x; t <= a.nrbins; t += B) thr_l[t] = a.thr[t];
         thr = thr_l;
         if constexpr (PLACE == kTablesLds) {
             double *iw_l = (double *)(thr_l + a.nrbins + 1 + ((a.nrbins + 1) & 1));  // 8-byte aligned
-            for (int t = threadIdx.x; t < a.dims; t += 64 * WAVES) iw_l[t] = a.iw[t];
+            for (int t = threadIdx.x; t < a.dims; t += B) iw_l[t] = a.iw[t];
             iw = iw_l;
-        } else {
-            iw = a.iw;
         }
     }
     __syncthreads();
-    double *const all = hist;
-    if constexpr (OWN) hist += wave * a.nrbins;
-    double2 *stage = stage_all + (size_t)wave * 64 * RUN;
-    const Step sS = a.step;
-    Pos p = pos_of(wave * CH + lane * RUN, r0, rowlen, a.dims);
-    for (; c < m1; c += S) {
-        double2 nxt[RUN];
+    double *const mine = hist + (OWN ? (wave * a.nrbins) << cshift : 0) + (lane & ((1 << cshift) - 1));
+    Pos p = pos_of(m, rowlen, a.dims);
+    for (; m < n; m += S) {
+        // the wavefront's rows: z of its first mode, kx^2 + ky^2, x and y there and in the next row
+        int z0[U], kxy[U][2], gx[U][2], gy[U][2];
+        if constexpr (WIDE) {
 #pragma unroll
-        for (int u = 0; u < RUN; u++) {
-            const long long mu = c + S + 64 * u + lane;
-            nxt[u] = mu < m1 ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+            for (int u = 0; u < U; u++) {
+                const int x0 = a.startslab + p.i;
+                int x1 = x0, j1 = p.j + 1;
+                if (j1 == a.dims) {
+                    j1 = 0;
+                    x1 = x0 + 1;
+                }
+                const int kx0 = kval(x0, a.dims), ky0 = kval(p.j, a.dims), kx1 = kval(x1, a.dims), ky1 = kval(j1, a.dims);
+                z0[u] = p.z;
+                kxy[u][0] = kx0 * kx0 + ky0 * ky0;
+                kxy[u][1] = kx1 * kx1 + ky1 * ky1;
+                gx[u][0] = x0, gx[u][1] = x1, gy[u][0] = p.j, gy[u][1] = j1;
+                advance(p, u + 1 < U ? a.in_tile : a.to_next, rowlen, a.dims);
+            }
         }
-        // transpose through LDS: lane l wrote modes l, 64 + l, ...; reads 4l .. 4l + 3.
-        // LDS operations of one wavefront complete in order, so the fences only
-        // keep the compiler from moving the reads above the writes (and the next
-        // chunk's writes above these reads).
 #pragma unroll
-        for (int u = 0; u < RUN; u++) stage[stage_slot(64 * u + lane)] = cur[u];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        double2 f[RUN];
-#pragma unroll
-        for (int r = 0; r < RUN; r++) f[r] = stage[stage_slot(RUN * lane + r)];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const long long mrun = c + (long long)RUN * lane;
-        Pos q = p;
-        int curb = -1, b = -1, bnext = 0;
-        double acc = 0.0;
-        // the row's kx^2 + ky^2 and window product, at the run start and at a new row
-        int kx = kval(a.startslab + q.i, a.dims), ky = kval(q.j, a.dims);
-        int kxy2 = kx * kx + ky * ky;
-        double iwxy = __dmul_rn(iw[a.startslab + q.i], iw[q.j]);
-#pragma unroll
-        for (int r = 0; r < RUN; r++) {
-            if (mrun + r >= m1) break;
-            if (r && ++q.z == rowlen) {
-                q.z = 0;
-                if (++q.j == a.dims) {
-                    q.j = 0;
-                    q.i++;
-                }
-                kx = kval(a.startslab + q.i, a.dims);
-                ky = kval(q.j, a.dims);
-                kxy2 = kx * kx + ky * ky;
-                iwxy = __dmul_rn(iw[a.startslab + q.i], iw[q.j]);
-            }
-            const int k2 = kxy2 + q.z * q.z;
-            if (k2 == 0) continue;
-            if (b < 0 || q.z == 0) {
-                b = find_bin(k2, a.half_bpu, thr, a.nrbins);
-                bnext = thr[b + 1];
-            } else if (k2 >= bnext) {
-                const int t2 = thr[b + 2];  // b + 1 <= nrbins - 1 here, so b + 2 <= nrbins
-                if (k2 < t2) {
-                    b++;
-                    bnext = t2;
-                } else {
-                    b = find_bin(k2, a.half_bpu, thr, a.nrbins);
-                    bnext = thr[b + 1];
-                }
-            }
-            const double v = mode_weight(f[r], iwxy, iw[q.z], q.z, half);
-            if (b != curb) {
-                if (curb >= 0) atomicAdd(&hist[curb], acc);
-                curb = b;
-                acc = v;
+        for (int u = 0; u < U; u++) {
+            const long long mu = m + B * u + lane;
+            int z, k2, x, y;
+            if constexpr (WIDE) {
+                z = z0[u] + lane;
+                const bool next = z >= rowlen;
+                z -= next ? rowlen : 0;
+                k2 = (next ? kxy[u][1] : kxy[u][0]) + __mul24(z, z);
+                x = next ? gx[u][1] : gx[u][0];
+                y = next ? gy[u][1] : gy[u][0];
             } else {
-                acc += v;
+                const Pos q = pos_of(mu < n ? mu : 0, rowlen, a.dims);
+                x = a.startslab + q.i;
+                y = q.j;
+                z = q.z;
+                const int kx = kval(x, a.dims), ky = kval(y, a.dims);
+                k2 = kx * kx + ky * ky + z * z;
             }
+            if (mu >= n || k2 == 0) continue;
+            int b;
+            if constexpr (PLACE == kTablesGlobal) {  // so many bins that the estimate may be further off
+                b = find_bin(k2, a.half_bpu, thr, a.nrbins);
+            } else {
+                b = (int)(__logf((float)k2) * a.half_bpu);
+                b = b > a.nrbins - 1 ? a.nrbins - 1 : b;
+                const int t0 = thr[b], t1 = thr[b + 1];
+                b += (k2 >= t1) - (k2 < t0);
+            }
+            const double v = mode_weight(cur[u], __dmul_rn(iw[x], iw[y]), iw[z], z, half);
+            atomicAdd((double *)((char *)mine + ((unsigned)b << cbyte)), v);
         }
-        if (curb >= 0) atomicAdd(&hist[curb], acc);
 #pragma unroll
-        for (int u = 0; u < RUN; u++) cur[u] = nxt[u];
-        advance(p, sS, rowlen, a.dims);
+        for (int u = 0; u < U; u++) {
+            const long long mu = m + S + B * u + lane;
+            cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+        }
     }
     if constexpr (PLACE != kTablesGlobal) {
         __syncthreads();
-        for (int t = threadIdx.x; t < a.nrbins; t += 64 * WAVES) {
-            double v = all[t];
-            if constexpr (OWN)
-#pragma unroll
-                for (int w = 1; w < WAVES; w++) v += all[w * a.nrbins + t];
+        for (int t = threadIdx.x; t < a.nrbins; t += B) {
+            double v = 0.0;
+            for (int w = 0; w < (OWN ? WAVES : 1); w++)
+                for (int c = 0; c < 1 << cshift; c++) v += hist[((w * a.nrbins + t) << cshift) + c];
             a.partial[(size_t)blockIdx.x * a.nrbins + t] = v;
         }
     }

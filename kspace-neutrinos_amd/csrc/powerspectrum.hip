@@ -12,18 +12,19 @@
 //    (powerspectrum.c:97-116).
 //
 // MI355X design: the pass streams the grid once from HBM (16 B per mode,
-// coalesced non-temporal dwordx4 loads, transposed through LDS so that each
-// lane bins a run of consecutive modes; see bin_kernels.h).  The bin index is
-// integer-exact: the host evaluates the reference expression once per integer
-// |k|^2 and stores, per bin, the smallest |k|^2 that reaches it; the kernel
-// takes an fp32 estimate of the bin and corrects it against that threshold
-// table, so counts are bit-exact with the reference's libm.  The wavefronts of
-// a block add into one set of bin sums in LDS (ds_add_f64; the order of the
+// coalesced non-temporal dwordx4 loads, each lane one mode of a wavefront's 64
+// consecutive ones; see bin_kernels.h).  The bin index is integer-exact: the
+// host evaluates the reference expression once per integer |k|^2 and stores,
+// per bin, the smallest |k|^2 that reaches it; the kernel takes an fp32
+// estimate of the bin and corrects it against that threshold table, so counts
+// are bit-exact with the reference's libm.  The wavefronts of a block add into
+// one set of bin sums in LDS (ds_add_f64, in several copies; the order of the
 // adds between wavefronts is not fixed, so a sum can differ in its last bit
-// from run to run), blocks write partial sums and a second kernel adds them in
-// a fixed order.  Tables go to LDS when they fit, else are read from global
-// memory, so any number of bins works.  Mode counts and <|k|> depend only on
-// the geometry; they are computed once per (dims, nrbins, slab range) by a
+// from run to run, except where each wavefront has its own), blocks write
+// partial sums and a second kernel adds them in a fixed order.  Tables go to
+// LDS when they fit, else are read from global memory, so any number of bins
+// works.  Mode counts and <|k|> depend only on the geometry; they are computed
+// once per (dims, nrbins, slab range) by a
 // read-free kernel and cached (bit-exact, deterministic).
 #include <math.h>
 #include <string.h>
@@ -42,15 +43,17 @@ using kn_bin::kval;
 
 constexpr int kBlock = 256;  // geometry pass
 constexpr int kWaves = kBlock / 64;
-constexpr int kSweepSlots = 2;  // bin sweep blocks per resident slot (1.41-1.44 ms at 1024^3 against 1.45 at three)
-constexpr int kSweepPasses = 8;  // passes a block gets before a slot takes a second block (sweep_grid)
+constexpr int kSweepPerCu = 3;  // bin sweep blocks per CU (k_bin_sweep)
+constexpr size_t kSweepSumBytes = 16 * 1024;  // bin sums of one block, all copies
+constexpr int kSweepOwnBins = 32;             // most bins for own sums per wavefront on a large grid
 constexpr size_t kLdsMax = 160 * 1024;
 
-// How one geometry is swept: where the tables are, whether every wavefront has
-// its own bin sums, the blocks and their LDS.
+// How one geometry is swept: where the tables are, the blocks and their
+// wavefronts, the copies of the bin sums (2^cshift) and whether every wavefront
+// has its own, and the LDS.
 struct SweepPlan {
-    int place = 0, grid = 0;
-    bool own = false;
+    int place = 0, grid = 0, waves = 0, cshift = 0;
+    bool wide = false, own = false;
     size_t smem = 0;
 };
 
@@ -233,56 +236,82 @@ int resident_blocks(K kernel, int threads, size_t smem)
 }
 
 typedef void (*SweepKernel)(kn_bin::BinArgs);
-SweepKernel sweep_kernel(const SweepPlan &p)
+template <int WAVES, int U, bool OWN, bool WIDE>
+SweepKernel sweep_kernel_at(int place)
 {
-    if (p.place == kn_bin::kTablesLds)
-        return p.own ? kn_bin::k_bin_sweep<kn_bin::kTablesLds, true> : kn_bin::k_bin_sweep<kn_bin::kTablesLds>;
-    if (p.place == kn_bin::kWindowGlobal)
-        return p.own ? kn_bin::k_bin_sweep<kn_bin::kWindowGlobal, true> : kn_bin::k_bin_sweep<kn_bin::kWindowGlobal>;
-    return kn_bin::k_bin_sweep<kn_bin::kTablesGlobal>;
+    if (place == kn_bin::kTablesLds) return kn_bin::k_bin_sweep<kn_bin::kTablesLds, WAVES, U, OWN, WIDE>;
+    if (place == kn_bin::kWindowGlobal) return kn_bin::k_bin_sweep<kn_bin::kWindowGlobal, WAVES, U, OWN, WIDE>;
+    return kn_bin::k_bin_sweep<kn_bin::kTablesGlobal, WAVES, U, false, WIDE>;
 }
 
-// The tables' placement: the first whose LDS leaves room for two blocks per
-// CU, else the first that fits at all (kTablesGlobal always does).  Own bin
-// sums where they leave three blocks per CU their LDS (as many as the sweep's
-// registers allow).
-// Blocks: a pass is 64 kSweepRun modes per wavefront of a block.  A block with
-// less than one spends its time on its tables and its partial row, so a small
-// grid gets one block per pass (with own bin sums, now whatever their LDS:
-// no second block waits for it); then one block per resident slot; and two per
-// slot (a better balanced tail) only from kSweepPasses passes per block on.
-// A small grid with so many bins that own sums do not fit gets a block per
-// row: there, too, its sums are the same on every run.
-// us per call, sweep and reduction, at two per slot whatever the size, and by
-// this rule: 64^3 24.3 -> 10.1, 128^3 27.0 -> 14.4, 192^3 36.6 -> 22.0, 256^3
-// 49.2 -> 35.2, 512^3 199.6 -> 191, 1024^3 1429 -> 1419 (its grid unchanged).
+SweepKernel sweep_kernel(const SweepPlan &p)
+{
+    constexpr int W = kn_bin::kSweepWaves, U = kn_bin::kSweepUnroll;
+    if (p.waves == 1) return sweep_kernel_at<1, 1, false, false>(p.place);
+    if (p.wide) return p.own ? sweep_kernel_at<W, U, true, true>(p.place) : sweep_kernel_at<W, U, false, true>(p.place);
+    return p.own ? sweep_kernel_at<W, 1, true, false>(p.place) : sweep_kernel_at<W, 1, false, false>(p.place);
+}
+
+// The plan of a sweep over `rows` rows.
+// Tables: the first placement whose LDS leaves room for two blocks per CU,
+// else the first that fits at all (kTablesGlobal always does).
+// Rows of 64 modes or more take the wide form.  Blocks: one per tile, up to
+// kSweepPerCu per CU.
+// Copies of the sums: as many as kSweepSumBytes hold, up to 32: the fewer the
+// bins, the more neighbouring lanes share one.  Own sums per wavefront take
+// eight times the LDS, so up to kSweepOwnBins bins (eight copies each), and
+// for grids of up to two tiles per CU, where all blocks are resident at once
+// anyway, as long as their LDS allows it.  (1024^3 with 400 bins: own sums without copies 2.20 ms,
+// four shared copies 1.32.  32 KB of copies instead of 16: 192^3 19.3 us
+// against 16.9, for their clearing and adding; 1024^3 the same.)  A small grid
+// with so many bins that own sums do not fit is swept by blocks of one
+// wavefront: its sums, too, are the same on every run.
+// us per call, sweep and reduction, before the wide form and now: 64^3 10.3 ->
+// 7.8, 128^3 14.4 -> 12.7, 256^3 34.5 -> 30.1, 512^3 189 -> 174, 1024^3 1411
+// -> 1322 (1320 with 12 to 400 bins); 1024^3 with 9000 bins 3220 -> 2170, 512^3
+// with 20000 3140 -> 2390.
 SweepPlan sweep_plan(long long rows, int dims, int nrbins)
 {
     SweepPlan p;
     p.place = kn_bin::kTablesGlobal;
     for (size_t most : {kLdsMax, kLdsMax / 2})
         for (int pl : {kn_bin::kWindowGlobal, kn_bin::kTablesLds})
-            if (kn_bin::sweep_smem_bytes(pl, dims, nrbins) <= most) p.place = pl;
-    const long long pass = 64LL * kn_bin::kSweepRun * kn_bin::kSweepWaves;
-    const long long passes = (rows * (dims / 2 + 1) + pass - 1) / pass;
-    const size_t own = kn_bin::sweep_smem_bytes(p.place, dims, nrbins, true);
-    const bool few = passes < num_cus();  // no CU gets a second block
-    p.own = p.place != kn_bin::kTablesGlobal && own <= (few ? kLdsMax : kLdsMax / 3);
-    p.smem = p.own ? own : kn_bin::sweep_smem_bytes(p.place, dims, nrbins);
-    const long long slots = (long long)resident_blocks(sweep_kernel(p), 64 * kn_bin::kSweepWaves, p.smem) * num_cus();
-    long long g = passes < slots ? passes : slots;
-    if (passes >= kSweepPasses * kSweepSlots * slots || (few && !p.own)) g = kSweepSlots * slots;
-    if (g > 65535) g = 65535;  // the sweep's 32-bit row shares
-    p.grid = (int)(rows < g ? rows : g);
+            if (kn_bin::sweep_smem_bytes(pl, dims, nrbins, 1) <= most) p.place = pl;
+    p.wide = dims / 2 + 1 >= 64;
+    p.waves = kn_bin::kSweepWaves;
+    const long long modes = rows * (dims / 2 + 1);
+    long long tile = 64LL * p.waves * (p.wide ? kn_bin::kSweepUnroll : 1), tiles = (modes + tile - 1) / tile;
+    const bool few = tiles <= 2 * num_cus();
+    const size_t own = kn_bin::sweep_smem_bytes(p.place, dims, nrbins, p.waves);
+    p.own = p.place != kn_bin::kTablesGlobal && 
+            (few ? own * (tiles <= num_cus() ? 1 : 2) <= kLdsMax : nrbins <= kSweepOwnBins);
+    if (few && !p.own && !p.wide) {
+        p.waves = 1;
+        tile = 64;
+        tiles = (modes + tile - 1) / tile;
+    }
+    const int sets = p.own ? p.waves : 1;
+    while (p.place != kn_bin::kTablesGlobal && p.cshift < 5 &&
+           sizeof(double) * ((size_t)nrbins * sets << (p.cshift + 1)) <= kSweepSumBytes)
+        p.cshift++;
+    p.smem = kn_bin::sweep_smem_bytes(p.place, dims, nrbins, sets << p.cshift);
+    if (p.smem > 64 * 1024)
+        KN_CHECK(hipFuncSetAttribute((const void *)sweep_kernel(p), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)p.smem));
+    long long per_cu = p.smem ? (long long)(kLdsMax / p.smem) : kSweepPerCu;
+    per_cu = p.waves == 1 ? 8 : (per_cu < kSweepPerCu ? per_cu : kSweepPerCu);
+    p.grid = (int)(tiles < per_cu * num_cus() ? tiles : per_cu * num_cus());
     return p;
 }
 
 void launch_sweep(kn_bin::BinArgs &a, const SweepPlan &p, hipStream_t st, double *sum_out, double *mass_out)
 {
-    a.rq = a.rows / p.grid;
-    a.rr = (unsigned)(a.rows % p.grid);
-    a.step = kn_bin::step_of(64LL * kn_bin::kSweepRun * kn_bin::kSweepWaves, a.dims / 2 + 1, a.dims);
-    hipLaunchKernelGGL(sweep_kernel(p), dim3(p.grid), dim3(64 * kn_bin::kSweepWaves), p.smem, st, a);
+    const int rowlen = a.dims / 2 + 1, B = 64 * p.waves;
+    const long long tile = (long long)B * (p.wide ? kn_bin::kSweepUnroll : 1);
+    a.in_tile = kn_bin::step_of(B, rowlen, a.dims);
+    a.to_next = kn_bin::step_of((p.grid - 1) * tile + B, rowlen, a.dims);
+    a.cshift = p.cshift;
+    hipLaunchKernelGGL(sweep_kernel(p), dim3(p.grid), dim3(B), p.smem, st, a);
     KN_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_reduce_partials, dim3((a.nrbins + kRedBins - 1) / kRedBins), dim3(kRedBins * kRedGroups), 0,
                        st, a.partial, p.grid, a.nrbins, sum_out, a.F, a.startslab == 0 ? 1 : 0, mass_out);
@@ -361,7 +390,7 @@ void launch_power(BinGeom *g, const double2 *F, hipStream_t st, double *sum_out 
     a.dims = g->dims;
     a.startslab = g->startslab;
     a.nrbins = g->nrbins;
-    a.rows = (long long)g->nslab * g->dims;
+    a.modes = (long long)g->nslab * g->dims * (g->dims / 2 + 1);
     a.thr = g->d_thr;
     a.iw = g->d_iw;
     a.half_bpu = g->half_bpu;
@@ -406,7 +435,7 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_bin_adjoint(const double2 *_
     const long long r0 = rows * blockIdx.x / gridDim.x, r1 = rows * (blockIdx.x + 1) / gridDim.x;
     const long long m1 = r1 * rowlen;
     constexpr long long S = (long long)B * kAdjUnroll;
-    Pos p = kn_bin::pos_of((int)threadIdx.x, r0, rowlen, dims);
+    Pos p = kn_bin::pos_of(r0 * rowlen + threadIdx.x, rowlen, dims);
     long long m = r0 * rowlen + threadIdx.x;
     double2 cur[kAdjUnroll];
 #pragma unroll
@@ -562,7 +591,7 @@ extern "C" int kn_bin_power_device_noalloc(const fftw_complex *d_field, int dims
     a.dims = dims;
     a.startslab = startslab;
     a.nrbins = nrbins;
-    a.rows = rows;
+    a.modes = rows * (dims / 2 + 1);
     a.thr = (const int *)sd.ptr;
     a.iw = (const double *)(sd.ptr + off_iw);
     a.half_bpu = (float)(0.5 * (nrbins - 1) / log(sqrt(3) * dims / 2.0));

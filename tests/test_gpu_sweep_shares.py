@@ -38,9 +38,12 @@ def test_rescale_shares(kn, torch_cuda, N, start, nslab, green):
 
 
 @pytest.mark.parametrize("N,start,nslab,nb", [(4, 0, 4, 15), (5, 3, 1, 7), (33, 0, 33, 9), (96, 0, 96, 96), (192, 0, 192, 64),
-                                              (250, 100, 37, 64), (250, 0, 250, 1000), (64, 0, 64, 12000)])
+                                              (250, 100, 37, 64), (250, 0, 250, 1000), (64, 0, 64, 12000), (125, 3, 122, 40),
+                                              (126, 1, 5, 2), (127, 120, 7, 33), (128, 0, 128, 1), (200, 0, 200, 13500),
+                                              (40, 0, 40, 15000), (160, 1, 159, 15000)])
 def test_bin_shares(kn, torch_cuda, N, start, nslab, nb):
-    """One block and one partial row, a pass per block, a block per resident slot; few and many bins for the reduction
+    """One block and one partial row, a tile per block, all resident blocks; rows of just under and over 64 modes; one bin,
+    and the bin counts where own sums, copies, LDS tables and one-wavefront blocks begin and end
     (counts equal, sums to 1e-12 as the other tests of the sums: they are added in another order)."""
     torch = torch_cuda
     F = _rand_grid(N, 7, nslab)
@@ -57,10 +60,10 @@ def test_bin_shares(kn, torch_cuda, N, start, nslab, nb):
         assert got[nb] == 0.0
 
 
-@pytest.mark.parametrize("N,nb", [(8, 10), (32, 1500), (36, 12000), (64, 64), (256, 128)])
+@pytest.mark.parametrize("N,nb", [(8, 10), (32, 1500), (36, 12000), (64, 64), (130, 20), (256, 32)])
 def test_bin_sums_repeat(kn, torch_cuda, N, nb):
-    """Own bin sums per wavefront (small grids, and few bins at any size), and small grids with a block per row for want of
-    LDS: the same bits on every run."""
+    """Own bin sums per wavefront (small grids, and few bins at any size), and small grids with one wavefront per block for
+    want of LDS: the same bits on every run."""
     torch = torch_cuda
     print("bin repeat", N, nb, flush=True)
     d = torch.from_numpy(_rand_grid(N, 9)).cuda()
