@@ -117,8 +117,8 @@ __device__ inline void fs_node_wave(const HTab &H, int nfs, double x0, double xa
 }
 
 // The fslength nodes in two passes with the result of one QAG per node.
-// Pass 1 (k_fs_first, no LDS): sixteen nodes per wavefront, four lanes
-// each (gk61_q4), forming the first 61-point Gauss-Kronrod estimate over
+// Pass 1 (k_fs_first): sixteen nodes per wavefront, four lanes each
+// (gk61_first), forming the first 61-point Gauss-Kronrod estimate over
 // [x_i, log a] exactly as wave_qag61's first step does, and accepting it by
 // the same test (QUADPACK returns that estimate when it already meets the
 // tolerance); a node that needs bisection is appended to a list.  Pass 2
@@ -127,33 +127,25 @@ __device__ inline void fs_node_wave(const HTab &H, int nfs, double x0, double xa
 // quarter hold 16 neighbouring nodes ((log a - log T0) / (16 Na - 1) apart,
 // far below a panel's width), so their points at one abscissa lie in one or
 // two H panels and a coefficient load touches a few cache lines, not one per
-// lane.  `push(node)` lists a node for pass 2.
-template <class Push>
-__device__ inline void fs_first_q4(const HTab &H, int nfs, double x0, double xa, double light,
-                                   double *__restrict__ fx, double *__restrict__ fy, int *__restrict__ status,
-                                   int wave, const Push &push)
+// lane.  `push(node)` lists a node for pass 2; f: the integrand.
+template <class F, class K, class Push>
+__device__ __forceinline__ void fs_first_tile(const F &f, const K &k, int nfs, double x0, double xa, double light,
+                                              double *__restrict__ fx, double *__restrict__ fy,
+                                              int *__restrict__ status, int tile, const Push &push)
 {
-    if (16 * wave >= nfs) return;  // wave-uniform
+    if (16 * tile >= nfs) return;  // wave-uniform
     const int lane = threadIdx.x & 63;
-    const int node = 16 * wave + (lane & 15);
+    const int node = 16 * tile + (lane & 15);
     // delta_tot_table.c:582: log T0 + i (log a - log T0) / (Nfs - 1.)
     const double xi = node < nfs ? x0 + node * (xa - x0) / (nfs - 1.) : xa;
-    FslIntegrand f;
-    f.H = H;
-    const GK g = gk61_q4(f, xi < xa ? xi : xa, xa);
+    double r;
+    const int rc = gk61_first(f, k, xi < xa ? xi : xa, xa, 1e-6, &r);
     if (lane < 16 && node < nfs) {
         double v = 0.0;
         if (xi < xa) {  // fslength returns 0 when logai >= logaf (:402)
-            const double tol = 1e-6 * fabs(g.res);
-            if (g.err <= 50 * DBL_EPSILON * g.resabs && g.err > tol) {
-                atomicOr(status, 1);  // roundoff on the first estimate (wave_qag61 returns 18)
-                v = light * g.res;
-            } else if ((g.err <= tol && g.err != g.resasc) || g.err == 0.0) {
-                v = light * g.res;
-            } else {
-                push(node);
-                v = 0.0;
-            }
+            if (rc == 18) atomicOr(status, 1);  // roundoff on the first estimate
+            if (rc < 0) push(node);
+            else v = light * r;
         }
         fx[node] = xi;
         fy[node] = v;
@@ -171,7 +163,9 @@ __global__ __launch_bounds__(256) void k_fs_first(HTab H, int nfs, double x0, do
                                                   int *__restrict__ count)
 {
     const ListPush push = {list, count};
-    fs_first_q4(H, nfs, x0, xa, light, fx, fy, status, (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), push);
+    FslIntegrand f;
+    f.H = H;
+    fs_first_tile(f, RuleConst(), nfs, x0, xa, light, fx, fy, status, (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), push);
 }
 
 // Pass 2: full QAG for the listed nodes (a bounded loop over the list).
@@ -363,7 +357,7 @@ __device__ inline DnuIntegrand dnu_integrand(const QagArgs &a, const SpeciesDev 
     f.H = a.H;
     f.fy = a.fy;
     f.fc = a.fc;
-    f.fk.x0 = a.x0;  // the fslength knots' own expression (fs_first_q4)
+    f.fk.x0 = a.x0;  // the fslength knots' own expression (fs_first_tile)
     f.fk.span = a.xa - a.x0;
     f.fk.den = a.nfs - 1.;
     f.nfs = a.nfs;
@@ -622,7 +616,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, double *lds)
     const double kk = A.wavenum[k], mnubykT = A.sp->mnubykT, gb = A.gbar[item];
     const JPar &J = A.sp->J;
     const double fx0 = fx[0], finv_h = (nfs - 1) / (fx[nfs - 1] - fx[0]), sx0 = sx[0];
-    UniformKnots fk;  // the fslength knots (fs_first_q4's expression)
+    UniformKnots fk;  // the fslength knots (fs_first_tile's expression)
     fk.x0 = A.x0;
     fk.span = A.xa - A.x0;
     fk.den = nfs - 1.;
@@ -999,9 +993,10 @@ __global__ __launch_bounds__(64) void k_bg_panels(const BgJob *__restrict__ jobs
     if (p >= J.npanel) return;
     const BgHub hub{J.b};
     const double lo = J.x0 + p * J.w, hi = J.x0 + (p + 1) * J.w;
-    double *c = J.coef + (size_t)p * kHStride;
-    h_fit(lo, hi, hub, c);
-    J.miss[p] = h_fit_err(c, lo, hi, hub);
+    double fit[kHStride];
+    h_fit(lo, hi, hub, fit);
+    J.miss[p] = h_fit_err(fit, lo, hi, hub);
+    h_store(fit, J.coef + (size_t)p * kHStride);
 }
 
 // One wavefront per table: the panels that miss are gathered (a strided scan,
@@ -1065,6 +1060,7 @@ __global__ __launch_bounds__(64) void k_bg_splits(const BgJob *__restrict__ jobs
         const int q = sp_p[s];
         h_split_wave(J.x0 + q * J.w, J.x0 + (q + 1) * J.w, hub,
                      J.coef + (size_t)J.npanel * kHStride + (size_t)s * kHSplitStride, L);
+        if (lane < kHStride) J.coef[(size_t)q * kHStride + lane] = NAN;  // a split panel (HTab)
     }
 }
 
@@ -1373,7 +1369,10 @@ extern "C" void kn_htable_ensure(double origin, double xlo, double xhi)
         g_h.dirty = true;
     }
     if (g_h.dirty) {
-        KN_CHECK(hipMemcpy(g_h.d_coef, g_h.coef.data(), sizeof(double) * nreg, hipMemcpyHostToDevice));
+        std::vector<double> up(g_h.coef);  // split panels as NaN (HTab)
+        for (int i = 0; i < g_h.splits.n; i++)
+            std::fill_n(up.begin() + (size_t)g_h.splits.p[i] * kHStride, kHStride, NAN);
+        KN_CHECK(hipMemcpy(g_h.d_coef, up.data(), sizeof(double) * nreg, hipMemcpyHostToDevice));
         if (g_h.splits.n)
             KN_CHECK(hipMemcpy(g_h.d_coef + nreg, g_h.splits.rec, sizeof(double) * kHSplitStride * g_h.splits.n,
                                hipMemcpyHostToDevice));
@@ -1389,7 +1388,7 @@ extern "C" double kn_htable_eval_host(double x)
     p = p < 0 ? 0 : (p >= g_h.npanel ? g_h.npanel - 1 : p);
     for (int s = 0; s < g_h.splits.n; s++)
         if (p == g_h.splits.p[s]) return exp(-x) / h_split_eval((const double *)g_h.splits.rec[s], x, 1);
-    return exp(-x) / h_clenshaw(g_h.coef.data() + (size_t)p * kHStride + kHnc, 2.0 * (u - p) - 1.0);
+    return exp(-x) / h_horner(g_h.coef.data() + (size_t)p * kHStride + kHnc, u - p);
 }
 
 extern "C" int kn_dnu_last_max_intervals(void) { return g_last_max_intervals; }
@@ -1991,8 +1990,49 @@ __global__ __launch_bounds__(256) void k_m_fs_first(const GroupDesc *__restrict_
     const GroupDesc &d = D[h];
     if (!d.integ) return;
     const GroupPush push = {list, count, h};
-    fs_first_q4(d.H, d.nfs, d.x0, d.xa, d.light, d.fx, d.fy, d.status,
-                (int)(((blk - pre[h]) * blockDim.x + threadIdx.x) >> 6), push);
+    FslIntegrand f;
+    f.H = d.H;
+    fs_first_tile(f, RuleConst(), d.nfs, d.x0, d.xa, d.light, d.fx, d.fy, d.status,
+                  (int)(((blk - pre[h]) * blockDim.x + threadIdx.x) >> 6), push);
+}
+
+// The same for large groups: a block takes kFsChunk nodes of one history and
+// first copies the panels they read (from its first node's to log a's) and the
+// rule to LDS.  The evaluations load ten coefficients each: through the L1 (64
+// bytes per clock and CU) that alone is 80 clocks per wavefront and point, from
+// LDS 40, about what the arithmetic takes; that bounds it.  256 histories,
+// 6.35e6 nodes, 387e6 points: 1252 us with Chebyshev sums through the L1, an
+// index compare per split panel and both error sums always formed; 561 us now
+// (53 clocks per wavefront and point).  With the copy's one block per CU a
+// group needs a chunk for every CU: kFsLdsNodes.
+constexpr int kFsWaves = 16, kFsChunk = 2048;
+constexpr long long kFsLdsNodes = 256LL * kFsChunk;
+__global__ __launch_bounds__(64 * kFsWaves) void k_m_fs_first_lds(const GroupDesc *__restrict__ D,
+                                                                  const int *__restrict__ pre, int nhist,
+                                                                  long long *__restrict__ list,
+                                                                  int *__restrict__ count)
+{
+    HIP_DYNAMIC_SHARED(double, lds)  // kHnc doubles per panel of the longest table
+    __shared__ double rule[kRuleLds];
+    const int blk = xcd_block();
+    const int h = hist_of(pre, nhist, blk);
+    const GroupDesc &d = D[h];
+    const int n0 = (blk - pre[h]) * kFsChunk;
+    if (!d.integ || n0 >= d.nfs) return;  // block-uniform
+    const double xi = d.x0 + n0 * (d.xa - d.x0) / (d.nfs - 1.);
+    FslIntegrandLds f;
+    f.H = d.H;
+    f.c = (const HPair *)lds;
+    f.p0 = h_locate(d.H, xi).p;
+    const int np = h_locate(d.H, d.xa).p + 1 - f.p0;
+    rule_to_lds(rule);
+    gconst_double *src = (gconst_double *)d.H.coef + (size_t)f.p0 * kHStride;
+    for (int t = threadIdx.x; t < np * kHnc; t += 64 * kFsWaves) lds[t] = src[t / kHnc * kHStride + t % kHnc];
+    __syncthreads();
+    const GroupPush push = {list, count, h};
+    const int t1 = (n0 + kFsChunk) / 16;
+    for (int t = n0 / 16 + (threadIdx.x >> 6); t < t1; t += kFsWaves)
+        fs_first_tile(f, RuleLds{rule}, d.nfs, d.x0, d.xa, d.light, d.fx, d.fy, d.status, t, push);
 }
 
 __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_fs_rest(const GroupDesc *__restrict__ D,
@@ -2281,6 +2321,7 @@ struct kn_group {
     long long *mlist = nullptr;  // pass-2 fslength list (fs_tot entries)
     std::vector<GroupDesc> desc_h;
     size_t qag_lds = 0;  // staged log a values of the longest stageable history
+    size_t fs_lds = 0;   // k_m_fs_first_lds: the longest H table's coefficients (0: k_m_fs_first)
     int tot[kPhases] = {};
     size_t adj_lds[kAdjClasses] = {};
     hipStream_t st[kGroupStreams] = {};
@@ -2408,6 +2449,23 @@ void group_plan(kn_group *g)
     std::vector<int> pre((size_t)kPhases * (n + 1), 0);
     std::vector<long long> acc(kPhases, 0);
     size_t lds[kAdjClasses] = {};
+    // the fslength nodes with the panels in LDS: where every table fits and
+    // there are enough nodes to give each CU some chunks of them
+    g->fs_lds = 0;
+    {
+        long long nodes = 0;
+        for (int i = 0; i < n; i++) {
+            const GroupHist &q = g->h[i];
+            if (!(g->cap_plan || q.integ)) continue;
+            nodes += 16LL * (g->cap_plan ? q.spec.na_max : q.na);
+            const size_t b = sizeof(double) * kHnc * (size_t)g->htabs[q.htab].npanel;
+            g->fs_lds = b > g->fs_lds ? b : g->fs_lds;
+        }
+        if (nodes < kFsLdsNodes || g->fs_lds > 160 * 1024 - sizeof(double) * kRuleLds) g->fs_lds = 0;
+        if (g->fs_lds > 64 * 1024)
+            KN_CHECK(hipFuncSetAttribute((const void *)k_m_fs_first_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)g->fs_lds));
+    }
     for (int i = 0; i < n; i++) {
         const GroupHist &q = g->h[i];
         GroupDesc &d = g->desc_h[i];
@@ -2465,7 +2523,7 @@ void group_plan(kn_group *g)
         const bool p_integ = g->cap_plan || q.integ, p_ic = g->cap_plan || !q.integ;
         long long cnt[kPhases] = {};
         if (p_integ) {
-            cnt[kPhFs] = fs_first_blocks(16 * np);
+            cnt[kPhFs] = g->fs_lds ? (16LL * np + kFsChunk - 1) / kFsChunk : fs_first_blocks(16 * np);
             cnt[kPhFactor] = factor_blocks(np);
             cnt[kPhRows] = rows_prep_blocks(rows_prep_spline_blocks(np, d.nk), 4 * np);
             cnt[kPhFsSpline] = spline_blocks(16 * np, 1);
@@ -2622,8 +2680,12 @@ void group_launch_merged(kn_group *g, hipStream_t s, bool forward, bool adjoint)
     auto pre = [&](int ph) { return g->pre + (size_t)ph * (n + 1); };
     if (forward) {
         if (g->tot[kPhFs]) {
-            hipLaunchKernelGGL(k_m_fs_first, dim3(g->tot[kPhFs]), dim3(256), 0, s, g->desc, pre(kPhFs), n, g->mlist,
-                               g->status + 3 * n);
+            if (g->fs_lds)
+                hipLaunchKernelGGL(k_m_fs_first_lds, dim3(g->tot[kPhFs]), dim3(64 * kFsWaves), g->fs_lds, s, g->desc,
+                                   pre(kPhFs), n, g->mlist, g->status + 3 * n);
+            else
+                hipLaunchKernelGGL(k_m_fs_first, dim3(g->tot[kPhFs]), dim3(256), 0, s, g->desc, pre(kPhFs), n,
+                                   g->mlist, g->status + 3 * n);
             hipLaunchKernelGGL(k_m_fs_rest, dim3(kMergedRestBlocks), dim3(64 * kWavesPerBlock), 0, s, g->desc,
                                g->mlist, g->status + 3 * n);
         }

@@ -17,6 +17,7 @@
 #include <float.h>
 #include <math.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "kn_gk61.h"
@@ -24,7 +25,8 @@
 namespace kn_dnu {
 
 constexpr int kLimit = 200;   // QAG subinterval limit (GSL_VAL)
-constexpr int kHnc = 10;      // Chebyshev coefficients per function per H panel
+constexpr int kHnc = 10;      // coefficients per function per H panel
+static_assert(kHnc == 10, "FslIntegrandLds steps five pairs a panel");
 constexpr int kHStride = 2 * kHnc;  // one panel: 1/(a^2 H) coefficients, then 1/(a H)
 // A panel whose fit misses H by more than this (relative, at test points
 // between the interpolation nodes) holds a jump or a kink of H: it is split
@@ -44,13 +46,17 @@ __constant__ double c_wg[15];
 // ---- H(a) factors as functions of x = ln a: Chebyshev panels of width 1/inv_w from origin x0 ----
 // Each panel holds the coefficients of 1/(a^2 H) (the fslength integrand,
 // delta_tot_table.c:378-383) and of 1/(a H) (the delta_nu integrand's factor,
-// :492-500), so neither integrand forms an exponential.  H may be only
+// :492-500), so neither integrand forms an exponential: fitted in Chebyshev
+// polynomials, stored as powers of the place v in [0, 1] across the panel,
+// which take half the operations (the coefficients fall by a factor of a
+// thousand per degree, so nothing is lost).  H may be only
 // piecewise smooth (the host's neutrino density switches from its spline
 // table to the non-relativistic series at a = 100 kT/m, omega_nu_single.c:
 // 171-183, where H jumps by ~1e-8 relative): a panel that holds such a point
 // is split there into two fits, stored after the npanel regular panels; the
-// table lists the split panels' indices, so the regular evaluation loads
-// nothing more than before.
+// table lists the split panels' indices.  A split panel's own coefficients are
+// NaN in the device's table: the regular evaluation knows one by its value and
+// compares no index.
 struct HTab {
     const double *coef;  // npanel * kHStride, then nsplit * kHSplitStride
     double x0, inv_w;
@@ -97,6 +103,41 @@ __host__ __device__ __forceinline__ double h_clenshaw(P c, double t)
     return fma(t, b1, c[0] - b2);
 }
 
+// One function of a panel at v in [0, 1]: sum_k c[k] v^k.
+template <typename P>
+__host__ __device__ __forceinline__ double h_horner(P c, double v)
+{
+    double r = c[kHnc - 1];
+#pragma unroll
+    for (int k = kHnc - 2; k >= 0; k--) r = fma(r, v, c[k]);
+    return r;
+}
+
+// A fit's Chebyshev coefficients (t = 2 v - 1) into the panel's powers of v,
+// for both functions.
+__host__ __device__ inline void h_store(const double *fit, double *panel)
+{
+    for (int w = 0; w < 2; w++) {
+        const double *c = fit + w * kHnc;
+        double *pw = panel + w * kHnc;
+        double a[kHnc] = {}, b[kHnc] = {};  // T_{k-1}, T_k as powers of v
+        a[0] = 1.0;
+        b[0] = -1.0;
+        b[1] = 2.0;
+        for (int i = 0; i < kHnc; i++) pw[i] = c[0] * a[i] + c[1] * b[i];
+        for (int k = 2; k < kHnc; k++) {
+            double prev = 0.0;  // b[i - 1]
+            for (int i = 0; i < kHnc; i++) {
+                const double n = 4.0 * prev - 2.0 * b[i] - a[i];
+                prev = b[i];
+                a[i] = b[i];
+                b[i] = n;
+                pw[i] += c[k] * n;
+            }
+        }
+    }
+}
+
 // A split panel's value: the piece left or right of the split point.
 template <typename P>
 __host__ __device__ __forceinline__ double h_split_eval(P rec, double x, int which)
@@ -133,18 +174,20 @@ __host__ __device__ inline void h_piece(double lo, double hi, Hub hub, double *p
     h_fit(lo, hi, hub, piece + 2);
 }
 
-// The panel [lo, hi] into coef[kHStride].  Where the fit misses H by
+// The panel [lo, hi] into panel[kHStride].  Where the fit misses H by
 // more than kHSplitTol the panel is also split, into rec[kHSplitStride], at
 // the point that bisection finds (the half whose own fit misses more is
 // kept, until both halves fit or the bracket is a few units in the last
 // place wide).  Returns the fit's miss (above kHSplitTol: rec was written).
 template <typename Hub>
-__host__ __device__ inline double h_panel(double lo, double hi, Hub hub, double *coef, double *rec)
+__host__ __device__ inline double h_panel(double lo, double hi, Hub hub, double *panel, double *rec)
 {
-    h_fit(lo, hi, hub, coef);
-    const double err = h_fit_err(coef, lo, hi, hub);
+    double tmp[kHStride];
+    h_fit(lo, hi, hub, tmp);
+    const double err = h_fit_err(tmp, lo, hi, hub);
+    h_store(tmp, panel);
     if (err <= kHSplitTol) return err;
-    double l = lo, r = hi, tmp[kHStride];
+    double l = lo, r = hi;
     for (;;) {
         const double m = l + 0.5 * (r - l);
         if (!(m > l && m < r)) break;
@@ -204,24 +247,15 @@ inline void h_table(double x0, double w, int npanel, Hub hub, std::vector<double
         const double e = h_panel(x0 + p * w, x0 + (p + 1) * w, hub, &coef[(size_t)p * kHStride], rec);
         if (e > kHSplitTol) sp.offer(p, e, rec);
     }
-    for (int i = 0; i < sp.n; i++) coef.insert(coef.end(), sp.rec[i], sp.rec[i] + kHSplitStride);
+    for (int i = 0; i < sp.n; i++) {
+        std::fill_n(coef.begin() + (size_t)sp.p[i] * kHStride, kHStride, NAN);
+        coef.insert(coef.end(), sp.rec[i], sp.rec[i] + kHSplitStride);
+    }
     H.x0 = x0;
     H.inv_w = 1.0 / w;
     H.npanel = npanel;
     H.nsplit = sp.n;
     for (int i = 0; i < kHSplitMax; i++) H.split_p[i] = i < sp.n ? sp.p[i] : -1;
-}
-
-// Evaluation of one function (which = 0: 1/(a^2 H), 1: 1/(a H)) at x.
-__host__ __device__ __forceinline__ double h_cheb(const double *coef, double x0, double inv_w, int npanel, int nsplit,
-                                                  const int *split_p, double x, int which)
-{
-    const double u = (x - x0) * inv_w;
-    int p = (int)floor(u);
-    p = p < 0 ? 0 : (p >= npanel ? npanel - 1 : p);
-    for (int s = 0; s < nsplit; s++)
-        if (p == split_p[s]) return h_split_eval(coef + (size_t)npanel * kHStride + (size_t)s * kHSplitStride, x, which);
-    return h_clenshaw(coef + (size_t)p * kHStride + which * kHnc, 2.0 * (u - p) - 1.0);
 }
 
 // Device form: the table lives in global memory, so its loads are global
@@ -230,43 +264,48 @@ __host__ __device__ __forceinline__ double h_cheb(const double *coef, double x0,
 // out-of-line pieces.
 typedef const __attribute__((address_space(1))) double gconst_double;
 
-// x's panel p (clamped to the table), its split record s (-1: none) and the
-// local coordinate t in [-1, 1]; one expression for every evaluation form.
+// x's panel p (clamped to the table) and the place v in [0, 1] across it.
 struct HLoc {
-    int p, s;
-    double t;
+    int p;
+    double v;
 };
 __device__ __forceinline__ HLoc h_locate(const HTab &H, double x)
 {
     const double u = (x - H.x0) * H.inv_w;
-    int p = (int)floor(u);
-    p = p < 0 ? 0 : (p >= H.npanel ? H.npanel - 1 : p);
-    int s = -1;
-    if (H.nsplit > 0)  // the table's (uniform): most tables have no split panel
-#pragma unroll
-        for (int i = 0; i < kHSplitMax; i++)
-            if (i < H.nsplit && p == H.split_p[i]) s = i;
     HLoc L;
-    L.p = p;
-    L.s = s;
-    L.t = 2.0 * (u - p) - 1.0;
+    L.p = (int)u;
+    L.p = L.p < 0 ? 0 : (L.p > H.npanel - 1 ? H.npanel - 1 : L.p);
+    L.v = u - L.p;
     return L;
 }
 
-__device__ __forceinline__ gconst_double *h_split_rec(const HTab &H, int s)
+// Panel p's value at x from its split record; NaN when it has none.
+__device__ __forceinline__ double h_split(const HTab &H, int p, double x, int which)
 {
-    return (gconst_double *)(H.coef + (size_t)H.npanel * kHStride + (size_t)s * kHSplitStride);
+    int s = -1;
+#pragma unroll
+    for (int i = 0; i < kHSplitMax; i++)  // constant indices: the list stays in registers
+        if (i < H.nsplit && p == H.split_p[i]) s = i;
+    if (s >= 0)
+        return h_split_eval((gconst_double *)(H.coef + (size_t)H.npanel * kHStride + (size_t)s * kHSplitStride), x,
+                            which);
+    return NAN;
 }
 
-__device__ __forceinline__ double h_cheb_dev(const HTab &H, double x, int which)
+// One function (which = 0: 1/(a^2 H), 1: 1/(a H)) at x; regular: NaN in a split panel.
+__device__ __forceinline__ double h_regular(const HTab &H, const HLoc &L, int which)
+{
+    return h_horner((gconst_double *)H.coef + (unsigned)(L.p * kHStride + which * kHnc), L.v);
+}
+__device__ __forceinline__ double h_eval(const HTab &H, double x, int which)
 {
     const HLoc L = h_locate(H, x);
-    if (H.nsplit > 0 && L.s >= 0) return h_split_eval(h_split_rec(H, L.s), x, which);
-    return h_clenshaw((gconst_double *)(H.coef + (size_t)L.p * kHStride + which * kHnc), L.t);
+    const double r = h_regular(H, L, which);
+    return r == r ? r : h_split(H, L.p, x, which);
 }
 
-__device__ __forceinline__ double inv_a2h(const HTab &H, double x) { return h_cheb_dev(H, x, 0); }
-__device__ __forceinline__ double inv_ah(const HTab &H, double x) { return h_cheb_dev(H, x, 1); }
+__device__ __forceinline__ double inv_a2h(const HTab &H, double x) { return h_eval(H, x, 0); }
+__device__ __forceinline__ double inv_ah(const HTab &H, double x) { return h_eval(H, x, 1); }
 
 // ---- the background: Omega_nu(a) and H(a), host and device ----
 // The neutrino density of omega_nu_single.c:55-205 (a table of kRhoTab log-a
@@ -643,7 +682,36 @@ __device__ __forceinline__ int settle(const double *xa, int n, int i, double x)
 // ---- integrands ----
 struct FslIntegrand {  // delta_tot_table.c:378-383: 1 / a / (a H(a))
     HTab H;
+    // NaN in a split panel, and the value there
+    __device__ __forceinline__ double regular(double x) const { return h_regular(H, h_locate(H, x), 0); }
+    __device__ __forceinline__ double split(double x) const { return h_split(H, h_locate(H, x).p, x, 0); }
     __device__ __forceinline__ double operator()(double x) const { return inv_a2h(H, x); }
+};
+
+// The same with the panels' 1/(a^2 H) coefficients in LDS: kHnc doubles a
+// panel from panel p0 on (p0 at or below every point's panel).
+struct alignas(16) HPair {
+    double x, y;
+};
+struct FslIntegrandLds {
+    HTab H;
+    const HPair *c;  // 16-byte aligned: a pair is one LDS read, whose passes of 16 lanes take one or two panels each
+    int p0;
+    __device__ __forceinline__ double regular(double x) const
+    {
+        const HLoc L = h_locate(H, x);
+        const int i0 = L.p - p0;
+        const HPair *q = c + (i0 + (i0 << 2));  // kHnc / 2 pairs a panel (shifts: a 32-bit multiply takes four times as long)
+        HPair k = q[kHnc / 2 - 1];
+        double r = fma(k.y, L.v, k.x);
+#pragma unroll
+        for (int i = kHnc / 2 - 2; i >= 0; i--) {
+            k = q[i];
+            r = fma(fma(r, L.v, k.y), L.v, k.x);
+        }
+        return r;
+    }
+    __device__ __forceinline__ double split(double x) const { return h_split(H, h_locate(H, x).p, x, 0); }
 };
 
 struct DnuIntegrand {  // delta_tot_table.c:492-500
@@ -826,7 +894,34 @@ __device__ __forceinline__ void gk61_pair(const F &f, double a1, double b1, doub
     g2.resasc = __shfl(r.resasc, 32, 64);
 }
 
-// The first 61-point Gauss-Kronrod estimate on [a, b] by four lanes of a
+// The rule's nodes and weights by gk61_pair's lane j (0 at j = 31, and Gauss
+// weights at even j), from constant memory or from a copy in LDS: with j
+// different from lane to lane, constant memory means vector loads.
+struct RuleConst {
+    __device__ __forceinline__ double x(int j) const { return j <= 30 ? c_xgk[j] : 0.0; }
+    __device__ __forceinline__ double wk(int j) const { return j <= 30 ? c_wgk[j] : 0.0; }
+    __device__ __forceinline__ double wg(int j) const { return (j < 30 && (j & 1)) ? c_wg[j >> 1] : 0.0; }
+};
+constexpr int kRuleLds = 96;  // doubles
+struct RuleLds {
+    const double *k;
+    __device__ __forceinline__ double x(int j) const { return k[j]; }
+    __device__ __forceinline__ double wk(int j) const { return k[32 + j]; }
+    __device__ __forceinline__ double wg(int j) const { return k[64 + j]; }
+};
+// The copy, by the first 32 threads of a block.
+__device__ __forceinline__ void rule_to_lds(double *k)
+{
+    const RuleConst c;
+    const int j = threadIdx.x;
+    if (j < 32) {
+        k[j] = c.x(j);
+        k[32 + j] = c.wk(j);
+        k[64 + j] = c.wg(j);
+    }
+}
+
+// QAG's first step on [a, b], a <= b, by four lanes of a
 // wavefront, lanes l, l ^ 16, l ^ 32, l ^ 48 (quarter q = (l >> 4) & 3; the
 // other 15 lanes of each quarter take 15 other intervals, so that lanes of
 // one load instruction evaluate nearby points of nearby intervals).  Quarter
@@ -834,34 +929,55 @@ __device__ __forceinline__ void gk61_pair(const F &f, double a1, double b1, doub
 // and adds their terms as gk61_pair's butterfly does (xor 16, 8 and 4 within
 // the quarter), then xor 2 and xor 1 across quarters (lane xor 32, 16): the
 // sums, and so the estimate, are gk61_pair's bit for bit, in all four lanes.
-template <class F>
-__device__ __forceinline__ GK gk61_q4(const F &f, double a, double b)
+// Returns what wave_qag61 does with the first estimate *res at relative
+// tolerance epsrel: 0 it is the result, 18 roundoff, -1 bisect (valid in
+// quarter 0).
+// The error estimate asks for two more sums over the points, |f| and
+// |f - mean|, but most integrals are accepted without them.  With f > 0
+// throughout, resabs is the result itself.  For two points of weight w, resasc
+// >= h w |f1 - f2| =: s; and with e the difference of the two rules, t = 200 e
+// / resasc < 1/2 gives err = max(resasc t^1.5, 50 eps resabs) <= max(200 e, 50
+// eps resabs), below resasc if s > 100 eps resabs.  So 200 e < s / 2, 200 e
+// below the tolerance and s above that floor mean acceptance; where that is
+// not so for some lane the wavefront forms the sums.
+template <class F, class K>
+__device__ __forceinline__ int gk61_first(const F &f, const K &k, double a, double b, double epsrel, double *res)
 {
 #pragma clang fp contract(off)  // as gk61_pair
     const int q = (threadIdx.x >> 4) & 3;
     const double c = 0.5 * (a + b), h = 0.5 * (b - a);
-    double f01[4], f02[4], f11[4], f12[4];
+    double f01[4], f02[4], f11[4], f12[4], tk[4], tg[4];
+    // four points at a time in straight-line code (sixteen would take 478 registers)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int j0 = q + 4 * r, j1 = j0 + 16;
-        const double dx0 = h * c_xgk[j0];
-        const double dx1 = j1 <= 30 ? h * c_xgk[j1] : 0.0;
-        f01[r] = f(c - dx0);
-        f02[r] = f(c + dx0);
-        f11[r] = j1 <= 30 ? f(c - dx1) : 0.0;
-        f12[r] = j1 < 30 ? f(c + dx1) : 0.0;
+        const double dx0 = h * k.x(j0), dx1 = h * k.x(j1);
+        const double x01 = c - dx0, x02 = c + dx0, x11 = c - dx1, x12 = c + dx1;
+        double v01 = f.regular(x01), v02 = f.regular(x02), v11 = f.regular(x11), v12 = f.regular(x12);
+        const double any = (v01 + v02) + (v11 + v12);
+        if (__ballot(any != any)) {  // points in split panels
+            if (v01 != v01) v01 = f.split(x01);
+            if (v02 != v02) v02 = f.split(x02);
+            if (v11 != v11) v11 = f.split(x11);
+            if (v12 != v12) v12 = f.split(x12);
+        }
+        f01[r] = v01;
+        f02[r] = v02;
+        f11[r] = j1 <= 30 ? v11 : 0.0;  // j1 = 30 is the centre, which the right point repeats; 31 (quarter 3) no point
+        f12[r] = j1 < 30 ? v12 : 0.0;
     }
-    double tk[4], tg[4], ta[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int j0 = q + 4 * r, j1 = j0 + 16;
-        const double wk0 = c_wgk[j0], wk1 = j1 <= 30 ? c_wgk[j1] : 0.0;
-        const double wg0 = (j0 & 1) ? c_wg[j0 >> 1] : 0.0;
-        const double wg1 = (j1 < 30 && (j1 & 1)) ? c_wg[j1 >> 1] : 0.0;
-        tk[r] = wk0 * (f01[r] + f02[r]) + (j1 == 30 ? wk1 * f11[r] : wk1 * (f11[r] + f12[r]));
-        tg[r] = wg0 * (f01[r] + f02[r]) + wg1 * (f11[r] + f12[r]);
-        ta[r] = wk0 * (fabs(f01[r]) + fabs(f02[r])) +
-                (j1 == 30 ? wk1 * fabs(f11[r]) : wk1 * (fabs(f11[r]) + fabs(f12[r])));
+        tk[r] = k.wk(j0) * (f01[r] + f02[r]) + k.wk(j1) * (f11[r] + f12[r]);  // the centre: f12 = 0
+        tg[r] = k.wg(j0) * (f01[r] + f02[r]) + k.wg(j1) * (f11[r] + f12[r]);
+    }
+    double least = fmin(f01[0], f02[0]);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        least = fmin(least, fmin(f01[r], f02[r]));
+        if (q + 4 * r + 16 < 30) least = fmin(least, fmin(f11[r], f12[r]));
+        else if (q + 4 * r + 16 == 30) least = fmin(least, f11[r]);
     }
     // xor 8 (j, j + 8: r, r + 2), xor 4 (j, j + 4: r 0, 1), then across quarters
     auto sum4 = [](const double(&t)[4]) {
@@ -870,7 +986,21 @@ __device__ __forceinline__ GK gk61_q4(const F &f, double a, double b)
         v += __shfl_xor(v, 16, 64);
         return v;
     };
-    const double sk = sum4(tk), sg = sum4(tg), sa = sum4(ta);
+    const double sk = sum4(tk), sg = sum4(tg);
+    *res = sk * h;
+    const double tol = epsrel * fabs(*res);
+    const double e200 = 200 * fabs((sk - sg) * h), s = h * k.wk(q) * fabs(f01[0] - f02[0]);
+    const bool sure = least > 0 && e200 < 0.5 * s && e200 < 0.99 * tol && s > 101 * DBL_EPSILON * *res &&
+                      51 * DBL_EPSILON * *res < tol;
+    if (!__ballot(a < b && !sure)) return 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int j0 = q + 4 * r, j1 = j0 + 16;
+        const double wk0 = c_wgk[j0], wk1 = j1 <= 30 ? c_wgk[j1] : 0.0;
+        tk[r] = wk0 * (fabs(f01[r]) + fabs(f02[r])) +
+                (j1 == 30 ? wk1 * fabs(f11[r]) : wk1 * (fabs(f11[r]) + fabs(f12[r])));
+    }
+    const double sa = sum4(tk);
     const double mean = sk * 0.5;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -880,13 +1010,10 @@ __device__ __forceinline__ GK gk61_q4(const F &f, double a, double b)
                 (j1 == 30 ? wk1 * fabs(f11[r] - mean)
                           : (j1 < 30 ? wk1 * (fabs(f11[r] - mean) + fabs(f12[r] - mean)) : 0.0));
     }
-    const double sasc = sum4(tk);
-    GK r;
-    r.res = sk * h;
-    r.resabs = sa * fabs(h);
-    r.resasc = sasc * fabs(h);
-    r.err = gk_rescale((sk - sg) * h, r.resabs, r.resasc);
-    return r;
+    const double resasc = sum4(tk) * fabs(h), resabs = sa * fabs(h);
+    const double err = gk_rescale((sk - sg) * h, resabs, resasc);
+    if (err <= 50 * DBL_EPSILON * resabs && err > tol) return 18;
+    return ((err <= tol && err != resasc) || err == 0.0) ? 0 : -1;
 }
 
 // Interval list of one wavefront (QUADPACK workspace), in LDS.  QUADPACK's

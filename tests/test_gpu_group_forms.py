@@ -1,0 +1,59 @@
+"""The forms a group's launches take by its size, against the per-history
+launches (streams mode), which do not change with it: equal bit for bit."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+
+import knhip
+from batch_common import Cosmo
+from dnu_common import synthetic_history
+
+pytestmark = pytest.mark.gpu
+
+HUB = C.CFUNCTYPE(C.c_double, C.c_double, C.c_void_p)
+
+
+def _merged_and_streams(hists, data, keep):
+    B = knhip.Batch(hists, keep=keep)
+    for i, (logs, rows, k, init) in enumerate(data):
+        B.load(i, logs, rows, k, init)
+    g = np.random.default_rng(1).uniform(-1, 1, B.off_k[B.n])
+    out = []
+    for streams in (0, 4):
+        print("group of %d histories, streams %d" % (B.n, streams), flush=True)
+        B.set_streams(streams)
+        B.solve()
+        B.adjoint(g)
+        out.append([B.delta_nu(), B._get("dtot_bar", 0, B.off_y[B.n]), B._get("init_bar", 0, B.off_k[B.n]), B.mnu_bar()])
+    B.close()
+    return out
+
+
+@pytest.mark.parametrize("steps", [32760, 33000, 40001])
+def test_fslength_nodes_by_group_size(kn, torch_cuda, steps):
+    """Below, just above and well above the nodes from which the H panels are copied to LDS; chunks that end inside a
+    history; tables with a split panel (the density switch of 0.379 eV), without one, and of a stepped H(a) (nodes for the
+    second pass, panels whose split records do not all fit)."""
+    c = [Cosmo([0.379, 0, 0]), Cosmo([0.0, 0, 0])]
+    hub = HUB(lambda a, ctx: 0.1 * math.sqrt(0.3 / a ** 3 + 0.7) *
+              (1.3 + 0.3 * math.tanh((math.log(a) - math.log(0.1)) / 0.002)))
+    hists, data, left = [], [], steps
+    while left > 1:
+        na = min(left, [2500, 1111, 129, 3000][len(hists) % 4])
+        i = len(hists)
+        logs, rows, k, init = synthetic_history(na, 3, 0.6, seed=i, noise=0.0)
+        h = c[i % 2].history(3, na, na, 0.6, 0.6, 0.379)
+        if i % 5 == 4:
+            h.hubble, h.hubble_ctx = C.cast(hub, C.c_void_p).value, None
+            h.light, h.delta_nu_prefac = 1.0e5, 1e-9
+        hists.append(h)
+        data.append((logs, rows, k, init))
+        left -= na
+    a, b = _merged_and_streams(hists, data, (c, hub))
+    assert np.all(np.isfinite(a[0])) and np.all(a[0] != 0)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    for x in c:
+        x.free()
