@@ -13,7 +13,8 @@
 //                wavefront per row window: scans of the substitution recurrences);
 //   k_rows_prep  the same for every delta_tot[k][0..Na-1] row, and a uniform
 //                bucket index over the stored log a values, in one launch;
-//   k_dnu_qag    one wavefront per (species, k): QAG-GK61 of the integrand
+//   k_dnu_qag_spec, k_dnu_qag_mix
+//                one block or wavefront per (species, k): QAG-GK61 of
 //                fsl/(a H) * specialJ * S_k over [log T0, log a] at the
 //                species' tolerance, as the reference does per k.
 // H(a) enters the device integrands as Chebyshev interpolants of 1/(a^2 H) and
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(256) void k_spline(const double *__restrict__ x, co
     spline_item_wave(x, y, c, n, ystride, cstride, item);
 }
 
-// Blocks of k_spline / k_adj_solve for nrows rows of n knots.
+// Blocks of k_spline for nrows rows of n knots.
 __host__ __device__ inline int spline_blocks(int n, int nrows)
 {
     const long long items = (long long)((n + kKeep - 1) / kKeep) * nrows;
@@ -276,9 +277,7 @@ __device__ inline void rows_prep_block(const double *__restrict__ sx, const doub
         const long long item = (long long)b * 4 + (threadIdx.x >> 6);
         if (item < (long long)nwin * nk) {  // wave-uniform
             const int r = (int)(item / nwin), w = (int)(item % nwin);
-            const int lo = w * kKeep, hi = lo + kKeep < na ? lo + kKeep : na;
-            tri_window_staged<false>(sx, na, Y + r * ystride, lo, hi, C + r * ystride, fac,
-                                     lds + (threadIdx.x >> 6) * kTriLds);
+            tri_window_staged(sx, na, Y + r * ystride, w, C + r * ystride, fac, lds + (threadIdx.x >> 6) * kTriLds);
         }
         return;
     }
@@ -299,7 +298,10 @@ __global__ __launch_bounds__(256, 3) void k_rows_prep(const double *__restrict__
 
 inline int rows_prep_blocks(int b_sp, int nsb) { return b_sp + (nsb + 256) / 256; }
 
-__host__ __device__ inline int rows_prep_spline_blocks(int na, int nk) { return na > 2 ? spline_blocks(na, nk) : 0; }
+__host__ __device__ inline int rows_prep_spline_blocks(int na, int nk)
+{
+    return na > 2 ? (int)(((long long)fac_windows(na) * nk + 3) / 4) : 0;
+}
 
 struct SpeciesDev {
     double mnubykT, relerr;
@@ -435,19 +437,7 @@ __device__ inline void dnu_qag_item_block(const QagArgs &a, const SpeciesDev &sp
     dnu_qag_store(a, sp, item, k, S.ws, r, ni, rc, threadIdx.x, 64 * W);
 }
 
-__global__ __launch_bounds__(64 * kWavesPerBlock) void k_dnu_qag(QagArgs a, const SpeciesDev *__restrict__ sp,
-                                                                  const int *__restrict__ item_species, int nk,
-                                                                  int nitems)
-{
-    __shared__ QagWs ws[kWavesPerBlock];
-    HIP_DYNAMIC_SHARED(double, sxs)  // a.ns doubles when a.ns <= kStageMax
-    const int wave = threadIdx.x >> 6;
-    const int item = blockIdx.x * kWavesPerBlock + wave;
-    if (item >= nitems) return;
-    dnu_qag_item(a, sp[item_species[item / nk]], item, item % nk, ws[wave], a.ns <= kStageMax ? sxs : nullptr);
-}
-
-// The same items, one block of kQagSpec wavefronts each, the highest k first
+// A call's (species, k) items, one block of kQagSpec wavefronts each, the highest k first
 // (the longest bisection chains are at high k).
 #ifndef KN_QAG_SPEC
 #define KN_QAG_SPEC 4
@@ -519,11 +509,10 @@ __device__ __forceinline__ void ic_adjoint_at(int k, const double *__restrict__ 
 }
 
 // Adjoint of one item's integral with its recorded subdivision held fixed:
-// node weights onto delta_tot[k][.] (y) and the spline coefficients (c) are
-// accumulated in LDS (ds_add_f64: the row belongs to this wave alone), plus
-// the derivative in m/kT.  One wavefront per block, one item per block.
-// Rows of Y, C, ybar and cbar are `ystride` doubles apart; entries
-// [ns, ystride) of the item's ybar row are written as zeros.
+// the points' weights onto delta_tot[k][.] and, through the spline's
+// coefficients, onto it again, plus the derivative in m/kT.
+// Rows of Y, C and ybar are `ystride` doubles apart; entries [ns, ystride) of
+// the item's ybar row are written as zeros.
 struct AdjArgs {
     HTab H;
     const double *fx, *fy, *fc;
@@ -541,202 +530,192 @@ struct AdjArgs {
     const int *nint;
     const double *gbar;
     double prefac;
-    double *ybar, *cbar, *mu_bar;  // mu_bar: [item][part]
-    int nparts, plen;              // knots split in parts of plen (see adj_parts)
+    double *ybar, *mu_bar;  // mu_bar: [item][window]
+    const double *fac;      // spline factors of sx (fac_windows(ns) windows, then the reciprocal spacings)
     IcAdjArgs ica;
 };
 
-// An item's knots [0, ns) are split in nparts parts of plen knots, one block
-// each, so that a block's LDS rows stay small (more wavefronts per CU).
-constexpr int kAdjPartKnots = 1024;
-__host__ __device__ inline int adj_parts(int ns) { return (ns + kAdjPartKnots - 1) / kAdjPartKnots; }
-__host__ __device__ inline int adj_plen(int ns) { return (ns + adj_parts(ns) - 1) / adj_parts(ns); }
-// LDS of one block: ybar and cbar rows of plen doubles, the selected interval
-// list and the queue of points to evaluate (kAdjQueue)
+// One window's weights, the intervals that reach it and the queue of points
+// to evaluate.
 constexpr int kAdjQueue = 128;
-inline size_t adj_lds_bytes(int ns)
-{
-    return sizeof(double) * 2 * (size_t)adj_plen(ns) + sizeof(int) * (kLimit + kAdjQueue);
-}
+struct AdjLds {
+    double c[kTriSpan], y[kTriSpan];
+    double a[64], b[64];
+    double x[kAdjQueue], w[kAdjQueue];
+};
 
-// Block `blk` of one history's adjoint: (item, part) blocks [0, nk nparts),
-// then the initial-condition piece, 64 k per block.  The part owning knots
-// [K0, K1) evaluates the points of the recorded intervals that can reach
-// them (a point in knot interval si feeds knots si and si+1: x within
-// [sx[K0 - 1], sx[K1]]) and keeps the terms that land in [K0, K1); a point's
-// d/d(m/kT) term goes to the part owning its si, so every term is counted
-// once.  The points that pass are queued in LDS and evaluated 64 at a time,
-// one per lane, so a part evaluates its own share of a long interval's
-// points, not all of them.  `lds`: adj_lds_bytes(ns).
-__device__ inline void dnu_adj_block(const AdjArgs &A, int blk, double *lds)
+// Block `blk` of one history's adjoint, one wavefront: (item, window) blocks
+// [0, nk fac_windows(ns)), then the initial-condition piece, 64 k per block.
+// A point at x in knot interval si puts weights on y and on the spline's
+// quadratic coefficients c at knots si and si + 1.  The coefficients solve M c
+// = rhs(y) (natural-spline matrix, symmetric), so their weights cbar go onto y
+// as rhs^T(M^-1 cbar): the window keeps knots [lo, hi) and gathers cbar kHalo
+// knots further on either side, which is all that M^-1 lets reach them; the
+// weights stay in LDS from the points to the finished row.  (The points in
+// parts of up to 1024 knots, their weights through memory to a solve of their
+// own, took 1131 + 1157 us for 256 histories of 64-512 k x 100-3000 steps;
+// this takes 1339: 284 in the solve, 740 in the points' FP64, the rest in
+// gathering them and in the rows' one write.  Three waves per SIMD: with the
+// compiler's own choice of registers, which lets two run, 1411; with four,
+// which spill more, 1412.)
+// Points that reach the window (x within [sx[E0 - 1], sx[E1]]) are queued and
+// evaluated 64 at a time, one per lane; a point's d/d(m/kT) term belongs to
+// the window that keeps its si, so every term is counted once.
+__device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
 {
-    const int nk = A.nk, ns = A.ns, nfs = A.nfs;
-    const double *__restrict__ fx = A.fx, *__restrict__ fy = A.fy, *__restrict__ fc = A.fc, *__restrict__ sx = A.sx;
-    const int *__restrict__ sb = A.sb;
-    const double prefac = A.prefac, vcrit = A.vcrit, sinv_bw = A.sinv_bw;
-    const int nsb = A.nsb;
-    const HTab &H = A.H;
-    const int P = A.nparts, L = A.plen;
+    const int nk = A.nk, ns = A.ns, nfs = A.nfs, lane = threadIdx.x & 63;
+    const int P = fac_windows(ns), keep = fac_keep(ns);
     if (blk >= nk * P) {
-        const int kk = (blk - nk * P) * 64 + (int)(threadIdx.x & 63);
+        const int kk = (blk - nk * P) * 64 + lane;
         if (kk < nk) ic_adjoint_at(kk, A.wavenum, A.gbar, *A.sp, A.ica);
         return;
     }
-    const int lane = threadIdx.x & 63, item = blk / P, part = blk % P, k = item % nk;
-    const int K0 = part * L, K1 = K0 + L < ns ? K0 + L : ns;
-    int *sel = (int *)(lds + 2 * L);
-    for (int t = lane; t < 2 * L; t += 64) lds[t] = 0.0;
-    const double *__restrict__ ivl = A.ivl;
+    const double *__restrict__ fx = A.fx, *__restrict__ fy = A.fy, *__restrict__ fc = A.fc, *__restrict__ sx = A.sx;
+    const int item = blk / P, win = blk % P, k = item % nk;
+    const int lo = win * keep, hi = lo + keep < ns ? lo + keep : ns;
+    const int E0 = lo > kHalo ? lo - kHalo : 0, E1 = hi + kHalo < ns ? hi + kHalo : ns;
+    const double xlo = sx[E0 > 0 ? E0 - 1 : 0], xhi = sx[E1 < ns ? E1 : ns - 1];
+    const double *__restrict__ ivl = A.ivl + (size_t)item * kLimit * 2;
     const int ni = A.nint[item];
-    // the recorded intervals that reach this part's knots, in their order:
-    // x in [sx[K0 - 1], sx[K1]] (clamped to the table)
-    int nsel = 0;
-    const double xlo = sx[K0 > 0 ? K0 - 1 : 0], xhi = sx[K1 < ns ? K1 : ns - 1];
-    {
-        for (int t0 = 0; t0 < ni; t0 += 64) {
-            const int t = t0 + lane;
-            int hit = 0;
-            if (t < ni) {
-                const double a = ivl[((size_t)item * kLimit + t) * 2], b = ivl[((size_t)item * kLimit + t) * 2 + 1];
-                hit = (a <= xhi && b >= xlo) ? 1 : 0;
-            }
-            double sc = hit;  // inclusive prefix count over the wavefront
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const double o = __shfl_up(sc, d, 64);
-                if (lane >= d) sc += o;
-            }
-            if (hit) sel[nsel + (int)sc - 1] = t;
-            nsel += (int)__shfl(sc, 63, 64);
-        }
-    }
-    __syncthreads();
     const double *syk = A.Y + (size_t)k * A.ystride, *sck = A.C + (size_t)k * A.ystride;
     const bool linear = ns <= 2;
-    const double kk = A.wavenum[k], mnubykT = A.sp->mnubykT, gb = A.gbar[item];
+    const double kk = A.wavenum[k], mnubykT = A.sp->mnubykT, gb = A.gbar[item] * A.prefac;
     const JPar &J = A.sp->J;
     const double fx0 = fx[0], finv_h = (nfs - 1) / (fx[nfs - 1] - fx[0]), sx0 = sx[0];
     UniformKnots fk;  // the fslength knots (fs_first_tile's expression)
     fk.x0 = A.x0;
     fk.span = A.xa - A.x0;
     fk.den = nfs - 1.;
+#pragma unroll
+    for (int p = 0; p < kTriPass; p++) {
+        const int t = p * 64 + lane;
+        if (t < kTriSpan) S.c[t] = S.y[t] = 0.0;
+    }
     double mu_acc = 0.0;
-    // point g of the selected intervals: interval sel[g / 61], node jj = g % 61
-    // (jj < 30: c - h xgk[jj]; 30: c; jj > 30: c + h xgk[60 - jj])
-    auto point = [&](int g, double &x, double &w) {
-        const int t = sel[g / 61], jj = g % 61, jn = jj <= 30 ? jj : 60 - jj;
-        const double a = ivl[((size_t)item * kLimit + t) * 2], b = ivl[((size_t)item * kLimit + t) * 2 + 1];
-        const double c = 0.5 * (a + b), hl = 0.5 * (b - a);
-        x = jj < 30 ? c - hl * c_xgk[jn] : (jj == 30 ? c : c + hl * c_xgk[jn]);
-        w = c_wgk[jn] * hl * prefac * gb;
-    };
-    auto eval = [&](int g) {
-        double x, w;
-        point(g, x, w);
-        // the pieces of delta_tot_table.c:492-500
+    auto eval = [&](double x, double w) {
+        // the pieces of delta_tot_table.c:492-500; the spline's knots and values at the bucket's knot and the next
+        // two, loaded before the knot walk (as DnuIntegrand::eval2)
+        int q = (int)((x - sx0) * A.sinv_bw);
+        q = q < 0 ? 0 : (q > A.nsb ? A.nsb : q);
+        const int b = A.sb[q], i0 = b < 0 ? 0 : (b > ns - 2 ? ns - 2 : b), i2 = i0 + 2 < ns ? i0 + 2 : ns - 1;
+        const double s0 = sx[i0], s1 = sx[i0 + 1], s2 = sx[i2], y0 = syk[i0], y1 = syk[i0 + 1], y2 = syk[i2];
+        double c0 = 0.0, c1 = 0.0, c2 = 0.0;
+        if (!linear) c0 = sck[i0], c1 = sck[i0 + 1], c2 = sck[i2];
         double xl, xr;
         const int fi = settle_uniform(fk, nfs, (int)((x - fx0) * finv_h), x, xl, xr);
         const double fsl = cspline_val(xl, xr, fy[fi], fy[fi + 1], fc[fi], fc[fi + 1], x);
-        int q = (int)((x - sx0) * sinv_bw);
-        q = q < 0 ? 0 : (q > nsb ? nsb : q);
-        const int si = settle(sx, ns, sb[q], x);
+        const double base = fsl * inv_ah(A.H, x);  // fsl / (a H), as the forward
+        int si = i0;
+        double sl = s0, sr = s1, yl = y0, yr = y1, cl = c0, cr = c1;
+        if (s0 > x || (i0 < ns - 2 && s1 <= x)) {
+            if (s0 <= x && (i0 + 1 >= ns - 2 || s2 > x)) {
+                si = i0 + 1;
+                sl = s1, sr = s2, yl = y1, yr = y2, cl = c1, cr = c2;
+            } else {
+                si = settle(sx, ns, i0, x);
+                sl = sx[si], sr = sx[si + 1], yl = syk[si], yr = syk[si + 1];
+                if (!linear) cl = sck[si], cr = sck[si + 1];
+            }
+        }
         const double kx = kk * fsl / mnubykT;
         double Jx, Jq;
         const double Jv = specialJ_d(kx, J, Jx, Jq);
-        const double base = fsl * inv_ah(H, x);  // fsl / (a H), as the forward
-        const double S = linear ? linear_at(sx, syk, si, x) : cspline_at(sx, syk, sck, si, x);
-        const bool own0 = si >= K0 && si < K1, own1 = si + 1 >= K0 && si + 1 < K1;
-        if (own0)  // d/d(m/kT), qc = vcrit m/kT
-            mu_acc += w * base * S * (Jx * (-kx / mnubykT) + Jq * vcrit);
+        const double dx = x - sl, h = sr - sl;
+        const double S0 = linear ? (h > 0.0 ? yl + dx / h * (yr - yl) : yl) : cspline_val(sl, sr, yl, yr, cl, cr, x);
+        const bool own = si >= lo && si < hi, own1 = si + 1 >= lo && si + 1 < hi;
+        if (own)  // d/d(m/kT), qc = vcrit m/kT
+            mu_acc += w * base * S0 * (Jx * (-kx / mnubykT) + Jq * A.vcrit);
         const double wj = w * base * Jv;
         if (linear) {
-            const double t1 = (x - sx[si]) / (sx[si + 1] - sx[si]);
-            if (own0) atomicAdd(&lds[si - K0], wj * (1.0 - t1));
-            if (own1) atomicAdd(&lds[si + 1 - K0], wj * t1);
+            const double t1 = dx / h;
+            if (own) atomicAdd(&S.y[si - lo], wj * (1.0 - t1));
+            if (own1) atomicAdd(&S.y[si + 1 - lo], wj * t1);
         } else {
             double wy0, wy1, wc0, wc1;
-            cspline_grad(sx, si, x, wy0, wy1, wc0, wc1);
-            if (own0) {
-                atomicAdd(&lds[si - K0], wj * wy0);
-                atomicAdd(&lds[L + si - K0], wj * wc0);
-            }
-            if (own1) {
-                atomicAdd(&lds[si + 1 - K0], wj * wy1);
-                atomicAdd(&lds[L + si + 1 - K0], wj * wc1);
-            }
+            cspline_grad(sl, sr, x, wy0, wy1, wc0, wc1);
+            if (own) atomicAdd(&S.y[si - lo], wj * wy0);
+            if (own1) atomicAdd(&S.y[si + 1 - lo], wj * wy1);
+            if (si >= E0 && si < E1) atomicAdd(&S.c[si - E0], wj * wc0);
+            if (si + 1 >= E0 && si + 1 < E1) atomicAdd(&S.c[si + 1 - E0], wj * wc1);
         }
     };
-    int *queue = sel + kLimit;  // kAdjQueue point indices
-    const int npts = nsel * 61;
     int nq = 0;  // queued points (wavefront-uniform), below 64 between rounds
-    for (int g0 = 0; g0 < npts; g0 += 64) {
-        const int g = g0 + lane;
-        bool in = false;
-        if (g < npts) {
-            double x, w;
-            point(g, x, w);
-            in = x >= xlo && x <= xhi;
+    for (int t0 = 0; t0 < ni; t0 += 64) {
+        // of 64 recorded intervals, those that reach the window, in their order
+        const int t = t0 + lane;
+        const double ia = t < ni ? ivl[2 * t] : 0.0, ib = t < ni ? ivl[2 * t + 1] : 0.0;
+        const bool hit = t < ni && ia <= xhi && ib >= xlo;
+        const unsigned long long m = __ballot(hit);
+        if (hit) {
+            const int r = __popcll(m & ((1ull << lane) - 1));
+            S.a[r] = ia;
+            S.b[r] = ib;
         }
-        const unsigned long long m = __ballot(in);
-        if (in) queue[nq + __popcll(m & ((1ull << lane) - 1))] = g;
-        nq += __popcll(m);
-        __builtin_amdgcn_wave_barrier();  // the queue is written before any lane reads it
-        if (nq >= 64) {
-            eval(queue[lane]);
-            const int rest = nq - 64;
-            const int v = lane < rest ? queue[64 + lane] : 0;
-            __builtin_amdgcn_wave_barrier();  // every lane has read before any lane moves
-            if (lane < rest) queue[lane] = v;
-            __builtin_amdgcn_wave_barrier();
-            nq = rest;
+        wave_lds_sync();
+        const int npts = __popcll(m) * 61;
+        for (int g0 = 0; g0 < npts; g0 += 64) {
+            // point g: interval g / 61, node jj = g % 61 (jj < 30: c - h xgk[jj]; 30: c; jj > 30: c + h xgk[60 - jj])
+            const int g = g0 + lane < npts ? g0 + lane : npts - 1, jj = g % 61, jn = jj <= 30 ? jj : 60 - jj;
+            const double pa = S.a[g / 61], pb = S.b[g / 61], c = 0.5 * (pa + pb), hl = 0.5 * (pb - pa);
+            const double x = jj < 30 ? c - hl * c_xgk[jn] : (jj == 30 ? c : c + hl * c_xgk[jn]);
+            const bool in = g0 + lane < npts && x >= xlo && x <= xhi;
+            const unsigned long long mi = __ballot(in);
+            if (in) {
+                const int r = nq + __popcll(mi & ((1ull << lane) - 1));
+                S.x[r] = x;
+                S.w[r] = c_wgk[jn] * hl * gb;
+            }
+            nq += __popcll(mi);
+            wave_lds_sync();
+            if (nq >= 64) {
+                eval(S.x[lane], S.w[lane]);
+                nq -= 64;
+                const double qx = lane < nq ? S.x[64 + lane] : 0.0, qw = lane < nq ? S.w[64 + lane] : 0.0;
+                wave_lds_sync();
+                if (lane < nq) {
+                    S.x[lane] = qx;
+                    S.w[lane] = qw;
+                }
+                wave_lds_sync();
+            }
         }
     }
-    if (lane < nq) eval(queue[lane]);
+    if (lane < nq) eval(S.x[lane], S.w[lane]);
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) mu_acc += __shfl_xor(mu_acc, m, 64);
-    __syncthreads();
-    double *yrow = A.ybar + (size_t)k * A.ystride, *crow = A.cbar + (size_t)k * A.ystride;
-    for (int t = lane; t < K1 - K0; t += 64) {
-        yrow[K0 + t] = lds[t];
-        crow[K0 + t] = lds[L + t];
+    if (lane == 0) A.mu_bar[(size_t)item * P + win] = mu_acc;
+    wave_lds_sync();
+    if (ns > 2) {
+        const TriLane t = tri_lane(ns, lo, hi);
+        const double *ih = A.fac + (size_t)P * kFacStride;
+        double rv[kRun], g[kRun], ial[kRun], before, vi[kTriPass];
+        tri_factor_load(A.fac, win, g, ial, before);
+        const int base = t.wa - 1, cnt = t.wb - base;
+#pragma unroll
+        for (int p = 0; p < kTriPass; p++) vi[p] = p * 64 + lane < cnt ? ih[base + p * 64 + lane] : 0.0;
+#pragma unroll
+        for (int j = 0; j < kRun; j++) rv[j] = j < t.len ? S.c[t.s + j - E0] : 0.0;
+        wave_lds_sync();  // the reciprocal spacings take the place of cbar
+#pragma unroll
+        for (int p = 0; p < kTriPass; p++)
+            if (p * 64 + lane < cnt) S.c[p * 64 + lane] = vi[p];
+        wave_lds_sync();
+        tri_solve<RunRhs, true>(sx, ns, RunRhs{rv, t.s}, lo, hi, OutLds{S.y, lo}, t, g, ial, before,
+                                IhLds{S.c, base});
+        wave_lds_sync();
     }
-    if (part == P - 1)
+    double *yrow = A.ybar + (size_t)k * A.ystride;
+#pragma unroll
+    for (int p = 0; p < kTriPass; p++)
+        if (p * 64 + lane < hi - lo) yrow[lo + p * 64 + lane] = S.y[p * 64 + lane];
+    if (win == P - 1)
         for (int t = ns + lane; t < A.ystride; t += 64) yrow[t] = 0.0;
-    if (lane == 0) A.mu_bar[(size_t)item * P + part] = mu_acc;
 }
 
-__global__ __launch_bounds__(64) void k_dnu_adj(AdjArgs A)
+__global__ __launch_bounds__(64, 3) void k_dnu_adj(AdjArgs A)
 {
-    HIP_DYNAMIC_SHARED(double, lds)  // adj_lds_bytes(ns): part rows of ybar and cbar, interval list
-    dnu_adj_block(A, blockIdx.x, lds);
-}
-
-// Per row of the adjoint, M z = cbar (the natural-spline matrix is
-// symmetric, so its transpose is itself) by wavefronts as k_spline, and z
-// added through the right-hand side 3((y_{i+1}-y_i)/h_i - (y_i-y_{i-1})/h_{i-1})
-// onto ybar in the same pass.
-// Rows `stride` doubles apart, on the stored factors of x; block `b` of
-// spline_blocks(n, nrows).
-// lds: kTriLds doubles per wavefront of the block
-__device__ inline void adj_solve_block(const double *__restrict__ x, int n, int nrows, long long stride,
-                                       const double *__restrict__ cbar, double *__restrict__ ybar,
-                                       const double *__restrict__ fac, int b, double *lds)
-{
-    const int nwin = (n + kKeep - 1) / kKeep;
-    const long long item = (long long)b * 4 + (threadIdx.x >> 6);
-    if (item >= (long long)nwin * nrows) return;  // wave-uniform
-    const int r = (int)(item / nwin), w = (int)(item % nwin);
-    const int lo = w * kKeep, hi = lo + kKeep < n ? lo + kKeep : n;
-    tri_window_staged<true>(x, n, cbar + (size_t)r * stride, lo, hi, ybar + (size_t)r * stride, fac,
-                            lds + (threadIdx.x >> 6) * kTriLds);
-}
-
-__global__ __launch_bounds__(256) void k_adj_solve(const double *__restrict__ x, int n, int nrows, long long stride,
-                                                   const double *__restrict__ cbar, double *__restrict__ ybar,
-                                                   const double *__restrict__ fac)
-{
-    __shared__ double lds[4 * kTriLds];
-    adj_solve_block(x, n, nrows, stride, cbar, ybar, fac, blockIdx.x, lds);
+    __shared__ AdjLds S;
+    dnu_adj_block(A, blockIdx.x, S);
 }
 
 // ---------------------------------------------------------------- state
@@ -755,7 +734,7 @@ struct DnuDev {
     double *ivl = nullptr;                                            // recorded subdivisions
     size_t cap_fac = 0;
     double *fac = nullptr;  // spline factors of scalefact (fac_doubles(Na))
-    double *gbar = nullptr, *ybar = nullptr, *cbar = nullptr, *mubar = nullptr;  // adjoint
+    double *gbar = nullptr, *ybar = nullptr, *mubar = nullptr;  // adjoint
     // the delta_tot rows held in Y (row stride namax, the host table's), and a
     // host copy of what Y holds: each call uploads a row only from its first
     // entry that differs from that copy (an appended or overwritten step is
@@ -771,7 +750,7 @@ struct DnuDev {
 std::unordered_map<const void *, DnuDev *> g_dev;
 int g_last_max_intervals = 0, g_last_items = 0;
 long long g_last_intervals = 0;
-// optional HIP-event timing of the QAG launch (k_dnu_qag) of each get_delta_nu
+// optional HIP-event timing of the QAG launch of each get_delta_nu
 int g_qag_timing = 0;
 hipEvent_t g_qag_ev[2];
 float g_qag_ms = 0.0f;
@@ -1429,8 +1408,8 @@ extern "C" void kn_dnu_release(const _delta_tot_table *d)
     if (it == g_dev.end()) return;
     DnuDev *v = it->second;
     void *ptrs[] = {v->fs_list, v->fx,  v->fy,   v->fc,   v->sx,   v->Y,    v->C,    v->wavenum, v->bucket, v->out,
-                    v->nint, v->item_species, v->sp, v->status, v->ivl, v->gbar, v->ybar, v->cbar,
-                    v->mubar, v->fac, v->order};
+                    v->nint, v->item_species, v->sp, v->status, v->ivl, v->gbar, v->ybar, v->mubar,
+                    v->fac, v->order};
     for (void *p : ptrs)
         if (p) KN_CHECK(hipFree(p));
     delete v;
@@ -1737,17 +1716,15 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
     if (dtot_bar && (s.ic_only || Na < 2)) memset(dtot_bar, 0, sizeof(double) * (size_t)nk * Na);
     if (!s.ic_only && Na >= 2) {
         DnuDev *dev = g_dev[d];
-        const int namax = dev->ystride;  // rows of Y, C, ybar and cbar are namax doubles apart
+        const int namax = dev->ystride;  // rows of Y, C and ybar are namax doubles apart
         const size_t ny = (size_t)nk * Na, nyd = (size_t)nk * namax;
         if (dev->cap_adj < nyd) {
-            for (double **p : {&dev->ybar, &dev->cbar}) {
-                if (*p) KN_CHECK(hipFree(*p));
-                KN_CHECK(hipMalloc(p, sizeof(double) * nyd));
-            }
+            if (dev->ybar) KN_CHECK(hipFree(dev->ybar));
+            KN_CHECK(hipMalloc(&dev->ybar, sizeof(double) * nyd));
             dev->cap_adj = nyd;
         }
-        const int P = adj_parts(Na);
-        if (dev->cap_adj_k < (size_t)nk * P) {  // gbar (nk), mubar (nk x parts)
+        const int P = fac_windows(Na);
+        if (dev->cap_adj_k < (size_t)nk * P) {  // gbar (nk), mubar (nk x windows)
             for (double **p : {&dev->gbar, &dev->mubar}) {
                 if (*p) KN_CHECK(hipFree(*p));
                 KN_CHECK(hipMalloc(p, sizeof(double) * nk * P));
@@ -1755,7 +1732,6 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
             dev->cap_adj_k = (size_t)nk * P;
         }
         KN_CHECK(hipMemcpy(dev->gbar, gbar, sizeof(double) * nk, hipMemcpyHostToDevice));
-        const size_t lds = adj_lds_bytes(Na);
         const int nfs = 16 * Na, nsb = 4 * Na;
         const double sinv_bw = nsb / (d->scalefact[Na - 1] - d->scalefact[0]);
         const double vcrit = s.qc > 0 ? d->omnu->hybnu.vcrit : 0.0;
@@ -1784,19 +1760,12 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
         A.gbar = dev->gbar;
         A.prefac = d->delta_nu_prefac;
         A.ybar = dev->ybar;
-        A.cbar = dev->cbar;
         A.mu_bar = dev->mubar;
-        A.nparts = P;
-        A.plen = adj_plen(Na);
+        A.fac = dev->fac;
         A.ica = IcAdjArgs{nullptr, 0.0, 0.0, nullptr, nullptr};
-        hipLaunchKernelGGL(k_dnu_adj, dim3(nk * P), dim3(64), lds, 0, A);
+        hipLaunchKernelGGL(k_dnu_adj, dim3(nk * P), dim3(64), 0, 0, A);
         KN_CHECK(hipGetLastError());
-        if (Na > 2) {
-            hipLaunchKernelGGL(k_adj_solve, dim3(spline_blocks(Na, nk)), dim3(256), 0, 0, dev->sx, Na, nk,
-                               (long long)namax, dev->cbar, dev->ybar, dev->fac);
-            KN_CHECK(hipGetLastError());
-        }
-        // results through the pinned stage: [mu_bar (nk x parts) | dL/d delta_tot (nk Na)]
+        // results through the pinned stage: [mu_bar (nk x windows) | dL/d delta_tot (nk Na)]
         const size_t nmu = (size_t)nk * P;
         double *mub = (double *)pinned_stage(sizeof(double) * (nmu + (dtot_bar ? ny : 0))), *yb = mub + nmu;
         KN_CHECK(hipMemcpyAsync(mub, dev->mubar, sizeof(double) * nmu, hipMemcpyDeviceToHost, 0));
@@ -1813,7 +1782,7 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
             KN_CHECK(hipEventRecord(done[c], 0));
         }
         KN_CHECK(chunks ? hipEventSynchronize(done[0]) : hipStreamSynchronize(0));  // mu_bar went first
-        for (size_t i = 0; i < nmu; i++) mb += mub[i];  // k-major, parts in order
+        for (size_t i = 0; i < nmu; i++) mb += mub[i];  // k-major, windows in order
         for (int c = 0; c < chunks; c++) {
             KN_CHECK(hipEventSynchronize(done[c]));
             const size_t i0 = (size_t)((long long)nk * c / chunks) * Na, i1 = (size_t)((long long)nk * (c + 1) / chunks) * Na;
@@ -1922,13 +1891,13 @@ struct GroupHist {
 // that history's block b - pre[h] of the per-call kernel's grid, running the
 // same device code on the history's arrays (descriptor below).
 
-// Per-history arrays and scalars (device copy; rows of Y, C, dbar and cbar
-// are na_max doubles apart).
+// Per-history arrays and scalars (device copy; rows of Y, C and dbar are
+// na_max doubles apart).
 struct GroupDesc {
     HTab H;
     double *sx, *Y;
     const double *wavenum, *init, *gbar;
-    double *C, *fx, *fy, *fc, *out, *ivl, *dbar, *cbar, *mubar, *ibar, *mbic, *fac;
+    double *C, *fx, *fy, *fc, *out, *ivl, *dbar, *mubar, *ibar, *mbic, *fac;
     int *bucket, *nint, *status;
     const SpeciesDev *sp;
     // the stored steps and what they set: live in device memory (the device
@@ -1940,12 +1909,8 @@ struct GroupDesc {
     double xmax, nu_crit_time, nufrac_low, vcrit_spec, mnu, kBtnu, deriv_prefac;
 };
 
-// phases (rows of the prefix table); the adjoint's (item, part) blocks are
-// split in classes of part length (LDS rows of 2 adj_plen(na) doubles):
-// class c holds adj_plen(na) <= 128 << c
-enum { kPhFs, kPhFactor, kPhRows, kPhFsSpline, kPhQag, kPhIc, kPhSolve, kPhAdj0 };
-constexpr int kAdjClasses = 4;
-constexpr int kPhases = kPhAdj0 + kAdjClasses;
+// phases (rows of the prefix table)
+enum { kPhFs, kPhFactor, kPhRows, kPhFsSpline, kPhQag, kPhIc, kPhAdj, kPhases };
 constexpr int kMergedRestBlocks = 1280;
 
 // The hardware deals the blocks of a grid to the 8 XCDs in turn (block b to
@@ -2165,10 +2130,10 @@ __global__ __launch_bounds__(64) void k_m_ic_adj(const GroupDesc *__restrict__ D
     }
 }
 
-__global__ __launch_bounds__(64) void k_m_dnu_adj(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
+__global__ __launch_bounds__(64, 3) void k_m_dnu_adj(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
                                                   int nhist)
 {
-    HIP_DYNAMIC_SHARED(double, lds)  // adj_lds_bytes of the class's longest part
+    __shared__ AdjLds S;
     const int blk = xcd_block();
     const int h = hist_of(pre, nhist, blk);
     const GroupDesc &d = D[h];
@@ -2198,23 +2163,10 @@ __global__ __launch_bounds__(64) void k_m_dnu_adj(const GroupDesc *__restrict__ 
     A.gbar = d.gbar;
     A.prefac = d.prefac;
     A.ybar = d.dbar;
-    A.cbar = d.cbar;
     A.mu_bar = d.mubar;
-    A.nparts = adj_parts(d.na);
-    A.plen = adj_plen(d.na);
+    A.fac = d.fac;
     A.ica = group_ica(d);
-    dnu_adj_block(A, blk - pre[h], lds);
-}
-
-__global__ __launch_bounds__(256) void k_m_adj_solve(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
-                                                     int nhist)
-{
-    const int blk = xcd_block();
-    const int h = hist_of(pre, nhist, blk);
-    const GroupDesc &d = D[h];
-    if (!d.integ) return;
-    __shared__ double lds[4 * kTriLds];
-    adj_solve_block(d.sx, d.na, d.nk, (long long)d.na_max, d.cbar, d.dbar, d.fac, blk - pre[h], lds);
+    dnu_adj_block(A, blk - pre[h], S);
 }
 
 // One more stored step per history, on the device (one wavefront per
@@ -2296,7 +2248,7 @@ __global__ __launch_bounds__(64) void k_group_step(GroupDesc *__restrict__ D, Sp
         sp[h].relerr = relerr;
         sp[h].J.qc = qc;
         meta[h].integ = integ;
-        meta[h].nparts = adj_parts(n1);
+        meta[h].nparts = fac_windows(n1);
     }
 }
 
@@ -2309,7 +2261,7 @@ struct kn_group {
     std::vector<HTab> htabs;
     std::vector<double *> hcoef;
     std::vector<int> order;
-    double *sx = nullptr, *Y = nullptr, *C = nullptr, *dbar = nullptr, *cbar = nullptr, *fx = nullptr,
+    double *sx = nullptr, *Y = nullptr, *C = nullptr, *dbar = nullptr, *fx = nullptr,
            *fy = nullptr, *fc = nullptr, *wavenum = nullptr, *init = nullptr, *out = nullptr, *gbar = nullptr,
            *ibar = nullptr, *mbic = nullptr, *mubar = nullptr, *mbar = nullptr, *ivl = nullptr, *fac = nullptr;
     int *bucket = nullptr, *nint = nullptr, *status = nullptr, *zeros = nullptr, *spec0 = nullptr, *fs_list = nullptr;
@@ -2323,7 +2275,6 @@ struct kn_group {
     size_t qag_lds = 0;  // staged log a values of the longest stageable history
     size_t fs_lds = 0;   // k_m_fs_first_lds: the longest H table's coefficients (0: k_m_fs_first)
     int tot[kPhases] = {};
-    size_t adj_lds[kAdjClasses] = {};
     hipStream_t st[kGroupStreams] = {};
     hipEvent_t fork = nullptr, join[kGroupStreams] = {};
     hipGraph_t graph = nullptr;
@@ -2424,7 +2375,7 @@ void group_meta_upload(kn_group *g)
     for (int i = 0; i < g->nhist; i++) {
         m[i].off_k = g->h[i].off_k;
         m[i].off_mu = g->h[i].off_mu;
-        m[i].nparts = adj_parts(g->h[i].na);
+        m[i].nparts = fac_windows(g->h[i].na);
         m[i].nk = g->h[i].spec.nk;
         m[i].integ = g->h[i].integ;
         m[i].kBtnu = g->h[i].spec.kBtnu;
@@ -2448,7 +2399,6 @@ void group_plan(kn_group *g)
     g->desc_h.resize(n);
     std::vector<int> pre((size_t)kPhases * (n + 1), 0);
     std::vector<long long> acc(kPhases, 0);
-    size_t lds[kAdjClasses] = {};
     // the fslength nodes with the panels in LDS: where every table fits and
     // there are enough nodes to give each CU some chunks of them
     g->fs_lds = 0;
@@ -2482,7 +2432,6 @@ void group_plan(kn_group *g)
         d.out = g->out + q.off_k;
         d.ivl = g->ivl + (size_t)q.off_k * kLimit * 2;
         d.dbar = g->dbar + q.off_y;
-        d.cbar = g->cbar + q.off_y;
         d.mubar = g->mubar + q.off_mu;
         d.ibar = g->ibar + q.off_k;
         d.mbic = g->mbic + q.off_k;
@@ -2528,16 +2477,7 @@ void group_plan(kn_group *g)
             cnt[kPhRows] = rows_prep_blocks(rows_prep_spline_blocks(np, d.nk), 4 * np);
             cnt[kPhFsSpline] = spline_blocks(16 * np, 1);
             cnt[kPhQag] = blocks_for(d.nk);
-            cnt[kPhSolve] = np > 2 ? spline_blocks(np, d.nk) : 0;
-            // part length: adj_plen is not monotone in the step count (1024 at
-            // 1024 knots, 513 at 1025), so the capacity plan takes the longest
-            // part any count up to na_max has, min(na_max, kAdjPartKnots)
-            const int nl = g->cap_plan ? (np < kAdjPartKnots ? np : kAdjPartKnots) : np;
-            int c = 0;
-            while (c < kAdjClasses - 1 && adj_plen(nl) > (128 << c)) c++;
-            cnt[kPhAdj0 + c] = (long long)d.nk * adj_parts(np) + (d.nk + 63) / 64;
-            const size_t b = adj_lds_bytes(nl);
-            lds[c] = b > lds[c] ? b : lds[c];
+            cnt[kPhAdj] = (long long)d.nk * fac_windows(np) + (d.nk + 63) / 64;
         }
         if (p_ic) cnt[kPhIc] = (d.nk + 63) / 64;
         for (int p = 0; p < kPhases; p++) {
@@ -2553,7 +2493,6 @@ void group_plan(kn_group *g)
         if ((g->cap_plan || g->h[i].integ) && np <= kStageMax && sizeof(double) * np > g->qag_lds)
             g->qag_lds = sizeof(double) * np;
     }
-    for (int c = 0; c < kAdjClasses; c++) g->adj_lds[c] = lds[c];
     KN_CHECK(hipMemcpy(g->desc, g->desc_h.data(), sizeof(GroupDesc) * n, hipMemcpyHostToDevice));
     KN_CHECK(hipMemcpy(g->pre, pre.data(), sizeof(int) * pre.size(), hipMemcpyHostToDevice));
     group_meta_upload(g);
@@ -2661,16 +2600,11 @@ void group_adjoint_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
     A.gbar = d.gbar;
     A.prefac = q.spec.delta_nu_prefac;
     A.ybar = dbar;  // rows written whole: [0, na) the item's terms, [na, na_max) zeros
-    A.cbar = d.cbar;
     A.mu_bar = d.mubar;
-    A.nparts = adj_parts(na);
-    A.plen = adj_plen(na);
+    A.fac = d.fac;
     A.ica = ica;
-    // nk x parts item blocks, then the initial-condition piece's blocks
-    hipLaunchKernelGGL(k_dnu_adj, dim3(nk * A.nparts + (nk + 63) / 64), dim3(64), adj_lds_bytes(na), s, A);
-    if (na > 2)
-        hipLaunchKernelGGL(k_adj_solve, dim3(spline_blocks(na, nk)), dim3(256), 0, s, d.sx, na, nk, (long long)na_max,
-                           d.cbar, dbar, d.fac);
+    // nk x windows item blocks, then the initial-condition piece's blocks
+    hipLaunchKernelGGL(k_dnu_adj, dim3(nk * fac_windows(na) + (nk + 63) / 64), dim3(64), 0, s, A);
 }
 
 // The whole group in one grid per phase, on stream s.
@@ -2701,12 +2635,8 @@ void group_launch_merged(kn_group *g, hipStream_t s, bool forward, bool adjoint)
         if (g->tot[kPhIc]) hipLaunchKernelGGL(k_m_ic, dim3(g->tot[kPhIc]), dim3(64), 0, s, g->desc, pre(kPhIc), n);
     }
     if (adjoint) {
-        for (int c = 0; c < kAdjClasses; c++)
-            if (g->tot[kPhAdj0 + c])
-                hipLaunchKernelGGL(k_m_dnu_adj, dim3(g->tot[kPhAdj0 + c]), dim3(64), g->adj_lds[c], s, g->desc,
-                                   pre(kPhAdj0 + c), n);
-        if (g->tot[kPhSolve])
-            hipLaunchKernelGGL(k_m_adj_solve, dim3(g->tot[kPhSolve]), dim3(256), 0, s, g->desc, pre(kPhSolve), n);
+        if (g->tot[kPhAdj])
+            hipLaunchKernelGGL(k_m_dnu_adj, dim3(g->tot[kPhAdj]), dim3(64), 0, s, g->desc, pre(kPhAdj), n);
         if (g->tot[kPhIc])
             hipLaunchKernelGGL(k_m_ic_adj, dim3(g->tot[kPhIc]), dim3(64), 0, s, g->desc, pre(kPhIc), n);
     }
@@ -2828,7 +2758,7 @@ extern "C" void kn_group_destroy(kn_group *g)
         KN_CHECK(hipGraphExecDestroy(g->exec));
         KN_CHECK(hipGraphDestroy(g->graph));
     }
-    void *ptrs[] = {g->sx,   g->Y,    g->C,      g->dbar, g->cbar,   g->fx,     g->fy,    g->fc,
+    void *ptrs[] = {g->sx,   g->Y,    g->C,      g->dbar, g->fx,     g->fy,    g->fc,
                     g->wavenum, g->init, g->out,  g->gbar,   g->ibar, g->mbic,   g->mubar,  g->mbar,  g->ivl,
                     g->bucket, g->nint, g->status, g->zeros, g->spec0, g->sp,    g->fs_list, g->meta, g->desc,
                     g->pre,  g->mlist, g->fac,  g->step_fsl, g->step_err, g->step_sticky};
@@ -2875,7 +2805,7 @@ extern "C" int kn_group_create(kn_group **out, int nhist, const kn_batch_history
         q.off_fac = g->fac_tot;
         g->fac_tot += (long long)fac_doubles(q.spec.na_max);
         q.off_mu = g->mu_tot;
-        g->mu_tot += (long long)q.spec.nk * adj_parts(q.spec.na_max);
+        g->mu_tot += (long long)q.spec.nk * fac_windows(q.spec.na_max);
         g->nk_tot += q.spec.nk;
         g->y_tot += (long long)q.spec.nk * q.spec.na_max;
         g->s_tot += q.spec.na_max;
@@ -2928,11 +2858,11 @@ extern "C" int kn_group_create(kn_group **out, int nhist, const kn_batch_history
     }
     const size_t ny = (size_t)g->y_tot, nk = (size_t)g->nk_tot;
     g->sx = group_alloc<double>(g->s_tot);
-    for (double **p : {&g->Y, &g->C, &g->dbar, &g->cbar}) *p = group_alloc<double>(ny);
+    for (double **p : {&g->Y, &g->C, &g->dbar}) *p = group_alloc<double>(ny);
     for (double **p : {&g->fx, &g->fy, &g->fc}) *p = group_alloc<double>(g->fs_tot);
     for (double **p : {&g->wavenum, &g->init, &g->out, &g->gbar, &g->ibar, &g->mbic})
         *p = group_alloc<double>(nk);
-    g->mubar = group_alloc<double>(g->mu_tot);  // [k][part] per history
+    g->mubar = group_alloc<double>(g->mu_tot);  // [k][window] per history
     g->mbar = group_alloc<double>(nhist);
     g->fac = group_alloc<double>(g->fac_tot);
     g->ivl = group_alloc<double>(nk * kLimit * 2);

@@ -1534,89 +1534,17 @@ __device__ int block_qag61(const F &f, double a, double b, double epsrel, int li
 // ---- natural cubic spline coefficients, windowed parallel solve ----
 // The interior system h_{i-1} c_{i-1} + 2(h_{i-1}+h_i) c_i + h_i c_{i+1} = g_i is
 // 2:1 diagonally dominant, so the influence of a row decays at least as
-// 0.268^distance.  A thread solves rows [lo-halo, hi+halo) with zero
+// 0.268^distance.  A window solves rows [lo-halo, hi+halo) with zero
 // boundary values at the window edges and keeps rows [lo, hi): the edge error
 // reaching the kept rows is below 0.268^48 ~ 1e-27 relative.
 constexpr int kHalo = 48;
-
-// Rows per batch of loads: a thread issues the loads of kSB rows at once
-// and then runs their (serial) elimination steps, so the window's memory
-// round trips are m / kSB instead of m.  Same arithmetic, step by step, as
-// the one-row-at-a-time loops.
-constexpr int kSB = 16;
-
-__device__ inline void spline_window(const double *x, const double *y, int n, int lo, int hi, double *c)
-{
-    // unknowns c[1..n-2]; c[0] = c[n-1] = 0
-    if (n < 3) {
-        for (int i = lo; i < hi; i++) c[i] = 0.0;
-        return;
-    }
-    int a = lo - kHalo, b = hi + kHalo;  // window of interior unknowns [a, b)
-    if (a < 1) a = 1;
-    if (b > n - 1) b = n - 1;
-    const int m = b - a;
-    // forward elimination (L D L^T of the window), then back substitution into c;
-    // the window is at most hi-lo+2*kHalo rows
-    double gam_prev = 0.0, z_prev = 0.0;
-    double gam[64 + 2 * kHalo + 2], zz[64 + 2 * kHalo + 2];
-    for (int r0 = 0; r0 < m; r0 += kSB) {
-        double xs[kSB + 2], ys[kSB + 2];  // x, y at rows a+r0-1 .. a+r0+kSB (only up to b is read)
-#pragma unroll
-        for (int j = 0; j < kSB + 2; j++) {
-            const int i = a + r0 - 1 + j;
-            xs[j] = i <= b ? x[i] : 0.0;
-            ys[j] = i <= b ? y[i] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r0 + j;  // unknown c[a+r], row couples c[i-1], c[i], c[i+1]
-            if (r < m) {
-                const double hl = xs[j + 1] - xs[j], hr = xs[j + 2] - xs[j + 1];
-                const double gl = hl != 0.0 ? 1.0 / hl : 0.0, gr = hr != 0.0 ? 1.0 / hr : 0.0;
-                const double diag = 2.0 * (hr + hl);
-                const double rhs = 3.0 * ((ys[j + 2] - ys[j + 1]) * gr - (ys[j + 1] - ys[j]) * gl);
-                const double alp = r == 0 ? diag : diag - hl * gam_prev;
-                const double g = hr / alp;
-                const double z = r == 0 ? rhs : rhs - gam_prev * z_prev;
-                gam[r] = g;
-                zz[r] = z / alp;
-                gam_prev = g;
-                z_prev = z;
-            }
-        }
-    }
-    double cnext = 0.0;
-    for (int r1 = m; r1 > 0; r1 -= kSB) {
-        double gs[kSB], zs[kSB];
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r1 - 1 - j;
-            gs[j] = r >= 0 ? gam[r] : 0.0;
-            zs[j] = r >= 0 ? zz[r] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r1 - 1 - j;
-            if (r >= 0) {
-                const double ci = zs[j] - (r == m - 1 ? 0.0 : gs[j] * cnext);
-                const int i = a + r;
-                if (i >= lo && i < hi) c[i] = ci;
-                cnext = ci;
-            }
-        }
-    }
-    if (lo == 0) c[0] = 0.0;
-    if (hi >= n) c[n - 1] = 0.0;
-    if (lo <= n - 1 && n - 1 < hi) c[n - 1] = 0.0;
-}
 
 // ---- natural-spline rows by wavefront scans -------------------------------
 // One wavefront solves a window of up to 64 kRun interior rows of
 // M c = rhs (rows i = 1..n-2, c_0 = c_{n-1} = 0), lane l taking kRun
 // consecutive rows in registers, and keeps the rows [lo, hi) that lie kHalo
-// rows or more inside the window (zero values are assumed just outside it,
-// as in spline_window).  M's L D L^T factors
+// rows or more inside the window (zero values are assumed just outside it).
+// M's L D L^T factors
 //   alp_i = 2(hl_i + hr_i) - hl_i gam_{i-1},  gam_i = hr_i / alp_i
 // are those of the elimination from row 1; the gam recurrence contracts by
 // at most (hl/alp)(hr/alp) <= 1/4 per row, so a lane that starts it kWarm
@@ -1639,11 +1567,6 @@ struct SplineRhs {
         const double gl = hl != 0.0 ? 1.0 / hl : 0.0, gr = hr != 0.0 ? 1.0 / hr : 0.0;
         return 3.0 * ((y[i + 1] - y[i]) * gr - (y[i] - y[i - 1]) * gl);
     }
-};
-
-struct ArrayRhs {
-    const double *r;
-    __device__ __forceinline__ double operator()(int i) const { return r[i]; }
 };
 
 // A lane's share of a window: rows [s, s + len) of the window's interior
@@ -1702,7 +1625,7 @@ __device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, do
 // ADJ_RHS: instead of storing the solution z, add its image under the
 // transpose of the natural-spline right-hand side's y-derivative onto out
 // (the second half of the spline adjoint) for the kept rows, with the
-// reciprocal knot spacings ih (as SplineRhsIh's).
+// reciprocal knot spacings ih.
 // OUT: where the kept rows go (set for the solution, add for ADJ_RHS); IH:
 // the reciprocal spacings.  Each kept row receives exactly one set or add.
 struct OutDirect {
@@ -1847,17 +1770,25 @@ __device__ inline void tridiag_window_wave(const double *x, int n, const RHS &rh
     tri_solve<RHS, false>(x, n, rhs, lo, hi, OutDirect{out}, t, g, al, gb, IhDirect{nullptr});
 }
 
+// The windows of rows that share their knots: one for up to 64 kRun interior
+// rows, else equal shares of at most kKeep kept rows (window w keeps
+// [w keep, (w + 1) keep)).
+__host__ __device__ inline int fac_windows(int n) { return n <= 64 * kRun + 2 ? 1 : (n + kKeep - 1) / kKeep; }
+__host__ __device__ inline int fac_keep(int n)
+{
+    const int w = fac_windows(n);
+    return (n + w - 1) / w;
+}
+
 // Factors of the knots x[0..n) stored once for every row that shares them:
 // window w at fac + w kFacStride, [j][lane] for gam, then 1 / alp, then
 // gam_{s-1} per lane (from the values tri_factor forms in each wavefront).
 constexpr int kFacStride = (2 * kRun + 1) * 64;
 
-__host__ __device__ inline int fac_windows(int n) { return (n + kKeep - 1) / kKeep; }
-
 __device__ inline void tri_factor_store(const double *x, int n, int w, double *fac)
 {
     const int lane = threadIdx.x & 63;
-    const int lo = w * kKeep, hi = lo + kKeep < n ? lo + kKeep : n;
+    const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
     const TriLane t = tri_lane(n, lo, hi);
     double g[kRun], al[kRun], gb;
     tri_factor(x, t, g, al, gb);
@@ -1905,7 +1836,7 @@ __device__ __forceinline__ void stage_span(double *dst, const double *__restrict
     }
 }
 
-// SplineRhsIh's values, bit for bit, from staged y and ih (ys[k] = y[base + k]).
+// SplineRhs's values, bit for bit, from staged y and ih (ys[k] = y[base + k]).
 struct SplineRhsLds {
     const double *ys, *ihs;
     int base;
@@ -1915,98 +1846,74 @@ struct SplineRhsLds {
         return 3.0 * ((ys[k + 1] - ys[k]) * ihs[k] - (ys[k] - ys[k - 1]) * ihs[k - 1]);
     }
 };
-struct ArrayRhsLds {
-    const double *rs;
-    int base;
-    __device__ __forceinline__ double operator()(int i) const { return rs[i - base]; }
-};
-struct OutLds {  // kept row i at o[i - lo]; add stores the row's one contribution
+struct OutLds {  // kept row i at o[i - lo]
     double *o;
     int lo;
     __device__ __forceinline__ void set(int i, double v) const { o[i - lo] = v; }
-    __device__ __forceinline__ void add(int i, double v) const { o[i - lo] = v; }
+    __device__ __forceinline__ void add(int i, double v) const { o[i - lo] += v; }
 };
 struct IhLds {
     const double *ihs;
     int base;
     __device__ __forceinline__ double operator()(int i) const { return ihs[i - base]; }
 };
+struct RunRhs {  // the lane's own rows, in registers
+    const double (&v)[kRun];
+    int s;
+    __device__ __forceinline__ double operator()(int i) const { return v[i - s]; }
+};
 
-// tridiag_window_wave for window w = lo / kKeep with the stored factors
+// The lane's stored factors of window w.
+__device__ __forceinline__ void tri_factor_load(const double *__restrict__ fac, int w, double (&g)[kRun],
+                                                double (&ial)[kRun], double &gb)
+{
+    const int lane = threadIdx.x & 63;
+    const double *f = fac + (size_t)w * kFacStride;
+#pragma unroll
+    for (int j = 0; j < kRun; j++) {
+        g[j] = f[j * 64 + lane];
+        ial[j] = f[(kRun + j) * 64 + lane];
+    }
+    gb = f[2 * kRun * 64 + lane];
+}
+
+// tridiag_window_wave for window w of a row on knots whose factors are stored
 // (fac_windows(n) windows, then the reciprocal spacings), the window staged
 // through the wavefront's LDS (lds: kTriLds doubles): lane l solves rows
 // s .. s + kRun - 1, kRun rows from its neighbours', so read from global
 // memory directly each load's 64 lanes would touch ~40 cache lines (and a
 // CU's wavefronts together more lines than its L1 holds); staged, the rows
 // come in and go out by loads and stores of consecutive doubles across the
-// lanes.  src: the y row (natural-spline coefficients set on out) or, with
-// ADJ_RHS, the right-hand side (its adjoint added onto out).
-template <bool ADJ_RHS>
-__device__ inline void tri_window_staged(const double *x, int n, const double *__restrict__ src, int lo, int hi,
+// lanes.  src: the y row; the natural-spline coefficients are set on out.
+__device__ inline void tri_window_staged(const double *x, int n, const double *__restrict__ src, int w,
                                          double *__restrict__ out, const double *__restrict__ fac, double *lds)
 {
     const int lane = threadIdx.x & 63;
+    const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
     if (n < 3) {
-        if (!ADJ_RHS)
-            for (int i = lo + lane; i < hi; i += 64) out[i] = 0.0;
+        for (int i = lo + lane; i < hi; i += 64) out[i] = 0.0;
         return;
     }
     const TriLane t = tri_lane(n, lo, hi);
-    const double *f = fac + (size_t)(lo / kKeep) * kFacStride;
     const double *ih = fac + (size_t)fac_windows(n) * kFacStride;
     double *sa = lds, *sb = lds + kTriSpan;
     const int base = t.wa - 1;
-    // ih[wa - 1 .. wb - 1]; y[wa - 1 .. wb] or rhs[wa .. wb - 1]
+    // ih[wa - 1 .. wb - 1]; y[wa - 1 .. wb]
     stage_span(sb, ih + base, t.wb - base);
-    if (ADJ_RHS) stage_span(sa, src + t.wa, t.wb - t.wa);
-    else stage_span(sa, src + base, t.wb - base + 1);
+    stage_span(sa, src + base, t.wb - base + 1);
     wave_lds_sync();
-    double g[kRun], ial[kRun];
-#pragma unroll
-    for (int j = 0; j < kRun; j++) {
-        g[j] = f[j * 64 + lane];
-        ial[j] = f[(kRun + j) * 64 + lane];
-    }
-    const double gb = f[2 * kRun * 64 + lane];
+    double g[kRun], ial[kRun], gb;
+    tri_factor_load(fac, w, g, ial, gb);
     const OutLds o{sa, lo};  // the staged rows are all read before the first kept row is written
-    if (ADJ_RHS)
-        tri_solve<ArrayRhsLds, true>(x, n, ArrayRhsLds{sa, t.wa}, lo, hi, o, t, g, ial, gb, IhLds{sb, base});
-    else
-        tri_solve<SplineRhsLds, false>(x, n, SplineRhsLds{sa, sb, base}, lo, hi, o, t, g, ial, gb,
-                                       IhLds{sb, base});
+    tri_solve<SplineRhsLds, false>(x, n, SplineRhsLds{sa, sb, base}, lo, hi, o, t, g, ial, gb, IhLds{sb, base});
     wave_lds_sync();
     const int cnt = hi - lo;
-    if (ADJ_RHS) {  // out += the staged contributions, every load issued first
-        double v[kTriPass];
 #pragma unroll
-        for (int p = 0; p < kTriPass; p++) {
-            const int k = p * 64 + lane;
-            v[p] = k < cnt ? out[lo + k] : 0.0;
-        }
-#pragma unroll
-        for (int p = 0; p < kTriPass; p++) {
-            const int k = p * 64 + lane;
-            if (k < cnt) out[lo + k] = v[p] + sa[k];
-        }
-    } else {
-#pragma unroll
-        for (int p = 0; p < kTriPass; p++) {
-            const int k = p * 64 + lane;
-            if (k < cnt) out[lo + k] = sa[k];
-        }
+    for (int p = 0; p < kTriPass; p++) {
+        const int k = p * 64 + lane;
+        if (k < cnt) out[lo + k] = sa[k];
     }
 }
-
-// Right-hand side of the natural-spline system with the reciprocal knot
-// spacings ih[i] = 1 / (x[i+1] - x[i]) (0 for a zero spacing) stored: the
-// values of SplineRhs, bit for bit.
-struct SplineRhsIh {
-    const double *ih, *y;
-    __device__ __forceinline__ double operator()(int i) const
-    {
-        return 3.0 * ((y[i + 1] - y[i]) * ih[i] - (y[i] - y[i - 1]) * ih[i - 1]);
-    }
-};
 
 // ---- derivatives for the adjoint ----------------------------------------
 
@@ -2071,77 +1978,15 @@ __device__ inline double specialJ_d(double x, const JPar &P, double &dJdx, doubl
 }
 
 // Weights of S(x) = y_i + dx (b + dx (c_i + dx d)) on y_i, y_{i+1}, c_i, c_{i+1}.
-__device__ __forceinline__ void cspline_grad(const double *xa, int i, double x, double &wy0, double &wy1, double &wc0,
+__device__ __forceinline__ void cspline_grad(double xl, double xr, double x, double &wy0, double &wy1, double &wc0,
                                              double &wc1)
 {
-    const double h = xa[i + 1] - xa[i], dx = x - xa[i], ih = rcp_fast(h);
+    const double h = xr - xl, dx = x - xl, ih = rcp_fast(h);
     const double t = dx * ih, dx3 = dx * dx * dx * ih * (1.0 / 3.0);
     wy0 = 1.0 - t;
     wy1 = t;
     wc0 = -dx * h * (2.0 / 3.0) + dx * dx - dx3;
     wc1 = -dx * h * (1.0 / 3.0) + dx3;
-}
-
-// Windowed solve of the natural-spline system M z = rhs (interior rows
-// 1..n-2, z[0] = z[n-1] = 0); same window scheme as spline_window.
-__device__ inline void tridiag_window(const double *x, const double *rhs, int n, int lo, int hi, double *z_out)
-{
-    if (n < 3) {
-        for (int i = lo; i < hi; i++) z_out[i] = 0.0;
-        return;
-    }
-    int a = lo - kHalo, b = hi + kHalo;
-    if (a < 1) a = 1;
-    if (b > n - 1) b = n - 1;
-    const int m = b - a;
-    double gam[64 + 2 * kHalo + 2], zz[64 + 2 * kHalo + 2];
-    double gam_prev = 0.0, z_prev = 0.0;
-    for (int r0 = 0; r0 < m; r0 += kSB) {
-        double xs[kSB + 2], rs[kSB];  // x at rows a+r0-1 .. a+r0+kSB (up to b), rhs at a+r0 .. a+r0+kSB-1
-#pragma unroll
-        for (int j = 0; j < kSB + 2; j++) {
-            const int i = a + r0 - 1 + j;
-            xs[j] = i <= b ? x[i] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kSB; j++) rs[j] = r0 + j < m ? rhs[a + r0 + j] : 0.0;
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r0 + j;
-            if (r < m) {
-                const double hl = xs[j + 1] - xs[j], hr = xs[j + 2] - xs[j + 1];
-                const double diag = 2.0 * (hr + hl);
-                const double alp = r == 0 ? diag : diag - hl * gam_prev;
-                const double zr = r == 0 ? rs[j] : rs[j] - gam_prev * z_prev;
-                gam[r] = hr / alp;
-                zz[r] = zr / alp;
-                gam_prev = gam[r];
-                z_prev = zr;
-            }
-        }
-    }
-    double next = 0.0;
-    for (int r1 = m; r1 > 0; r1 -= kSB) {
-        double gs[kSB], zs[kSB];
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r1 - 1 - j;
-            gs[j] = r >= 0 ? gam[r] : 0.0;
-            zs[j] = r >= 0 ? zz[r] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < kSB; j++) {
-            const int r = r1 - 1 - j;
-            if (r >= 0) {
-                const double v = zs[j] - (r == m - 1 ? 0.0 : gs[j] * next);
-                const int i = a + r;
-                if (i >= lo && i < hi) z_out[i] = v;
-                next = v;
-            }
-        }
-    }
-    if (lo == 0) z_out[0] = 0.0;
-    if (lo <= n - 1 && n - 1 < hi) z_out[n - 1] = 0.0;
 }
 
 }  // namespace kn_dnu

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import knhip
-from batch_common import Cosmo
+from batch_common import Cosmo, compare_adjoint
 from dnu_common import synthetic_history
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +57,30 @@ def test_fslength_nodes_by_group_size(kn, torch_cuda, steps):
         assert np.array_equal(x, y)
     for x in c:
         x.free()
+
+
+@pytest.mark.parametrize("na,noise", [(3, 0.0), (49, 0.1), (400, 0.1), (642, 0.03), (643, 0.03), (1088, 0.0), (1089, 0.0)])
+def test_adjoint_by_history_length(kn, torch_cuda, na, noise):
+    """The adjoint's windows: shorter than a window's halo, the longest single window, the shortest and longest pair, the
+    shortest triple, with a spare step (row stride na + 1); noise per entry makes up to 148 recorded intervals (rounds of
+    64, and fewer).  Against the oracle, and merged launches against streams."""
+    c = Cosmo([0.3, 0, 0])
+    logs, rows, k, init = synthetic_history(na, 3, 0.9, noise=noise)
+    h = c.history(3, na, na + 1, 0.9, 0.9, 0.3)
+    B = knhip.Batch([h], keep=c)
+    B.load(0, logs, rows, k, init)
+    g = np.array([0.3, -1.0, 0.7])
+    orc = c.oracle(3, logs, rows, init).get_delta_nu_adjoint(0.9, k, 0.3, g)
+    assert orc[0] == 0
+    out = []
+    for streams in (0, 4):
+        print("adjoint of %d steps, streams %d" % (na, streams), flush=True)
+        B.set_streams(streams)
+        B.solve()
+        B.adjoint(g)
+        out.append((B.delta_nu(0), B.dtot_bar(0, na), B.init_bar(0), B.mnu_bar()[0]))
+        compare_adjoint("Na=%d streams %d" % (na, streams), out[-1], orc)
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+    B.close()
+    c.free()
