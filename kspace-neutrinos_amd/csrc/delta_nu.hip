@@ -263,44 +263,53 @@ __device__ inline void bucket_at(const double *__restrict__ x, int n, double inv
 }
 
 // The delta_tot rows' splines (on the stored factors of the knots sx, see
-// factor_block) and the bucket index in one launch: blocks [0, b_sp) four
-// row windows each (none when na <= 2), the rest the bucket.  Rows of Y and
-// C are `ystride` doubles apart.
-// lds: kTriLds doubles per wavefront of the block
-__device__ inline void rows_prep_block(const double *__restrict__ sx, const double *__restrict__ Y,
+// factor_block) and the bucket index in one launch: blocks [0, b_sp) one
+// window of 4 rpw rows each (none when na <= 2), the rest the bucket.  Rows of
+// Y and C are `ystride` doubles apart.
+// lds: kTriSpan doubles per wavefront of the block and one more
+__device__ __forceinline__ void rows_prep_block(const double *__restrict__ sx, const double *__restrict__ Y,
                                        double *__restrict__ C, int na, int nk, long long ystride, int b_sp, int nsb,
                                        double sinv_bw, int *__restrict__ bucket, const double *__restrict__ fac,
-                                       int b, double *lds)
+                                       int rpw, int b, double *lds)
 {
-    if (b < b_sp) {
-        const int nwin = fac_windows(na);
-        const long long item = (long long)b * 4 + (threadIdx.x >> 6);
-        if (item < (long long)nwin * nk) {  // wave-uniform
-            const int r = (int)(item / nwin), w = (int)(item % nwin);
-            tri_window_staged(sx, na, Y + r * ystride, w, C + r * ystride, fac, lds + (threadIdx.x >> 6) * kTriLds);
-        }
+    if (b < b_sp) {  // window b % nwin of 4 rpw rows, every fourth by one wavefront
+        const int nwin = fac_windows(na), wave = threadIdx.x >> 6;
+        const int r0 = (int)(b / nwin) * 4 * rpw, rend = r0 + 4 * rpw < nk ? r0 + 4 * rpw : nk;
+        tri_rows_staged(na, b % nwin, Y, C, ystride, r0 + wave, 4, rend, fac, lds + (1 + wave) * kTriSpan, lds);
         return;
     }
     const int q = (b - b_sp) * 256 + threadIdx.x;
     if (q <= nsb) bucket_at(sx, na, sinv_bw, bucket, q);
 }
 
-// three wavefronts per SIMD (168 registers, a 20-byte spill): 0.91 ms against
-// 1.06 ms at two for the 256-history group's rows
-__global__ __launch_bounds__(256, 3) void k_rows_prep(const double *__restrict__ sx, const double *__restrict__ Y,
+// Bound by memory: 256 histories of 64-512 k x 100-3000 steps, 1.83 GB read and
+// written, take 385 us (4.75 TB/s) with four wavefronts per SIMD (128
+// registers), 402 with three; a row at a time, with the factors read for each,
+// took 750.
+__global__ __launch_bounds__(256, 4) void k_rows_prep(const double *__restrict__ sx, const double *__restrict__ Y,
                                                    double *__restrict__ C, int na, int nk, long long ystride,
                                                    int b_sp, int nsb, double sinv_bw, int *__restrict__ bucket,
-                                                   const double *__restrict__ fac)
+                                                   const double *__restrict__ fac, int rpw)
 {
-    __shared__ double lds[4 * kTriLds];
-    rows_prep_block(sx, Y, C, na, nk, ystride, b_sp, nsb, sinv_bw, bucket, fac, blockIdx.x, lds);
+    __shared__ double lds[5 * kTriSpan];
+    rows_prep_block(sx, Y, C, na, nk, ystride, b_sp, nsb, sinv_bw, bucket, fac, rpw, blockIdx.x, lds);
 }
 
 inline int rows_prep_blocks(int b_sp, int nsb) { return b_sp + (nsb + 256) / 256; }
 
-__host__ __device__ inline int rows_prep_spline_blocks(int na, int nk)
+__host__ __device__ inline int rows_prep_spline_blocks(int na, int nk, int rpw)
 {
-    return na > 2 ? (int)(((long long)fac_windows(na) * nk + 3) / 4) : 0;
+    return na > 2 ? fac_windows(na) * ((nk + 4 * rpw - 1) / (4 * rpw)) : 0;
+}
+
+// Rows per wavefront, for launches of that many (row, window) items: more pay
+// the factors' loads and scan products once (the 243k items of 256 histories:
+// 2 rows 495 us, 4 427, 8 402, 16 414, 32 438) as long as each of the chip's
+// 4096 wavefronts still gets one or two.
+inline int rows_per_wave(long long items)
+{
+    const long long r = items / 8192;
+    return r < 1 ? 1 : (r > 8 ? 8 : (int)r);
 }
 
 struct SpeciesDev {
@@ -554,10 +563,10 @@ struct AdjLds {
 // weights stay in LDS from the points to the finished row.  (The points in
 // parts of up to 1024 knots, their weights through memory to a solve of their
 // own, took 1131 + 1157 us for 256 histories of 64-512 k x 100-3000 steps;
-// this takes 1339: 284 in the solve, 740 in the points' FP64, the rest in
+// this took 1339: 284 in the solve, 740 in the points' FP64, the rest in
 // gathering them and in the rows' one write.  Three waves per SIMD: with the
 // compiler's own choice of registers, which lets two run, 1411; with four,
-// which spill more, 1412.)
+// which spill more, 1412.  With the scans' three steps, 1304.)
 // Points that reach the window (x within [sx[E0 - 1], sx[E1]]) are queued and
 // evaluated 64 at a time, one per lane; a point's d/d(m/kT) term belongs to
 // the window that keeps its si, so every term is counted once.
@@ -700,7 +709,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
         for (int p = 0; p < kTriPass; p++)
             if (p * 64 + lane < cnt) S.c[p * 64 + lane] = vi[p];
         wave_lds_sync();
-        tri_solve<RunRhs, true>(sx, ns, RunRhs{rv, t.s}, lo, hi, OutLds{S.y, lo}, t, g, ial, before,
+        tri_solve<RunRhs, true>(ns, RunRhs{rv, t.s}, lo, hi, OutLds{S.y, lo}, t, g, ial, before, tri_scan(g, before),
                                 IhLds{S.c, base});
         wave_lds_sync();
     }
@@ -1611,11 +1620,11 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
 
     const double sinv_bw = nsb / (d->scalefact[Na - 1] - d->scalefact[0]);
     {
-        const int bsp = rows_prep_spline_blocks(Na, nk);
+        const int rpw = rows_per_wave((long long)fac_windows(Na) * nk), bsp = rows_prep_spline_blocks(Na, nk, rpw);
         hipLaunchKernelGGL(k_factor, dim3(factor_blocks(Na)), dim3(256), 0, 0, dev->sx, Na, dev->fac,
                            dev->fac + (size_t)fac_windows(Na) * kFacStride);
         hipLaunchKernelGGL(k_rows_prep, dim3(rows_prep_blocks(bsp, nsb)), dim3(256), 0, 0, dev->sx, dev->Y, dev->C, Na,
-                           nk, (long long)namax, bsp, nsb, sinv_bw, dev->bucket, dev->fac);
+                           nk, (long long)namax, bsp, nsb, sinv_bw, dev->bucket, dev->fac, rpw);
     }
     QagArgs qa;
     qa.H = H;
@@ -1902,7 +1911,7 @@ struct GroupDesc {
     const SpeciesDev *sp;
     // the stored steps and what they set: live in device memory (the device
     // append updates them), read by every launch
-    int nk, na, na_max, nfs, nsb, bsp, integ, ic_only;
+    int nk, na, na_max, nfs, nsb, bsp, rpw, integ, ic_only;
     double x0, xa, a, light, sinv_bw, fsl0, lin, prefac, vcrit;
     // constants of the history that the device append derives from
     int hybrid;
@@ -2024,16 +2033,16 @@ __global__ __launch_bounds__(256) void k_m_factor(const GroupDesc *__restrict__ 
     factor_block(d.sx, d.na, d.fac, d.fac + (size_t)fac_windows(d.na) * kFacStride, blk - pre[h]);
 }
 
-__global__ __launch_bounds__(256, 3) void k_m_rows_prep(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
+__global__ __launch_bounds__(256, 4) void k_m_rows_prep(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
                                                      int nhist)
 {
     const int blk = xcd_block();
     const int h = hist_of(pre, nhist, blk);
     const GroupDesc &d = D[h];
     if (!d.integ) return;
-    __shared__ double lds[4 * kTriLds];
+    __shared__ double lds[5 * kTriSpan];
     rows_prep_block(d.sx, d.Y, d.C, d.na, d.nk, (long long)d.na_max, d.bsp, d.nsb, d.sinv_bw, d.bucket, d.fac,
-                    blk - pre[h], lds);
+                    d.rpw, blk - pre[h], lds);
 }
 
 __global__ __launch_bounds__(256) void k_m_fs_spline(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
@@ -2236,7 +2245,7 @@ __global__ __launch_bounds__(64) void k_group_step(GroupDesc *__restrict__ D, Sp
         d.na = n1;
         d.nfs = 16 * n1;
         d.nsb = 4 * n1;
-        d.bsp = rows_prep_spline_blocks(n1, nk);
+        d.bsp = rows_prep_spline_blocks(n1, nk, d.rpw);
         d.integ = integ;
         d.ic_only = ic_only;
         d.xa = la;
@@ -2402,12 +2411,15 @@ void group_plan(kn_group *g)
     // the fslength nodes with the panels in LDS: where every table fits and
     // there are enough nodes to give each CU some chunks of them
     g->fs_lds = 0;
+    long long items = 0;  // (row, window)
     {
         long long nodes = 0;
         for (int i = 0; i < n; i++) {
             const GroupHist &q = g->h[i];
             if (!(g->cap_plan || q.integ)) continue;
-            nodes += 16LL * (g->cap_plan ? q.spec.na_max : q.na);
+            const int np = g->cap_plan ? q.spec.na_max : q.na;
+            nodes += 16LL * np;
+            items += (long long)fac_windows(np) * q.spec.nk;
             const size_t b = sizeof(double) * kHnc * (size_t)g->htabs[q.htab].npanel;
             g->fs_lds = b > g->fs_lds ? b : g->fs_lds;
         }
@@ -2416,6 +2428,7 @@ void group_plan(kn_group *g)
             KN_CHECK(hipFuncSetAttribute((const void *)k_m_fs_first_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)g->fs_lds));
     }
+    const int rpw = rows_per_wave(items);
     for (int i = 0; i < n; i++) {
         const GroupHist &q = g->h[i];
         GroupDesc &d = g->desc_h[i];
@@ -2445,7 +2458,8 @@ void group_plan(kn_group *g)
         d.na_max = q.spec.na_max;
         d.nfs = 16 * q.na;
         d.nsb = 4 * q.na;
-        d.bsp = rows_prep_spline_blocks(q.na, q.spec.nk);
+        d.rpw = rpw;
+        d.bsp = rows_prep_spline_blocks(q.na, q.spec.nk, rpw);
         d.integ = q.integ;
         d.ic_only = q.spec.ic_only;
         d.x0 = q.x0;
@@ -2474,7 +2488,7 @@ void group_plan(kn_group *g)
         if (p_integ) {
             cnt[kPhFs] = g->fs_lds ? (16LL * np + kFsChunk - 1) / kFsChunk : fs_first_blocks(16 * np);
             cnt[kPhFactor] = factor_blocks(np);
-            cnt[kPhRows] = rows_prep_blocks(rows_prep_spline_blocks(np, d.nk), 4 * np);
+            cnt[kPhRows] = rows_prep_blocks(rows_prep_spline_blocks(np, d.nk, rpw), 4 * np);
             cnt[kPhFsSpline] = spline_blocks(16 * np, 1);
             cnt[kPhQag] = blocks_for(d.nk);
             cnt[kPhAdj] = (long long)d.nk * fac_windows(np) + (d.nk + 63) / 64;
@@ -2525,7 +2539,7 @@ void group_forward_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
     hipLaunchKernelGGL(k_factor, dim3(factor_blocks(na)), dim3(256), 0, s, d.sx, na, d.fac,
                        d.fac + (size_t)fac_windows(na) * kFacStride);
     hipLaunchKernelGGL(k_rows_prep, dim3(rows_prep_blocks(d.bsp, d.nsb)), dim3(256), 0, s, d.sx, d.Y, d.C, na, nk,
-                       (long long)na_max, d.bsp, d.nsb, d.sinv_bw, d.bucket, d.fac);
+                       (long long)na_max, d.bsp, d.nsb, d.sinv_bw, d.bucket, d.fac, d.rpw);
     hipLaunchKernelGGL(k_spline, dim3(spline_blocks(nfs, 1)), dim3(256), 0, s, fx, fy, fc, nfs, 1, 0LL, 0LL);
     QagArgs a;
     a.H = d.H;

@@ -1588,9 +1588,10 @@ __device__ __forceinline__ TriLane tri_lane(int n, int lo, int hi)
     return t;
 }
 
-// The lane's factors gam (g) and alp (al) over its run, and gam_{s-1}; past
-// the run al = 1, g = 0.
-__device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, double (&g)[kRun], double (&al)[kRun],
+// The lane's factors gam (g) and 1 / alp (ial) over its run, and gam_{s-1} (0
+// before the window's first row); past the run both are 0, so that the solve
+// gives 0 there.
+__device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, double (&g)[kRun], double (&ial)[kRun],
                                            double &g_before)
 {
     const int s = t.s, wb = t.wb, len = t.len;
@@ -1603,25 +1604,57 @@ __device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, do
         const double alr = r == a ? diag : diag - hl * gp;
         gp = hr / alr;
     }
-    g_before = gp;
+    g_before = s == t.wa ? 0.0 : gp;
 #pragma unroll
     for (int j = 0; j < kRun; j++) {
         if (j < len) {
             const int i = s + j;
             const double hl = x[i] - x[i - 1], hr = x[i + 1] - x[i];
             const double diag = 2.0 * (hr + hl);
-            al[j] = i == a ? diag : diag - hl * gp;
-            g[j] = hr / al[j];
+            const double al = i == a ? diag : diag - hl * gp;
+            g[j] = hr / al;
+            ial[j] = 1.0 / al;
             gp = g[j];
         } else {
-            al[j] = 1.0;
-            g[j] = 0.0;
+            g[j] = ial[j] = 0.0;
         }
     }
 }
 
+// What the substitutions' scans over the lanes multiply by, from the factors
+// alone: a lane's run composes to z_out = A - f[0] z_in (A from the row's
+// values), and f[k] is the factor of the 2^k runs that end with the lane's;
+// b[k] likewise backwards.  Three levels reach 8 runs, 80 rows, and a row's
+// influence is below 0.268^80 ~ 1e-46 there (all six levels: the coefficient
+// rows of 256 histories took 754 us for 721).
+constexpr int kScan = 3;
+static_assert((kRun << kScan) >= kHalo, "the scans reach as far as a window's halo");
+struct TriScan {
+    double f[kScan], b[kScan];
+};
+
+__device__ __forceinline__ TriScan tri_scan(const double (&g)[kRun], double g_before)
+{
+    const int lane = threadIdx.x & 63;
+    TriScan S;
+    double f = -g_before, b = 1.0;
+#pragma unroll
+    for (int j = 1; j < kRun; j++) f = -g[j - 1] * f;
+#pragma unroll
+    for (int j = kRun - 1; j >= 0; j--) b = -g[j] * b;
+#pragma unroll
+    for (int k = 0; k < kScan; k++) {
+        S.f[k] = f;
+        S.b[k] = b;
+        const double fp = __shfl_up(f, 1 << k, 64), bn = __shfl_down(b, 1 << k, 64);
+        f = lane >= (1 << k) ? f * fp : f;
+        b = lane + (1 << k) < 64 ? b * bn : b;
+    }
+    return S;
+}
+
 // Called by all 64 lanes of a wavefront together, with hi - lo <= kKeep and
-// n >= 3, given the lane's factors gam and 1 / alp.
+// n >= 3, given the lane's factors and their scan products.
 // ADJ_RHS: instead of storing the solution z, add its image under the
 // transpose of the natural-spline right-hand side's y-derivative onto out
 // (the second half of the spline adjoint) for the kept rows, with the
@@ -1639,74 +1672,48 @@ struct IhDirect {
 };
 
 template <class RHS, bool ADJ_RHS, class OUT = OutDirect, class IH = IhDirect>
-__device__ __forceinline__ void tri_solve(const double *x, int n, const RHS &rhs, int lo, int hi, const OUT &out,
-                                          const TriLane &t, const double (&g)[kRun], const double (&ial)[kRun],
-                                          double g_before, const IH &ih)
+__device__ __forceinline__ void tri_solve(int n, const RHS &rhs, int lo, int hi, const OUT &out, const TriLane &t,
+                                          const double (&g)[kRun], const double (&ial)[kRun], double g_before,
+                                          const TriScan &S, const IH &ih)
 {
     const int lane = threadIdx.x & 63;
-    const int wa = t.wa, wb = t.wb, s = t.s, len = t.len;
+    const int wb = t.wb, s = t.s, len = t.len;
     double zz[kRun];
-    double rv[kRun];
 #pragma unroll
-    for (int j = 0; j < kRun; j++) rv[j] = j < len ? rhs(s + j) : 0.0;
+    for (int j = 0; j < kRun; j++) zz[j] = j < len ? rhs(s + j) : 0.0;
     // forward: z_i = rhs_i - gam_{i-1} z_{i-1}, z_{wa-1} = 0
-    double A = 0.0, B = 1.0;
+    double A = zz[0];
 #pragma unroll
-    for (int j = 0; j < kRun; j++) {
-        if (j < len) {
-            const double gm = s + j == wa ? 0.0 : (j == 0 ? g_before : g[j - 1]);
-            A = rv[j] - gm * A;
-            B = -gm * B;
-        }
-    }
+    for (int j = 1; j < kRun; j++) A = zz[j] - g[j - 1] * A;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Ap = __shfl_up(A, d, 64), Bp = __shfl_up(B, d, 64);
-        if (lane >= d) {
-            A = A + B * Ap;
-            B = B * Bp;
-        }
+    for (int k = 0; k < kScan; k++) {
+        const double Ap = __shfl_up(A, 1 << k, 64);
+        if (lane >= (1 << k)) A = A + S.f[k] * Ap;
     }
     double z = __shfl_up(A, 1, 64);
     if (lane == 0) z = 0.0;
 #pragma unroll
     for (int j = 0; j < kRun; j++) {
-        if (j < len) {
-            const double gm = s + j == wa ? 0.0 : (j == 0 ? g_before : g[j - 1]);
-            z = rv[j] - gm * z;
-            zz[j] = z * ial[j];
-        } else {
-            zz[j] = 0.0;
-        }
+        z = zz[j] - (j == 0 ? g_before : g[j - 1]) * z;
+        zz[j] = z * ial[j];
     }
     // back: c_i = zz_i - gam_i c_{i+1}, c_{wb} = 0
     A = 0.0;
-    B = 1.0;
 #pragma unroll
-    for (int j = kRun - 1; j >= 0; j--) {
-        if (j < len) {
-            A = zz[j] - g[j] * A;
-            B = -g[j] * B;
-        }
-    }
+    for (int j = kRun - 1; j >= 0; j--) A = zz[j] - g[j] * A;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double An = __shfl_down(A, d, 64), Bn = __shfl_down(B, d, 64);
-        if (lane + d < 64) {
-            A = A + B * An;
-            B = B * Bn;
-        }
+    for (int k = 0; k < kScan; k++) {
+        const double An = __shfl_down(A, 1 << k, 64);
+        if (lane + (1 << k) < 64) A = A + S.b[k] * An;
     }
     double c = __shfl_down(A, 1, 64);
     if (lane == 63) c = 0.0;
     if (!ADJ_RHS) {
 #pragma unroll
         for (int j = kRun - 1; j >= 0; j--) {
-            if (j < len) {
-                const int i = s + j;
-                c = zz[j] - g[j] * c;
-                if (i >= lo && i < hi) out.set(i, c);
-            }
+            const int i = s + j;
+            c = zz[j] - g[j] * c;
+            if (j < len && i >= lo && i < hi) out.set(i, c);
         }
         if (lane == 0) {
             if (lo == 0) out.set(0, 0.0);
@@ -1718,14 +1725,7 @@ __device__ __forceinline__ void tri_solve(const double *x, int n, const RHS &rhs
     // rhs_i = 3 ((y_{i+1} - y_i) / h_i - (y_i - y_{i-1}) / h_{i-1}) and z_0 = z_{n-1} = 0
     double zv[kRun];
 #pragma unroll
-    for (int j = kRun - 1; j >= 0; j--) {
-        if (j < len) {
-            c = zz[j] - g[j] * c;
-            zv[j] = c;
-        } else {
-            zv[j] = 0.0;
-        }
-    }
+    for (int j = kRun - 1; j >= 0; j--) zv[j] = c = zz[j] - g[j] * c;
     // z just before and after this lane's run (0 at the natural ends; a
     // window's inner ends are never next to a kept row)
     double zp = __shfl_up(zv[kRun - 1], 1, 64), zn = __shfl_down(zv[0], 1, 64);
@@ -1755,7 +1755,7 @@ __device__ __forceinline__ void tri_solve(const double *x, int n, const RHS &rhs
 // One window [lo, hi) of natural-spline rows by one wavefront (factors
 // formed in place).
 template <class RHS>
-__device__ inline void tridiag_window_wave(const double *x, int n, const RHS &rhs, int lo, int hi, double *out)
+__device__ __forceinline__ void tridiag_window_wave(const double *x, int n, const RHS &rhs, int lo, int hi, double *out)
 {
     const int lane = threadIdx.x & 63;
     if (n < 3) {
@@ -1763,11 +1763,9 @@ __device__ inline void tridiag_window_wave(const double *x, int n, const RHS &rh
         return;
     }
     const TriLane t = tri_lane(n, lo, hi);
-    double g[kRun], al[kRun], gb;
-    tri_factor(x, t, g, al, gb);
-#pragma unroll
-    for (int j = 0; j < kRun; j++) al[j] = 1.0 / al[j];
-    tri_solve<RHS, false>(x, n, rhs, lo, hi, OutDirect{out}, t, g, al, gb, IhDirect{nullptr});
+    double g[kRun], ial[kRun], gb;
+    tri_factor(x, t, g, ial, gb);
+    tri_solve<RHS, false>(n, rhs, lo, hi, OutDirect{out}, t, g, ial, gb, tri_scan(g, gb), IhDirect{nullptr});
 }
 
 // The windows of rows that share their knots: one for up to 64 kRun interior
@@ -1790,21 +1788,19 @@ __device__ inline void tri_factor_store(const double *x, int n, int w, double *f
     const int lane = threadIdx.x & 63;
     const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
     const TriLane t = tri_lane(n, lo, hi);
-    double g[kRun], al[kRun], gb;
-    tri_factor(x, t, g, al, gb);
+    double g[kRun], ial[kRun], gb;
+    tri_factor(x, t, g, ial, gb);
     double *f = fac + (size_t)w * kFacStride;
 #pragma unroll
     for (int j = 0; j < kRun; j++) {
         f[j * 64 + lane] = g[j];
-        f[(kRun + j) * 64 + lane] = 1.0 / al[j];
+        f[(kRun + j) * 64 + lane] = ial[j];
     }
     f[2 * kRun * 64 + lane] = gb;
 }
 
-// A window's rows staged in LDS: the span [wa - 1, wb] of a window and its
-// two neighbours, twice (kTriLds doubles per wavefront).
+// The span of a window in LDS: its rows and their two neighbours.
 constexpr int kTriSpan = 64 * kRun + 2;
-constexpr int kTriLds = 2 * kTriSpan;
 constexpr int kTriPass = (kTriSpan + 63) / 64;  // 64-wide passes over a span
 
 // A wavefront's LDS writes ordered before its lanes' reads of them (LDS
@@ -1817,18 +1813,21 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// dst[k] = src[k] for k < cnt (cnt <= kTriSpan) by the 64 lanes: every load
-// issued before the first LDS store, so that the passes' loads are in flight
-// together.
-__device__ __forceinline__ void stage_span(double *dst, const double *__restrict__ src, int cnt)
+// v = src[0 .. cnt), cnt <= kTriSpan, spread over the 64 lanes: every load
+// issued at once.
+__device__ __forceinline__ void load_span(double (&v)[kTriPass], const double *__restrict__ src, int cnt)
 {
     const int lane = threadIdx.x & 63;
-    double v[kTriPass];
 #pragma unroll
     for (int p = 0; p < kTriPass; p++) {
         const int k = p * 64 + lane;
         v[p] = k < cnt ? src[k] : 0.0;
     }
+}
+
+__device__ __forceinline__ void store_span(double *dst, const double (&v)[kTriPass], int cnt)
+{
+    const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int p = 0; p < kTriPass; p++) {
         const int k = p * 64 + lane;
@@ -1877,41 +1876,47 @@ __device__ __forceinline__ void tri_factor_load(const double *__restrict__ fac, 
     gb = f[2 * kRun * 64 + lane];
 }
 
-// tridiag_window_wave for window w of a row on knots whose factors are stored
-// (fac_windows(n) windows, then the reciprocal spacings), the window staged
-// through the wavefront's LDS (lds: kTriLds doubles): lane l solves rows
-// s .. s + kRun - 1, kRun rows from its neighbours', so read from global
-// memory directly each load's 64 lanes would touch ~40 cache lines (and a
-// CU's wavefronts together more lines than its L1 holds); staged, the rows
-// come in and go out by loads and stores of consecutive doubles across the
-// lanes.  src: the y row; the natural-spline coefficients are set on out.
-__device__ inline void tri_window_staged(const double *x, int n, const double *__restrict__ src, int w,
-                                         double *__restrict__ out, const double *__restrict__ fac, double *lds)
+// tridiag_window_wave for window w of a wavefront's rows r0, r0 + step, ... <
+// rend, on knots whose factors are stored (fac_windows(n) windows, then the
+// reciprocal spacings): the coefficients of row Y + r ystride go to C + r
+// ystride.  The window is staged through LDS (sa: kTriSpan doubles of the
+// wavefront's own; sb: the reciprocal spacings, the same for the block's
+// wavefronts, which come here together): lane l solves rows s .. s + kRun - 1,
+// kRun rows from its neighbours', so read from global memory directly each
+// load's 64 lanes would touch ~40 cache lines (and a CU's wavefronts together
+// more lines than its L1 holds); staged, the rows come in and go out by loads
+// and stores of consecutive doubles across the lanes.  The factors and scan
+// products stay in registers from row to row (they are five times a row's own
+// bytes), and the next row is on its way while one is solved.
+__device__ __forceinline__ void tri_rows_staged(int n, int w, const double *__restrict__ Y, double *__restrict__ C,
+                                       long long ystride, int r0, int step, int rend, const double *__restrict__ fac,
+                                       double *sa, double *sb)
 {
     const int lane = threadIdx.x & 63;
     const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
-    if (n < 3) {
-        for (int i = lo + lane; i < hi; i += 64) out[i] = 0.0;
-        return;
-    }
     const TriLane t = tri_lane(n, lo, hi);
     const double *ih = fac + (size_t)fac_windows(n) * kFacStride;
-    double *sa = lds, *sb = lds + kTriSpan;
-    const int base = t.wa - 1;
-    // ih[wa - 1 .. wb - 1]; y[wa - 1 .. wb]
-    stage_span(sb, ih + base, t.wb - base);
-    stage_span(sa, src + base, t.wb - base + 1);
-    wave_lds_sync();
-    double g[kRun], ial[kRun], gb;
+    const int base = t.wa - 1, cnt = t.wb - base + 1;  // y[wa - 1 .. wb]
+    double v[kTriPass], g[kRun], ial[kRun], gb;
+    if (r0 < rend) load_span(v, Y + r0 * ystride + base, cnt);
     tri_factor_load(fac, w, g, ial, gb);
-    const OutLds o{sa, lo};  // the staged rows are all read before the first kept row is written
-    tri_solve<SplineRhsLds, false>(x, n, SplineRhsLds{sa, sb, base}, lo, hi, o, t, g, ial, gb, IhLds{sb, base});
-    wave_lds_sync();
-    const int cnt = hi - lo;
+    for (int k = threadIdx.x; k < cnt - 1; k += blockDim.x) sb[k] = ih[base + k];  // ih[wa - 1 .. wb - 1]
+    const TriScan S = tri_scan(g, gb);
+    __syncthreads();
+    for (int r = r0; r < rend; r += step) {
+        store_span(sa, v, cnt);
+        wave_lds_sync();
+        if (r + step < rend) load_span(v, Y + (r + step) * ystride + base, cnt);
+        const OutLds o{sa, lo};  // the staged row is all read before the first kept row is written
+        tri_solve<SplineRhsLds, false>(n, SplineRhsLds{sa, sb, base}, lo, hi, o, t, g, ial, gb, S, IhLds{sb, base});
+        wave_lds_sync();
+        double *out = C + r * ystride + lo;
 #pragma unroll
-    for (int p = 0; p < kTriPass; p++) {
-        const int k = p * 64 + lane;
-        if (k < cnt) out[lo + k] = sa[k];
+        for (int p = 0; p < kTriPass; p++) {
+            const int k = p * 64 + lane;
+            if (k < hi - lo) out[k] = sa[k];
+        }
+        wave_lds_sync();
     }
 }
 

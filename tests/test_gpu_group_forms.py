@@ -84,3 +84,36 @@ def test_adjoint_by_history_length(kn, torch_cuda, na, noise):
         assert np.array_equal(x, y)
     B.close()
     c.free()
+
+
+@pytest.mark.parametrize("rows", [20000, 70000])
+def test_rows_per_wavefront(kn, torch_cuda, rows):
+    """Histories whose k counts end inside a wavefront's share of rows, of one, two and three windows, in a group with so
+    many rows (a history of 3 steps) that wavefronts take 2 and 8 each: equal bit for bit to the same history alone in its
+    group, one row per wavefront.  (Noise per entry at 643 and more steps: the oracle's QAG fails too.)"""
+    c = Cosmo([0.3, 0, 0])
+    hists, data = [], []
+    for i, (nk, na) in enumerate([(1, 642), (7, 3), (8, 643), (31, 60), (33, 1089), (65, 1500), (rows, 3)]):
+        logs, r, k, init = synthetic_history(na, nk, 0.6, seed=i, noise=0.01 if na < 100 else 0.0)
+        hists.append(c.history(nk, na, na + i % 2, 0.6, 0.6, 0.3))
+        data.append((logs, r, k, init))
+    g = np.random.default_rng(2).uniform(-1, 1, sum(h.nk for h in hists))
+
+    def run(sel):
+        B = knhip.Batch([hists[i] for i in sel], keep=c)
+        for j, i in enumerate(sel):
+            B.load(j, *data[i])
+        print("%d rows in %d histories" % (B.off_k[B.n], B.n), flush=True)
+        B.solve()
+        off = sum(h.nk for h in hists[:sel[0]])
+        B.adjoint(g[off:off + B.off_k[B.n]])
+        out = [[B.delta_nu(j), B.dtot_bar(j, len(data[i][0])), B.init_bar(j), B.mnu_bar()[j]] for j, i in enumerate(sel)]
+        B.close()
+        return out
+
+    whole = run(list(range(len(hists))))
+    assert all(np.all(np.isfinite(x)) for o in whole for x in o)
+    for i in range(len(hists) - 1):
+        for x, y in zip(whole[i], run([i])[0]):
+            assert np.array_equal(x, y)
+    c.free()
