@@ -354,8 +354,7 @@ struct QagArgs {
 };
 
 // Histories of at most this many stored steps have their log a values copied
-// to LDS by the QAG kernels (48 KB; a block's four wavefronts share the copy,
-// which every wavefront writes whole before it reads, so no block barrier).
+// to LDS by the QAG kernels (48 KB, one copy for the block's four wavefronts).
 constexpr int kStageMax = 6144;
 
 // Item `item` (species sp, wavenumber k) by one wavefront; sxs: LDS for the
@@ -371,6 +370,7 @@ __device__ inline DnuIntegrand dnu_integrand(const QagArgs &a, const SpeciesDev 
     f.fk.x0 = a.x0;  // the fslength knots' own expression (fs_first_tile)
     f.fk.span = a.xa - a.x0;
     f.fk.den = a.nfs - 1.;
+    f.fk.rden = 1.0 / f.fk.den;
     f.nfs = a.nfs;
     f.fx0 = a.fx[0];
     f.fxhi = a.fx[a.nfs - 1];
@@ -410,16 +410,25 @@ __device__ inline void dnu_qag_store(const QagArgs &a, const SpeciesDev &sp, int
     }
 }
 
+// The stored log a values to LDS by the block's `threads` threads, eight loads
+// of each in flight; every thread of the block comes here.
+__device__ __forceinline__ void stage_knots(const double *__restrict__ sx, int ns, double *sxs, int threads)
+{
+    for (int t0 = threadIdx.x; t0 < ns; t0 += 8 * threads) {
+        double v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = t0 + j * threads < ns ? sx[t0 + j * threads] : 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (t0 + j * threads < ns) sxs[t0 + j * threads] = v[j];
+    }
+    __syncthreads();
+}
+
 __device__ inline void dnu_qag_item(const QagArgs &a, const SpeciesDev &sp, int item, int k, QagWs &ws,
-                                    double *sxs)
+                                    const double *sx)
 {
     const int lane = threadIdx.x & 63;
-    const double *sx = a.sx;
-    if (sxs) {
-        for (int t = lane; t < a.ns; t += 64) sxs[t] = a.sx[t];
-        __builtin_amdgcn_wave_barrier();  // every lane's entries written before any lane reads
-        sx = sxs;
-    }
     const DnuIntegrand f = dnu_integrand(a, sp, k, sx);
     double r;
     int ni;
@@ -435,8 +444,7 @@ __device__ inline void dnu_qag_item_block(const QagArgs &a, const SpeciesDev &sp
 {
     const double *sx = a.sx;
     if (sxs) {
-        for (int t = threadIdx.x; t < a.ns; t += 64 * W) sxs[t] = a.sx[t];
-        __syncthreads();
+        stage_knots(a.sx, a.ns, sxs, 64 * W);
         sx = sxs;
     }
     const DnuIntegrand f = dnu_integrand(a, sp, k, sx);
@@ -485,9 +493,10 @@ __global__ __launch_bounds__(64 * kQagSpec) void k_dnu_qag_mix(QagArgs a, const 
         return;
     }
     const int wave = threadIdx.x >> 6, j = nlong + (b - nlong) * kQagSpec + wave;
+    if (st) stage_knots(a.sx, a.ns, st, 64 * kQagSpec);
     if (j >= nitems) return;
     const int item = order[j];
-    dnu_qag_item(a, sp[item_species[item / nk]], item, item % nk, U.ws[wave], st);
+    dnu_qag_item(a, sp[item_species[item / nk]], item, item % nk, U.ws[wave], st ? st : a.sx);
 }
 
 // Interval counts at or above which an item is expected to gain from the
@@ -595,6 +604,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
     fk.x0 = A.x0;
     fk.span = A.xa - A.x0;
     fk.den = nfs - 1.;
+    fk.rden = 1.0 / fk.den;
 #pragma unroll
     for (int p = 0; p < kTriPass; p++) {
         const int t = p * 64 + lane;
@@ -2066,7 +2076,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDe
     const GroupDesc &d = D[h];
     const int wave = threadIdx.x >> 6;
     const int k = (blk - pre[h]) * kWavesPerBlock + wave;
-    if (!d.integ || k >= d.nk) return;
+    if (!d.integ) return;
+    const bool staged = d.na <= kStageMax;
+    if (staged) stage_knots(d.sx, d.na, sxs, 64 * kWavesPerBlock);
+    if (k >= d.nk) return;
     QagArgs a;
     a.H = d.H;
     a.fx = d.fx;
@@ -2092,7 +2105,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDe
     a.ic.fsl0 = d.fsl0;
     a.ic.lin = d.lin;
     a.ic.prefac = d.prefac;
-    dnu_qag_item(a, *d.sp, k, k, ws[wave], d.na <= kStageMax ? sxs : nullptr);
+    dnu_qag_item(a, *d.sp, k, k, ws[wave], staged ? sxs : d.sx);
 }
 
 // initial-condition-only histories, 64 k per block

@@ -651,9 +651,16 @@ __device__ __forceinline__ double linear_at(const double *xa, const double *ya, 
 // The fslength table's knots are x0 + i (xa - x0) / (n - 1.) (delta_tot_table.c:582),
 // the expression the fslength kernels store them with: knot i recomputed here
 // equals the stored one, so the spline is evaluated without loading knots.
+// The quotient is formed from 1 / den, rounded, and one correction by its
+// exact remainder (Markstein 1990), which gives the division's own result in a
+// quarter of its instructions.
 struct UniformKnots {
-    double x0, span, den;  // x0, xa - x0, n - 1.
-    __device__ __forceinline__ double at(int i) const { return x0 + i * span / den; }
+    double x0, span, den, rden;  // x0, xa - x0, n - 1., 1 / (n - 1.)
+    __device__ __forceinline__ double at(int i) const
+    {
+        const double p = i * span, q = p * rden;
+        return x0 + fma(fma(-q, den, p), rden, q);
+    }
 };
 
 // settle() on those knots: i and its interval [xl, xr]
@@ -812,13 +819,79 @@ __device__ __forceinline__ void eval_pair<DnuIntegrand>(const DnuIntegrand &f, d
     r2 = use2 ? r2 : 0.0;
 }
 
-// ---- wave reductions over 32-lane halves ----
+// ---- moves between lanes ----
+// A wavefront that runs one QAG spends its time in a serial chain: a rule's
+// four sums of five steps each were most of it while every step went through
+// the LDS crossbar (over 100 clocks).  These run in the vector unit (8 to 16).
+// All 64 lanes take part.  (The host build of this file, a test's emulation,
+// has the shuffles.)
+#if defined(__HIP_DEVICE_COMPILE__)
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v)
+{
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);  // a lane without a source keeps its own
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v)
+{
+    return __hiloint2double(dpp<CTRL>(__double2hiint(v)), dpp<CTRL>(__double2loint(v)));
+}
+// v of the next lane (lane 63: its own), of the one before (lane 0: its own)
+template <class T>
+__device__ __forceinline__ T lane_next(T v)
+{
+    return dpp<0x130>(v);  // wave_shl:1
+}
+template <class T>
+__device__ __forceinline__ T lane_prev(T v)
+{
+    return dpp<0x138>(v);  // wave_shr:1
+}
+template <int LANE>
+__device__ __forceinline__ double lane_value(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), LANE),
+                            __builtin_amdgcn_readlane(__double2loint(v), LANE));
+}
+
+// The sum over each 32-lane half in every lane, by the butterfly v += v[lane ^
+// m], m = 16, 8, 4, 2, 1 (a step's two orders of its pair give one sum).
 __device__ __forceinline__ double half_sum(double v)
 {
-#pragma unroll
+    // rows 0 and 1 (2 and 3) of 16 lanes: the swap leaves one row's values in both rows, the other's likewise
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    v += dpp<0x128>(v);  // row_ror:8
+    v += dpp<0x124>(v);  // row_ror:4, lane ^ 4's value now that lane ^ 8 holds the same
+    v += dpp<0x4e>(v);   // quad_perm [2,3,0,1]
+    v += dpp<0xb1>(v);   // quad_perm [1,0,3,2]
+    return v;
+}
+#else
+template <class T>
+__device__ __forceinline__ T lane_next(T v)
+{
+    const int p = threadIdx.x & 63;
+    return __shfl(v, p < 63 ? p + 1 : 63, 64);
+}
+template <class T>
+__device__ __forceinline__ T lane_prev(T v)
+{
+    const int p = threadIdx.x & 63;
+    return __shfl(v, p > 0 ? p - 1 : 0, 64);
+}
+template <int LANE>
+__device__ __forceinline__ double lane_value(double v)
+{
+    return __shfl(v, LANE, 64);
+}
+__device__ __forceinline__ double half_sum(double v)
+{
     for (int m = 16; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
     return v;
 }
+#endif
 
 // t^1.5 rounded once: t sqrt(t) carried in two parts (the products' and the
 // square root's rounding errors recovered exactly by fma), then summed.  The
@@ -884,14 +957,14 @@ __device__ __forceinline__ void gk61_pair(const F &f, double a1, double b1, doub
     r.resasc = sasc * fabs(h);
     r.err = gk_rescale((sk - sg) * h, r.resabs, r.resasc);
     // broadcast each half's result to every lane
-    g1.res = __shfl(r.res, 0, 64);
-    g1.err = __shfl(r.err, 0, 64);
-    g1.resabs = __shfl(r.resabs, 0, 64);
-    g1.resasc = __shfl(r.resasc, 0, 64);
-    g2.res = __shfl(r.res, 32, 64);
-    g2.err = __shfl(r.err, 32, 64);
-    g2.resabs = __shfl(r.resabs, 32, 64);
-    g2.resasc = __shfl(r.resasc, 32, 64);
+    g1.res = lane_value<0>(r.res);
+    g1.err = lane_value<0>(r.err);
+    g1.resabs = lane_value<0>(r.resabs);
+    g1.resasc = lane_value<0>(r.resasc);
+    g2.res = lane_value<32>(r.res);
+    g2.err = lane_value<32>(r.err);
+    g2.resabs = lane_value<32>(r.resabs);
+    g2.resasc = lane_value<32>(r.resasc);
 }
 
 // The rule's nodes and weights by gk61_pair's lane j (0 at j = 31, and Gauss
@@ -1140,9 +1213,8 @@ __device__ __forceinline__ int wave_ord_insert(double &es, int &os, int im, doub
     const unsigned long long m1 = __ballot(p >= 1 && p < top && !(emax < es));
     const int i = m1 ? __ffsll((long long)m1) - 1 : top;
     // ord[p - 1] = ord[p] for p in [1, i), then ord[i - 1] = im
-    const int dn = p < 63 ? p + 1 : 63;
-    const double es_dn = __shfl(es, dn, 64);
-    const int os_dn = __shfl(os, dn, 64);
+    const double es_dn = lane_next(es);
+    const int os_dn = lane_next(os);
     if (p < i - 1) {
         es = es_dn;
         os = os_dn;
@@ -1154,9 +1226,8 @@ __device__ __forceinline__ int wave_ord_insert(double &es, int &os, int im, doub
     const unsigned long long m2 = __ballot(p >= i - 1 && p <= top - 1 && !(emin >= es));
     const int k = m2 ? 63 - __builtin_clzll(m2) : i - 2;
     // ord[p + 1] = ord[p] for p in [k + 1, top - 1], then ord[k + 1] = last
-    const int up = p > 0 ? p - 1 : 0;
-    const double es_up = __shfl(es, up, 64);
-    const int os_up = __shfl(os, up, 64);
+    const double es_up = lane_prev(es);
+    const int os_up = lane_prev(os);
     if (p > k + 1 && p <= top) {
         es = es_up;
         os = os_up;
@@ -1164,7 +1235,7 @@ __device__ __forceinline__ int wave_ord_insert(double &es, int &os, int im, doub
         es = emin;
         os = last;
     }
-    return __shfl(os, 0, 64);
+    return __builtin_amdgcn_readfirstlane(os);
 }
 
 // The order after appending interval n - 1: in registers while it fits,
@@ -1201,71 +1272,83 @@ template <class F>
 __device__ int wave_qag61(const F &f, double a, double b, double epsrel, int limit, QagWs &w, double *result,
                           int *nint)
 {
+    // the first estimate and the bisections share one copy of the rule's code
+    // (the integrand inlined at two places is beyond the instruction cache)
     const bool lead = (threadIdx.x & 63) == 0;
-    GK g0, gx;
-    gk61_pair(f, a, b, a, b, g0, gx);
-    *result = g0.res;
-    *nint = 1;
-    if (lead) {
-        w.lo[0] = a;
-        w.hi[0] = b;
-        w.r[0] = g0.res;
-        w.e[0] = g0.err;
-        w.ord[0] = 0;
-    }
-    int imax = __shfl(0, 0, 64);
-    double es = g0.err;  // the error order in registers (ord_insert)
-    int os = 0;
+    int imax = 0, os = 0;
     bool ord_lds = false;
-    double tol = epsrel * fabs(g0.res);
-    if (g0.err <= 50 * DBL_EPSILON * g0.resabs && g0.err > tol) return 18;
-    if ((g0.err <= tol && g0.err != g0.resasc) || g0.err == 0.0) return 0;
-    if (limit == 1) return 11;
-    double area = g0.res, errsum = g0.err;
-    int n = 1, it = 1, rt1 = 0, rt2 = 0, etype = 0;
-    do {
-        const int im = imax;
-        const double ai = w.lo[im], bi = w.hi[im], ri = w.r[im], ei = w.e[im];
-        const double a1 = ai, b1 = 0.5 * (ai + bi), a2 = b1, b2 = bi;
+    double es = 0.0, tol = 0.0, area = 0.0, errsum = 0.0;  // es, os: the error order in registers (ord_insert)
+    double ri = 0.0, ei = 0.0, a1 = a, b1 = b, a2 = a, b2 = b;
+    int n = 0, it = 1, rt1 = 0, rt2 = 0, etype = 0;
+    for (;;) {
         GK g1, g2;
         gk61_pair(f, a1, b1, a2, b2, g1, g2);
-        const double r12 = g1.res + g2.res, e12 = g1.err + g2.err;
-        errsum += e12 - ei;
-        area += r12 - ri;
-        if (g1.resasc != g1.err && g2.resasc != g2.err) {
-            if (fabs(ri - r12) <= 1.0e-5 * fabs(r12) && e12 >= 0.99 * ei) rt1++;
-            if (it >= 10 && e12 > ei) rt2++;
-        }
-        tol = epsrel * fabs(area);
-        if (errsum > tol) {
-            const double t = (1 + 100 * DBL_EPSILON) * (fabs(a2) + 1000 * DBL_MIN);
-            if (rt1 >= 6 || rt2 >= 20) etype = 2;
-            if (fabs(a1) <= t && fabs(b2) <= t) etype = 3;
-        }
-        if (lead) {
-            if (g2.err > g1.err) {
-                w.lo[im] = a2;
-                w.r[im] = g2.res;
-                w.e[im] = g2.err;
-                w.lo[n] = a1;
-                w.hi[n] = b1;
-                w.r[n] = g1.res;
-                w.e[n] = g1.err;
-            } else {
-                w.hi[im] = b1;
-                w.r[im] = g1.res;
-                w.e[im] = g1.err;
-                w.lo[n] = a2;
-                w.hi[n] = b2;
-                w.r[n] = g2.res;
-                w.e[n] = g2.err;
+        if (n == 0) {
+            *result = g1.res;
+            *nint = 1;
+            if (lead) {
+                w.lo[0] = a;
+                w.hi[0] = b;
+                w.r[0] = g1.res;
+                w.e[0] = g1.err;
+                w.ord[0] = 0;
             }
+            imax = __shfl(0, 0, 64);
+            es = g1.err;
+            tol = epsrel * fabs(g1.res);
+            if (g1.err <= 50 * DBL_EPSILON * g1.resabs && g1.err > tol) return 18;
+            if ((g1.err <= tol && g1.err != g1.resasc) || g1.err == 0.0) return 0;
+            if (limit == 1) return 11;
+            area = g1.res;
+            errsum = g1.err;
+            n = 1;
+        } else {
+            const int im = imax;
+            const double r12 = g1.res + g2.res, e12 = g1.err + g2.err;
+            errsum += e12 - ei;
+            area += r12 - ri;
+            if (g1.resasc != g1.err && g2.resasc != g2.err) {
+                if (fabs(ri - r12) <= 1.0e-5 * fabs(r12) && e12 >= 0.99 * ei) rt1++;
+                if (it >= 10 && e12 > ei) rt2++;
+            }
+            tol = epsrel * fabs(area);
+            if (errsum > tol) {
+                const double t = (1 + 100 * DBL_EPSILON) * (fabs(a2) + 1000 * DBL_MIN);
+                if (rt1 >= 6 || rt2 >= 20) etype = 2;
+                if (fabs(a1) <= t && fabs(b2) <= t) etype = 3;
+            }
+            if (lead) {
+                if (g2.err > g1.err) {
+                    w.lo[im] = a2;
+                    w.r[im] = g2.res;
+                    w.e[im] = g2.err;
+                    w.lo[n] = a1;
+                    w.hi[n] = b1;
+                    w.r[n] = g1.res;
+                    w.e[n] = g1.err;
+                } else {
+                    w.hi[im] = b1;
+                    w.r[im] = g1.res;
+                    w.e[im] = g1.err;
+                    w.lo[n] = a2;
+                    w.hi[n] = b2;
+                    w.r[n] = g2.res;
+                    w.e[n] = g2.err;
+                }
+            }
+            const bool hi2 = g2.err > g1.err;
+            imax = ord_insert(w, es, os, ord_lds, im, hi2 ? g2.err : g1.err, hi2 ? g1.err : g2.err, n + 1, limit);
+            n++;
+            it++;
+            if (!(it < limit && !etype && errsum > tol)) break;
         }
-        const bool hi2 = g2.err > g1.err;
-        imax = ord_insert(w, es, os, ord_lds, im, hi2 ? g2.err : g1.err, hi2 ? g1.err : g2.err, n + 1, limit);
-        n++;
-        it++;
-    } while (it < limit && !etype && errsum > tol);
+        const double ai = w.lo[imax], bi = w.hi[imax];
+        ri = w.r[imax];
+        ei = w.e[imax];
+        a1 = ai;
+        b1 = a2 = 0.5 * (ai + bi);
+        b2 = bi;
+    }
     double s = 0.0;
     for (int k = 0; k < n; k++) s += w.r[k];
     *result = s;
@@ -1318,20 +1401,15 @@ __device__ int block_qag61(const F &f, double a, double b, double epsrel, int li
     QagWs &w = S.ws;
     // pass 0: wavefront 0 the first estimate; wavefront 1 the halves of [a, b] (the first bisection)
     GK g0, gx;
-    if (wave == 0) {
-        gk61_pair(f, a, b, a, b, g0, gx);
-    } else if constexpr (W > 1) {
-        if (wave == 1) {
-            const double m = 0.5 * (a + b);
-            GK g1, g2;
-            gk61_pair(f, a, m, m, b, g1, g2);
-            if ((threadIdx.x & 63) == 0) {
-                S.slot[1].used = 1;
-                S.slot[1].lo = a;
-                S.slot[1].hi = b;
-                S.slot[1].g1 = g1;
-                S.slot[1].g2 = g2;
-            }
+    if (wave <= 1) {
+        const double m = 0.5 * (a + b);
+        gk61_pair(f, a, wave ? m : b, wave ? m : a, b, g0, gx);
+        if (wave == 1 && (threadIdx.x & 63) == 0) {
+            S.slot[1].used = 1;
+            S.slot[1].lo = a;
+            S.slot[1].hi = b;
+            S.slot[1].g1 = g0;
+            S.slot[1].g2 = gx;
         }
     }
     if (lead)
