@@ -5,14 +5,16 @@
 // with the host's own hubble_function (the initial-condition piece,
 // fslength(T0, a), delta_tot_table.c:522-535) and the per-species parameters
 // (:539-548); the device computes, in order:
-//   k_fs_first,  the 16 Na free-streaming lengths fslength(x_i, log a) on the
+//   k_dnu_first, the 16 Na free-streaming lengths fslength(x_i, log a) on the
 //   k_fs_rest    reference's uniform log-a grid, each a QAG-GK61 integral of
-//                1/(a^2 H) (relerr 1e-6): the first estimate for two nodes per
-//                wavefront, full QAG (one wavefront each) for those it leaves;
-//   k_spline     natural cubic spline coefficients of that table (one
-//                wavefront per row window: scans of the substitution recurrences);
-//   k_rows_prep  the same for every delta_tot[k][0..Na-1] row, and a uniform
-//                bucket index over the stored log a values, in one launch;
+//                1/(a^2 H) (relerr 1e-6): the first estimate for sixteen nodes
+//                per wavefront (with it, in the same launch, the factors of the
+//                delta_tot rows' splines and a uniform bucket index over the
+//                stored log a values), then full QAG (one wavefront each) for
+//                the nodes it leaves;
+//   k_prep       natural cubic spline coefficients of that table and of every
+//                delta_tot[k][0..Na-1] row (one wavefront per row window: scans
+//                of the substitution recurrences);
 //   k_dnu_qag_spec, k_dnu_qag_mix
 //                one block or wavefront per (species, k): QAG-GK61 of
 //                fsl/(a H) * specialJ * S_k over [log T0, log a] at the
@@ -185,65 +187,28 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_fs_rest(HTab H, int nfs
 
 constexpr int kFsRestBlocks = 64;
 
-inline int fs_first_blocks(int nfs) { return (nfs + 63) / 64; }  // 4 waves x 16 nodes per block
-
-// Rows of natural-spline coefficients (row r: x[0..n), y + r*ystride,
-// c + r*cstride): one wavefront per (row, window of kKeep rows).
-__device__ inline void spline_item_wave(const double *__restrict__ x, const double *__restrict__ y,
-                                        double *__restrict__ c, int n, long long ystride, long long cstride,
-                                        long long item)
-{
-    const int nwin = (n + kKeep - 1) / kKeep;
-    const int r = (int)(item / nwin), w = (int)(item % nwin);
-    const int lo = w * kKeep, hi = lo + kKeep < n ? lo + kKeep : n;
-    SplineRhs rhs;
-    rhs.x = x;
-    rhs.y = y + r * ystride;
-    tridiag_window_wave(x, n, rhs, lo, hi, c + r * cstride);
-}
-
-__global__ __launch_bounds__(256) void k_spline(const double *__restrict__ x, const double *__restrict__ y,
-                                                double *__restrict__ c, int n, int nrows, long long ystride,
-                                                long long cstride)
-{
-    const long long item = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= (long long)((n + kKeep - 1) / kKeep) * nrows) return;  // wave-uniform
-    spline_item_wave(x, y, c, n, ystride, cstride, item);
-}
-
-// Blocks of k_spline for nrows rows of n knots.
-__host__ __device__ inline int spline_blocks(int n, int nrows)
-{
-    const long long items = (long long)((n + kKeep - 1) / kKeep) * nrows;
-    return (int)((items + 3) / 4);
-}
+__host__ __device__ inline int fs_first_blocks(int nfs) { return (nfs + 63) / 64; }  // 4 waves x 16 nodes per block
 
 // Spline factors of the knots x[0..n) shared by all rows on them (fac,
 // kFacStride doubles per window; none when n < 3) and the reciprocal knot
-// spacings ih[0..n-1): block b's waves factor windows 4b .. 4b+3, its threads
-// the spacings 256b + t.
-__device__ inline void factor_block(const double *__restrict__ x, int n, double *__restrict__ fac,
+// spacings ih[0..n-1): of a block with W wavefronts, block b's factor windows
+// Wb .. Wb + W - 1, its threads the spacings 64 Wb + t.
+__device__ __forceinline__ void factor_block(const double *__restrict__ x, int n, double *__restrict__ fac,
                                     double *__restrict__ ih, int b)
 {
-    const int w = b * 4 + (threadIdx.x >> 6);
+    const int w = b * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6);
     if (n >= 3 && w < fac_windows(n)) tri_factor_store(x, n, w, fac);  // wave-uniform
-    const int i = b * 256 + threadIdx.x;
+    const int i = b * (int)blockDim.x + (int)threadIdx.x;
     if (i < n - 1) {
         const double h = x[i + 1] - x[i];
         ih[i] = h != 0.0 ? 1.0 / h : 0.0;
     }
 }
 
-inline int factor_blocks(int n)
+__host__ __device__ inline int factor_blocks(int n, int threads)
 {
-    const int bw = (fac_windows(n) + 3) / 4, bi = (n - 1 + 255) / 256;
+    const int wpb = threads / 64, bw = (fac_windows(n) + wpb - 1) / wpb, bi = (n - 1 + threads - 1) / threads;
     return bw > bi ? bw : bi;
-}
-
-__global__ __launch_bounds__(256) void k_factor(const double *__restrict__ x, int n, double *__restrict__ fac,
-                                                double *__restrict__ ih)
-{
-    factor_block(x, n, fac, ih, blockIdx.x);
 }
 
 // doubles of factor storage for n knots: windows, then the spacings
@@ -262,44 +227,102 @@ __device__ inline void bucket_at(const double *__restrict__ x, int n, double inv
     bucket[q] = lo;
 }
 
-// The delta_tot rows' splines (on the stored factors of the knots sx, see
-// factor_block) and the bucket index in one launch: blocks [0, b_sp) one
-// window of 4 rpw rows each (none when na <= 2), the rest the bucket.  Rows of
-// Y and C are `ystride` doubles apart.
-// lds: kTriSpan doubles per wavefront of the block and one more
-__device__ __forceinline__ void rows_prep_block(const double *__restrict__ sx, const double *__restrict__ Y,
-                                       double *__restrict__ C, int na, int nk, long long ystride, int b_sp, int nsb,
-                                       double sinv_bw, int *__restrict__ bucket, const double *__restrict__ fac,
-                                       int rpw, int b, double *lds)
+// What a history's integrals need of its knots sx alone: the spline factors and
+// the bucket index, blocks [0, knots_blocks).
+struct KnotsArgs {
+    const double *sx;
+    int na, nsb;
+    double sinv_bw;
+    double *fac;
+    int *bucket;
+};
+__device__ __forceinline__ void knots_block(const KnotsArgs &k, int b)
 {
-    if (b < b_sp) {  // window b % nwin of 4 rpw rows, every fourth by one wavefront
-        const int nwin = fac_windows(na), wave = threadIdx.x >> 6;
-        const int r0 = (int)(b / nwin) * 4 * rpw, rend = r0 + 4 * rpw < nk ? r0 + 4 * rpw : nk;
-        tri_rows_staged(na, b % nwin, Y, C, ystride, r0 + wave, 4, rend, fac, lds + (1 + wave) * kTriSpan, lds);
+    const int nf = factor_blocks(k.na, blockDim.x);
+    if (b < nf) {  // block-uniform
+        factor_block(k.sx, k.na, k.fac, k.fac + (size_t)fac_windows(k.na) * kFacStride, b);
         return;
     }
-    const int q = (b - b_sp) * 256 + threadIdx.x;
-    if (q <= nsb) bucket_at(sx, na, sinv_bw, bucket, q);
+    const int q = (b - nf) * (int)blockDim.x + (int)threadIdx.x;
+    if (q <= k.nsb) bucket_at(k.sx, k.na, k.sinv_bw, k.bucket, q);
+}
+
+__host__ __device__ inline int knots_blocks(int na, int nsb, int threads)
+{
+    return factor_blocks(na, threads) + (nsb + threads) / threads;
+}
+
+__global__ __launch_bounds__(256) void k_knots(KnotsArgs k) { knots_block(k, blockIdx.x); }
+
+// k_fs_first and k_knots in one launch: neither fills the chip at one history's
+// sizes, and a launch by itself is a few microseconds (their 7-11 and 8 us, one
+// after the other, were a fifth of a small call's device time).
+__global__ __launch_bounds__(256) void k_dnu_first(HTab H, int nfs, double x0, double xa, double light,
+                                                   double *__restrict__ fx, double *__restrict__ fy,
+                                                   int *__restrict__ status, int *__restrict__ list,
+                                                   int *__restrict__ count, KnotsArgs kn)
+{
+    const int fsb = fs_first_blocks(nfs);
+    if ((int)blockIdx.x >= fsb) {
+        knots_block(kn, blockIdx.x - fsb);
+        return;
+    }
+    const ListPush push = {list, count};
+    FslIntegrand f;
+    f.H = H;
+    fs_first_tile(f, RuleConst(), nfs, x0, xa, light, fx, fy, status, (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), push);
+}
+
+// The splines in one launch: blocks [0, b_sp) the delta_tot rows' (on the
+// stored factors of their knots), one window of 4 rpw rows each (none when na <=
+// 2), the rest the fslength table's, four windows each.  Rows of Y and C are
+// `ystride` doubles apart.
+struct PrepArgs {
+    const double *Y;
+    double *C;
+    int na, nk;
+    long long ystride;
+    int b_sp, rpw;
+    const double *fac;
+    UniformKnots fk;
+    const double *fy;
+    double *fc;
+    int nfs;
+};
+// lds: kTriSpan doubles per wavefront of the block and one more
+__device__ __forceinline__ void prep_block(const PrepArgs &a, int b, double *lds)
+{
+    const int wave = threadIdx.x >> 6;
+    if (b < a.b_sp) {  // window b % nwin of 4 rpw rows, every fourth by one wavefront
+        const int nwin = fac_windows(a.na);
+        const int r0 = (int)(b / nwin) * 4 * a.rpw, rend = r0 + 4 * a.rpw < a.nk ? r0 + 4 * a.rpw : a.nk;
+        tri_rows_staged(a.na, b % nwin, a.Y, a.C, a.ystride, r0 + wave, 4, rend, a.fac, lds + (1 + wave) * kTriSpan,
+                        lds);
+        return;
+    }
+    const int w = (b - a.b_sp) * 4 + wave;
+    if (w < fac_windows(a.nfs)) uniform_spline_wave(a.fk, a.fy, a.fc, a.nfs, w, lds + wave * kTriSpan);
 }
 
 // Bound by memory: 256 histories of 64-512 k x 100-3000 steps, 1.83 GB read and
 // written, take 385 us (4.75 TB/s) with four wavefronts per SIMD (128
 // registers), 402 with three; a row at a time, with the factors read for each,
 // took 750.
-__global__ __launch_bounds__(256, 4) void k_rows_prep(const double *__restrict__ sx, const double *__restrict__ Y,
-                                                   double *__restrict__ C, int na, int nk, long long ystride,
-                                                   int b_sp, int nsb, double sinv_bw, int *__restrict__ bucket,
-                                                   const double *__restrict__ fac, int rpw)
+__global__ __launch_bounds__(256, 4) void k_prep(PrepArgs a)
 {
     __shared__ double lds[5 * kTriSpan];
-    rows_prep_block(sx, Y, C, na, nk, ystride, b_sp, nsb, sinv_bw, bucket, fac, rpw, blockIdx.x, lds);
+    prep_block(a, blockIdx.x, lds);
 }
-
-inline int rows_prep_blocks(int b_sp, int nsb) { return b_sp + (nsb + 256) / 256; }
 
 __host__ __device__ inline int rows_prep_spline_blocks(int na, int nk, int rpw)
 {
     return na > 2 ? fac_windows(na) * ((nk + 4 * rpw - 1) / (4 * rpw)) : 0;
+}
+__host__ __device__ inline int prep_blocks(int b_sp, int nfs) { return b_sp + (fac_windows(nfs) + 3) / 4; }
+
+__host__ __device__ inline UniformKnots fs_knots(double x0, double xa, int nfs)
+{
+    return {x0, xa - x0, nfs - 1., 1.0 / (nfs - 1.)};
 }
 
 // Rows per wavefront, for launches of that many (row, window) items: more pay
@@ -367,10 +390,7 @@ __device__ inline DnuIntegrand dnu_integrand(const QagArgs &a, const SpeciesDev 
     f.H = a.H;
     f.fy = a.fy;
     f.fc = a.fc;
-    f.fk.x0 = a.x0;  // the fslength knots' own expression (fs_first_tile)
-    f.fk.span = a.xa - a.x0;
-    f.fk.den = a.nfs - 1.;
-    f.fk.rden = 1.0 / f.fk.den;
+    f.fk = fs_knots(a.x0, a.xa, a.nfs);
     f.nfs = a.nfs;
     f.fx0 = a.fx[0];
     f.fxhi = a.fx[a.nfs - 1];
@@ -600,11 +620,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
     const double kk = A.wavenum[k], mnubykT = A.sp->mnubykT, gb = A.gbar[item] * A.prefac;
     const JPar &J = A.sp->J;
     const double fx0 = fx[0], finv_h = (nfs - 1) / (fx[nfs - 1] - fx[0]), sx0 = sx[0];
-    UniformKnots fk;  // the fslength knots (fs_first_tile's expression)
-    fk.x0 = A.x0;
-    fk.span = A.xa - A.x0;
-    fk.den = nfs - 1.;
-    fk.rden = 1.0 / fk.den;
+    const UniformKnots fk = fs_knots(A.x0, A.xa, nfs);
 #pragma unroll
     for (int p = 0; p < kTriPass; p++) {
         const int t = p * 64 + lane;
@@ -740,15 +756,17 @@ __global__ __launch_bounds__(64, 3) void k_dnu_adj(AdjArgs A)
 // ---------------------------------------------------------------- state
 
 struct DnuDev {
-    size_t cap_fs = 0, cap_y = 0, cap_x = 0, cap_k = 0, cap_items = 0, cap_b = 0;
+    size_t cap_fs = 0, cap_y = 0, cap_b = 0;
     double *fx = nullptr, *fy = nullptr, *fc = nullptr;
-    int *fs_list = nullptr;  // fslength nodes that need bisection, then their count at [cap_fs]
-    double *sx = nullptr, *Y = nullptr, *C = nullptr, *wavenum = nullptr;
+    int *fs_list = nullptr;  // fslength nodes that need bisection
+    double *Y = nullptr, *C = nullptr;
     int *bucket = nullptr;
-    double *out = nullptr;
-    int *nint = nullptr, *item_species = nullptr;
+    // a call's small inputs and its results, one block each way (IoLayout)
+    char *io = nullptr;
+    size_t cap_io = 0;
+    double *sx = nullptr, *wavenum = nullptr, *out = nullptr;
+    int *nint = nullptr, *item_species = nullptr, *order = nullptr, *status = nullptr;
     SpeciesDev *sp = nullptr;
-    int *status = nullptr;
     size_t cap_ivl = 0, cap_adj = 0, cap_adj_k = 0;
     double *ivl = nullptr;                                            // recorded subdivisions
     size_t cap_fac = 0;
@@ -764,7 +782,6 @@ struct DnuDev {
     // each item's final interval count in the last call, which orders the
     // next call's QAG items (the same k bins are integrated every step)
     std::vector<int> prev_nint;
-    int *order = nullptr;
 };
 std::unordered_map<const void *, DnuDev *> g_dev;
 int g_last_max_intervals = 0, g_last_items = 0;
@@ -876,26 +893,50 @@ HostPool &host_pool()
     return *p;
 }
 
-char *g_stage = nullptr;
-size_t g_stage_cap = 0;
+// Pinned buffers: 0 the history's columns and the adjoint's results, 1 the
+// rest of a call's inputs and results (each may be in flight while the other
+// grows).
+char *g_stage[2];
+size_t g_stage_cap[2];
 hipStream_t g_copy = nullptr;
 hipEvent_t g_copied = nullptr;
 
-char *pinned_stage(size_t bytes)
+char *pinned_stage(int which, size_t bytes)
 {
-    if (bytes > g_stage_cap) {
-        if (g_stage) KN_CHECK(hipHostFree(g_stage));
-        KN_CHECK(hipHostMalloc((void **)&g_stage, bytes, 0));
-        g_stage_cap = bytes;
+    if (bytes > g_stage_cap[which]) {
+        if (g_stage[which]) KN_CHECK(hipHostFree(g_stage[which]));
+        KN_CHECK(hipHostMalloc((void **)&g_stage[which], bytes, 0));
+        g_stage_cap[which] = bytes;
     }
     if (!g_copy) {
         KN_CHECK(hipStreamCreateWithFlags(&g_copy, hipStreamNonBlocking));
         KN_CHECK(hipEventCreateWithFlags(&g_copied, hipEventDisableTiming));
     }
-    return g_stage;
+    return g_stage[which];
 }
 
 inline size_t align64(size_t n) { return (n + 63) & ~(size_t)63; }
+
+// A call's small arrays in one block, on the device and in pinned memory: up
+// goes [0, out) in one copy (the status words and the count of listed nodes as
+// zeros), back comes [status, end) in one copy.  (Five and three copies and two
+// fills before: each is a launch of its own.)
+struct IoLayout {
+    size_t sx, wavenum, sp, species, order, status, count, out, nint, end;
+    IoLayout(int Na, int nk, int nitems)
+    {
+        sx = 0;
+        wavenum = sx + sizeof(double) * Na;
+        sp = wavenum + sizeof(double) * nk;
+        species = sp + sizeof(SpeciesDev) * NUSPECIES;
+        order = species + sizeof(int) * NUSPECIES;
+        status = align64(order + sizeof(int) * nitems);
+        count = status + sizeof(int) * 2;
+        out = align64(count + sizeof(int));
+        nint = out + sizeof(double) * nitems;
+        end = nint + sizeof(int) * nitems;
+    }
+};
 
 }  // namespace
 
@@ -1426,9 +1467,8 @@ extern "C" void kn_dnu_release(const _delta_tot_table *d)
     auto it = g_dev.find(d);
     if (it == g_dev.end()) return;
     DnuDev *v = it->second;
-    void *ptrs[] = {v->fs_list, v->fx,  v->fy,   v->fc,   v->sx,   v->Y,    v->C,    v->wavenum, v->bucket, v->out,
-                    v->nint, v->item_species, v->sp, v->status, v->ivl, v->gbar, v->ybar, v->mubar,
-                    v->fac, v->order};
+    void *ptrs[] = {v->fs_list, v->fx, v->fy, v->fc, v->Y, v->C, v->bucket, v->io, v->ivl, v->gbar, v->ybar, v->mubar,
+                    v->fac};
     for (void *p : ptrs)
         if (p) KN_CHECK(hipFree(p));
     delete v;
@@ -1454,19 +1494,23 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
     const double x0 = log(d->TimeTransfer), xa = log(a);
     const double nfl0 = d->omnu->hybnu.nufrac_low[0];
     // initial-condition piece, on the host exactly as delta_tot_table.c:522-535
-    const double fsl_A0a = fslength(x0, xa, d->light);
-    const double deriv_prefac = kn_deriv_prefac(d);
-    for (int s = 0; s < nspecies; s++)
-        for (int k = 0; k < nk; k++) {
-            const double m = sp[s].mnubykT > 0 ? sp[s].mnubykT : 1;
-            const double specJ = specialJ(wavenum[k] * fsl_A0a / m, 0, nfl0);
-            out[(size_t)s * nk + k] = specJ * d->delta_nu_init[k] * (1. + deriv_prefac * fsl_A0a);
-        }
+    auto initial_piece = [&] {
+        const double fsl_A0a = fslength(x0, xa, d->light);
+        const double deriv_prefac = kn_deriv_prefac(d);
+        for (int s = 0; s < nspecies; s++)
+            for (int k = 0; k < nk; k++) {
+                const double m = sp[s].mnubykT > 0 ? sp[s].mnubykT : 1;
+                const double specJ = specialJ(wavenum[k] * fsl_A0a / m, 0, nfl0);
+                out[(size_t)s * nk + k] = specJ * d->delta_nu_init[k] * (1. + deriv_prefac * fsl_A0a);
+            }
+    };
     std::vector<int> need;
     for (int s = 0; s < nspecies; s++)
         if (!sp[s].ic_only) need.push_back(s);
-    if (need.empty()) return 0;
-    if (Na < 2) return 0;
+    if (need.empty() || Na < 2) {
+        initial_piece();
+        return 0;
+    }
 
     upload_constants();
     kn_htable_ensure(x0, x0, xa);
@@ -1481,10 +1525,9 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
             KN_CHECK(hipMalloc(p, sizeof(double) * nfs));
         }
         if (dev->fs_list) KN_CHECK(hipFree(dev->fs_list));
-        KN_CHECK(hipMalloc(&dev->fs_list, sizeof(int) * ((size_t)nfs + 1)));
+        KN_CHECK(hipMalloc(&dev->fs_list, sizeof(int) * nfs));
         dev->cap_fs = nfs;
     }
-    grow(dev->sx, dev->cap_x, (size_t)Na);
     const int namax = d->namax;
     if (dev->ystride != namax || dev->have_nk != nk) {  // a new layout: nothing of the history is on the device
         dev->ystride = namax;
@@ -1501,40 +1544,62 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
         dev->cap_y = (size_t)nk * namax;
         dev->have_na = 0;
     }
-    grow(dev->wavenum, dev->cap_k, (size_t)nk);
     grow(dev->bucket, dev->cap_b, (size_t)nsb + 1);
     grow(dev->fac, dev->cap_fac, fac_doubles(Na));
-    if (dev->cap_items < (size_t)nitems) {
-        if (dev->out) KN_CHECK(hipFree(dev->out));
-        if (dev->nint) KN_CHECK(hipFree(dev->nint));
-        KN_CHECK(hipMalloc(&dev->out, sizeof(double) * nitems));
-        KN_CHECK(hipMalloc(&dev->nint, sizeof(int) * nitems));
-        if (dev->order) KN_CHECK(hipFree(dev->order));
-        KN_CHECK(hipMalloc(&dev->order, sizeof(int) * nitems));
-        dev->cap_items = nitems;
-    }
-    if (!dev->sp) {
-        KN_CHECK(hipMalloc(&dev->sp, sizeof(SpeciesDev) * NUSPECIES));
-        KN_CHECK(hipMalloc(&dev->item_species, sizeof(int) * NUSPECIES));
-        KN_CHECK(hipMalloc(&dev->status, sizeof(int) * 2));
-    }
+    const IoLayout L(Na, nk, nitems);
+    grow(dev->io, dev->cap_io, L.end);
+    dev->sx = (double *)(dev->io + L.sx);
+    dev->wavenum = (double *)(dev->io + L.wavenum);
+    dev->sp = (SpeciesDev *)(dev->io + L.sp);
+    dev->item_species = (int *)(dev->io + L.species);
+    dev->order = (int *)(dev->io + L.order);
+    dev->status = (int *)(dev->io + L.status);
+    dev->out = (double *)(dev->io + L.out);
+    dev->nint = (int *)(dev->io + L.nint);
     if (record && dev->cap_ivl < (size_t)nitems) {
         if (dev->ivl) KN_CHECK(hipFree(dev->ivl));
         KN_CHECK(hipMalloc(&dev->ivl, sizeof(double) * (size_t)nitems * kLimit * 2));
         dev->cap_ivl = nitems;
     }
-    // the fslength nodes and their spline need only (T0, a): they start
+    char *io = pinned_stage(1, L.end);
+    memcpy(io + L.sx, d->scalefact, sizeof(double) * Na);
+    memcpy(io + L.wavenum, wavenum, sizeof(double) * nk);
+    SpeciesDev *sd = (SpeciesDev *)(io + L.sp);
+    int *ispec = (int *)(io + L.species), *ord = (int *)(io + L.order);
+    for (size_t i = 0; i < need.size(); i++) {
+        const kn_species &q = sp[need[i]];
+        sd[i].mnubykT = q.mnubykT;
+        sd[i].relerr = q.relerr;
+        sd[i].J.qc = q.qc;
+        sd[i].J.nufrac_low = nfl0;
+        sd[i].J.en[0] = 1.0;
+        for (int n = 1; n < 20; n++) sd[i].J.en[n] = exp(-n * q.qc);
+        ispec[i] = (int)i;
+    }
+    // the QAG items' order: those that needed kLongChain intervals or more in
+    // the last call first (longest first), then the rest in item order
+    int nlong = 0;
+    {
+        const bool pred = dev->prev_nint.size() == (size_t)nitems;
+        for (int i = 0; i < nitems; i++)
+            if (pred && dev->prev_nint[i] >= kLongChain) ord[nlong++] = i;
+        std::stable_sort(ord, ord + nlong, [&](int x, int y) { return dev->prev_nint[x] > dev->prev_nint[y]; });
+        int j = nlong;
+        for (int i = 0; i < nitems; i++)
+            if (!(pred && dev->prev_nint[i] >= kLongChain)) ord[j++] = i;
+    }
+    memset(io + L.status, 0, L.out - L.status);
+    KN_CHECK(hipMemcpyAsync(dev->io, io, L.out, hipMemcpyHostToDevice, 0));
+    // the fslength nodes and the knots' factors need no history: they start
     // first, and run while the host finds and packs the missing columns
     const HTab H = device_htab();
-    KN_CHECK(hipMemsetAsync(dev->status, 0, sizeof(int) * 2, 0));
-    int *fs_count = dev->fs_list + dev->cap_fs;
-    KN_CHECK(hipMemsetAsync(fs_count, 0, sizeof(int), 0));
-    hipLaunchKernelGGL(k_fs_first, dim3(fs_first_blocks(nfs)), dim3(256), 0, 0, H, nfs, x0, xa, d->light, dev->fx,
-                       dev->fy, dev->status, dev->fs_list, fs_count);
+    const double sinv_bw = nsb / (d->scalefact[Na - 1] - d->scalefact[0]);
+    int *fs_count = (int *)(dev->io + L.count);
+    hipLaunchKernelGGL(k_dnu_first, dim3(fs_first_blocks(nfs) + knots_blocks(Na, nsb, 256)), dim3(256), 0, 0, H, nfs,
+                       x0, xa, d->light, dev->fx, dev->fy, dev->status, dev->fs_list, fs_count,
+                       KnotsArgs{dev->sx, Na, nsb, sinv_bw, dev->fac, dev->bucket});
     hipLaunchKernelGGL(k_fs_rest, dim3(kFsRestBlocks), dim3(64 * kWavesPerBlock), 0, 0, H, nfs, x0, xa, d->light,
                        dev->fx, dev->fy, dev->status, dev->fs_list, fs_count);
-    hipLaunchKernelGGL(k_spline, dim3(spline_blocks(nfs, 1)), dim3(256), 0, 0, dev->fx, dev->fy, dev->fc, nfs, 1, 0LL,
-                       0LL);
     KN_CHECK(hipGetLastError());
     // which columns of the history the device lacks: per row, the first entry
     // that differs from the shadow (entries past the shadow's count differ)
@@ -1565,23 +1630,15 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
     dev->have_na = Na;
     const int ncol = Na - col0;  // columns [col0, Na) of every row go up
     g_last_upload_cols = ncol;
-    // pinned staging: inputs [Y columns col0..Na | scalefact | wavenum | species | species index], then outputs
     const size_t nY = (size_t)nk * ncol;
-    const size_t b_sp = sizeof(double) * (nY + Na + nk);
-    const size_t b_in = align64(b_sp + sizeof(SpeciesDev) * NUSPECIES + sizeof(int) * NUSPECIES + sizeof(int) * nitems);
-    char *stage = pinned_stage(b_in + align64(sizeof(double) * nitems) + sizeof(int) * ((size_t)nitems + 2));
-    double *stY = (double *)stage, *stX = stY + nY, *stK = stX + Na;
-    SpeciesDev *sd = (SpeciesDev *)(stage + b_sp);
-    int *ispec = (int *)(sd + NUSPECIES);
-    int *ord = ispec + NUSPECIES;
-    double *res = (double *)(stage + b_in);
-    int *nint = (int *)(stage + b_in + align64(sizeof(double) * nitems)), *status = nint + nitems;
 
     // meanwhile the missing columns are packed (ncol per row) and uploaded on
     // the copy stream into rows of stride namax, in chunks of rows: a chunk's
     // upload runs while the next is packed
     if (ncol > 0) {
+        double *stY = (double *)pinned_stage(0, sizeof(double) * nY);
         const int chunks = nY < (1u << 16) ? 1 : 4, parts = nY < (1u << 16) ? 1 : 8;
+        const hipStream_t cs = chunks > 1 ? g_copy : 0;  // a few columns: no second stream to wait for
         for (int c = 0; c < chunks; c++) {
             const int c0 = (int)((long long)nk * c / chunks), c1 = (int)((long long)nk * (c + 1) / chunks);
             host_pool().run(parts, [&](int p) {
@@ -1593,48 +1650,18 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
             if (c1 > c0)
                 KN_CHECK(hipMemcpy2DAsync(dev->Y + (size_t)c0 * namax + col0, sizeof(double) * namax,
                                           stY + (size_t)c0 * ncol, sizeof(double) * ncol, sizeof(double) * ncol,
-                                          c1 - c0, hipMemcpyHostToDevice, g_copy));
+                                          c1 - c0, hipMemcpyHostToDevice, cs));
+        }
+        if (cs) {
+            KN_CHECK(hipEventRecord(g_copied, cs));
+            KN_CHECK(hipStreamWaitEvent(0, g_copied, 0));
         }
     }
-    memcpy(stX, d->scalefact, sizeof(double) * Na);
-    memcpy(stK, wavenum, sizeof(double) * nk);
-    for (size_t i = 0; i < need.size(); i++) {
-        const kn_species &q = sp[need[i]];
-        sd[i].mnubykT = q.mnubykT;
-        sd[i].relerr = q.relerr;
-        sd[i].J.qc = q.qc;
-        sd[i].J.nufrac_low = nfl0;
-        sd[i].J.en[0] = 1.0;
-        for (int n = 1; n < 20; n++) sd[i].J.en[n] = exp(-n * q.qc);
-        ispec[i] = (int)i;
-    }
-    KN_CHECK(hipMemcpyAsync(dev->sx, stX, sizeof(double) * Na, hipMemcpyHostToDevice, g_copy));
-    KN_CHECK(hipMemcpyAsync(dev->wavenum, stK, sizeof(double) * nk, hipMemcpyHostToDevice, g_copy));
-    KN_CHECK(hipMemcpyAsync(dev->sp, sd, sizeof(SpeciesDev) * need.size(), hipMemcpyHostToDevice, g_copy));
-    KN_CHECK(hipMemcpyAsync(dev->item_species, ispec, sizeof(int) * need.size(), hipMemcpyHostToDevice, g_copy));
-    // the QAG items' order: those that needed kLongChain intervals or more in
-    // the last call first (longest first), then the rest in item order
-    int nlong = 0;
-    {
-        const bool pred = dev->prev_nint.size() == (size_t)nitems;
-        for (int i = 0; i < nitems; i++)
-            if (pred && dev->prev_nint[i] >= kLongChain) ord[nlong++] = i;
-        std::stable_sort(ord, ord + nlong, [&](int x, int y) { return dev->prev_nint[x] > dev->prev_nint[y]; });
-        int j = nlong;
-        for (int i = 0; i < nitems; i++)
-            if (!(pred && dev->prev_nint[i] >= kLongChain)) ord[j++] = i;
-    }
-    KN_CHECK(hipMemcpyAsync(dev->order, ord, sizeof(int) * nitems, hipMemcpyHostToDevice, g_copy));
-    KN_CHECK(hipEventRecord(g_copied, g_copy));
-    KN_CHECK(hipStreamWaitEvent(0, g_copied, 0));
-
-    const double sinv_bw = nsb / (d->scalefact[Na - 1] - d->scalefact[0]);
     {
         const int rpw = rows_per_wave((long long)fac_windows(Na) * nk), bsp = rows_prep_spline_blocks(Na, nk, rpw);
-        hipLaunchKernelGGL(k_factor, dim3(factor_blocks(Na)), dim3(256), 0, 0, dev->sx, Na, dev->fac,
-                           dev->fac + (size_t)fac_windows(Na) * kFacStride);
-        hipLaunchKernelGGL(k_rows_prep, dim3(rows_prep_blocks(bsp, nsb)), dim3(256), 0, 0, dev->sx, dev->Y, dev->C, Na,
-                           nk, (long long)namax, bsp, nsb, sinv_bw, dev->bucket, dev->fac, rpw);
+        hipLaunchKernelGGL(k_prep, dim3(prep_blocks(bsp, nfs)), dim3(256), 0, 0,
+                           PrepArgs{dev->Y, dev->C, Na, nk, (long long)namax, bsp, rpw, dev->fac,
+                                    fs_knots(x0, xa, nfs), dev->fy, dev->fc, nfs});
     }
     QagArgs qa;
     qa.H = H;
@@ -1665,10 +1692,11 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
                        dev->order, nlong);
     KN_CHECK(hipGetLastError());
     if (g_qag_timing) KN_CHECK(hipEventRecord(g_qag_ev[1], 0));
-    KN_CHECK(hipMemcpyAsync(res, dev->out, sizeof(double) * nitems, hipMemcpyDeviceToHost, 0));
-    KN_CHECK(hipMemcpyAsync(nint, dev->nint, sizeof(int) * nitems, hipMemcpyDeviceToHost, 0));
-    KN_CHECK(hipMemcpyAsync(status, dev->status, sizeof(int) * 2, hipMemcpyDeviceToHost, 0));
+    KN_CHECK(hipMemcpyAsync(io + L.status, dev->io + L.status, L.end - L.status, hipMemcpyDeviceToHost, 0));
+    initial_piece();  // while the device works
     KN_CHECK(hipStreamSynchronize(0));
+    const int *status = (const int *)(io + L.status), *nint = (const int *)(io + L.nint);
+    const double *res = (const double *)(io + L.out);
     if (status[1] || status[0]) {
         if (status[1])
             kn_set_last_error("GSL_ERROR-equivalent: interpolation outside the stored table (GSL_EDOM)");
@@ -1721,19 +1749,23 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
     const int rc = dnu_solve(d, a, wavenum, 1, &s, out.data(), true, true);
     if (rc) return rc;
     if (delta_nu) memcpy(delta_nu, out.data(), sizeof(double) * nk);
-    // initial-condition piece (delta_tot_table.c:522-535)
-    const double fsl_A0a = fslength(log(d->TimeTransfer), log(a), d->light);
-    const double lin = 1. + kn_deriv_prefac(d) * fsl_A0a;
-    const double m = s.mnubykT > 0 ? s.mnubykT : 1;
-    const double nfl0 = d->omnu->hybnu.nufrac_low[0];
     double mb = 0.0;
-    for (int k = 0; k < nk; k++) {
-        const double kk = wavenum[k] * fsl_A0a / m;
-        if (init_bar) init_bar[k] = gbar[k] * specialJ(kk, 0, nfl0) * lin;
-        if (s.mnubykT > 0) mb += gbar[k] * fit_dJdx(kk) * (-kk / m) * d->delta_nu_init[k] * lin;
-    }
+    // initial-condition piece (delta_tot_table.c:522-535)
+    auto initial_piece = [&] {
+        const double fsl_A0a = fslength(log(d->TimeTransfer), log(a), d->light);
+        const double lin = 1. + kn_deriv_prefac(d) * fsl_A0a;
+        const double m = s.mnubykT > 0 ? s.mnubykT : 1;
+        const double nfl0 = d->omnu->hybnu.nufrac_low[0];
+        for (int k = 0; k < nk; k++) {
+            const double kk = wavenum[k] * fsl_A0a / m;
+            if (init_bar) init_bar[k] = gbar[k] * specialJ(kk, 0, nfl0) * lin;
+            if (s.mnubykT > 0) mb += gbar[k] * fit_dJdx(kk) * (-kk / m) * d->delta_nu_init[k] * lin;
+        }
+    };
     if (dtot_bar && (s.ic_only || Na < 2)) memset(dtot_bar, 0, sizeof(double) * (size_t)nk * Na);
-    if (!s.ic_only && Na >= 2) {
+    if (s.ic_only || Na < 2) {
+        initial_piece();
+    } else {
         DnuDev *dev = g_dev[d];
         const int namax = dev->ystride;  // rows of Y, C and ybar are namax doubles apart
         const size_t ny = (size_t)nk * Na, nyd = (size_t)nk * namax;
@@ -1750,7 +1782,9 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
             }
             dev->cap_adj_k = (size_t)nk * P;
         }
-        KN_CHECK(hipMemcpy(dev->gbar, gbar, sizeof(double) * nk, hipMemcpyHostToDevice));
+        double *stg = (double *)pinned_stage(1, sizeof(double) * nk);
+        memcpy(stg, gbar, sizeof(double) * nk);
+        KN_CHECK(hipMemcpyAsync(dev->gbar, stg, sizeof(double) * nk, hipMemcpyHostToDevice, 0));
         const int nfs = 16 * Na, nsb = 4 * Na;
         const double sinv_bw = nsb / (d->scalefact[Na - 1] - d->scalefact[0]);
         const double vcrit = s.qc > 0 ? d->omnu->hybnu.vcrit : 0.0;
@@ -1786,7 +1820,7 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
         KN_CHECK(hipGetLastError());
         // results through the pinned stage: [mu_bar (nk x windows) | dL/d delta_tot (nk Na)]
         const size_t nmu = (size_t)nk * P;
-        double *mub = (double *)pinned_stage(sizeof(double) * (nmu + (dtot_bar ? ny : 0))), *yb = mub + nmu;
+        double *mub = (double *)pinned_stage(0, sizeof(double) * (nmu + (dtot_bar ? ny : 0))), *yb = mub + nmu;
         KN_CHECK(hipMemcpyAsync(mub, dev->mubar, sizeof(double) * nmu, hipMemcpyDeviceToHost, 0));
         // dL/d delta_tot comes back in chunks: the host copies one out while the next is in flight
         static hipEvent_t done[4];
@@ -1800,6 +1834,7 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
                                           0));
             KN_CHECK(hipEventRecord(done[c], 0));
         }
+        initial_piece();  // while the device works
         KN_CHECK(chunks ? hipEventSynchronize(done[0]) : hipStreamSynchronize(0));  // mu_bar went first
         for (size_t i = 0; i < nmu; i++) mb += mub[i];  // k-major, windows in order
         for (int c = 0; c < chunks; c++) {
@@ -1929,7 +1964,7 @@ struct GroupDesc {
 };
 
 // phases (rows of the prefix table)
-enum { kPhFs, kPhFactor, kPhRows, kPhFsSpline, kPhQag, kPhIc, kPhAdj, kPhases };
+enum { kPhFs, kPhKnots, kPhPrep, kPhQag, kPhIc, kPhAdj, kPhases };
 constexpr int kMergedRestBlocks = 1280;
 
 // The hardware deals the blocks of a grid to the 8 XCDs in turn (block b to
@@ -1966,6 +2001,11 @@ struct GroupPush {
     __device__ void operator()(int node) const { list[atomicAdd(count, 1)] = ((long long)h << 32) | node; }
 };
 
+// A history's blocks: its fslength nodes, then (knots_block) its knots.  (Beside
+// the form with panels in LDS, one block per CU, the knots have a launch of their
+// own: 20 us for 256 histories, 45 as blocks of that one.)
+__device__ inline KnotsArgs group_knots(const GroupDesc &d) { return {d.sx, d.na, d.nsb, d.sinv_bw, d.fac, d.bucket}; }
+
 __global__ __launch_bounds__(256) void k_m_fs_first(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
                                                     int nhist, long long *__restrict__ list, int *__restrict__ count)
 {
@@ -1973,14 +2013,26 @@ __global__ __launch_bounds__(256) void k_m_fs_first(const GroupDesc *__restrict_
     const int h = hist_of(pre, nhist, blk);
     const GroupDesc &d = D[h];
     if (!d.integ) return;
+    const int b = blk - pre[h], fsb = fs_first_blocks(d.nfs);
+    if (b >= fsb) {
+        knots_block(group_knots(d), b - fsb);
+        return;
+    }
     const GroupPush push = {list, count, h};
     FslIntegrand f;
     f.H = d.H;
     fs_first_tile(f, RuleConst(), d.nfs, d.x0, d.xa, d.light, d.fx, d.fy, d.status,
-                  (int)(((blk - pre[h]) * blockDim.x + threadIdx.x) >> 6), push);
+                  (int)((b * blockDim.x + threadIdx.x) >> 6), push);
 }
 
-// The same for large groups: a block takes kFsChunk nodes of one history and
+__global__ __launch_bounds__(256) void k_m_knots(const GroupDesc *__restrict__ D, const int *__restrict__ pre, int nhist)
+{
+    const int blk = xcd_block();
+    const int h = hist_of(pre, nhist, blk);
+    if (D[h].integ) knots_block(group_knots(D[h]), blk - pre[h]);
+}
+
+// k_m_fs_first's nodes for large groups: a block takes kFsChunk nodes of one history and
 // first copies the panels they read (from its first node's to log a's) and the
 // rule to LDS.  The evaluations load ten coefficients each: through the L1 (64
 // bytes per clock and CU) that alone is 80 clocks per wavefront and point, from
@@ -2033,37 +2085,20 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_fs_rest(const GroupDe
     }
 }
 
-__global__ __launch_bounds__(256) void k_m_factor(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
-                                                  int nhist)
+__device__ inline PrepArgs group_prep(const GroupDesc &d)
 {
-    const int blk = xcd_block();
-    const int h = hist_of(pre, nhist, blk);
-    const GroupDesc &d = D[h];
-    if (!d.integ) return;
-    factor_block(d.sx, d.na, d.fac, d.fac + (size_t)fac_windows(d.na) * kFacStride, blk - pre[h]);
+    return {d.Y, d.C, d.na, d.nk, (long long)d.na_max, d.bsp, d.rpw, d.fac, fs_knots(d.x0, d.xa, d.nfs), d.fy, d.fc, d.nfs};
 }
 
-__global__ __launch_bounds__(256, 4) void k_m_rows_prep(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
-                                                     int nhist)
+__global__ __launch_bounds__(256, 4) void k_m_prep(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
+                                                   int nhist)
 {
     const int blk = xcd_block();
     const int h = hist_of(pre, nhist, blk);
     const GroupDesc &d = D[h];
     if (!d.integ) return;
     __shared__ double lds[5 * kTriSpan];
-    rows_prep_block(d.sx, d.Y, d.C, d.na, d.nk, (long long)d.na_max, d.bsp, d.nsb, d.sinv_bw, d.bucket, d.fac,
-                    d.rpw, blk - pre[h], lds);
-}
-
-__global__ __launch_bounds__(256) void k_m_fs_spline(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
-                                                     int nhist)
-{
-    const int blk = xcd_block();
-    const int h = hist_of(pre, nhist, blk);
-    const GroupDesc &d = D[h];
-    const long long item = (long long)(blk - pre[h]) * 4 + (threadIdx.x >> 6);
-    if (!d.integ || item >= (d.nfs + kKeep - 1) / kKeep) return;  // wave-uniform
-    spline_item_wave(d.fx, d.fy, d.fc, d.nfs, 0LL, 0LL, item);
+    prep_block(group_prep(d), blk - pre[h], lds);
 }
 
 __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDesc *__restrict__ D,
@@ -2500,9 +2535,8 @@ void group_plan(kn_group *g)
         long long cnt[kPhases] = {};
         if (p_integ) {
             cnt[kPhFs] = g->fs_lds ? (16LL * np + kFsChunk - 1) / kFsChunk : fs_first_blocks(16 * np);
-            cnt[kPhFactor] = factor_blocks(np);
-            cnt[kPhRows] = rows_prep_blocks(rows_prep_spline_blocks(np, d.nk, rpw), 4 * np);
-            cnt[kPhFsSpline] = spline_blocks(16 * np, 1);
+            cnt[g->fs_lds ? kPhKnots : kPhFs] += knots_blocks(np, 4 * np, 256);
+            cnt[kPhPrep] = prep_blocks(rows_prep_spline_blocks(np, d.nk, rpw), 16 * np);
             cnt[kPhQag] = blocks_for(d.nk);
             cnt[kPhAdj] = (long long)d.nk * fac_windows(np) + (d.nk + 63) / 64;
         }
@@ -2549,11 +2583,11 @@ void group_forward_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
                        fy, d.status, fs_list, fs_count);
     hipLaunchKernelGGL(k_fs_rest, dim3(kFsRestBlocks), dim3(64 * kWavesPerBlock), 0, s, d.H, nfs, q.x0, q.xa,
                        q.spec.light, fx, fy, d.status, fs_list, fs_count);
-    hipLaunchKernelGGL(k_factor, dim3(factor_blocks(na)), dim3(256), 0, s, d.sx, na, d.fac,
-                       d.fac + (size_t)fac_windows(na) * kFacStride);
-    hipLaunchKernelGGL(k_rows_prep, dim3(rows_prep_blocks(d.bsp, d.nsb)), dim3(256), 0, s, d.sx, d.Y, d.C, na, nk,
-                       (long long)na_max, d.bsp, d.nsb, d.sinv_bw, d.bucket, d.fac, d.rpw);
-    hipLaunchKernelGGL(k_spline, dim3(spline_blocks(nfs, 1)), dim3(256), 0, s, fx, fy, fc, nfs, 1, 0LL, 0LL);
+    hipLaunchKernelGGL(k_knots, dim3(knots_blocks(na, d.nsb, 256)), dim3(256), 0, s,
+                       KnotsArgs{d.sx, na, d.nsb, d.sinv_bw, d.fac, d.bucket});
+    hipLaunchKernelGGL(k_prep, dim3(prep_blocks(d.bsp, nfs)), dim3(256), 0, s,
+                       PrepArgs{d.Y, d.C, na, nk, (long long)na_max, d.bsp, d.rpw, d.fac, fs_knots(q.x0, q.xa, nfs), fy,
+                                fc, nfs});
     QagArgs a;
     a.H = d.H;
     a.fx = fx;
@@ -2650,12 +2684,10 @@ void group_launch_merged(kn_group *g, hipStream_t s, bool forward, bool adjoint)
             hipLaunchKernelGGL(k_m_fs_rest, dim3(kMergedRestBlocks), dim3(64 * kWavesPerBlock), 0, s, g->desc,
                                g->mlist, g->status + 3 * n);
         }
-        if (g->tot[kPhFactor])
-            hipLaunchKernelGGL(k_m_factor, dim3(g->tot[kPhFactor]), dim3(256), 0, s, g->desc, pre(kPhFactor), n);
-        if (g->tot[kPhRows])
-            hipLaunchKernelGGL(k_m_rows_prep, dim3(g->tot[kPhRows]), dim3(256), 0, s, g->desc, pre(kPhRows), n);
-        if (g->tot[kPhFsSpline])
-            hipLaunchKernelGGL(k_m_fs_spline, dim3(g->tot[kPhFsSpline]), dim3(256), 0, s, g->desc, pre(kPhFsSpline), n);
+        if (g->tot[kPhKnots])
+            hipLaunchKernelGGL(k_m_knots, dim3(g->tot[kPhKnots]), dim3(256), 0, s, g->desc, pre(kPhKnots), n);
+        if (g->tot[kPhPrep])
+            hipLaunchKernelGGL(k_m_prep, dim3(g->tot[kPhPrep]), dim3(256), 0, s, g->desc, pre(kPhPrep), n);
         if (g->tot[kPhQag])
             hipLaunchKernelGGL(k_m_dnu_qag, dim3(g->tot[kPhQag]), dim3(64 * kWavesPerBlock), g->qag_lds, s,
                                g->desc, pre(kPhQag), n);

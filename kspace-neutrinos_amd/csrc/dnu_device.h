@@ -567,7 +567,9 @@ __device__ __forceinline__ double sph_j0(double x)
 //   al = qc j0 + qc c, be = qc^2 j0, ga = qc^2 x^2 j0 + 2c, de = qc x^2 c - qc x^2 j0,
 // so that a term is three fused multiply-adds, the squared denominator's
 // reciprocal and one more fused multiply-add.  SJTerms holds one point's
-// per-x factors; specialJ and specialJ2 run the same operations per point.
+// per-x factors; specialJ and specialJ2 run the same operations per point, four
+// terms at a time: their weights come by one scalar load (757 k x 2000 steps:
+// 103 us, with two at a time 108, with all nineteen 130 for the registers).
 struct SJTerms {
     double y, al, be, ga, de, integ;
 };
@@ -597,7 +599,7 @@ __device__ __forceinline__ double specialJ(double x, const JPar &P)
 {
     if (P.qc > 0) {
         SJTerms t = sj_terms(x, P.qc);
-#pragma unroll 2
+#pragma unroll 4
         for (int n = 1; n < 20; n++) sj_term(t, n, ((n & 1) ? 1.0 : -1.0) * P.en[n]);
         return t.integ / (1.5 * 1.202056903159594 * (1 - P.nufrac_low));
     }
@@ -610,7 +612,7 @@ __device__ __forceinline__ void specialJ2(double x1, double x2, const JPar &P, d
 {
     if (P.qc > 0) {
         SJTerms t1 = sj_terms(x1, P.qc), t2 = sj_terms(x2, P.qc);
-#pragma unroll 2
+#pragma unroll 4
         for (int n = 1; n < 20; n++) {
             const double w = ((n & 1) ? 1.0 : -1.0) * P.en[n];
             sj_term(t1, n, w);
@@ -1636,17 +1638,6 @@ constexpr int kWarm = 32;
 constexpr int kRun = 10;                        // rows per lane
 constexpr int kKeep = 64 * kRun - 2 * kHalo;    // rows kept per window (544)
 
-// Right-hand side of the natural-spline system (GSL cspline): 3 (dy/h right - dy/h left).
-struct SplineRhs {
-    const double *x, *y;
-    __device__ __forceinline__ double operator()(int i) const
-    {
-        const double hl = x[i] - x[i - 1], hr = x[i + 1] - x[i];
-        const double gl = hl != 0.0 ? 1.0 / hl : 0.0, gr = hr != 0.0 ? 1.0 / hr : 0.0;
-        return 3.0 * ((y[i + 1] - y[i]) * gr - (y[i] - y[i - 1]) * gl);
-    }
-};
-
 // A lane's share of a window: rows [s, s + len) of the window's interior
 // rows [wa, wb).
 struct TriLane {
@@ -1739,17 +1730,7 @@ __device__ __forceinline__ TriScan tri_scan(const double (&g)[kRun], double g_be
 // reciprocal knot spacings ih.
 // OUT: where the kept rows go (set for the solution, add for ADJ_RHS); IH:
 // the reciprocal spacings.  Each kept row receives exactly one set or add.
-struct OutDirect {
-    double *o;
-    __device__ __forceinline__ void set(int i, double v) const { o[i] = v; }
-    __device__ __forceinline__ void add(int i, double v) const { o[i] += v; }
-};
-struct IhDirect {
-    const double *ih;
-    __device__ __forceinline__ double operator()(int i) const { return ih[i]; }
-};
-
-template <class RHS, bool ADJ_RHS, class OUT = OutDirect, class IH = IhDirect>
+template <class RHS, bool ADJ_RHS, class OUT, class IH>
 __device__ __forceinline__ void tri_solve(int n, const RHS &rhs, int lo, int hi, const OUT &out, const TriLane &t,
                                           const double (&g)[kRun], const double (&ial)[kRun], double g_before,
                                           const TriScan &S, const IH &ih)
@@ -1830,22 +1811,6 @@ __device__ __forceinline__ void tri_solve(int n, const RHS &rhs, int lo, int hi,
     }
 }
 
-// One window [lo, hi) of natural-spline rows by one wavefront (factors
-// formed in place).
-template <class RHS>
-__device__ __forceinline__ void tridiag_window_wave(const double *x, int n, const RHS &rhs, int lo, int hi, double *out)
-{
-    const int lane = threadIdx.x & 63;
-    if (n < 3) {
-        for (int i = lo + lane; i < hi; i += 64) out[i] = 0.0;
-        return;
-    }
-    const TriLane t = tri_lane(n, lo, hi);
-    double g[kRun], ial[kRun], gb;
-    tri_factor(x, t, g, ial, gb);
-    tri_solve<RHS, false>(n, rhs, lo, hi, OutDirect{out}, t, g, ial, gb, tri_scan(g, gb), IhDirect{nullptr});
-}
-
 // The windows of rows that share their knots: one for up to 64 kRun interior
 // rows, else equal shares of at most kKeep kept rows (window w keeps
 // [w keep, (w + 1) keep)).
@@ -1861,7 +1826,7 @@ __host__ __device__ inline int fac_keep(int n)
 // gam_{s-1} per lane (from the values tri_factor forms in each wavefront).
 constexpr int kFacStride = (2 * kRun + 1) * 64;
 
-__device__ inline void tri_factor_store(const double *x, int n, int w, double *fac)
+__device__ __forceinline__ void tri_factor_store(const double *x, int n, int w, double *fac)
 {
     const int lane = threadIdx.x & 63;
     const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
@@ -1913,7 +1878,8 @@ __device__ __forceinline__ void store_span(double *dst, const double (&v)[kTriPa
     }
 }
 
-// SplineRhs's values, bit for bit, from staged y and ih (ys[k] = y[base + k]).
+// Right-hand side of the natural-spline system (GSL cspline): 3 (dy/h right -
+// dy/h left), from staged y and ih (ys[k] = y[base + k]).
 struct SplineRhsLds {
     const double *ys, *ihs;
     int base;
@@ -1954,7 +1920,7 @@ __device__ __forceinline__ void tri_factor_load(const double *__restrict__ fac, 
     gb = f[2 * kRun * 64 + lane];
 }
 
-// tridiag_window_wave for window w of a wavefront's rows r0, r0 + step, ... <
+// Spline coefficients for window w of a wavefront's rows r0, r0 + step, ... <
 // rend, on knots whose factors are stored (fac_windows(n) windows, then the
 // reciprocal spacings): the coefficients of row Y + r ystride go to C + r
 // ystride.  The window is staged through LDS (sa: kTriSpan doubles of the
@@ -1995,6 +1961,82 @@ __device__ __forceinline__ void tri_rows_staged(int n, int w, const double *__re
             if (k < hi - lo) out[k] = sa[k];
         }
         wave_lds_sync();
+    }
+}
+
+// ---- the fslength table's spline: knots evenly spaced but for their rounding ----
+// With one spacing h the factors need no knots: alp_i = h / gam_i, gam_i = 1 /
+// (4 - gam_{i-1}) from gam_0 = 0, at its limit 2 - sqrt(3) to the last bit by
+// row 16.  The stored knots differ from even ones by their rounding, d <= 4e-16
+// in x; what that changes in the factors (relative d / h) reaches the spline's
+// values as h^2 c d / h, below what d itself changes in them, dy/dx d.  The
+// right-hand side, where a second difference would magnify it, takes each
+// interval's own length: 1 / h corrected by one Newton step (relative (d /
+// h)^2).  Small solves wait for a chain of divisions in the general factors:
+// 1600 knots 11.6 us with them.
+constexpr int kGamRows = 20;
+struct GamTab {
+    double g[kGamRows + 1];
+    constexpr GamTab() : g()
+    {
+        for (int i = 1; i <= kGamRows; i++) g[i] = 1.0 / (4.0 - g[i - 1]);
+    }
+};
+static_assert(kGamRows == 2 * kRun, "rows 1 .. 20 are those of a first window's lanes 0 and 1");
+
+struct UniformRhsLds {
+    const double *ys;
+    UniformKnots kn;
+    double ih0;
+    int base;
+    __device__ __forceinline__ double slope(double xl, double xr, double yl, double yr) const
+    {
+        return (yr - yl) * fma(fma(xl - xr, ih0, 1.0), ih0, ih0);
+    }
+    __device__ __forceinline__ double operator()(int i) const
+    {
+        const int k = i - base;
+        const double xm = kn.at(i), ym = ys[k];
+        return 3.0 * (slope(xm, kn.at(i + 1), ym, ys[k + 1]) - slope(kn.at(i - 1), xm, ys[k - 1], ym));
+    }
+};
+struct NoIh {
+    __device__ __forceinline__ double operator()(int) const { return 0.0; }
+};
+
+// Window w (of fac_windows(n), n >= 3) of the fslength table's coefficients c
+// by one wavefront; sa: kTriSpan doubles of its own LDS.
+__device__ __forceinline__ void uniform_spline_wave(const UniformKnots &kn, const double *__restrict__ y,
+                                                    double *__restrict__ c, int n, int w, double *sa)
+{
+    constexpr GamTab kGam;
+    const int lane = threadIdx.x & 63;
+    const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
+    const TriLane t = tri_lane(n, lo, hi);
+    const int base = t.wa - 1, cnt = t.wb - base + 1;  // y[wa - 1 .. wb]
+    double v[kTriPass], g[kRun], ial[kRun];
+    load_span(v, y + base, cnt);
+    const double h = kn.span * kn.rden, ih0 = h > 0.0 ? 1.0 / h : 0.0;
+    // rows 1 .. 20 of a first window (its rows start at 1; the other windows' start beyond 20)
+    const bool l0 = t.wa == 1 && lane == 0, l1 = t.wa == 1 && lane == 1;
+#pragma unroll
+    for (int j = 0; j < kRun; j++) {
+        const double gj = l0 ? kGam.g[1 + j] : (l1 ? kGam.g[kRun + 1 + j] : kGam.g[kGamRows]);
+        g[j] = j < t.len ? gj : 0.0;
+        ial[j] = g[j] * ih0;
+    }
+    const double before = lane == 0 ? 0.0 : (l1 ? kGam.g[kRun] : kGam.g[kGamRows]);
+    const TriScan S = tri_scan(g, before);
+    store_span(sa, v, cnt);
+    wave_lds_sync();
+    // the staged row is all read before the first kept row is written
+    tri_solve<UniformRhsLds, false>(n, UniformRhsLds{sa, kn, ih0, base}, lo, hi, OutLds{sa, lo}, t, g, ial, before, S,
+                                    NoIh{});
+    wave_lds_sync();
+#pragma unroll
+    for (int p = 0; p < kTriPass; p++) {
+        const int k = p * 64 + lane;
+        if (k < hi - lo) c[lo + k] = sa[k];
     }
 }
 
