@@ -377,6 +377,8 @@ struct QagArgs {
 };
 
 // Histories of at most this many stored steps have their log a values copied
+// (STAGED: a form of its own, so that the compiler knows the copy for LDS and
+// does not read it by flat accesses)
 // to LDS by the QAG kernels (48 KB, one copy for the block's four wavefronts).
 constexpr int kStageMax = 6144;
 
@@ -384,9 +386,10 @@ constexpr int kStageMax = 6144;
 // stored log a values (na <= kStageMax), or null to read them from memory.
 // The integrand of item (species sp, wavenumber index k), with the stored
 // log a values read from sx (device memory or their LDS copy).
-__device__ inline DnuIntegrand dnu_integrand(const QagArgs &a, const SpeciesDev &sp, int k, const double *sx)
+template <bool HYB>
+__device__ inline DnuIntegrand<HYB> dnu_integrand(const QagArgs &a, const SpeciesDev &sp, int k, const double *sx)
 {
-    DnuIntegrand f;
+    DnuIntegrand<HYB> f;
     f.H = a.H;
     f.fy = a.fy;
     f.fc = a.fc;
@@ -445,11 +448,12 @@ __device__ __forceinline__ void stage_knots(const double *__restrict__ sx, int n
     __syncthreads();
 }
 
+template <bool HYB>
 __device__ inline void dnu_qag_item(const QagArgs &a, const SpeciesDev &sp, int item, int k, QagWs &ws,
                                     const double *sx)
 {
     const int lane = threadIdx.x & 63;
-    const DnuIntegrand f = dnu_integrand(a, sp, k, sx);
+    const DnuIntegrand<HYB> f = dnu_integrand<HYB>(a, sp, k, sx);
     double r;
     int ni;
     const int rc = wave_qag61(f, a.x0, a.xa, sp.relerr, kLimit, ws, &r, &ni);
@@ -458,16 +462,11 @@ __device__ inline void dnu_qag_item(const QagArgs &a, const SpeciesDev &sp, int 
 
 // One item by the W wavefronts of a block (block_qag61: speculative
 // bisections on the wavefronts other than the first).
-template <int W>
+template <bool HYB, int W>
 __device__ inline void dnu_qag_item_block(const QagArgs &a, const SpeciesDev &sp, int item, int k, QagBlock<W> &S,
-                                          double *sxs)
+                                          const double *sx)
 {
-    const double *sx = a.sx;
-    if (sxs) {
-        stage_knots(a.sx, a.ns, sxs, 64 * W);
-        sx = sxs;
-    }
-    const DnuIntegrand f = dnu_integrand(a, sp, k, sx);
+    const DnuIntegrand<HYB> f = dnu_integrand<HYB>(a, sp, k, sx);
     double r;
     int ni;
     const int rc = block_qag61<W>(f, a.x0, a.xa, sp.relerr, kLimit, S, &r, &ni);
@@ -480,15 +479,17 @@ __device__ inline void dnu_qag_item_block(const QagArgs &a, const SpeciesDev &sp
 #define KN_QAG_SPEC 4
 #endif
 constexpr int kQagSpec = KN_QAG_SPEC;
+template <bool STAGED, bool HYB>
 __global__ __launch_bounds__(64 * kQagSpec) void k_dnu_qag_spec(QagArgs a, const SpeciesDev *__restrict__ sp,
                                                                  const int *__restrict__ item_species, int nk,
                                                                  int nitems)
 {
     __shared__ QagBlock<kQagSpec> S;
-    HIP_DYNAMIC_SHARED(double, sxs)  // a.ns doubles when a.ns <= kStageMax
+    HIP_DYNAMIC_SHARED(double, sxs)  // STAGED: a.ns doubles
     const int nsp = nitems / nk, b = (int)blockIdx.x;
     const int k = nk - 1 - b / nsp, item = (b % nsp) * nk + k;
-    dnu_qag_item_block<kQagSpec>(a, sp[item_species[item / nk]], item, k, S, a.ns <= kStageMax ? sxs : nullptr);
+    if constexpr (STAGED) stage_knots(a.sx, a.ns, sxs, 64 * kQagSpec);
+    dnu_qag_item_block<HYB, kQagSpec>(a, sp[item_species[item / nk]], item, k, S, STAGED ? sxs : a.sx);
 }
 
 // Items in a given order: the first nlong (expected to need long bisection
@@ -499,24 +500,38 @@ union QagMixLds {
     QagBlock<kQagSpec> blk;
     QagWs ws[kQagSpec];
 };
+template <bool STAGED, bool HYB>
 __global__ __launch_bounds__(64 * kQagSpec) void k_dnu_qag_mix(QagArgs a, const SpeciesDev *__restrict__ sp,
                                                                 const int *__restrict__ item_species, int nk,
                                                                 int nitems, const int *__restrict__ order, int nlong)
 {
     __shared__ QagMixLds U;
-    HIP_DYNAMIC_SHARED(double, sxs)  // a.ns doubles when a.ns <= kStageMax
-    double *st = a.ns <= kStageMax ? sxs : nullptr;
+    HIP_DYNAMIC_SHARED(double, sxs)  // STAGED: a.ns doubles
     const int b = (int)blockIdx.x;
+    if constexpr (STAGED) stage_knots(a.sx, a.ns, sxs, 64 * kQagSpec);
+    const double *sx = STAGED ? sxs : a.sx;
     if (b < nlong) {  // block-uniform
         const int item = order[b];
-        dnu_qag_item_block<kQagSpec>(a, sp[item_species[item / nk]], item, item % nk, U.blk, st);
+        dnu_qag_item_block<HYB, kQagSpec>(a, sp[item_species[item / nk]], item, item % nk, U.blk, sx);
         return;
     }
     const int wave = threadIdx.x >> 6, j = nlong + (b - nlong) * kQagSpec + wave;
-    if (st) stage_knots(a.sx, a.ns, st, 64 * kQagSpec);
     if (j >= nitems) return;
     const int item = order[j];
-    dnu_qag_item(a, sp[item_species[item / nk]], item, item % nk, U.ws[wave], st ? st : a.sx);
+    dnu_qag_item<HYB>(a, sp[item_species[item / nk]], item, item % nk, U.ws[wave], sx);
+}
+
+// The form for stored steps that fit in LDS or not, and for launches with a
+// hybrid species (qc > 0) or none.
+inline auto qag_spec(bool staged, bool hyb)
+{
+    return staged ? (hyb ? k_dnu_qag_spec<true, true> : k_dnu_qag_spec<true, false>)
+                  : (hyb ? k_dnu_qag_spec<false, true> : k_dnu_qag_spec<false, false>);
+}
+inline auto qag_mix(bool staged, bool hyb)
+{
+    return staged ? (hyb ? k_dnu_qag_mix<true, true> : k_dnu_qag_mix<true, false>)
+                  : (hyb ? k_dnu_qag_mix<false, true> : k_dnu_qag_mix<false, false>);
 }
 
 // Interval counts at or above which an item is expected to gain from the
@@ -595,10 +610,14 @@ struct AdjLds {
 // this took 1339: 284 in the solve, 740 in the points' FP64, the rest in
 // gathering them and in the rows' one write.  Three waves per SIMD: with the
 // compiler's own choice of registers, which lets two run, 1411; with four,
-// which spill more, 1412.  With the scans' three steps, 1304.)
+// which spill more, 1412.  With the scans' three steps, 1304; in launches without
+// a hybrid species, whose series would take 33 registers through the fit's code
+// and spill 52 bytes a lane, and by global instead of flat accesses, 1075.  Its
+// LDS allows three waves anyway.)
 // Points that reach the window (x within [sx[E0 - 1], sx[E1]]) are queued and
 // evaluated 64 at a time, one per lane; a point's d/d(m/kT) term belongs to
 // the window that keeps its si, so every term is counted once.
+template <bool HYB>
 __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
 {
     const int nk = A.nk, ns = A.ns, nfs = A.nfs, lane = threadIdx.x & 63;
@@ -629,7 +648,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
     double mu_acc = 0.0;
     auto eval = [&](double x, double w) {
         // the pieces of delta_tot_table.c:492-500; the spline's knots and values at the bucket's knot and the next
-        // two, loaded before the knot walk (as DnuIntegrand::eval2)
+        // two, loaded before the knot walk
         int q = (int)((x - sx0) * A.sinv_bw);
         q = q < 0 ? 0 : (q > A.nsb ? A.nsb : q);
         const int b = A.sb[q], i0 = b < 0 ? 0 : (b > ns - 2 ? ns - 2 : b), i2 = i0 + 2 < ns ? i0 + 2 : ns - 1;
@@ -654,7 +673,7 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
         }
         const double kx = kk * fsl / mnubykT;
         double Jx, Jq;
-        const double Jv = specialJ_d(kx, J, Jx, Jq);
+        const double Jv = specialJ_d<HYB>(kx, J, Jx, Jq);
         const double dx = x - sl, h = sr - sl;
         const double S0 = linear ? (h > 0.0 ? yl + dx / h * (yr - yl) : yl) : cspline_val(sl, sr, yl, yr, cl, cr, x);
         const bool own = si >= lo && si < hi, own1 = si + 1 >= lo && si + 1 < hi;
@@ -747,10 +766,11 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
         for (int t = ns + lane; t < A.ystride; t += 64) yrow[t] = 0.0;
 }
 
+template <bool HYB>
 __global__ __launch_bounds__(64, 3) void k_dnu_adj(AdjArgs A)
 {
     __shared__ AdjLds S;
-    dnu_adj_block(A, blockIdx.x, S);
+    dnu_adj_block<HYB>(A, blockIdx.x, S);
 }
 
 // ---------------------------------------------------------------- state
@@ -1566,11 +1586,13 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
     memcpy(io + L.wavenum, wavenum, sizeof(double) * nk);
     SpeciesDev *sd = (SpeciesDev *)(io + L.sp);
     int *ispec = (int *)(io + L.species), *ord = (int *)(io + L.order);
+    bool hyb = false;
     for (size_t i = 0; i < need.size(); i++) {
         const kn_species &q = sp[need[i]];
         sd[i].mnubykT = q.mnubykT;
         sd[i].relerr = q.relerr;
         sd[i].J.qc = q.qc;
+        hyb = hyb || q.qc > 0;
         sd[i].J.nufrac_low = nfl0;
         sd[i].J.en[0] = 1.0;
         for (int n = 1; n < 20; n++) sd[i].J.en[n] = exp(-n * q.qc);
@@ -1687,7 +1709,7 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
     qa.ic.init = nullptr;
     qa.ic.fsl0 = qa.ic.lin = qa.ic.prefac = 0.0;
     if (g_qag_timing) KN_CHECK(hipEventRecord(g_qag_ev[0], 0));
-    hipLaunchKernelGGL(k_dnu_qag_mix, dim3(nlong + (nitems - nlong + kQagSpec - 1) / kQagSpec), dim3(64 * kQagSpec),
+    hipLaunchKernelGGL(qag_mix(Na <= kStageMax, hyb), dim3(nlong + (nitems - nlong + kQagSpec - 1) / kQagSpec), dim3(64 * kQagSpec),
                        Na <= kStageMax ? sizeof(double) * Na : 0, 0, qa, dev->sp, dev->item_species, nk, nitems,
                        dev->order, nlong);
     KN_CHECK(hipGetLastError());
@@ -1816,7 +1838,7 @@ extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, cons
         A.mu_bar = dev->mubar;
         A.fac = dev->fac;
         A.ica = IcAdjArgs{nullptr, 0.0, 0.0, nullptr, nullptr};
-        hipLaunchKernelGGL(k_dnu_adj, dim3(nk * P), dim3(64), 0, 0, A);
+        hipLaunchKernelGGL(s.qc > 0 ? k_dnu_adj<true> : k_dnu_adj<false>, dim3(nk * P), dim3(64), 0, 0, A);
         KN_CHECK(hipGetLastError());
         // results through the pinned stage: [mu_bar (nk x windows) | dL/d delta_tot (nk Na)]
         const size_t nmu = (size_t)nk * P;
@@ -1949,11 +1971,11 @@ struct GroupHist {
 // na_max doubles apart).
 struct GroupDesc {
     HTab H;
-    double *sx, *Y;
-    const double *wavenum, *init, *gbar;
-    double *C, *fx, *fy, *fc, *out, *ivl, *dbar, *mubar, *ibar, *mbic, *fac;
-    int *bucket, *nint, *status;
-    const SpeciesDev *sp;
+    GlobalPtr<double> sx, Y;
+    GlobalPtr<const double> wavenum, init, gbar;
+    GlobalPtr<double> C, fx, fy, fc, out, ivl, dbar, mubar, ibar, mbic, fac;
+    GlobalPtr<int> bucket, nint, status;
+    GlobalPtr<const SpeciesDev> sp;
     // the stored steps and what they set: live in device memory (the device
     // append updates them), read by every launch
     int nk, na, na_max, nfs, nsb, bsp, rpw, integ, ic_only;
@@ -2101,19 +2123,19 @@ __global__ __launch_bounds__(256, 4) void k_m_prep(const GroupDesc *__restrict__
     prep_block(group_prep(d), blk - pre[h], lds);
 }
 
+template <bool STAGED, bool HYB>
 __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDesc *__restrict__ D,
                                                                     const int *__restrict__ pre, int nhist)
 {
     __shared__ QagWs ws[kWavesPerBlock];
-    HIP_DYNAMIC_SHARED(double, sxs)  // min(largest na, kStageMax) doubles
+    HIP_DYNAMIC_SHARED(double, sxs)  // STAGED: the largest na doubles
     const int blk = xcd_block();
     const int h = hist_of(pre, nhist, blk);
     const GroupDesc &d = D[h];
     const int wave = threadIdx.x >> 6;
     const int k = (blk - pre[h]) * kWavesPerBlock + wave;
     if (!d.integ) return;
-    const bool staged = d.na <= kStageMax;
-    if (staged) stage_knots(d.sx, d.na, sxs, 64 * kWavesPerBlock);
+    if constexpr (STAGED) stage_knots(d.sx, d.na, sxs, 64 * kWavesPerBlock);
     if (k >= d.nk) return;
     QagArgs a;
     a.H = d.H;
@@ -2140,7 +2162,16 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDe
     a.ic.fsl0 = d.fsl0;
     a.ic.lin = d.lin;
     a.ic.prefac = d.prefac;
-    dnu_qag_item(a, *d.sp, k, k, ws[wave], staged ? sxs : d.sx);
+    dnu_qag_item<HYB>(a, *d.sp, k, k, ws[wave], STAGED ? sxs : a.sx);
+}
+
+// k_m_dnu_qag's form (qag_spec).  256 histories, 73 k items: 647 us with the
+// integrand's knot walks as loops, flat accesses and the hybrid series in every
+// launch; 462 us now, three wavefronts per SIMD.
+inline auto m_qag(bool staged, bool hyb)
+{
+    return staged ? (hyb ? k_m_dnu_qag<true, true> : k_m_dnu_qag<true, false>)
+                  : (hyb ? k_m_dnu_qag<false, true> : k_m_dnu_qag<false, false>);
 }
 
 // initial-condition-only histories, 64 k per block
@@ -2187,6 +2218,7 @@ __global__ __launch_bounds__(64) void k_m_ic_adj(const GroupDesc *__restrict__ D
     }
 }
 
+template <bool HYB>
 __global__ __launch_bounds__(64, 3) void k_m_dnu_adj(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
                                                   int nhist)
 {
@@ -2223,7 +2255,7 @@ __global__ __launch_bounds__(64, 3) void k_m_dnu_adj(const GroupDesc *__restrict
     A.mu_bar = d.mubar;
     A.fac = d.fac;
     A.ica = group_ica(d);
-    dnu_adj_block(A, blk - pre[h], S);
+    dnu_adj_block<HYB>(A, blk - pre[h], S);
 }
 
 // One more stored step per history, on the device (one wavefront per
@@ -2330,6 +2362,8 @@ struct kn_group {
     long long *mlist = nullptr;  // pass-2 fslength list (fs_tot entries)
     std::vector<GroupDesc> desc_h;
     size_t qag_lds = 0;  // staged log a values of the longest stageable history
+    bool qag_staged = true;
+    bool hyb = true;  // a history has, or (device append) may get, a hybrid species
     size_t fs_lds = 0;   // k_m_fs_first_lds: the longest H table's coefficients (0: k_m_fs_first)
     int tot[kPhases] = {};
     hipStream_t st[kGroupStreams] = {};
@@ -2550,10 +2584,13 @@ void group_plan(kn_group *g)
     for (int p = 0; p < kPhases; p++) g->tot[p] = (int)acc[p];
     g->qag_lds = 0;
     for (int i = 0; i < n; i++) {
-        const int np = g->cap_plan ? (g->h[i].spec.na_max < kStageMax ? g->h[i].spec.na_max : kStageMax) : g->h[i].na;
-        if ((g->cap_plan || g->h[i].integ) && np <= kStageMax && sizeof(double) * np > g->qag_lds)
-            g->qag_lds = sizeof(double) * np;
+        const int np = g->cap_plan ? g->h[i].spec.na_max : g->h[i].na;
+        if ((g->cap_plan || g->h[i].integ) && sizeof(double) * np > g->qag_lds) g->qag_lds = sizeof(double) * np;
     }
+    g->hyb = false;
+    for (const GroupHist &q : g->h) g->hyb = g->hyb || q.spec.hybrid || q.spec.qc > 0;
+    g->qag_staged = g->qag_lds <= sizeof(double) * kStageMax;
+    if (!g->qag_staged) g->qag_lds = 0;
     KN_CHECK(hipMemcpy(g->desc, g->desc_h.data(), sizeof(GroupDesc) * n, hipMemcpyHostToDevice));
     KN_CHECK(hipMemcpy(g->pre, pre.data(), sizeof(int) * pre.size(), hipMemcpyHostToDevice));
     group_meta_upload(g);
@@ -2613,7 +2650,7 @@ void group_forward_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
     a.ic.fsl0 = q.fsl0;
     a.ic.lin = q.lin;
     a.ic.prefac = q.spec.delta_nu_prefac;
-    hipLaunchKernelGGL(k_dnu_qag_spec, dim3(nk), dim3(64 * kQagSpec), na <= kStageMax ? sizeof(double) * na : 0, s,
+    hipLaunchKernelGGL(qag_spec(na <= kStageMax, g->hyb), dim3(nk), dim3(64 * kQagSpec), na <= kStageMax ? sizeof(double) * na : 0, s,
                        a, g->sp + i, g->spec0, nk, nk);
 }
 
@@ -2665,7 +2702,7 @@ void group_adjoint_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
     A.fac = d.fac;
     A.ica = ica;
     // nk x windows item blocks, then the initial-condition piece's blocks
-    hipLaunchKernelGGL(k_dnu_adj, dim3(nk * fac_windows(na) + (nk + 63) / 64), dim3(64), 0, s, A);
+    hipLaunchKernelGGL(g->hyb ? k_dnu_adj<true> : k_dnu_adj<false>, dim3(nk * fac_windows(na) + (nk + 63) / 64), dim3(64), 0, s, A);
 }
 
 // The whole group in one grid per phase, on stream s.
@@ -2689,13 +2726,13 @@ void group_launch_merged(kn_group *g, hipStream_t s, bool forward, bool adjoint)
         if (g->tot[kPhPrep])
             hipLaunchKernelGGL(k_m_prep, dim3(g->tot[kPhPrep]), dim3(256), 0, s, g->desc, pre(kPhPrep), n);
         if (g->tot[kPhQag])
-            hipLaunchKernelGGL(k_m_dnu_qag, dim3(g->tot[kPhQag]), dim3(64 * kWavesPerBlock), g->qag_lds, s,
-                               g->desc, pre(kPhQag), n);
+            hipLaunchKernelGGL(m_qag(g->qag_staged, g->hyb), dim3(g->tot[kPhQag]),
+                               dim3(64 * kWavesPerBlock), g->qag_lds, s, g->desc, pre(kPhQag), n);
         if (g->tot[kPhIc]) hipLaunchKernelGGL(k_m_ic, dim3(g->tot[kPhIc]), dim3(64), 0, s, g->desc, pre(kPhIc), n);
     }
     if (adjoint) {
         if (g->tot[kPhAdj])
-            hipLaunchKernelGGL(k_m_dnu_adj, dim3(g->tot[kPhAdj]), dim3(64), 0, s, g->desc, pre(kPhAdj), n);
+            hipLaunchKernelGGL(g->hyb ? k_m_dnu_adj<true> : k_m_dnu_adj<false>, dim3(g->tot[kPhAdj]), dim3(64), 0, s, g->desc, pre(kPhAdj), n);
         if (g->tot[kPhIc])
             hipLaunchKernelGGL(k_m_ic_adj, dim3(g->tot[kPhIc]), dim3(64), 0, s, g->desc, pre(kPhIc), n);
     }

@@ -264,6 +264,20 @@ inline void h_table(double x0, double w, int npanel, Hub hub, std::vector<double
 // out-of-line pieces.
 typedef const __attribute__((address_space(1))) double gconst_double;
 
+// A pointer kept in a descriptor in memory, known to point to global memory: as
+// a generic one it would be used by flat accesses, which wait for the LDS
+// counter too and cannot be told apart while in flight.
+template <class T>
+struct GlobalPtr {
+    __attribute__((address_space(1))) T *p;
+    __host__ __device__ __forceinline__ GlobalPtr &operator=(T *q)
+    {
+        p = (__attribute__((address_space(1))) T *)q;
+        return *this;
+    }
+    __host__ __device__ __forceinline__ operator T *() const { return (T *)p; }
+};
+
 // x's panel p (clamped to the table) and the place v in [0, 1] across it.
 struct HLoc {
     int p;
@@ -588,16 +602,20 @@ __device__ __forceinline__ void sj_term(SJTerms &t, int n, double w)
     const double d = n2 + t.y;
     t.integ = fma(w * rcp_fast(d * d), ii, t.integ);
 }
-__device__ __forceinline__ double sj_fit(double x)
+__device__ __forceinline__ double sj_fit(double x0)
 {
-    if (x <= 0.) return 1.;
+    const double x = x0 <= 0. ? 1. : x0;  // a select, not a branch: two points' chains then overlap
     const double x2 = x * x, x4 = x2 * x2, x8 = x4 * x4;
-    return (1. + 0.0168 * x2 + 0.0407 * x4) / (1. + 2.1734 * x2 + 1.6787 * exp(4.1811 * log(x)) + 0.1467 * x8);
+    const double v = (1. + 0.0168 * x2 + 0.0407 * x4) / (1. + 2.1734 * x2 + 1.6787 * exp(4.1811 * log(x)) + 0.1467 * x8);
+    return x0 <= 0. ? 1. : v;
 }
 
+// HYB false: every species of the launch has qc = 0, and the series is left out
+// (its registers, and the sine's, would be held through the fit's code too).
+template <bool HYB = true>
 __device__ __forceinline__ double specialJ(double x, const JPar &P)
 {
-    if (P.qc > 0) {
+    if (HYB && P.qc > 0) {
         SJTerms t = sj_terms(x, P.qc);
 #pragma unroll 4
         for (int n = 1; n < 20; n++) sj_term(t, n, ((n & 1) ? 1.0 : -1.0) * P.en[n]);
@@ -608,9 +626,10 @@ __device__ __forceinline__ double specialJ(double x, const JPar &P)
 
 // specialJ at two points, the two series in one loop (two independent
 // chains per term); each point's operations are specialJ's.
+template <bool HYB>
 __device__ __forceinline__ void specialJ2(double x1, double x2, const JPar &P, double &j1, double &j2)
 {
-    if (P.qc > 0) {
+    if (HYB && P.qc > 0) {
         SJTerms t1 = sj_terms(x1, P.qc), t2 = sj_terms(x2, P.qc);
 #pragma unroll 4
         for (int n = 1; n < 20; n++) {
@@ -638,16 +657,11 @@ __device__ __forceinline__ double cspline_val(double xl, double xr, double yl, d
     return yl + dx * (b + dx * (ci + dx * d));
 }
 
-__device__ __forceinline__ double cspline_at(const double *xa, const double *ya, const double *c, int i, double x)
+__device__ __forceinline__ double linear_val(double xl, double xr, double yl, double yr, double x)
 {
-    return cspline_val(xa[i], xa[i + 1], ya[i], ya[i + 1], c[i], c[i + 1], x);
-}
-
-__device__ __forceinline__ double linear_at(const double *xa, const double *ya, int i, double x)
-{
-    const double xl = xa[i], h = xa[i + 1] - xl;
-    if (h > 0.0) return ya[i] + (x - xl) / h * (ya[i + 1] - ya[i]);
-    return ya[i];
+    const double h = xr - xl;
+    if (h > 0.0) return yl + (x - xl) / h * (yr - yl);
+    return yl;
 }
 
 // The fslength table's knots are x0 + i (xa - x0) / (n - 1.) (delta_tot_table.c:582),
@@ -676,6 +690,22 @@ __device__ __forceinline__ int settle_uniform(const UniformKnots &u, int n, int 
         xl = xr;
         xr = u.at(++i + 1);
     }
+    return i;
+}
+
+// One step of settle_uniform either way from the guess, without its loops: the
+// rounding of (x - x0) / h moves the guess by one knot at most unless the knots
+// are a few units in the last place apart.  settled: whether x's interval was
+// reached, i.e. settle_uniform's answer.
+__device__ __forceinline__ int step_uniform(const UniformKnots &u, int n, int i, double x, double &xl, double &xr,
+                                            bool &settled)
+{
+    i = i < 0 ? 0 : (i > n - 2 ? n - 2 : i);
+    const double l = u.at(i), r = u.at(i + 1);
+    i += (int)(i < n - 2 && r <= x) - (int)(i > 0 && l > x);
+    xl = u.at(i);
+    xr = u.at(i + 1);
+    settled = !(i > 0 && xl > x) && !(i < n - 2 && xr <= x);
     return i;
 }
 
@@ -723,6 +753,7 @@ struct FslIntegrandLds {
     __device__ __forceinline__ double split(double x) const { return h_split(H, h_locate(H, x).p, x, 0); }
 };
 
+template <bool HYB>
 struct DnuIntegrand {  // delta_tot_table.c:492-500
     HTab H;
     const double *fy, *fc;  // fslength spline on the uniform knots fk
@@ -736,70 +767,75 @@ struct DnuIntegrand {  // delta_tot_table.c:492-500
     double k, mnubykT, k_by_m;  // k_by_m = k / mnubykT
     const JPar *J;  // in device memory: the series weights are read where used
     int *edom;
-    __device__ __forceinline__ double operator()(double x) const
+    // One point's place in the tables: its knot intervals, the fslength spline's values and 1 / (a H).
+    struct Point {
+        bool in;
+        int si;
+        double xl, xr, f0, f1, g0, g1;  // fslength: interval, values, coefficients
+        double sl, sr;                  // delta_tot's interval
+        double ih;
+    };
+    // Straight-line code, so that the loads of both points are in flight together:
+    // one step from the fslength guess, the bucket's knot or one of the next two.
+    // again: x lies further off (walk() finds it).
+    __device__ __forceinline__ Point place(double x, bool &again) const
     {
-        if (x < fx0 || x > fxhi || x < sx0 || x > sxhi) {
-            atomicOr(edom, 1);  // GSL_EDOM in gsl_interp_eval -> terminate(2001)
-            return 0.0;
-        }
-        double xl, xr;
-        const int fi = settle_uniform(fk, nfs, (int)((x - fx0) * finv_h), x, xl, xr);
-        const double fsl = cspline_val(xl, xr, fy[fi], fy[fi + 1], fc[fi], fc[fi + 1], x);
+        Point p;
+        p.in = !(x < fx0 || x > fxhi || x < sx0 || x > sxhi);
         int q = (int)((x - sx0) * sinv_bw);
         q = q < 0 ? 0 : (q > nsb ? nsb : q);
-        const int si = settle(sx, ns, sbucket[q], x);
-        const double dtot = linear ? linear_at(sx, sy, si, x) : cspline_at(sx, sy, sc, si, x);
-        const double specJ = specialJ(k_by_m * fsl, *J);
-        return fsl * inv_ah(H, x) * specJ * dtot;  // fsl / (a H) specJ dtot
+        const int b = sbucket[q];
+        bool settled;
+        const int fi = step_uniform(fk, nfs, (int)((x - fx0) * finv_h), x, p.xl, p.xr, settled);
+        p.f0 = fy[fi], p.f1 = fy[fi + 1], p.g0 = fc[fi], p.g1 = fc[fi + 1];
+        const HLoc L = h_locate(H, x);
+        p.ih = h_regular(H, L, 1);
+        const int i = b < 0 ? 0 : (b > ns - 2 ? ns - 2 : b), last = ns - 1;
+        const int i1 = i + 1, i2 = i + 2 < last ? i + 2 : last, i3 = i + 3 < last ? i + 3 : last;
+        const double t0 = sx[i], t1 = sx[i1], t2 = sx[i2], t3 = sx[i3];
+        const bool up1 = i1 < last && t1 <= x, up2 = i2 < last && t2 <= x, up3 = i3 < last && t3 <= x;
+        p.si = up1 ? (up2 ? i2 : i1) : i;
+        p.sl = up1 ? (up2 ? t2 : t1) : t0;
+        p.sr = up1 ? (up2 ? t3 : t2) : t1;
+        again = !settled || (i > 0 && t0 > x) || up3 || p.ih != p.ih;
+        return p;
     }
-    // Two points with operator()'s arithmetic, in straight-line code so that
-    // their dependent loads (bucket, knot walk, coefficients, H panel) overlap;
-    // use1 / use2 say which results are used.  A used point outside the
-    // tables flags GSL_EDOM and gives 0; the indices of every point are
-    // clamped into the tables, so an unused or outside point reads in bounds.
+    // The same from any distance, and in a split H panel.
+    __device__ __forceinline__ void walk(double x, Point &p) const
+    {
+        const int fi = settle_uniform(fk, nfs, (int)((x - fx0) * finv_h), x, p.xl, p.xr);
+        p.f0 = fy[fi], p.f1 = fy[fi + 1], p.g0 = fc[fi], p.g1 = fc[fi + 1];
+        p.si = settle(sx, ns, p.si, x);
+        p.sl = sx[p.si], p.sr = sx[p.si + 1];
+        if (p.ih != p.ih) p.ih = h_split(H, h_locate(H, x).p, x, 1);
+    }
+    // Two points.  A used point outside the tables flags GSL_EDOM and gives 0;
+    // the indices of every point are clamped into the tables, so an unused or
+    // outside point reads in bounds.  (With the knot walks as loops, a branch per
+    // spline interval and the series' code beside the fit's, a rule took 9000-11000
+    // clocks.)
     __device__ __forceinline__ void eval2(double x1, double x2, bool use1, bool use2, double &r1, double &r2) const
     {
-        const bool in1 = !(x1 < fx0 || x1 > fxhi || x1 < sx0 || x1 > sxhi);
-        const bool in2 = !(x2 < fx0 || x2 > fxhi || x2 < sx0 || x2 > sxhi);
-        if ((use1 && !in1) || (use2 && !in2)) atomicOr(edom, 1);
-        double xl1, xr1, xl2, xr2;
-        const int fi1 = settle_uniform(fk, nfs, (int)((x1 - fx0) * finv_h), x1, xl1, xr1);
-        const int fi2 = settle_uniform(fk, nfs, (int)((x2 - fx0) * finv_h), x2, xl2, xr2);
-        int q1 = (int)((x1 - sx0) * sinv_bw), q2 = (int)((x2 - sx0) * sinv_bw);
-        q1 = q1 < 0 ? 0 : (q1 > nsb ? nsb : q1);
-        q2 = q2 < 0 ? 0 : (q2 > nsb ? nsb : q2);
-        const int b1 = sbucket[q1], b2 = sbucket[q2];
-        // the delta_tot spline's values at the bucket's knot and the next two,
-        // loaded before the knot walk (which moves at most one knot up but
-        // rarely); the walk's result picks the pair
-        const int i1 = b1 < 0 ? 0 : (b1 > ns - 2 ? ns - 2 : b1), i2 = b2 < 0 ? 0 : (b2 > ns - 2 ? ns - 2 : b2);
-        const int u1 = i1 + 2 < ns ? i1 + 2 : ns - 1, u2 = i2 + 2 < ns ? i2 + 2 : ns - 1;
-        const double y10 = sy[i1], y11 = sy[i1 + 1], y12 = sy[u1], y20 = sy[i2], y21 = sy[i2 + 1], y22 = sy[u2];
-        double c10 = 0.0, c11 = 0.0, c12 = 0.0, c20 = 0.0, c21 = 0.0, c22 = 0.0;
-        if (!linear) {
-            c10 = sc[i1], c11 = sc[i1 + 1], c12 = sc[u1];
-            c20 = sc[i2], c21 = sc[i2 + 1], c22 = sc[u2];
-        }
-        const double fsl1 = cspline_val(xl1, xr1, fy[fi1], fy[fi1 + 1], fc[fi1], fc[fi1 + 1], x1);
-        const double fsl2 = cspline_val(xl2, xr2, fy[fi2], fy[fi2 + 1], fc[fi2], fc[fi2 + 1], x2);
-        const double ih1 = inv_ah(H, x1), ih2 = inv_ah(H, x2);
-        const int si1 = settle(sx, ns, b1, x1), si2 = settle(sx, ns, b2, x2);
-        double dt1, dt2;
+        bool again1, again2;
+        Point p1 = place(x1, again1), p2 = place(x2, again2);
+        if (again1) walk(x1, p1);
+        if (again2) walk(x2, p2);
+        const double y10 = sy[p1.si], y11 = sy[p1.si + 1], c10 = sc[p1.si], c11 = sc[p1.si + 1];
+        const double y20 = sy[p2.si], y21 = sy[p2.si + 1], c20 = sc[p2.si], c21 = sc[p2.si + 1];
+        const double fsl1 = cspline_val(p1.xl, p1.xr, p1.f0, p1.f1, p1.g0, p1.g1, x1);
+        const double fsl2 = cspline_val(p2.xl, p2.xr, p2.f0, p2.f1, p2.g0, p2.g1, x2);
+        double j1, j2, dt1, dt2;
+        specialJ2<HYB>(k_by_m * fsl1, k_by_m * fsl2, *J, j1, j2);
         if (linear) {
-            dt1 = linear_at(sx, sy, si1, x1);
-            dt2 = linear_at(sx, sy, si2, x2);
+            dt1 = linear_val(p1.sl, p1.sr, y10, y11, x1);
+            dt2 = linear_val(p2.sl, p2.sr, y20, y21, x2);
         } else {
-            dt1 = si1 == i1       ? cspline_val(sx[si1], sx[si1 + 1], y10, y11, c10, c11, x1)
-                  : si1 == i1 + 1 ? cspline_val(sx[si1], sx[si1 + 1], y11, y12, c11, c12, x1)
-                                  : cspline_at(sx, sy, sc, si1, x1);
-            dt2 = si2 == i2       ? cspline_val(sx[si2], sx[si2 + 1], y20, y21, c20, c21, x2)
-                  : si2 == i2 + 1 ? cspline_val(sx[si2], sx[si2 + 1], y21, y22, c21, c22, x2)
-                                  : cspline_at(sx, sy, sc, si2, x2);
+            dt1 = cspline_val(p1.sl, p1.sr, y10, y11, c10, c11, x1);
+            dt2 = cspline_val(p2.sl, p2.sr, y20, y21, c20, c21, x2);
         }
-        double j1, j2;
-        specialJ2(k_by_m * fsl1, k_by_m * fsl2, *J, j1, j2);
-        r1 = in1 ? fsl1 * ih1 * j1 * dt1 : 0.0;
-        r2 = in2 ? fsl2 * ih2 * j2 * dt2 : 0.0;
+        r1 = p1.in ? fsl1 * p1.ih * j1 * dt1 : 0.0;  // fsl / (a H) specJ dtot
+        r2 = p2.in ? fsl2 * p2.ih * j2 * dt2 : 0.0;
+        if ((use1 && !p1.in) || (use2 && !p2.in)) atomicOr(edom, 1);  // GSL_EDOM in gsl_interp_eval -> terminate(2001)
     }
 };
 
@@ -812,9 +848,9 @@ __device__ __forceinline__ void eval_pair(const F &f, double x1, double x2, bool
     r1 = use1 ? f(x1) : 0.0;
     r2 = use2 ? f(x2) : 0.0;
 }
-template <>
-__device__ __forceinline__ void eval_pair<DnuIntegrand>(const DnuIntegrand &f, double x1, double x2, bool use1,
-                                                        bool use2, double &r1, double &r2)
+template <bool HYB>
+__device__ __forceinline__ void eval_pair(const DnuIntegrand<HYB> &f, double x1, double x2, bool use1, bool use2,
+                                          double &r1, double &r2)
 {
     f.eval2(x1, x2, use1, use2, r1, r2);
     r1 = use1 ? r1 : 0.0;
@@ -930,9 +966,22 @@ struct GK {
     double res, err, resabs, resasc;
 };
 
+// The rule's node and weights of a lane of gk61_pair, read once per QAG.
+struct RuleLane {
+    double x, wk, wg;
+    __device__ __forceinline__ RuleLane()
+    {
+        const int j = threadIdx.x & 31;
+        x = j <= 30 ? c_xgk[j] : 0.0;
+        wk = j <= 30 ? c_wgk[j] : 0.0;
+        wg = (j < 30 && (j & 1)) ? c_wg[j >> 1] : 0.0;
+    }
+};
+
 // 61-point Gauss-Kronrod on [a1,b1] (lanes 0-31) and [a2,b2] (lanes 32-63).
 template <class F>
-__device__ __forceinline__ void gk61_pair(const F &f, double a1, double b1, double a2, double b2, GK &g1, GK &g2)
+__device__ __forceinline__ void gk61_pair(const F &f, const RuleLane &rule, double a1, double b1, double a2, double b2,
+                                          GK &g1, GK &g2)
 {
 #pragma clang fp contract(off)  // every product and sum rounded as written (gk61_q4's sums match bit for bit)
     const int lane = threadIdx.x & 63, hf = lane >> 5, j = lane & 31;
@@ -943,11 +992,10 @@ __device__ __forceinline__ void gk61_pair(const F &f, double a1, double b1, doub
     // integrand twice, not three times
     double f1 = 0.0, f2 = 0.0;
     {
-        const double dx = j <= 30 ? h * c_xgk[j] : 0.0;
+        const double dx = j <= 30 ? h * rule.x : 0.0;
         eval_pair(f, c - dx, c + dx, j <= 30, j < 30, f1, f2);
     }
-    const double wk = j <= 30 ? c_wgk[j] : 0.0;
-    const double wgv = (j < 30 && (j & 1)) ? c_wg[j >> 1] : 0.0;
+    const double wk = rule.wk, wgv = rule.wg;
     const double sk = half_sum(j == 30 ? wk * f1 : wk * (f1 + f2));
     const double sg = half_sum(wgv * (f1 + f2));
     const double sa = half_sum(j == 30 ? wk * fabs(f1) : wk * (fabs(f1) + fabs(f2)));
@@ -1277,6 +1325,7 @@ __device__ int wave_qag61(const F &f, double a, double b, double epsrel, int lim
     // the first estimate and the bisections share one copy of the rule's code
     // (the integrand inlined at two places is beyond the instruction cache)
     const bool lead = (threadIdx.x & 63) == 0;
+    const RuleLane rule;
     int imax = 0, os = 0;
     bool ord_lds = false;
     double es = 0.0, tol = 0.0, area = 0.0, errsum = 0.0;  // es, os: the error order in registers (ord_insert)
@@ -1284,7 +1333,7 @@ __device__ int wave_qag61(const F &f, double a, double b, double epsrel, int lim
     int n = 0, it = 1, rt1 = 0, rt2 = 0, etype = 0;
     for (;;) {
         GK g1, g2;
-        gk61_pair(f, a1, b1, a2, b2, g1, g2);
+        gk61_pair(f, rule, a1, b1, a2, b2, g1, g2);
         if (n == 0) {
             *result = g1.res;
             *nint = 1;
@@ -1402,10 +1451,11 @@ __device__ int block_qag61(const F &f, double a, double b, double epsrel, int li
     const bool lead = threadIdx.x == 0;  // lane 0 of wavefront 0 writes the list and the slots
     QagWs &w = S.ws;
     // pass 0: wavefront 0 the first estimate; wavefront 1 the halves of [a, b] (the first bisection)
+    const RuleLane rule;
     GK g0, gx;
     if (wave <= 1) {
         const double m = 0.5 * (a + b);
-        gk61_pair(f, a, wave ? m : b, wave ? m : a, b, g0, gx);
+        gk61_pair(f, rule, a, wave ? m : b, wave ? m : a, b, g0, gx);
         if (wave == 1 && (threadIdx.x & 63) == 0) {
             S.slot[1].used = 1;
             S.slot[1].lo = a;
@@ -1594,7 +1644,7 @@ __device__ int block_qag61(const F &f, double a, double b, double epsrel, int li
             if (sl.eval) {
                 const double lo = sl.lo, hi = sl.hi, m = 0.5 * (lo + hi);
                 GK g1, g2;
-                gk61_pair(f, lo, m, m, hi, g1, g2);
+                gk61_pair(f, rule, lo, m, m, hi, g1, g2);
                 if ((threadIdx.x & 63) == 0) {
                     sl.g1 = g1;
                     sl.g2 = g2;
@@ -2057,9 +2107,10 @@ __device__ __forceinline__ double sph_j0_prime(double z)
 }
 
 // specialJ(x, qc) with its partial derivatives d/dx and d/dqc.
+template <bool HYB = true>
 __device__ inline double specialJ_d(double x, const JPar &P, double &dJdx, double &dJdqc)
 {
-    if (P.qc > 0) {
+    if (HYB && P.qc > 0) {
         const double qc = P.qc;
         const double z = qc * x;
         double s, c;
