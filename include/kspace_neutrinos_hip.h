@@ -314,6 +314,19 @@ const char *kn_last_error(void);
 int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
                          const double *gbar, int nout, fftw_complex *d_field_bar, void *stream);
 
+/* The spectrum and its adjoint for callers that keep both on the device:
+ * d_power (room for nrbins) receives the values total_powerspectrum returns in
+ * power, *nout their number; the adjoint takes them back with d_gbar[nout] =
+ * dL/dpower and writes d_field_bar as kn_bin_power_adjoint does, without
+ * sweeping the field for the sums again.  Both run after the work stream has
+ * been given so far and before what it is given next, and do not wait for the
+ * device. */
+int kn_power_spectrum_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
+                             double *d_power, int *nout, void *stream);
+int kn_power_spectrum_adjoint_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
+                                     const double *d_power, const double *d_gbar, int nout,
+                                     fftw_complex *d_field_bar, void *stream);
+
 /* ---- (b) one history of a group: what one get_delta_nu call integrates ----
  * (delta_tot_table.c:507-611): its stored log a values and delta_tot rows,
  * its own H(a), mass and hybrid setting.  qc, relerr and ic_only are what

@@ -28,6 +28,7 @@
 // read-free kernel and cached (bit-exact, deterministic).
 #include <math.h>
 #include <string.h>
+#include <mutex>
 #include <vector>
 
 #include "kn_hip.h"
@@ -69,8 +70,11 @@ struct BinGeom {
     double *d_partial;      // max(grid, ggrid) * nrbins
     unsigned *d_cpartial;   // ggrid * nrbins (geometry pass)
     double *d_sum;          // nrbins + 1 (last: |F0|^2)
-    double *d_alpha;        // nrbins, adjoint coefficients (allocated on first use)
+    double *d_alpha;        // nrbins + 1, adjoint coefficients, then the zero mode's (allocated on first use)
     int agrid;              // adjoint-sweep grid
+    int nout;               // non-empty bins
+    int *d_slot;            // nrbins: a bin's place among them, -1 if empty (with d_count: allocated on first use)
+    double *d_count;        // nrbins
 };
 
 std::vector<BinGeom *> g_geoms;
@@ -398,8 +402,46 @@ void launch_power(BinGeom *g, const double2 *F, hipStream_t st, double *sum_out 
     launch_sweep(a, g->plan, st, sum_out, mass_out);
 }
 
+// kn_finish_powerspectrum's normalisation and compaction, with its operations:
+// the sums of the non-empty bins over |F0|^2, then over their counts.
+__global__ __launch_bounds__(256) void k_power_finish(const double *__restrict__ sums, const int *__restrict__ slot,
+                                                      const double *__restrict__ count, int nrbins,
+                                                      double *__restrict__ power)
+{
+    const int b = blockIdx.x * 256 + threadIdx.x;
+    if (b < nrbins && slot[b] >= 0) power[slot[b]] = sums[b] / sums[nrbins] / count[b];
+}
+
+// The adjoint sweep's coefficients from the spectrum and its gradient, one
+// block: alpha[b] = gbar / (|F0|^2 N_b), and beta = -2 sum gbar P / |F0|^2.
+constexpr int kAlphaThreads = 1024;
+__global__ __launch_bounds__(kAlphaThreads) void k_adjoint_alpha(const double2 *__restrict__ F,
+                                                                 const int *__restrict__ slot,
+                                                                 const double *__restrict__ count, int nrbins,
+                                                                 const double *__restrict__ power,
+                                                                 const double *__restrict__ gbar,
+                                                                 double *__restrict__ alpha)
+{
+    __shared__ double acc[kAlphaThreads];
+    const double2 f = F[0];
+    const double M = f.x * f.x + f.y * f.y;
+    double gp = 0.0;
+    for (int b = threadIdx.x; b < nrbins; b += kAlphaThreads) {
+        const int n = slot[b];
+        alpha[b] = n >= 0 ? gbar[n] / (M * count[b]) : 0.0;
+        if (n >= 0) gp += gbar[n] * power[n];
+    }
+    acc[threadIdx.x] = gp;
+#pragma unroll
+    for (int d = kAlphaThreads / 2; d >= 1; d >>= 1) {
+        __syncthreads();
+        if ((int)threadIdx.x < d) acc[threadIdx.x] += acc[threadIdx.x + d];
+    }
+    if (threadIdx.x == 0) alpha[nrbins] = -2.0 * acc[0] / M;
+}
+
 // Adjoint sweep of the binning: Fbar_m = s_m F_m with s_m = 2 c_m W_m^-4
-// alpha[bin(m)] (c_m the multiplicity) and s_0 = beta for the zero mode.
+// alpha[bin(m)] (c_m the multiplicity) and s_0 = alpha[nrbins] for the zero mode.
 // Reads 16 B and writes 16 B per mode; software-pipelined like the rescale sweep.
 constexpr int kAdjWaves = 8;
 constexpr int kAdjUnroll = 2;
@@ -412,9 +454,9 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_bin_adjoint(const double2 *_
                                                                 long long rows, int nrbins,
                                                                 const int *__restrict__ thr_g,
                                                                 const double *__restrict__ iw_g,
-                                                                const double *__restrict__ alpha_g, float half_bpu,
-                                                                double beta)
+                                                                const double *__restrict__ alpha_g, float half_bpu)
 {
+    const double beta = alpha_g[nrbins];
     extern __shared__ double smem[];
     const double *alpha = alpha_g, *iw = iw_g;
     const int *thr = thr_g;
@@ -475,6 +517,71 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_bin_adjoint(const double2 *_
 }
 
 size_t adjoint_smem(int dims, int nrbins) { return sizeof(double) * (size_t)(nrbins + dims) + sizeof(int) * (nrbins + 1); }
+
+// The adjoint sweep's coefficient buffer and grid, on first use.
+void adjoint_ready(BinGeom *g)
+{
+    if (g->d_alpha) return;
+    const bool global = adjoint_smem(g->dims, g->nrbins) > kLdsMax;
+    KN_CHECK(hipMalloc(&g->d_alpha, sizeof(double) * (g->nrbins + 1)));
+    const long long rows = (long long)g->nslab * g->dims;
+    const int per_cu = global ? resident_blocks(k_bin_adjoint<true>, 64 * kAdjWaves, 0)
+                              : resident_blocks(k_bin_adjoint<false>, 64 * kAdjWaves, adjoint_smem(g->dims, g->nrbins));
+    const long long ag = (long long)per_cu * num_cus();
+    g->agrid = (int)(rows < ag ? rows : ag);
+}
+
+// The sweep with the coefficients in d_alpha.
+void launch_adjoint(BinGeom *g, const double2 *F, double2 *Fb, hipStream_t st)
+{
+    const bool global = adjoint_smem(g->dims, g->nrbins) > kLdsMax;
+    hipLaunchKernelGGL(global ? k_bin_adjoint<true> : k_bin_adjoint<false>, dim3(g->agrid), dim3(64 * kAdjWaves),
+                       global ? 0 : adjoint_smem(g->dims, g->nrbins), st, F, Fb, g->dims, g->startslab,
+                       (long long)g->nslab * g->dims, g->nrbins, g->d_thr, g->d_iw, g->d_alpha, g->half_bpu);
+    KN_CHECK(hipGetLastError());
+}
+
+// The bins' places and counts on the device, on first use.
+void slots_ready(BinGeom *g)
+{
+    if (g->d_slot) return;
+    std::vector<int> slot(g->nrbins, -1);
+    std::vector<double> count(g->nrbins);
+    for (int b = 0; b < g->nrbins; b++) {
+        count[b] = (double)g->count[b];
+        if (g->count[b]) slot[b] = g->nout++;
+    }
+    int *d_slot;
+    KN_CHECK(hipMalloc(&d_slot, sizeof(int) * g->nrbins));
+    KN_CHECK(hipMalloc(&g->d_count, sizeof(double) * g->nrbins));
+    KN_CHECK(hipMemcpy(d_slot, slot.data(), sizeof(int) * g->nrbins, hipMemcpyHostToDevice));
+    KN_CHECK(hipMemcpy(g->d_count, count.data(), sizeof(double) * g->nrbins, hipMemcpyHostToDevice));
+    g->d_slot = d_slot;
+}
+
+// What a geometry keeps is shared by its calls, so those that do not wait run
+// in the order of the default stream, whatever stream they are for: after that
+// stream's work so far, and before what it is given next.
+std::mutex g_turn;  // one thread's launches of a call stay together
+struct DefaultStreamTurn {
+    std::lock_guard<std::mutex> lock{g_turn};
+    hipStream_t st;
+    hipEvent_t ev = nullptr;
+    explicit DefaultStreamTurn(hipStream_t s) : st(s)
+    {
+        if (!st) return;
+        KN_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        KN_CHECK(hipEventRecord(ev, st));
+        KN_CHECK(hipStreamWaitEvent(0, ev, 0));
+    }
+    void done()
+    {
+        if (!st) return;
+        KN_CHECK(hipEventRecord(ev, 0));
+        KN_CHECK(hipStreamWaitEvent(st, ev, 0));
+        KN_CHECK(hipEventDestroy(ev));
+    }
+};
 
 }  // namespace
 
@@ -684,7 +791,7 @@ extern "C" int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int n
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
     hipStream_t st = (hipStream_t)stream;
     launch_power(g, (const double2 *)d_field, st);
-    std::vector<double> sums(nrbins + 1), alpha(nrbins, 0.0);
+    std::vector<double> sums(nrbins + 1), alpha(nrbins + 1, 0.0);
     KN_CHECK(hipMemcpyAsync(sums.data(), g->d_sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost, st));
     KN_CHECK(hipStreamSynchronize(st));
     const double M = sums[nrbins];
@@ -704,26 +811,60 @@ extern "C" int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int n
         kn_set_last_error("kn_bin_power_adjoint: nout=%d but the forward has %d non-empty bins", nout, nonzero);
         return KN_ERR_ARG;
     }
-    const bool adj_global = adjoint_smem(dims, nrbins) > kLdsMax;
-    const size_t asmem = adj_global ? 0 : adjoint_smem(dims, nrbins);
-    if (!g->d_alpha) {
-        KN_CHECK(hipMalloc(&g->d_alpha, sizeof(double) * nrbins));
-        const long long rows = (long long)nslab * dims;
-        const int per_cu = adj_global ? resident_blocks(k_bin_adjoint<true>, 64 * kAdjWaves, 0)
-                                      : resident_blocks(k_bin_adjoint<false>, 64 * kAdjWaves, asmem);
-        const long long ag = (long long)per_cu * num_cus();
-        g->agrid = (int)(rows < ag ? rows : ag);
-    }
-    KN_CHECK(hipMemcpyAsync(g->d_alpha, alpha.data(), sizeof(double) * nrbins, hipMemcpyHostToDevice, st));
-    if (adj_global)
-        hipLaunchKernelGGL(k_bin_adjoint<true>, dim3(g->agrid), dim3(64 * kAdjWaves), 0, st, (const double2 *)d_field,
-                           (double2 *)d_field_bar, dims, startslab, (long long)nslab * dims, nrbins, g->d_thr,
-                           g->d_iw, g->d_alpha, g->half_bpu, -2.0 * gp / M);
-    else
-        hipLaunchKernelGGL(k_bin_adjoint<false>, dim3(g->agrid), dim3(64 * kAdjWaves), asmem, st,
-                           (const double2 *)d_field, (double2 *)d_field_bar, dims, startslab, (long long)nslab * dims,
-                           nrbins, g->d_thr, g->d_iw, g->d_alpha, g->half_bpu, -2.0 * gp / M);
-    KN_CHECK(hipGetLastError());
+    alpha[nrbins] = -2.0 * gp / M;
+    adjoint_ready(g);
+    KN_CHECK(hipMemcpyAsync(g->d_alpha, alpha.data(), sizeof(double) * (nrbins + 1), hipMemcpyHostToDevice, st));
+    launch_adjoint(g, (const double2 *)d_field, (double2 *)d_field_bar, st);
     KN_CHECK(hipStreamSynchronize(st));
+    return 0;
+}
+
+extern "C" int kn_power_spectrum_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
+                                        double *d_power, int *nout, void *stream)
+{
+    if (!d_field || !d_power || !nout) {
+        kn_set_last_error("kn_power_spectrum_device: null array");
+        return KN_ERR_ARG;
+    }
+    DefaultStreamTurn turn((hipStream_t)stream);
+    BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
+    slots_ready(g);
+    launch_power(g, (const double2 *)d_field, 0);
+    hipLaunchKernelGGL(k_power_finish, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->d_sum, g->d_slot, g->d_count,
+                       nrbins, d_power);
+    KN_CHECK(hipGetLastError());
+    if (kn_message_wanted()) {  // as total_powerspectrum; nobody to read it otherwise, and no wait
+        double mass2;
+        KN_CHECK(hipMemcpy(&mass2, g->d_sum + nrbins, sizeof(double), hipMemcpyDeviceToHost));
+        kn_message(0, "total mass of the grid, |F(k = 0)|: %g\n", sqrt(mass2));
+    }
+    turn.done();
+    *nout = g->nout;
+    return 0;
+}
+
+extern "C" int kn_power_spectrum_adjoint_device(const fftw_complex *d_field, int dims, int nrbins, int startslab,
+                                                int nslab, const double *d_power, const double *d_gbar, int nout,
+                                                fftw_complex *d_field_bar, void *stream)
+{
+    if (startslab != 0 || !d_field || !d_power || !d_gbar || !d_field_bar) {
+        kn_set_last_error("kn_power_spectrum_adjoint_device: needs startslab 0 (the zero mode) and non-null arrays");
+        return KN_ERR_ARG;
+    }
+    DefaultStreamTurn turn((hipStream_t)stream);
+    BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
+    slots_ready(g);
+    if (nout != g->nout) {
+        turn.done();
+        kn_set_last_error("kn_power_spectrum_adjoint_device: nout=%d but the forward has %d non-empty bins", nout,
+                          g->nout);
+        return KN_ERR_ARG;
+    }
+    adjoint_ready(g);
+    hipLaunchKernelGGL(k_adjoint_alpha, dim3(1), dim3(kAlphaThreads), 0, 0, (const double2 *)d_field, g->d_slot,
+                       g->d_count, nrbins, d_power, d_gbar, g->d_alpha);
+    KN_CHECK(hipGetLastError());
+    launch_adjoint(g, (const double2 *)d_field, (double2 *)d_field_bar, 0);
+    turn.done();
     return 0;
 }

@@ -137,6 +137,10 @@ SIGNATURES = {
     "kn_last_error": (C.c_char_p, []),
     "kn_bin_power_adjoint": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, dp, C.c_int, C.c_void_p,
                                        C.c_void_p]),
+    "kn_power_spectrum_device": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p,
+                                           C.POINTER(C.c_int), C.c_void_p]),
+    "kn_power_spectrum_adjoint_device": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p,
+                                                   C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
     "kn_batch_history_from_table": (C.c_int, [C.POINTER(DeltaTotTable), C.c_double, C.c_double,
                                               C.POINTER(BatchHistory)]),
     "kn_hubble_ctx": (C.c_double, [C.c_double, C.c_void_p]),
@@ -460,32 +464,34 @@ class Batch:
 def power_spectrum_function():
     """torch.autograd.Function over total_powerspectrum on a device grid:
     apply(field[dims, dims, dims/2+1, 2] float64 cuda, nrbins) -> power[n]
-    (the compacted, normalised bins); the gradient comes from
-    kn_bin_power_adjoint."""
-    import numpy as np
+    (the compacted, normalised bins), in the order of the current stream; the
+    gradient comes from kn_power_spectrum_adjoint_device and the forward's
+    spectrum."""
     import torch
 
     class PowerSpectrumFunction(torch.autograd.Function):
         @staticmethod
         def forward(ctx, field, nrbins):
             assert field.is_cuda and field.dtype == torch.float64 and field.is_contiguous()
-            dims = field.shape[0]
-            power, keffs = np.zeros(nrbins), np.zeros(nrbins)
-            count = np.zeros(nrbins, dtype=np.int64)
-            n = lib().total_powerspectrum(dims, field.data_ptr(), nrbins, 0, dims, power.ctypes.data_as(dp),
-                                          count.ctypes.data_as(llp), keffs.ctypes.data_as(dp), 0)
+            dims, n = field.shape[0], C.c_int()
+            power = torch.empty(nrbins, dtype=torch.float64, device=field.device)
+            _check(lib().kn_power_spectrum_device(field.data_ptr(), dims, nrbins, 0, dims, power.data_ptr(), C.byref(n),
+                                                  torch.cuda.current_stream(field.device).cuda_stream),
+                   "kn_power_spectrum_device")
             ctx.save_for_backward(field)
-            ctx.nrbins, ctx.n = nrbins, n
-            return torch.from_numpy(power[:n].copy()).to(field.device)
+            ctx.nrbins, ctx.n, ctx.power = nrbins, n.value, power  # a tensor of the function's own: the output is the caller's
+            return power[:n.value].clone()
 
         @staticmethod
         def backward(ctx, g):
             (field,) = ctx.saved_tensors
-            gb = np.ascontiguousarray(g.detach().cpu().numpy(), dtype=np.float64)
+            gb = g.detach().to(device=field.device, dtype=torch.float64).contiguous()
             fb = torch.empty_like(field)
-            _check(lib().kn_bin_power_adjoint(field.data_ptr(), field.shape[0], ctx.nrbins, 0, field.shape[0],
-                                              gb.ctypes.data_as(dp), ctx.n, fb.data_ptr(), None),
-                   "kn_bin_power_adjoint")
+            _check(lib().kn_power_spectrum_adjoint_device(field.data_ptr(), field.shape[0], ctx.nrbins, 0,
+                                                          field.shape[0], ctx.power.data_ptr(), gb.data_ptr(), ctx.n,
+                                                          fb.data_ptr(),
+                                                          torch.cuda.current_stream(field.device).cuda_stream),
+                   "kn_power_spectrum_adjoint_device")
             return fb, None
 
     return PowerSpectrumFunction
