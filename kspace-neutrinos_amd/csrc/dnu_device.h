@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "kn_gk61.h"
+#include "kn_powtab.h"
 
 namespace kn_dnu {
 
@@ -602,11 +603,31 @@ __device__ __forceinline__ void sj_term(SJTerms &t, int n, double w)
     const double d = n2 + t.y;
     t.integ = fma(w * rcp_fast(d * d), ii, t.integ);
 }
+// x^4.1811 of the fit, x > 0, within 2 units in the last place (kn_powtab.h:
+// two table entries and five terms) where exp(4.1811 log x), with the
+// product's rounding in the exponent, was off by up to 30, for a quarter of the
+// operations.  Outside 2^-64 .. 2^64, where the fit's other terms leave nothing of
+// it, and for infinities and NaN, which they carry, any finite value does.
+// QAG of 256 histories 455 -> 438 us, of 12 histories of 16-96 k 22.8 -> 18.2.
+__device__ __forceinline__ double pow_fit(double x)
+{
+    long long u;
+    __builtin_memcpy(&u, &x, sizeof u);
+    const int hi = (int)(u >> 32), e0 = (hi >> 20) - 1023, j = (hi >> 13) & (KN_POWTAB_N - 1);
+    const int e = e0 < -KN_POWTAB_E ? -KN_POWTAB_E : (e0 > KN_POWTAB_E ? KN_POWTAB_E : e0);
+    const long long mu = (u & 0xfffffffffffffLL) | 0x3ff0000000000000LL;
+    double m;
+    __builtin_memcpy(&m, &mu, sizeof m);
+    const double t = kn_powtab[2 * j + 1], r = fma(m, kn_powtab[2 * j], -1.0);
+    const double q = r * fma(r, fma(r, fma(r, fma(r, KN_POW_A5, KN_POW_A4), KN_POW_A3), KN_POW_A2), KN_POW_A1);
+    return kn_powexp[e + KN_POWTAB_E] * fma(t, q, t);
+}
+
 __device__ __forceinline__ double sj_fit(double x0)
 {
     const double x = x0 <= 0. ? 1. : x0;  // a select, not a branch: two points' chains then overlap
     const double x2 = x * x, x4 = x2 * x2, x8 = x4 * x4;
-    const double v = (1. + 0.0168 * x2 + 0.0407 * x4) / (1. + 2.1734 * x2 + 1.6787 * exp(4.1811 * log(x)) + 0.1467 * x8);
+    const double v = (1. + 0.0168 * x2 + 0.0407 * x4) / (1. + 2.1734 * x2 + 1.6787 * pow_fit(x) + 0.1467 * x8);
     return x0 <= 0. ? 1. : v;
 }
 
@@ -2144,7 +2165,7 @@ __device__ inline double specialJ_d(double x, const JPar &P, double &dJdx, doubl
         return 1.;
     }
     const double x2 = x * x, x3 = x2 * x, x4 = x2 * x2, x7 = x4 * x3, x8 = x4 * x4;
-    const double p = exp(4.1811 * log(x));
+    const double p = pow_fit(x);
     const double N = 1. + 0.0168 * x2 + 0.0407 * x4;
     const double D = 1. + 2.1734 * x2 + 1.6787 * p + 0.1467 * x8;
     const double Nx = 0.0336 * x + 0.1628 * x3;
