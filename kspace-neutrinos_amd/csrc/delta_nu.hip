@@ -588,12 +588,19 @@ struct AdjArgs {
     IcAdjArgs ica;
 };
 
-// One window's weights, the intervals that reach it and the queue of points
-// to evaluate.
+// A node of an interval with centre c and half-length h, rounded as gk61_pair's
+// (198 gradients within 5.7e-15 of the oracle's; with the product fused, which
+// moves points against the forward's, within 1.4e-13).
+__device__ __forceinline__ double rule_point(double c, double h, double node)
+{
+#pragma clang fp contract(off)
+    return c + h * node;
+}
+
+// One window's weights and the queue of points to evaluate.
 constexpr int kAdjQueue = 128;
 struct AdjLds {
     double c[kTriSpan], y[kTriSpan];
-    double a[64], b[64];
     double x[kAdjQueue], w[kAdjQueue];
 };
 
@@ -612,8 +619,11 @@ struct AdjLds {
 // compiler's own choice of registers, which lets two run, 1411; with four,
 // which spill more, 1412.  With the scans' three steps, 1304; in launches without
 // a hybrid species, whose series would take 33 registers through the fit's code
-// and spill 52 bytes a lane, and by global instead of flat accesses, 1075.  Its
-// LDS allows three waves anyway.)
+// and spill 52 bytes a lane, and by global instead of flat accesses, 1081; with
+// the points gathered interval by interval, a node per lane held in registers
+// (they took a division, two table loads and two LDS reads each), 985: 206 of
+// them write the rows, 240 solve, 450 evaluate.  Two to eight rows per block on
+// factors kept in registers spill 44 registers: 1474 to 1734.)
 // Points that reach the window (x within [sx[E0 - 1], sx[E1]]) are queued and
 // evaluated 64 at a time, one per lane; a point's d/d(m/kT) term belongs to
 // the window that keeps its si, so every term is counted once.
@@ -693,31 +703,25 @@ __device__ inline void dnu_adj_block(const AdjArgs &A, int blk, AdjLds &S)
             if (si + 1 >= E0 && si + 1 < E1) atomicAdd(&S.c[si + 1 - E0], wj * wc1);
         }
     };
+    // the rule's nodes in order, one per lane (61 used): point c + h node, weight h wgk gb
+    const int jn = lane <= 30 ? lane : (lane < 61 ? 60 - lane : 0);
+    const double node = lane < 30 ? -c_xgk[jn] : c_xgk[jn], wnode = lane < 61 ? c_wgk[jn] : 0.0;
     int nq = 0;  // queued points (wavefront-uniform), below 64 between rounds
     for (int t0 = 0; t0 < ni; t0 += 64) {
         // of 64 recorded intervals, those that reach the window, in their order
         const int t = t0 + lane;
         const double ia = t < ni ? ivl[2 * t] : 0.0, ib = t < ni ? ivl[2 * t + 1] : 0.0;
-        const bool hit = t < ni && ia <= xhi && ib >= xlo;
-        const unsigned long long m = __ballot(hit);
-        if (hit) {
-            const int r = __popcll(m & ((1ull << lane) - 1));
-            S.a[r] = ia;
-            S.b[r] = ib;
-        }
-        wave_lds_sync();
-        const int npts = __popcll(m) * 61;
-        for (int g0 = 0; g0 < npts; g0 += 64) {
-            // point g: interval g / 61, node jj = g % 61 (jj < 30: c - h xgk[jj]; 30: c; jj > 30: c + h xgk[60 - jj])
-            const int g = g0 + lane < npts ? g0 + lane : npts - 1, jj = g % 61, jn = jj <= 30 ? jj : 60 - jj;
-            const double pa = S.a[g / 61], pb = S.b[g / 61], c = 0.5 * (pa + pb), hl = 0.5 * (pb - pa);
-            const double x = jj < 30 ? c - hl * c_xgk[jn] : (jj == 30 ? c : c + hl * c_xgk[jn]);
-            const bool in = g0 + lane < npts && x >= xlo && x <= xhi;
+        unsigned long long m = __ballot(t < ni && ia <= xhi && ib >= xlo);
+        for (; m; m &= m - 1) {
+            const int r = __ffsll((long long)m) - 1;
+            const double pa = lane_value(ia, r), pb = lane_value(ib, r), c = 0.5 * (pa + pb), hl = 0.5 * (pb - pa);
+            const double x = rule_point(c, hl, node);
+            const bool in = lane < 61 && x >= xlo && x <= xhi;
             const unsigned long long mi = __ballot(in);
             if (in) {
-                const int r = nq + __popcll(mi & ((1ull << lane) - 1));
-                S.x[r] = x;
-                S.w[r] = c_wgk[jn] * hl * gb;
+                const int q = nq + __popcll(mi & ((1ull << lane) - 1));
+                S.x[q] = x;
+                S.w[q] = wnode * hl * gb;
             }
             nq += __popcll(mi);
             wave_lds_sync();

@@ -906,11 +906,10 @@ __device__ __forceinline__ T lane_prev(T v)
 {
     return dpp<0x138>(v);  // wave_shr:1
 }
-template <int LANE>
-__device__ __forceinline__ double lane_value(double v)
+__device__ __forceinline__ double lane_value(double v, int l)  // l the same in all lanes
 {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), LANE),
-                            __builtin_amdgcn_readlane(__double2loint(v), LANE));
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
 // The sum over each 32-lane half in every lane, by the butterfly v += v[lane ^
@@ -940,10 +939,9 @@ __device__ __forceinline__ T lane_prev(T v)
     const int p = threadIdx.x & 63;
     return __shfl(v, p > 0 ? p - 1 : 0, 64);
 }
-template <int LANE>
-__device__ __forceinline__ double lane_value(double v)
+__device__ __forceinline__ double lane_value(double v, int l)
 {
-    return __shfl(v, LANE, 64);
+    return __shfl(v, l, 64);
 }
 __device__ __forceinline__ double half_sum(double v)
 {
@@ -1028,14 +1026,14 @@ __device__ __forceinline__ void gk61_pair(const F &f, const RuleLane &rule, doub
     r.resasc = sasc * fabs(h);
     r.err = gk_rescale((sk - sg) * h, r.resabs, r.resasc);
     // broadcast each half's result to every lane
-    g1.res = lane_value<0>(r.res);
-    g1.err = lane_value<0>(r.err);
-    g1.resabs = lane_value<0>(r.resabs);
-    g1.resasc = lane_value<0>(r.resasc);
-    g2.res = lane_value<32>(r.res);
-    g2.err = lane_value<32>(r.err);
-    g2.resabs = lane_value<32>(r.resabs);
-    g2.resasc = lane_value<32>(r.resasc);
+    g1.res = lane_value(r.res, 0);
+    g1.err = lane_value(r.err, 0);
+    g1.resabs = lane_value(r.resabs, 0);
+    g1.resasc = lane_value(r.resasc, 0);
+    g2.res = lane_value(r.res, 32);
+    g2.err = lane_value(r.err, 32);
+    g2.resabs = lane_value(r.resabs, 32);
+    g2.resasc = lane_value(r.resasc, 32);
 }
 
 // The rule's nodes and weights by gk61_pair's lane j (0 at j = 31, and Gauss
