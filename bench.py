@@ -629,7 +629,7 @@ def main():
                      "frac": round(res_gbs / HBM_PEAK_GBS, 4),
                      "traffic": (round(1024 * (RESCALE_1024_FETCH_KIB * FETCH_SCALE + RESCALE_1024_WRITE_KIB * WRITE_SCALE))
                                  if N == 1024 else None),
-                     "kernel": "k_rescale_rows_pf (32 B/mode algorithmic, %d modes per launch)" % modes},
+                     "kernel": "k_rescale (32 B/mode algorithmic, %d modes per launch)" % modes},
         "bin_sweep": {"ms": round(t_bin.mean() * 1e3, 4), "GB/s": round(bin_gbs, 1),
                       "frac": round(bin_gbs / HBM_PEAK_GBS, 4)},
         "rescale_sweep": {"ms": round(t_res.mean() * 1e3, 4), "GB/s": round(res_gbs, 1)},

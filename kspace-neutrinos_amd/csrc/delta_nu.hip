@@ -2029,7 +2029,7 @@ struct GroupPush {
 
 // A history's blocks: its fslength nodes, then (knots_block) its knots.  (Beside
 // the form with panels in LDS, one block per CU, the knots have a launch of their
-// own: 20 us for 256 histories, 45 as blocks of that one.)
+// own: 30 us for 256 histories, 45 as blocks of that one.)
 __device__ inline KnotsArgs group_knots(const GroupDesc &d) { return {d.sx, d.na, d.nsb, d.sinv_bw, d.fac, d.bucket}; }
 
 __global__ __launch_bounds__(256) void k_m_fs_first(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
