@@ -249,7 +249,9 @@ int kn_synth_grid(fftw_complex *d_field, int dims, int startslab, int nslab, dou
 
 /* (a) on a device grid with device-side outputs left in HBM: power[nrbins]
  * holds the unnormalised bin sums, count/keffs the geometry sums, total_mass2
- * |F0|^2.  stream is a hipStream_t (NULL: default stream).  No host sync. */
+ * |F0|^2.  stream is a hipStream_t (NULL: default stream).  No host sync:
+ * calls for the same dims, nrbins and slabs share device buffers, so a program
+ * that gives them different streams orders those streams itself. */
 int kn_bin_power_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
                         double *d_power, double *d_total_mass2, void *stream);
 
@@ -320,7 +322,9 @@ int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int nrbins, int 
  * dL/dpower and writes d_field_bar as kn_bin_power_adjoint does, without
  * sweeping the field for the sums again.  Both run after the work stream has
  * been given so far and before what it is given next, and do not wait for the
- * device. */
+ * device, but for the first call of a geometry, which makes its tables.  They
+ * may overlap with any other call: their device buffers are their own, and
+ * among themselves they take turns. */
 int kn_power_spectrum_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,
                              double *d_power, int *nout, void *stream);
 int kn_power_spectrum_adjoint_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,

@@ -58,6 +58,13 @@ struct SweepPlan {
     size_t smem = 0;
 };
 
+// What a call writes on the device besides its results.
+struct BinBuffers {
+    double *partial = nullptr;  // rows of nrbins, one per block
+    double *sum = nullptr;      // nrbins + 1 (last: |F0|^2)
+    double *alpha = nullptr;    // nrbins + 1, adjoint coefficients, then the zero mode's (allocated on first use)
+};
+
 struct BinGeom {
     int dims, nrbins, startslab, nslab;
     int *d_thr;       // nrbins+1 thresholds on |k|^2
@@ -67,10 +74,9 @@ struct BinGeom {
     std::vector<double> keff_sum;
     SweepPlan plan;         // the power pass
     int ggrid;              // geometry-pass grid
-    double *d_partial;      // max(grid, ggrid) * nrbins
     unsigned *d_cpartial;   // ggrid * nrbins (geometry pass)
-    double *d_sum;          // nrbins + 1 (last: |F0|^2)
-    double *d_alpha;        // nrbins + 1, adjoint coefficients, then the zero mode's (allocated on first use)
+    BinBuffers b;           // of the calls that run on their caller's stream (and of the geometry pass)
+    BinBuffers dev;         // of those that take a DefaultStreamTurn (allocated on first use)
     int agrid;              // adjoint-sweep grid
     int nout;               // non-empty bins
     int *d_slot;            // nrbins: a bin's place among them, -1 if empty (with d_count: allocated on first use)
@@ -78,6 +84,7 @@ struct BinGeom {
 };
 
 std::vector<BinGeom *> g_geoms;
+std::mutex g_geoms_lock;  // the list, and what a geometry gets on first use
 
 // Geometry pass (no grid reads): multiplicity counts and sum of multiplicity*|k|.
 // GLOBAL: the per-block sums are added with global atomics into the block's
@@ -322,21 +329,32 @@ void launch_sweep(kn_bin::BinArgs &a, const SweepPlan &p, hipStream_t st, double
     KN_CHECK(hipGetLastError());
 }
 
-BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
+BinGeom *find_geom(int dims, int nrbins, int startslab, int nslab)
 {
     for (BinGeom *g : g_geoms)
         if (g->dims == dims && g->nrbins == nrbins && g->startslab == startslab && g->nslab == nslab) return g;
+    return nullptr;
+}
+
+BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_geoms_lock);
+        if (BinGeom *g = find_geom(dims, nrbins, startslab, nslab)) return g;
+    }
     if (dims < 2 || nrbins < 1 || nslab < 1 || startslab < 0 || startslab + nslab > dims)
         kn_terminate(KN_ERR_ARG, "total_powerspectrum: bad geometry dims=%d nrbins=%d slabs=[%d,%d)\n", dims,
                      nrbins, startslab, startslab + nslab);
+    std::vector<int> thr;
+    const long long bad = kn_bin::build_thresholds(dims, nrbins, thr);
+    if (bad) kn_terminate(KN_ERR_RANGE, "bin index of |k|^2 = %lld is not monotone or beyond %d bins\n", bad, nrbins);
+    std::lock_guard<std::mutex> lock(g_geoms_lock);
+    if (BinGeom *g = find_geom(dims, nrbins, startslab, nslab)) return g;  // another thread's, meanwhile
     BinGeom *g = new BinGeom();
     g->dims = dims;
     g->nrbins = nrbins;
     g->startslab = startslab;
     g->nslab = nslab;
-    std::vector<int> thr;
-    const long long bad = kn_bin::build_thresholds(dims, nrbins, thr);
-    if (bad) kn_terminate(KN_ERR_RANGE, "bin index of |k|^2 = %lld is not monotone or beyond %d bins\n", bad, nrbins);
     std::vector<double> iw;
     kn_bin::build_invwindow(dims, iw);
     g->half_bpu = (float)(0.5 * (nrbins - 1) / log(sqrt(3) * dims / 2.0));
@@ -346,9 +364,9 @@ BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
     const int pmax = g->plan.grid > g->ggrid ? g->plan.grid : g->ggrid;
     KN_CHECK(hipMalloc(&g->d_thr, sizeof(int) * (nrbins + 1)));
     KN_CHECK(hipMalloc(&g->d_iw, sizeof(double) * dims));
-    KN_CHECK(hipMalloc(&g->d_partial, sizeof(double) * (size_t)pmax * nrbins));
+    KN_CHECK(hipMalloc(&g->b.partial, sizeof(double) * (size_t)pmax * nrbins));
     KN_CHECK(hipMalloc(&g->d_cpartial, sizeof(unsigned) * (size_t)g->ggrid * nrbins));
-    KN_CHECK(hipMalloc(&g->d_sum, sizeof(double) * (nrbins + 1)));
+    KN_CHECK(hipMalloc(&g->b.sum, sizeof(double) * (nrbins + 1)));
     KN_CHECK(hipMemcpy(g->d_thr, thr.data(), sizeof(int) * (nrbins + 1), hipMemcpyHostToDevice));
     KN_CHECK(hipMemcpy(g->d_iw, iw.data(), sizeof(double) * dims, hipMemcpyHostToDevice));
     // geometry pass, once per geometry
@@ -362,13 +380,13 @@ BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
             KN_CHECK(hipFuncSetAttribute((const void *)k_bin_geometry<false>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)gsmem));
         hipLaunchKernelGGL(k_bin_geometry<false>, dim3(g->ggrid), dim3(kBlock), gsmem, 0, dims, startslab, rows,
-                           nrbins, g->d_thr, g->half_bpu, g->d_cpartial, g->d_partial);
+                           nrbins, g->d_thr, g->half_bpu, g->d_cpartial, g->b.partial);
     } else {
         hipLaunchKernelGGL(k_bin_geometry<true>, dim3(g->ggrid), dim3(kBlock), 0, 0, dims, startslab, rows, nrbins,
-                           g->d_thr, g->half_bpu, g->d_cpartial, g->d_partial);
+                           g->d_thr, g->half_bpu, g->d_cpartial, g->b.partial);
     }
     KN_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_reduce_counts, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->d_cpartial, g->d_partial,
+    hipLaunchKernelGGL(k_reduce_counts, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->d_cpartial, g->b.partial,
                        g->ggrid, nrbins, d_count, d_ksum);
     KN_CHECK(hipGetLastError());
     std::vector<unsigned long long> c(nrbins);
@@ -384,11 +402,12 @@ BinGeom *get_geom(int dims, int nrbins, int startslab, int nslab)
 }
 
 // Power pass; the bin sums land in sum_out[nrbins] and |F0|^2 in mass_out
-// (default: the geometry's own buffer, sums then |F0|^2).
-void launch_power(BinGeom *g, const double2 *F, hipStream_t st, double *sum_out = nullptr, double *mass_out = nullptr)
+// (default: the buffers' own, sums then |F0|^2).
+void launch_power(BinGeom *g, const BinBuffers &w, const double2 *F, hipStream_t st, double *sum_out = nullptr,
+                  double *mass_out = nullptr)
 {
-    if (!sum_out) sum_out = g->d_sum;
-    if (!mass_out) mass_out = g->d_sum + g->nrbins;
+    if (!sum_out) sum_out = w.sum;
+    if (!mass_out) mass_out = w.sum + g->nrbins;
     kn_bin::BinArgs a;
     a.F = F;
     a.dims = g->dims;
@@ -398,7 +417,7 @@ void launch_power(BinGeom *g, const double2 *F, hipStream_t st, double *sum_out 
     a.thr = g->d_thr;
     a.iw = g->d_iw;
     a.half_bpu = g->half_bpu;
-    a.partial = g->d_partial;
+    a.partial = w.partial;
     launch_sweep(a, g->plan, st, sum_out, mass_out);
 }
 
@@ -519,47 +538,58 @@ __global__ __launch_bounds__(64 * kAdjWaves) void k_bin_adjoint(const double2 *_
 size_t adjoint_smem(int dims, int nrbins) { return sizeof(double) * (size_t)(nrbins + dims) + sizeof(int) * (nrbins + 1); }
 
 // The adjoint sweep's coefficient buffer and grid, on first use.
-void adjoint_ready(BinGeom *g)
+void adjoint_ready(BinGeom *g, BinBuffers &w)
 {
-    if (g->d_alpha) return;
+    std::lock_guard<std::mutex> lock(g_geoms_lock);
+    if (w.alpha) return;
     const bool global = adjoint_smem(g->dims, g->nrbins) > kLdsMax;
-    KN_CHECK(hipMalloc(&g->d_alpha, sizeof(double) * (g->nrbins + 1)));
-    const long long rows = (long long)g->nslab * g->dims;
-    const int per_cu = global ? resident_blocks(k_bin_adjoint<true>, 64 * kAdjWaves, 0)
-                              : resident_blocks(k_bin_adjoint<false>, 64 * kAdjWaves, adjoint_smem(g->dims, g->nrbins));
-    const long long ag = (long long)per_cu * num_cus();
-    g->agrid = (int)(rows < ag ? rows : ag);
+    if (!g->agrid) {
+        const long long rows = (long long)g->nslab * g->dims;
+        const int per_cu = global ? resident_blocks(k_bin_adjoint<true>, 64 * kAdjWaves, 0)
+                                  : resident_blocks(k_bin_adjoint<false>, 64 * kAdjWaves,
+                                                    adjoint_smem(g->dims, g->nrbins));
+        const long long ag = (long long)per_cu * num_cus();
+        g->agrid = (int)(rows < ag ? rows : ag);
+    }
+    KN_CHECK(hipMalloc(&w.alpha, sizeof(double) * (g->nrbins + 1)));
 }
 
-// The sweep with the coefficients in d_alpha.
-void launch_adjoint(BinGeom *g, const double2 *F, double2 *Fb, hipStream_t st)
+// The sweep with the coefficients in w.alpha.
+void launch_adjoint(BinGeom *g, const BinBuffers &w, const double2 *F, double2 *Fb, hipStream_t st)
 {
     const bool global = adjoint_smem(g->dims, g->nrbins) > kLdsMax;
     hipLaunchKernelGGL(global ? k_bin_adjoint<true> : k_bin_adjoint<false>, dim3(g->agrid), dim3(64 * kAdjWaves),
                        global ? 0 : adjoint_smem(g->dims, g->nrbins), st, F, Fb, g->dims, g->startslab,
-                       (long long)g->nslab * g->dims, g->nrbins, g->d_thr, g->d_iw, g->d_alpha, g->half_bpu);
+                       (long long)g->nslab * g->dims, g->nrbins, g->d_thr, g->d_iw, w.alpha, g->half_bpu);
     KN_CHECK(hipGetLastError());
 }
 
-// The bins' places and counts on the device, on first use.
-void slots_ready(BinGeom *g)
+// The bins' places and counts on the device and the buffers of the calls that
+// leave their results there, on first use.
+void device_ready(BinGeom *g)
 {
+    std::lock_guard<std::mutex> lock(g_geoms_lock);
     if (g->d_slot) return;
     std::vector<int> slot(g->nrbins, -1);
     std::vector<double> count(g->nrbins);
+    int nout = 0;
     for (int b = 0; b < g->nrbins; b++) {
         count[b] = (double)g->count[b];
-        if (g->count[b]) slot[b] = g->nout++;
+        if (g->count[b]) slot[b] = nout++;
     }
+    g->nout = nout;
     int *d_slot;
     KN_CHECK(hipMalloc(&d_slot, sizeof(int) * g->nrbins));
     KN_CHECK(hipMalloc(&g->d_count, sizeof(double) * g->nrbins));
+    KN_CHECK(hipMalloc(&g->dev.partial, sizeof(double) * (size_t)g->plan.grid * g->nrbins));
+    KN_CHECK(hipMalloc(&g->dev.sum, sizeof(double) * (g->nrbins + 1)));
     KN_CHECK(hipMemcpy(d_slot, slot.data(), sizeof(int) * g->nrbins, hipMemcpyHostToDevice));
     KN_CHECK(hipMemcpy(g->d_count, count.data(), sizeof(double) * g->nrbins, hipMemcpyHostToDevice));
     g->d_slot = d_slot;
 }
 
-// What a geometry keeps is shared by its calls, so those that do not wait run
+// kn_power_spectrum_device and its adjoint return with work in flight in
+// buffers that their geometry keeps (BinGeom::dev, theirs alone), so they run
 // in the order of the default stream, whatever stream they are for: after that
 // stream's work so far, and before what it is given next.
 std::mutex g_turn;  // one thread's launches of a call stay together
@@ -589,7 +619,7 @@ extern "C" int kn_bin_power_device(const fftw_complex *d_field, int dims, int nr
                                    double *d_power, double *d_total_mass2, void *stream)
 {
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
-    launch_power(g, (const double2 *)d_field, (hipStream_t)stream, d_power, d_total_mass2);
+    launch_power(g, g->b, (const double2 *)d_field, (hipStream_t)stream, d_power, d_total_mass2);
     return 0;
 }
 
@@ -747,8 +777,8 @@ extern "C" void kn_bin_power_host_sums(const fftw_complex *d_field, int dims, in
 {
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
     std::vector<double> sums(nrbins + 1);
-    launch_power(g, (const double2 *)d_field, 0);
-    KN_CHECK(hipMemcpy(sums.data(), g->d_sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost));
+    launch_power(g, g->b, (const double2 *)d_field, 0);
+    KN_CHECK(hipMemcpy(sums.data(), g->b.sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost));
     memcpy(power, sums.data(), sizeof(double) * nrbins);
     *total_mass2 = sums[nrbins];
 }
@@ -767,9 +797,9 @@ extern "C" int total_powerspectrum(const int dims, fftw_complex *outfield, const
         KN_CHECK(hipMemcpy(staged, outfield, bytes, hipMemcpyHostToDevice));
         F = staged;
     }
-    launch_power(g, F, 0);
+    launch_power(g, g->b, F, 0);
     std::vector<double> sums(nrbins + 1);
-    KN_CHECK(hipMemcpy(sums.data(), g->d_sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost));
+    KN_CHECK(hipMemcpy(sums.data(), g->b.sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost));
     if (staged) KN_CHECK(hipFree(staged));
     memcpy(power, sums.data(), sizeof(double) * nrbins);
     memcpy(count, g->count.data(), sizeof(long long) * nrbins);
@@ -790,9 +820,9 @@ extern "C" int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int n
     }
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
     hipStream_t st = (hipStream_t)stream;
-    launch_power(g, (const double2 *)d_field, st);
+    launch_power(g, g->b, (const double2 *)d_field, st);
     std::vector<double> sums(nrbins + 1), alpha(nrbins + 1, 0.0);
-    KN_CHECK(hipMemcpyAsync(sums.data(), g->d_sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost, st));
+    KN_CHECK(hipMemcpyAsync(sums.data(), g->b.sum, sizeof(double) * (nrbins + 1), hipMemcpyDeviceToHost, st));
     KN_CHECK(hipStreamSynchronize(st));
     const double M = sums[nrbins];
     double gp = 0.0;
@@ -812,9 +842,9 @@ extern "C" int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int n
         return KN_ERR_ARG;
     }
     alpha[nrbins] = -2.0 * gp / M;
-    adjoint_ready(g);
-    KN_CHECK(hipMemcpyAsync(g->d_alpha, alpha.data(), sizeof(double) * (nrbins + 1), hipMemcpyHostToDevice, st));
-    launch_adjoint(g, (const double2 *)d_field, (double2 *)d_field_bar, st);
+    adjoint_ready(g, g->b);
+    KN_CHECK(hipMemcpyAsync(g->b.alpha, alpha.data(), sizeof(double) * (nrbins + 1), hipMemcpyHostToDevice, st));
+    launch_adjoint(g, g->b, (const double2 *)d_field, (double2 *)d_field_bar, st);
     KN_CHECK(hipStreamSynchronize(st));
     return 0;
 }
@@ -826,16 +856,16 @@ extern "C" int kn_power_spectrum_device(const fftw_complex *d_field, int dims, i
         kn_set_last_error("kn_power_spectrum_device: null array");
         return KN_ERR_ARG;
     }
-    DefaultStreamTurn turn((hipStream_t)stream);
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
-    slots_ready(g);
-    launch_power(g, (const double2 *)d_field, 0);
-    hipLaunchKernelGGL(k_power_finish, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->d_sum, g->d_slot, g->d_count,
+    device_ready(g);
+    DefaultStreamTurn turn((hipStream_t)stream);
+    launch_power(g, g->dev, (const double2 *)d_field, 0);
+    hipLaunchKernelGGL(k_power_finish, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->dev.sum, g->d_slot, g->d_count,
                        nrbins, d_power);
     KN_CHECK(hipGetLastError());
     if (kn_message_wanted()) {  // as total_powerspectrum; nobody to read it otherwise, and no wait
         double mass2;
-        KN_CHECK(hipMemcpy(&mass2, g->d_sum + nrbins, sizeof(double), hipMemcpyDeviceToHost));
+        KN_CHECK(hipMemcpy(&mass2, g->dev.sum + nrbins, sizeof(double), hipMemcpyDeviceToHost));
         kn_message(0, "total mass of the grid, |F(k = 0)|: %g\n", sqrt(mass2));
     }
     turn.done();
@@ -851,20 +881,19 @@ extern "C" int kn_power_spectrum_adjoint_device(const fftw_complex *d_field, int
         kn_set_last_error("kn_power_spectrum_adjoint_device: needs startslab 0 (the zero mode) and non-null arrays");
         return KN_ERR_ARG;
     }
-    DefaultStreamTurn turn((hipStream_t)stream);
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
-    slots_ready(g);
+    device_ready(g);
     if (nout != g->nout) {
-        turn.done();
         kn_set_last_error("kn_power_spectrum_adjoint_device: nout=%d but the forward has %d non-empty bins", nout,
                           g->nout);
         return KN_ERR_ARG;
     }
-    adjoint_ready(g);
+    adjoint_ready(g, g->dev);
+    DefaultStreamTurn turn((hipStream_t)stream);
     hipLaunchKernelGGL(k_adjoint_alpha, dim3(1), dim3(kAlphaThreads), 0, 0, (const double2 *)d_field, g->d_slot,
-                       g->d_count, nrbins, d_power, d_gbar, g->d_alpha);
+                       g->d_count, nrbins, d_power, d_gbar, g->dev.alpha);
     KN_CHECK(hipGetLastError());
-    launch_adjoint(g, (const double2 *)d_field, (double2 *)d_field_bar, 0);
+    launch_adjoint(g, g->dev, (const double2 *)d_field, (double2 *)d_field_bar, 0);
     turn.done();
     return 0;
 }
