@@ -322,7 +322,9 @@ int kn_bin_power_adjoint(const fftw_complex *d_field, int dims, int nrbins, int 
  * dL/dpower and writes d_field_bar as kn_bin_power_adjoint does, without
  * sweeping the field for the sums again.  Both run after the work stream has
  * been given so far and before what it is given next, and do not wait for the
- * device, but for the first call of a geometry, which makes its tables.  They
+ * device, but for the first call of a geometry, which makes its tables, and
+ * with KN_VERBOSE in the environment, when the spectrum's |F(0)| is reported as
+ * total_powerspectrum does (otherwise it is not: that needs a wait).  They
  * may overlap with any other call: their device buffers are their own, and
  * among themselves they take turns. */
 int kn_power_spectrum_device(const fftw_complex *d_field, int dims, int nrbins, int startslab, int nslab,

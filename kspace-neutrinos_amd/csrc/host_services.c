@@ -72,8 +72,6 @@ void kn_message(int level, const char *fmt, ...)
     if (getenv("KN_VERBOSE")) fputs(buf, stdout);
 }
 
-int kn_message_wanted(void) { return message || getenv("KN_VERBOSE"); }
-
 void *kn_malloc(const char *name, size_t n)
 {
     void *p;

@@ -37,7 +37,6 @@ double kn_hubble(double a);
 void kn_set_hubble_ctx(double (*fn)(double a, void *ctx), void *ctx);
 void kn_terminate(int code, const char *fmt, ...) __attribute__((noreturn, format(printf, 2, 3)));
 void kn_message(int level, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
-int kn_message_wanted(void); /* whether kn_message has anyone to tell */
 void *kn_malloc(const char *name, size_t n);
 void kn_free(void *p);
 void kn_set_last_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));

@@ -27,6 +27,7 @@
 // once per (dims, nrbins, slab range) by a
 // read-free kernel and cached (bit-exact, deterministic).
 #include <math.h>
+#include <stdlib.h>
 #include <string.h>
 #include <mutex>
 #include <vector>
@@ -858,17 +859,18 @@ extern "C" int kn_power_spectrum_device(const fftw_complex *d_field, int dims, i
     }
     BinGeom *g = get_geom(dims, nrbins, startslab, nslab);
     device_ready(g);
-    DefaultStreamTurn turn((hipStream_t)stream);
-    launch_power(g, g->dev, (const double2 *)d_field, 0);
-    hipLaunchKernelGGL(k_power_finish, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->dev.sum, g->d_slot, g->d_count,
-                       nrbins, d_power);
-    KN_CHECK(hipGetLastError());
-    if (kn_message_wanted()) {  // as total_powerspectrum; nobody to read it otherwise, and no wait
-        double mass2;
-        KN_CHECK(hipMemcpy(&mass2, g->dev.sum + nrbins, sizeof(double), hipMemcpyDeviceToHost));
-        kn_message(0, "total mass of the grid, |F(k = 0)|: %g\n", sqrt(mass2));
+    const bool report = getenv("KN_VERBOSE") != nullptr;  // what total_powerspectrum tells; waits for the sum
+    double mass2 = 0.0;
+    {
+        DefaultStreamTurn turn((hipStream_t)stream);
+        launch_power(g, g->dev, (const double2 *)d_field, 0);
+        hipLaunchKernelGGL(k_power_finish, dim3((nrbins + 255) / 256), dim3(256), 0, 0, g->dev.sum, g->d_slot,
+                           g->d_count, nrbins, d_power);
+        KN_CHECK(hipGetLastError());
+        if (report) KN_CHECK(hipMemcpy(&mass2, g->dev.sum + nrbins, sizeof(double), hipMemcpyDeviceToHost));
+        turn.done();
     }
-    turn.done();
+    if (report) kn_message(0, "total mass of the grid, |F(k = 0)|: %g\n", sqrt(mass2));
     *nout = g->nout;
     return 0;
 }

@@ -89,3 +89,40 @@ def test_two_streams_and_autograd(kn, torch_cuda):
             np.testing.assert_allclose(p.cpu().numpy(), op[:on], rtol=1e-12)
             e = np.max(np.abs(bar.cpu().numpy().view(np.complex128).reshape(ob.shape) / (1.0 + r) - ob))
             assert e < 1e-12 * np.max(np.abs(ob))
+
+
+def test_returns_with_the_work_in_flight(kn, host, torch_cuda, monkeypatch):
+    """Behind 200 ms of other work on its stream the spectrum and its gradient return at once (also in a program that
+    takes the library's messages), and what follows on that stream reads finished results."""
+    torch = torch_cuda
+    monkeypatch.delenv("KN_VERBOSE", raising=False)
+    N, nb = 64, 48
+    ((F, a),) = _grids(torch, N, 1)
+    on, op, _, _ = O.total_powerspectrum(F, nb)
+    rc, ob = O.bin_power_adjoint(F, nb, np.ones(on))
+    fn, st = knhip.power_spectrum_function(), torch.cuda.Stream()
+    big = torch.empty(1 << 28, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+
+    def step():
+        x = a.detach().requires_grad_(True)
+        p = fn.apply(x, nb)
+        (bar,) = torch.autograd.grad(p.sum(), x)
+        return p.detach() * 2.0, bar * 2.0
+
+    with torch.cuda.stream(st):
+        step()                      # the geometry's tables, the allocator's blocks
+        torch.cuda.synchronize()
+        messages = host.kn_test_messages()
+        print("work in flight", flush=True)
+        for _ in range(400):
+            big.zero_()
+        busy = torch.cuda.Event()
+        busy.record()
+        p, bar = step()
+        assert not busy.query()
+        assert host.kn_test_messages() == messages
+        p, bar = p.cpu().numpy(), bar.cpu().numpy()
+    np.testing.assert_allclose(p, 2.0 * op[:on], rtol=1e-12)
+    e = np.max(np.abs(bar.view(np.complex128).reshape(ob.shape) - 2.0 * ob))
+    assert rc == 0 and e < 1e-12 * np.max(np.abs(2.0 * ob))
