@@ -19,7 +19,7 @@ print("""// kn_logtab.h -- generated by gen_logtab.py; do not edit.
 
 #define KN_LOGTAB_N %d
 """ % N)
-print("static __device__ const double kn_logtab[2 * KN_LOGTAB_N] = {")
+print("static __device__ const __align__(16) double kn_logtab[2 * KN_LOGTAB_N] = {")
 for j in range(N):
     r = float(1 / (1 + (mp.mpf(j) + mp.mpf(1) / 2) / N))
     print("    %s, %s," % (r.hex(), float(-log(mp.mpf(r))).hex()))

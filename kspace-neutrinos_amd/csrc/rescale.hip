@@ -51,25 +51,42 @@ int res_cus()
     return cus;
 }
 
-// Buckets of a table of nbins: four per bin, one where those do not fit in LDS.
-int res_buckets(int nbins, int green_dims)
-{
-    return kn_res::smem_bytes(nbins, 4 * nbins, green_dims) <= 160 * 1024 ? 4 * nbins : nbins;
-}
+constexpr size_t kResLds = 160 * 1024;
 
 // A table of nbins (with green_dims Green's factors) is taken up to this many
-// bytes of log k, ratio and four buckets per bin: about 5100 bins.
+// bytes of log k, ratio and four buckets per bin: about 5100 bins.  Whatever is
+// taken fits in LDS by one of res_plan's forms.
 bool res_fits(int nbins, int green_dims)
 {
     return sizeof(double) * (2 * (size_t)nbins + green_dims) + sizeof(int) * ((4 * (size_t)nbins + 2) & ~(size_t)1) <=
-           160 * 1024;
+           kResLds;
 }
 
-template <int U, bool GREEN, bool WIDE>
-void res_launch_as(kn_res::ResArgs &a, hipStream_t st)
+// What the sweep keeps in LDS: four buckets per bin, one where those do not
+// fit; the logarithm's table, but in global memory where a grid's Green's
+// factors (from dims 18439) leave no room for it.  Without bins neither.
+struct ResPlan {
+    int nbuckets;
+    bool log_lds;
+    size_t smem;
+};
+
+ResPlan res_plan(int nbins, int green_dims)
 {
-    const size_t smem = kn_res::smem_bytes(a.nbins, a.nbuckets, GREEN ? a.dims : 0);
-    const void *k = (const void *)kn_res::k_rescale<kResWaves, U, GREEN, WIDE>;
+    ResPlan p = {0, true, kn_res::smem_bytes(0, 0, green_dims, false)};
+    if (nbins == 0) return p;
+    for (bool log_lds : {true, false})
+        for (int per_bin : {4, 1}) {
+            p = {per_bin * nbins, log_lds, kn_res::smem_bytes(nbins, per_bin * nbins, green_dims, log_lds)};
+            if (p.smem <= kResLds) return p;
+        }
+    return p;
+}
+
+template <int U, bool GREEN, bool WIDE, bool LOG_LDS>
+void res_launch_as(kn_res::ResArgs &a, size_t smem, hipStream_t st)
+{
+    const void *k = (const void *)kn_res::k_rescale<kResWaves, U, GREEN, WIDE, LOG_LDS>;
     if (smem > 64 * 1024) KN_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     const int rowlen = a.dims / 2 + 1, B = 64 * kResWaves;
     const long long T = (long long)B * U, slots = (smem <= 80 * 1024 ? 2LL : 1LL) * res_cus();
@@ -78,7 +95,7 @@ void res_launch_as(kn_res::ResArgs &a, hipStream_t st)
     if (g > slots) g = slots;
     a.in_tile = kn_res::step_of(B, rowlen, a.dims);
     a.to_next = kn_res::step_of((g - 1) * T + B, rowlen, a.dims);
-    hipLaunchKernelGGL((kn_res::k_rescale<kResWaves, U, GREEN, WIDE>), dim3((int)g), dim3(B), smem, st, a);
+    hipLaunchKernelGGL((kn_res::k_rescale<kResWaves, U, GREEN, WIDE, LOG_LDS>), dim3((int)g), dim3(B), smem, st, a);
     KN_CHECK(hipGetLastError());
 }
 
@@ -87,8 +104,13 @@ void res_launch_as(kn_res::ResArgs &a, hipStream_t st)
 template <bool GREEN>
 void res_launch(kn_res::ResArgs &a, hipStream_t st)
 {
-    if (a.dims / 2 + 1 >= 64) res_launch_as<kResUnroll, GREEN, true>(a, st);
-    else res_launch_as<1, GREEN, false>(a, st);
+    const ResPlan p = res_plan(a.nbins, GREEN ? a.dims : 0);
+    a.nbuckets = p.nbuckets;
+    if constexpr (GREEN) {
+        if (!p.log_lds) return res_launch_as<kResUnroll, GREEN, true, false>(a, p.smem, st);
+    }
+    if (a.dims / 2 + 1 >= 64) res_launch_as<kResUnroll, GREEN, true, true>(a, p.smem, st);
+    else res_launch_as<1, GREEN, false, true>(a, p.smem, st);
 }
 
 // ---- synthetic Gaussian random field -----------------------------------
@@ -162,7 +184,6 @@ extern "C" int kn_rescale_device(fftw_complex *d_field, int dims, int startslab,
     a.dims = dims;
     a.startslab = startslab;
     a.nbins = nbins;
-    a.nbuckets = res_buckets(nbins, 0);
     a.rows = (long long)nslab * dims;
     a.log_kunit = log(2 * M_PI / boxsize);
     a.norm = norm;
@@ -217,7 +238,6 @@ extern "C" int kn_rescale_green_device(fftw_complex *d_field, int dims, int star
     a.dims = dims;
     a.startslab = startslab;
     a.nbins = nbins;
-    a.nbuckets = res_buckets(nbins, dims);
     a.rows = (long long)nslab * dims;
     a.log_kunit = log(2 * M_PI / boxsize);
     a.norm = norm;

@@ -46,11 +46,11 @@ struct ResArgs {
     const double *__restrict__ gw;
 };
 
-// LDS of the sweep: the table's log k, ratio and slope, the logarithm's table,
-// the buckets, and the Green's factors of one axis.
-__host__ __device__ inline size_t smem_bytes(int nbins, int nbuckets, int green_dims = 0)
+// LDS of the sweep: the logarithm's table (log_lds), the ratio table's log k,
+// ratio and slope, the buckets, and the Green's factors of one axis.
+__host__ __device__ inline size_t smem_bytes(int nbins, int nbuckets, int green_dims, bool log_lds)
 {
-    return sizeof(double) * (3 * (size_t)nbins + 2 * KN_LOGTAB_N + (size_t)green_dims) +
+    return sizeof(double) * (3 * (size_t)nbins + (log_lds ? 2 * KN_LOGTAB_N : 0) + (size_t)green_dims) +
            sizeof(int) * (size_t)(nbuckets + 1 + ((nbuckets + 1) & 1));
 }
 
@@ -62,13 +62,15 @@ struct Tab {
     double x0, x1, inv_bw, norm, log_kunit;
 };
 
-// Ratio table, slopes, logarithm table and bucket index into LDS (all threads of the block).
+// Ratio table, slopes, bucket index and (LOG_LDS) logarithm table into LDS (all threads of the block).
+template <bool LOG_LDS>
 __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 {
     extern __shared__ double sm[];
-    double *lg = sm, *lk = lg + 2 * KN_LOGTAB_N, *rt = lk + a.nbins, *sl = rt + a.nbins;
+    double *lk = sm + (LOG_LDS ? 2 * KN_LOGTAB_N : 0), *rt = lk + a.nbins, *sl = rt + a.nbins;
     int *bucket = (int *)(sl + a.nbins);
-    for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) lg[t] = kn_logtab[t];
+    if (LOG_LDS)
+        for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) sm[t] = kn_logtab[t];
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
         lk[t] = a.logkk[t];
         rt[t] = a.ratio[t];
@@ -78,7 +80,7 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     T.lk = lk;
     T.rt = rt;
     T.sl = sl;
-    T.lg = (const double2 *)lg;
+    T.lg = (const double2 *)(LOG_LDS ? sm : kn_logtab);
     T.bucket = bucket;
     T.nbins = a.nbins;
     T.nbuckets = a.nbuckets;
@@ -214,7 +216,8 @@ __device__ __forceinline__ double green_of(int k2, double gxy, double gz)
 // G, the two roundings of the two passes it replaces) and zeroes the k = 0
 // mode; with nbins 0 it applies the Green's function alone.
 // WIDE: rows of 64 modes or more (else every lane finds its own row).
-template <int WAVES, int U, bool GREEN, bool WIDE>
+// LOG_LDS: the logarithm's table in LDS (else read through the caches).
+template <int WAVES, int U, bool GREEN, bool WIDE, bool LOG_LDS>
 __global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
 {
     constexpr int B = 64 * WAVES, T = B * U;
@@ -230,12 +233,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
     }
     Tab Tb;
     const double *gw = nullptr;
-    if (!GREEN || a.nbins > 0) Tb = load_tab(a, B);
+    if (!GREEN || a.nbins > 0) Tb = load_tab<LOG_LDS>(a, B);
     if constexpr (GREEN) {
         extern __shared__ double sm[];
-        double *gw_l = a.nbins > 0 ? (double *)((int *)(sm + 2 * KN_LOGTAB_N + 3 * (size_t)a.nbins) + a.nbuckets + 1 +
-                                                ((a.nbuckets + 1) & 1))
-                                   : sm;
+        double *gw_l = a.nbins > 0 ? (double *)((int *)(Tb.sl + a.nbins) + a.nbuckets + 1 + ((a.nbuckets + 1) & 1)) : sm;
         for (int t = threadIdx.x; t < a.dims; t += B) gw_l[t] = a.gw[t];
         __syncthreads();
         gw = gw_l;
