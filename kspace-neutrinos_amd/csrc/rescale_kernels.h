@@ -9,7 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include "kn_logtab.h"
+#include "half_log.h"
 #include "kn_mem.h"
 
 namespace kn_res {
@@ -106,26 +106,6 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     }
     __syncthreads();
     return T;
-}
-
-// log(sqrt(k2)), k2 >= 1, by kn_logtab: k2 = 2^e m with m in the table's
-// interval j, log m = -log r_j + log1p(m r_j - 1) with six terms of the series
-// (|m r_j - 1| <= 2^-8: the seventh is below 2e-18).  Within 1.8e-15 for all
-// int k2, as half of a log(k2) rounded to double is.  18 operations where the
-// math library's log and its double-double steps are about 75.
-__device__ __forceinline__ double half_log(int k2, const double2 *lg)
-{
-    const unsigned long long v = __double_as_longlong((double)k2);
-    const int hi = (int)(v >> 32), e = (hi >> 20) - 1023;
-    const double m = __longlong_as_double((v & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-    const double2 t = lg[(hi >> 13) & (KN_LOGTAB_N - 1)];
-    const double r = fma(m, t.x, -1.0), ef = (double)e;
-    double q = fma(r, -1.0 / 6.0, 1.0 / 5.0);
-    q = fma(r, q, -1.0 / 4.0);
-    q = fma(r, q, 1.0 / 3.0);
-    q = fma(r, q, -1.0 / 2.0);
-    const double p = fma(r * r, q, r);
-    return fma(ef, KN_HALF_LN2_HI, 0.5 * t.y) + fma(ef, KN_HALF_LN2_LO, 0.5 * p);
 }
 
 // 1 + get_dnudcdm_powerspec(log(|k|)) for k2 > 0, with |k| = sqrt(k2) 2 pi / BoxSize.

@@ -127,3 +127,10 @@ extern "C" double emu_gk_rescale(double err, double resabs, double resasc)
 {
     return kn_dnu::gk_rescale(err, resabs, resasc);
 }
+
+// The rescale sweep's logarithm (half_log.h) at n integers, for tests.
+#include "half_log.h"
+extern "C" void emu_half_log(int n, const int *k2, double *out)
+{
+    for (int i = 0; i < n; i++) out[i] = kn_res::half_log(k2[i], (const double2 *)kn_logtab);
+}

@@ -26,6 +26,7 @@
 #define __host__
 #define __forceinline__ inline
 #define __constant__
+#define __align__(n) alignas(n)
 #define __shared__ static
 #define __launch_bounds__(...)
 extern double emu_dyn_lds[];  // dynamic LDS of the running block (160 KiB)
@@ -35,6 +36,7 @@ struct dim3 {
     unsigned x, y, z;
     dim3(unsigned a = 1, unsigned b = 1, unsigned c = 1) : x(a), y(b), z(c) {}
 };
+struct double2 { double x, y; };
 struct emu_idx { unsigned x, y, z; };
 extern unsigned emu_tid, emu_bid, emu_bdim, emu_gdim, emu_bid_y, emu_gdim_y;
 inline emu_idx emu_threadIdx() { return {emu_tid, 0, 0}; }
