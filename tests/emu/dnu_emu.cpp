@@ -134,3 +134,18 @@ extern "C" void emu_half_log(int n, const int *k2, double *out)
 {
     for (int i = 0; i < n; i++) out[i] = kn_res::half_log(k2[i], (const double2 *)kn_logtab);
 }
+
+// specialJ's power, and specialJ with its derivatives (dnu_device.h), at n points, for tests.
+extern "C" void emu_pow_fit(int n, const double *x, double *out)
+{
+    for (int i = 0; i < n; i++) out[i] = kn_dnu::pow_fit(x[i]);
+}
+extern "C" void emu_specialJ_d(int n, const double *x, double qc, double nufrac_low, double *J, double *dJdx,
+                               double *dJdqc)
+{
+    kn_dnu::JPar P;
+    P.qc = qc;
+    P.nufrac_low = nufrac_low;
+    for (int m = 0; m < 20; m++) P.en[m] = exp(-m * qc);
+    for (int i = 0; i < n; i++) J[i] = kn_dnu::specialJ_d(x[i], P, dJdx[i], dJdqc[i]);
+}
