@@ -63,6 +63,7 @@ struct Tab {
 };
 
 // Ratio table, slopes, bucket index and (LOG_LDS) logarithm table into LDS (all threads of the block).
+// A table of one bin is its ratio at every k: its log k, which may be anything, is taken as 0.
 template <bool LOG_LDS>
 __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 {
@@ -72,7 +73,7 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     if (LOG_LDS)
         for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) sm[t] = kn_logtab[t];
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
-        lk[t] = a.logkk[t];
+        lk[t] = a.nbins > 1 ? a.logkk[t] : 0.0;
         rt[t] = a.ratio[t];
     }
     __syncthreads();
@@ -88,7 +89,7 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     T.x1 = lk[a.nbins - 1];
     T.inv_bw = a.nbins > 1 ? a.nbuckets / (T.x1 - T.x0) : 0.0;
     T.norm = a.norm;
-    T.log_kunit = a.log_kunit;
+    T.log_kunit = a.nbins > 1 ? a.log_kunit : 0.0;
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
         const double h = t + 1 < a.nbins ? lk[t + 1] - lk[t] : 0.0;
         sl[t] = h > 0.0 ? (rt[t + 1] - rt[t]) / h : 0.0;
