@@ -64,7 +64,7 @@ bool res_fits(int nbins, int green_dims)
 
 // What the sweep keeps in LDS: four buckets per bin, one where those do not
 // fit; the logarithm's table, but in global memory where a grid's Green's
-// factors (from dims 18439) leave no room for it.  Without bins neither.
+// factors (from dims 18435) leave no room for it.  Without bins neither.
 struct ResPlan {
     int nbuckets;
     bool log_lds;

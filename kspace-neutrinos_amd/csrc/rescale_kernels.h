@@ -46,12 +46,15 @@ struct ResArgs {
     const double *__restrict__ gw;
 };
 
+// The ints of load_tab: buckets 0 .. nbuckets and one flag, in whole doubles.
+__host__ __device__ inline int tab_ints(int nbuckets) { return nbuckets + 2 + (nbuckets & 1); }
+
 // LDS of the sweep: the logarithm's table (log_lds), the ratio table's log k,
-// ratio and slope, the buckets, and the Green's factors of one axis.
+// ratio and slope, its ints, and the Green's factors of one axis.
 __host__ __device__ inline size_t smem_bytes(int nbins, int nbuckets, int green_dims, bool log_lds)
 {
     return sizeof(double) * (3 * (size_t)nbins + (log_lds ? 2 * KN_LOGTAB_N : 0) + (size_t)green_dims) +
-           sizeof(int) * (size_t)(nbuckets + 1 + ((nbuckets + 1) & 1));
+           (nbins > 0 ? sizeof(int) * (size_t)tab_ints(nbuckets) : 0);
 }
 
 struct Tab {
@@ -59,6 +62,7 @@ struct Tab {
     const double2 *lg;           // kn_logtab
     const int *bucket;
     int nbins, nbuckets;
+    bool odd;  // a log k is not finite, or a slope overflows
     double x0, x1, inv_bw, norm, log_kunit;
 };
 
@@ -69,7 +73,8 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 {
     extern __shared__ double sm[];
     double *lk = sm + (LOG_LDS ? 2 * KN_LOGTAB_N : 0), *rt = lk + a.nbins, *sl = rt + a.nbins;
-    int *bucket = (int *)(sl + a.nbins);
+    int *bucket = (int *)(sl + a.nbins), *odd = bucket + a.nbuckets + 1;
+    if (threadIdx.x == 0) *odd = 0;
     if (LOG_LDS)
         for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) sm[t] = kn_logtab[t];
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
@@ -93,6 +98,7 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
         const double h = t + 1 < a.nbins ? lk[t + 1] - lk[t] : 0.0;
         sl[t] = h > 0.0 ? (rt[t + 1] - rt[t]) / h : 0.0;
+        if (!isfinite(lk[t]) || !isfinite(sl[t])) *odd = 1;
     }
     // bucket[q]: the GSL segment index (largest i <= n-2 with lk[i] <= x) at the bucket's left edge
     for (int q = threadIdx.x; q <= a.nbuckets; q += nthreads) {
@@ -106,6 +112,7 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
         bucket[q] = lo;
     }
     __syncthreads();
+    T.odd = __builtin_amdgcn_readfirstlane(*odd) != 0;
     return T;
 }
 
@@ -122,6 +129,10 @@ __device__ __forceinline__ double smth_of(int k2i, const Tab &T)
     q = q < 0 ? 0 : (q > T.nbuckets ? T.nbuckets : q);
     int i = T.bucket[q];
     while (i < T.nbins - 2 && T.lk[i + 1] <= kk) i++;
+    if (T.odd) {  // the whole table's: the reference's expression, which needs no slope
+        const double h = T.nbins > 1 ? T.lk[i + 1] - T.lk[i] : 0.0;
+        return fma(T.norm, h > 0.0 ? T.rt[i] + (kk - T.lk[i]) / h * (T.rt[i + 1] - T.rt[i]) : T.rt[i], 1.0);
+    }
     return fma(T.norm, fma(kk - T.lk[i], T.sl[i], T.rt[i]), 1.0);
 }
 
@@ -217,7 +228,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
     if (!GREEN || a.nbins > 0) Tb = load_tab<LOG_LDS>(a, B);
     if constexpr (GREEN) {
         extern __shared__ double sm[];
-        double *gw_l = a.nbins > 0 ? (double *)((int *)(Tb.sl + a.nbins) + a.nbuckets + 1 + ((a.nbuckets + 1) & 1)) : sm;
+        double *gw_l = a.nbins > 0 ? (double *)((int *)(Tb.sl + a.nbins) + tab_ints(a.nbuckets)) : sm;
         for (int t = threadIdx.x; t < a.dims; t += B) gw_l[t] = a.gw[t];
         __syncthreads();
         gw = gw_l;

@@ -37,8 +37,8 @@ def _want(torch, f, N, x, y0, lk, rt, norm, asmth):
 
 
 # 16 B per bin, four buckets of 4 B each, 8 B per axis index: 160 KB hold dims 20479 without bins, 20475 with one, 18439
-# with 510; with bins, from 20221 (one) and 18439 (510) the logarithm's table has no room beside them
-@pytest.mark.parametrize("N,nb", [(20223, 0), (20224, 0), (20479, 0), (20220, 1), (20221, 1), (20475, 1), (20399, 20),
+# with 510; with bins, from 20220 (one) and 18439 (510) the logarithm's table has no room beside them
+@pytest.mark.parametrize("N,nb", [(20223, 0), (20224, 0), (20479, 0), (20219, 1), (20220, 1), (20475, 1), (20399, 20),
                                   (19455, 256), (18438, 510), (18439, 510), (18435, 511)])
 def test_largest_grids(kn, torch_cuda, N, nb):
     """1e-14, as the fused sweep's other tests; the exponent is below 0.3 and the ratio's slope 0.3, so that neither its
