@@ -285,7 +285,7 @@ struct PrepArgs {
     int b_sp, rpw;
     const double *fac;
     UniformKnots fk;
-    const double *fy;
+    const double *fx, *fy;
     double *fc;
     int nfs;
 };
@@ -301,7 +301,7 @@ __device__ __forceinline__ void prep_block(const PrepArgs &a, int b, double *lds
         return;
     }
     const int w = (b - a.b_sp) * 4 + wave;
-    if (w < fac_windows(a.nfs)) uniform_spline_wave(a.fk, a.fy, a.fc, a.nfs, w, lds + wave * kTriSpan);
+    if (w < fac_windows(a.nfs)) uniform_spline_wave(a.fk, a.fx, a.fy, a.fc, a.nfs, w, lds + wave * kTriSpan);
 }
 
 // Bound by memory: 256 histories of 64-512 k x 100-3000 steps, 1.83 GB read and
@@ -1687,7 +1687,7 @@ static int dnu_solve(const _delta_tot_table *d, double a, const double *wavenum,
         const int rpw = rows_per_wave((long long)fac_windows(Na) * nk), bsp = rows_prep_spline_blocks(Na, nk, rpw);
         hipLaunchKernelGGL(k_prep, dim3(prep_blocks(bsp, nfs)), dim3(256), 0, 0,
                            PrepArgs{dev->Y, dev->C, Na, nk, (long long)namax, bsp, rpw, dev->fac,
-                                    fs_knots(x0, xa, nfs), dev->fy, dev->fc, nfs});
+                                    fs_knots(x0, xa, nfs), dev->fx, dev->fy, dev->fc, nfs});
     }
     QagArgs qa;
     qa.H = H;
@@ -2113,7 +2113,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_fs_rest(const GroupDe
 
 __device__ inline PrepArgs group_prep(const GroupDesc &d)
 {
-    return {d.Y, d.C, d.na, d.nk, (long long)d.na_max, d.bsp, d.rpw, d.fac, fs_knots(d.x0, d.xa, d.nfs), d.fy, d.fc, d.nfs};
+    return {d.Y, d.C, d.na, d.nk, (long long)d.na_max, d.bsp, d.rpw, d.fac, fs_knots(d.x0, d.xa, d.nfs), d.fx, d.fy, d.fc, d.nfs};
 }
 
 __global__ __launch_bounds__(256, 4) void k_m_prep(const GroupDesc *__restrict__ D, const int *__restrict__ pre,
@@ -2627,8 +2627,8 @@ void group_forward_one(kn_group *g, const GroupHist &q, int i, hipStream_t s)
     hipLaunchKernelGGL(k_knots, dim3(knots_blocks(na, d.nsb, 256)), dim3(256), 0, s,
                        KnotsArgs{d.sx, na, d.nsb, d.sinv_bw, d.fac, d.bucket});
     hipLaunchKernelGGL(k_prep, dim3(prep_blocks(d.bsp, nfs)), dim3(256), 0, s,
-                       PrepArgs{d.Y, d.C, na, nk, (long long)na_max, d.bsp, d.rpw, d.fac, fs_knots(q.x0, q.xa, nfs), fy,
-                                fc, nfs});
+                       PrepArgs{d.Y, d.C, na, nk, (long long)na_max, d.bsp, d.rpw, d.fac, fs_knots(q.x0, q.xa, nfs), fx,
+                                fy, fc, nfs});
     QagArgs a;
     a.H = d.H;
     a.fx = fx;

@@ -1746,17 +1746,17 @@ __device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, do
     g_before = s == t.wa ? 0.0 : gp;
 #pragma unroll
     for (int j = 0; j < kRun; j++) {
+        double gj = 0.0, aj = 0.0;
         if (j < len) {
             const int i = s + j;
             const double hl = x[i] - x[i - 1], hr = x[i + 1] - x[i];
             const double diag = 2.0 * (hr + hl);
             const double al = i == a ? diag : diag - hl * gp;
-            g[j] = hr / al;
-            ial[j] = 1.0 / al;
-            gp = g[j];
-        } else {
-            g[j] = ial[j] = 0.0;
+            gp = gj = hr / al;
+            aj = 1.0 / al;
         }
+        g[j] = gj;
+        ial[j] = aj;
     }
 }
 
@@ -2044,6 +2044,15 @@ __device__ __forceinline__ void tri_rows_staged(int n, int w, const double *__re
 // interval's own length: 1 / h corrected by one Newton step (relative (d /
 // h)^2).  Small solves wait for a chain of divisions in the general factors:
 // 1600 knots 11.6 us with them.
+// The knots count as even (uniform_even) where (d / h)^2 is below a rounding: h
+// at least 2^25 units in the last place of x, 1.4e-7 at log a = -4.6.  Closer
+// ones (2000 steps within 0.5% of the starting a) take the general factors and
+// divisions: with the constant ones the values of 80 knots over 1e-10 in log a
+// were off by 4e-10 of the largest, over 1e-6 by 1e-18.
+__device__ __forceinline__ bool uniform_even(const UniformKnots &kn)
+{
+    return kn.span * kn.rden >= 0x1p-25 * fmax(fabs(kn.x0), fabs(kn.x0 + kn.span));
+}
 constexpr int kGamRows = 20;
 struct GamTab {
     double g[kGamRows + 1];
@@ -2070,13 +2079,25 @@ struct UniformRhsLds {
         return 3.0 * (slope(xm, kn.at(i + 1), ym, ys[k + 1]) - slope(kn.at(i - 1), xm, ys[k - 1], ym));
     }
 };
+// The same on any knots x, in memory.
+struct KnotsRhsLds {
+    const double *ys, *x;
+    int base;
+    __device__ __forceinline__ double slope(int i) const  // of interval i
+    {
+        const double h = x[i + 1] - x[i];
+        return h != 0.0 ? (ys[i + 1 - base] - ys[i - base]) * (1.0 / h) : 0.0;
+    }
+    __device__ __forceinline__ double operator()(int i) const { return 3.0 * (slope(i) - slope(i - 1)); }
+};
 struct NoIh {
     __device__ __forceinline__ double operator()(int) const { return 0.0; }
 };
 
 // Window w (of fac_windows(n), n >= 3) of the fslength table's coefficients c
-// by one wavefront; sa: kTriSpan doubles of its own LDS.
-__device__ __forceinline__ void uniform_spline_wave(const UniformKnots &kn, const double *__restrict__ y,
+// by one wavefront; x: the knots as stored; sa: kTriSpan doubles of its own LDS.
+template <bool EVEN>
+__device__ __forceinline__ void uniform_spline_form(const UniformKnots &kn, const double *x, const double *__restrict__ y,
                                                     double *__restrict__ c, int n, int w, double *sa)
 {
     constexpr GamTab kGam;
@@ -2084,30 +2105,45 @@ __device__ __forceinline__ void uniform_spline_wave(const UniformKnots &kn, cons
     const int keep = fac_keep(n), lo = w * keep, hi = lo + keep < n ? lo + keep : n;
     const TriLane t = tri_lane(n, lo, hi);
     const int base = t.wa - 1, cnt = t.wb - base + 1;  // y[wa - 1 .. wb]
-    double v[kTriPass], g[kRun], ial[kRun];
+    double v[kTriPass], g[kRun], ial[kRun], before, ih0 = 0.0;
     load_span(v, y + base, cnt);
-    const double h = kn.span * kn.rden, ih0 = h > 0.0 ? 1.0 / h : 0.0;
-    // rows 1 .. 20 of a first window (its rows start at 1; the other windows' start beyond 20)
-    const bool l0 = t.wa == 1 && lane == 0, l1 = t.wa == 1 && lane == 1;
+    if constexpr (EVEN) {
+        ih0 = 1.0 / (kn.span * kn.rden);
+        // rows 1 .. 20 of a first window (its rows start at 1; the other windows' start beyond 20)
+        const bool l0 = t.wa == 1 && lane == 0, l1 = t.wa == 1 && lane == 1;
 #pragma unroll
-    for (int j = 0; j < kRun; j++) {
-        const double gj = l0 ? kGam.g[1 + j] : (l1 ? kGam.g[kRun + 1 + j] : kGam.g[kGamRows]);
-        g[j] = j < t.len ? gj : 0.0;
-        ial[j] = g[j] * ih0;
+        for (int j = 0; j < kRun; j++) {
+            const double gj = l0 ? kGam.g[1 + j] : (l1 ? kGam.g[kRun + 1 + j] : kGam.g[kGamRows]);
+            g[j] = j < t.len ? gj : 0.0;
+            ial[j] = g[j] * ih0;
+        }
+        before = lane == 0 ? 0.0 : (l1 ? kGam.g[kRun] : kGam.g[kGamRows]);
+    } else {
+        tri_factor(x, t, g, ial, before);
     }
-    const double before = lane == 0 ? 0.0 : (l1 ? kGam.g[kRun] : kGam.g[kGamRows]);
     const TriScan S = tri_scan(g, before);
     store_span(sa, v, cnt);
     wave_lds_sync();
     // the staged row is all read before the first kept row is written
-    tri_solve<UniformRhsLds, false>(n, UniformRhsLds{sa, kn, ih0, base}, lo, hi, OutLds{sa, lo}, t, g, ial, before, S,
-                                    NoIh{});
+    if constexpr (EVEN)
+        tri_solve<UniformRhsLds, false>(n, UniformRhsLds{sa, kn, ih0, base}, lo, hi, OutLds{sa, lo}, t, g, ial, before,
+                                        S, NoIh{});
+    else
+        tri_solve<KnotsRhsLds, false>(n, KnotsRhsLds{sa, x, base}, lo, hi, OutLds{sa, lo}, t, g, ial, before, S,
+                                      NoIh{});
     wave_lds_sync();
 #pragma unroll
     for (int p = 0; p < kTriPass; p++) {
         const int k = p * 64 + lane;
         if (k < hi - lo) c[lo + k] = sa[k];
     }
+}
+
+__device__ __forceinline__ void uniform_spline_wave(const UniformKnots &kn, const double *x, const double *__restrict__ y,
+                                                    double *__restrict__ c, int n, int w, double *sa)
+{
+    if (uniform_even(kn)) uniform_spline_form<true>(kn, x, y, c, n, w, sa);
+    else uniform_spline_form<false>(kn, x, y, c, n, w, sa);
 }
 
 // ---- derivatives for the adjoint ----------------------------------------

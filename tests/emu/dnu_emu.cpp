@@ -149,3 +149,12 @@ extern "C" void emu_specialJ_d(int n, const double *x, double qc, double nufrac_
     for (int m = 0; m < 20; m++) P.en[m] = exp(-m * qc);
     for (int i = 0; i < n; i++) J[i] = kn_dnu::specialJ_d(x[i], P, dJdx[i], dJdqc[i]);
 }
+
+// The fslength table's spline (dnu_device.h uniform_spline_wave) of y over n knots from x0 to xa, for tests.
+extern "C" void emu_fs_spline(double x0, double xa, int n, double *y, double *x, double *c)
+{
+    const UniformKnots kn = fs_knots(x0, xa, n);
+    for (int i = 0; i < n; i++) x[i] = kn.at(i);
+    hipLaunchKernelGGL(k_prep, dim3(prep_blocks(0, n)), dim3(256), 0, 0,
+                       PrepArgs{nullptr, nullptr, 2, 0, 0LL, 0, 1, nullptr, kn, x, y, c, n});
+}
