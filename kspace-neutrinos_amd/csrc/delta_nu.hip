@@ -2086,7 +2086,8 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_m_fs_first_lds(const GroupDes
     f.H = d.H;
     f.c = (const HPair *)lds;
     f.p0 = h_locate(d.H, xi).p;
-    const int np = h_locate(d.H, d.xa).p + 1 - f.p0;
+    f.p1 = h_locate(d.H, d.xa).p;
+    const int np = f.p1 + 1 - f.p0;
     rule_to_lds(rule);
     gconst_double *src = (gconst_double *)d.H.coef + (size_t)f.p0 * kHStride;
     for (int t = threadIdx.x; t < np * kHnc; t += 64 * kFsWaves) lds[t] = src[t / kHnc * kHStride + t % kHnc];

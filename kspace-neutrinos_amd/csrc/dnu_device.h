@@ -284,15 +284,16 @@ struct HLoc {
     int p;
     double v;
 };
-__device__ __forceinline__ HLoc h_locate(const HTab &H, double x)
+__device__ __forceinline__ HLoc h_locate(const HTab &H, double x, int first, int last)
 {
     const double u = (x - H.x0) * H.inv_w;
     HLoc L;
     L.p = (int)u;
-    L.p = L.p < 0 ? 0 : (L.p > H.npanel - 1 ? H.npanel - 1 : L.p);
+    L.p = L.p < first ? first : (L.p > last ? last : L.p);
     L.v = u - L.p;
     return L;
 }
+__device__ __forceinline__ HLoc h_locate(const HTab &H, double x) { return h_locate(H, x, 0, H.npanel - 1); }
 
 // Panel p's value at x from its split record; NaN when it has none.
 __device__ __forceinline__ double h_split(const HTab &H, int p, double x, int which)
@@ -749,18 +750,19 @@ struct FslIntegrand {  // delta_tot_table.c:378-383: 1 / a / (a H(a))
     __device__ __forceinline__ double operator()(double x) const { return inv_a2h(H, x); }
 };
 
-// The same with the panels' 1/(a^2 H) coefficients in LDS: kHnc doubles a
-// panel from panel p0 on (p0 at or below every point's panel).
+// The same with the 1/(a^2 H) coefficients of panels p0 .. p1 in LDS, kHnc
+// doubles a panel.  The points' panels lie among them, but for a point that its
+// rounding carries past the last: it takes the last panel's fit, as beyond a table.
 struct alignas(16) HPair {
     double x, y;
 };
 struct FslIntegrandLds {
     HTab H;
     const HPair *c;  // 16-byte aligned: a pair is one LDS read, whose passes of 16 lanes take one or two panels each
-    int p0;
+    int p0, p1;
     __device__ __forceinline__ double regular(double x) const
     {
-        const HLoc L = h_locate(H, x);
+        const HLoc L = h_locate(H, x, p0, p1);
         const int i0 = L.p - p0;
         const HPair *q = c + (i0 + (i0 << 2));  // kHnc / 2 pairs a panel (shifts: a 32-bit multiply takes four times as long)
         HPair k = q[kHnc / 2 - 1];
@@ -772,7 +774,7 @@ struct FslIntegrandLds {
         }
         return r;
     }
-    __device__ __forceinline__ double split(double x) const { return h_split(H, h_locate(H, x).p, x, 0); }
+    __device__ __forceinline__ double split(double x) const { return h_split(H, h_locate(H, x, p0, p1).p, x, 0); }
 };
 
 template <bool HYB>
