@@ -1765,9 +1765,11 @@ __device__ __forceinline__ void tri_factor(const double *x, const TriLane &t, do
 // What the substitutions' scans over the lanes multiply by, from the factors
 // alone: a lane's run composes to z_out = A - f[0] z_in (A from the row's
 // values), and f[k] is the factor of the 2^k runs that end with the lane's;
-// b[k] likewise backwards.  Three levels reach 8 runs, 80 rows, and a row's
-// influence is below 0.268^80 ~ 1e-46 there (all six levels: the coefficient
-// rows of 256 histories took 754 us for 721).
+// b[k] likewise backwards.  Three levels reach 8 runs, 80 rows: each row passes
+// on at most gam of what reaches it, 0.268 on even knots (1e-46 over 80 rows),
+// below 1/2 on any (alp_i > 2 hr_i + 1.5 hl_i): 0.5^80 = 8e-25, and to come near
+// that every interval has to be many times the one before it.  (All six levels:
+// the coefficient rows of 256 histories took 754 us for 721.)
 constexpr int kScan = 3;
 static_assert((kRun << kScan) >= kHalo, "the scans reach as far as a window's halo");
 struct TriScan {

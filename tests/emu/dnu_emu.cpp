@@ -158,3 +158,17 @@ extern "C" void emu_fs_spline(double x0, double xa, int n, double *y, double *x,
     hipLaunchKernelGGL(k_prep, dim3(prep_blocks(0, n)), dim3(256), 0, 0,
                        PrepArgs{nullptr, nullptr, 2, 0, 0LL, 0, 1, nullptr, kn, x, y, c, n});
 }
+
+// Spline coefficients of nk rows of n stored steps (k_knots, then k_prep's row blocks, rpw rows per wavefront), for tests.
+extern "C" void emu_rows_spline(int n, int nk, int rpw, double *x, double *Y, double *C)
+{
+    std::vector<double> fac(fac_doubles(n)), fx(32), fy(32, 0.0), fc(32);
+    std::vector<int> bucket(4 * n + 1);
+    const UniformKnots kn = fs_knots(0.0, 1.0, 32);
+    for (int i = 0; i < 32; i++) fx[i] = kn.at(i);
+    hipLaunchKernelGGL(k_knots, dim3(knots_blocks(n, 4 * n, 256)), dim3(256), 0, 0,
+                       KnotsArgs{x, n, 4 * n, 4.0 * n / (x[n - 1] - x[0]), fac.data(), bucket.data()});
+    const int bsp = rows_prep_spline_blocks(n, nk, rpw);
+    hipLaunchKernelGGL(k_prep, dim3(prep_blocks(bsp, 32)), dim3(256), 0, 0,
+                       PrepArgs{Y, C, n, nk, (long long)n, bsp, rpw, fac.data(), kn, fx.data(), fy.data(), fc.data(), 32});
+}
