@@ -10,12 +10,17 @@
 #include <math.h>
 #include <vector>
 
+#include "grid_pos.h"
 #include "kn_mem.h"
 
 namespace kn_bin {
 
-// KVAL of powerspectrum.c:27
-__host__ __device__ inline int kval(int n, int dims) { return n <= dims / 2 ? n : n - dims; }
+using kn_grid::Pos;
+using kn_grid::Step;
+using kn_grid::advance;
+using kn_grid::kval;
+using kn_grid::pos_of;
+using kn_grid::step_of;
 
 // Per-bin smallest |k|^2 reaching the bin under the reference expression
 // floor(binsperunit * log(sqrt(k2))) (powerspectrum.c:40, :67).  Returns 0,
@@ -66,10 +71,6 @@ __device__ __forceinline__ int find_bin(int k2, float half_bpu, const int *__res
     return b;
 }
 
-struct Pos {
-    int i, j, z;  // slab offset, row, z of a flat mode offset
-};
-
 __device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
 {
     p.z += step;
@@ -80,24 +81,6 @@ __device__ __forceinline__ void advance(Pos &p, int step, int rowlen, int dims)
             p.i++;
         }
     }
-}
-
-// Position of mode m of the rank's slabs.
-__device__ __forceinline__ Pos pos_of(long long m, int rowlen, int dims)
-{
-    Pos p;
-    if (m < 0x7fffffffLL) {  // 32-bit divisions
-        const unsigned r = (unsigned)m / (unsigned)rowlen;
-        p.z = (int)((unsigned)m - r * (unsigned)rowlen);
-        p.j = (int)(r % (unsigned)dims);
-        p.i = (int)(r / (unsigned)dims);
-    } else {
-        const long long r = m / rowlen;
-        p.z = (int)(m - r * rowlen);
-        p.j = (int)(r % dims);
-        p.i = (int)(r / dims);
-    }
-    return p;
 }
 
 // multiplicity * |F|^2 * ((iwx iwy iwz)^2)^2 in the reference's rounding order
@@ -112,22 +95,6 @@ __device__ __forceinline__ double mode_weight(double2 f, double iwxy, double iwz
     return v;
 }
 
-// A step of n modes along the flattened [slab][row][z] order, split so that
-// advancing a position costs two compares whatever n is.
-struct Step {
-    int di, dj, dz;
-};
-
-__host__ __device__ inline Step step_of(long long n, int rowlen, int dims)
-{
-    const long long r = n / rowlen;
-    Step s;
-    s.dz = (int)(n % rowlen);
-    s.dj = (int)(r % dims);
-    s.di = (int)(r / dims);
-    return s;
-}
-
 struct BinArgs {
     const double2 *F;
     int dims, startslab, nrbins;
@@ -139,21 +106,6 @@ struct BinArgs {
     double *partial;  // gridDim.x * nrbins
     int cshift;       // copies of the bin sums: 2^cshift
 };
-
-__device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int dims)
-{
-    p.z += s.dz;
-    p.j += s.dj;
-    p.i += s.di;
-    if (p.z >= rowlen) {
-        p.z -= rowlen;
-        p.j++;
-    }
-    if (p.j >= dims) {
-        p.j -= dims;
-        p.i++;
-    }
-}
 
 // Where the sweep keeps its tables: the bin thresholds, the per-axis inverse
 // window and the bin sums all in LDS (the fast form); the window read from

@@ -9,27 +9,18 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "grid_pos.h"
 #include "half_log.h"
 #include "kn_mem.h"
 
 namespace kn_res {
 
-__host__ __device__ inline int kval(int n, int dims) { return n <= dims / 2 ? n : n - dims; }
-
-// A step of n modes along the flattened [slab][row][z] order.
-struct Step {
-    int di, dj, dz;
-};
-
-inline Step step_of(long long n, int rowlen, int dims)
-{
-    const long long r = n / rowlen;
-    Step s;
-    s.dz = (int)(n % rowlen);
-    s.dj = (int)(r % dims);
-    s.di = (int)(r / dims);
-    return s;
-}
+using kn_grid::Pos;
+using kn_grid::Step;
+using kn_grid::advance;
+using kn_grid::kval;
+using kn_grid::pos_of;
+using kn_grid::step_of;
 
 struct ResArgs {
     double2 *F;
@@ -134,42 +125,6 @@ __device__ __forceinline__ double smth_of(int k2i, const Tab &T)
         return fma(T.norm, h > 0.0 ? T.rt[i] + (kk - T.lk[i]) / h * (T.rt[i + 1] - T.rt[i]) : T.rt[i], 1.0);
     }
     return fma(T.norm, fma(kk - T.lk[i], T.sl[i], T.rt[i]), 1.0);
-}
-
-struct Pos {
-    int i, j, z;  // slab, row and z of a mode
-};
-
-__device__ __forceinline__ Pos pos_of(long long m, int rowlen, int dims)
-{
-    Pos p;
-    if (m < 0x7fffffffLL) {  // 32-bit divisions
-        const unsigned r = (unsigned)m / (unsigned)rowlen;
-        p.z = (int)((unsigned)m - r * (unsigned)rowlen);
-        p.j = (int)(r % (unsigned)dims);
-        p.i = (int)(r / (unsigned)dims);
-    } else {
-        const long long r = m / rowlen;
-        p.z = (int)(m - r * rowlen);
-        p.j = (int)(r % dims);
-        p.i = (int)(r / dims);
-    }
-    return p;
-}
-
-__device__ __forceinline__ void advance(Pos &p, const Step &s, int rowlen, int dims)
-{
-    p.z += s.dz;
-    p.j += s.dj;
-    p.i += s.di;
-    if (p.z >= rowlen) {
-        p.z -= rowlen;
-        p.j++;
-    }
-    if (p.j >= dims) {
-        p.j -= dims;
-        p.i++;
-    }
 }
 
 // The PM Green's function with CiC deconvolution at k2 > 0, as the potential
