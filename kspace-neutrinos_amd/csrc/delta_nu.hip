@@ -376,14 +376,12 @@ struct QagArgs {
     IcArgs ic;
 };
 
-// Histories of at most this many stored steps have their log a values copied
-// (STAGED: a form of its own, so that the compiler knows the copy for LDS and
-// does not read it by flat accesses)
-// to LDS by the QAG kernels (48 KB, one copy for the block's four wavefronts).
+// Histories of at most this many stored steps have their log a values copied to
+// LDS by the QAG kernels (48 KB, one copy for the block's four wavefronts).
+// STAGED is a form of its own, so that the compiler knows the copy for LDS and
+// does not read it by flat accesses.
 constexpr int kStageMax = 6144;
 
-// Item `item` (species sp, wavenumber k) by one wavefront; sxs: LDS for the
-// stored log a values (na <= kStageMax), or null to read them from memory.
 // The integrand of item (species sp, wavenumber index k), with the stored
 // log a values read from sx (device memory or their LDS copy).
 template <bool HYB>
@@ -448,6 +446,7 @@ __device__ __forceinline__ void stage_knots(const double *__restrict__ sx, int n
     __syncthreads();
 }
 
+// One item (species sp, wavenumber k) by one wavefront.
 template <bool HYB>
 __device__ inline void dnu_qag_item(const QagArgs &a, const SpeciesDev &sp, int item, int k, QagWs &ws,
                                     const double *sx)
@@ -1761,8 +1760,8 @@ static double fit_dJdx(double x)
 }
 
 // Adjoint of get_delta_nu for one mass (delta_tot_table.c:507-611): the
-// forward above with its final QAG subdivisions recorded, then k_dnu_adj and
-// the two row passes on the device; the initial-condition piece on the host.
+// forward above with its final QAG subdivisions recorded, then k_dnu_adj; the
+// initial-condition piece on the host.
 extern "C" int kn_get_delta_nu_adjoint(const _delta_tot_table *d, double a, const double *wavenum, double mnu,
                                        const double *gbar, double *delta_nu, double *dtot_bar, double *init_bar,
                                        double *mnu_bar)
@@ -2172,7 +2171,12 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_m_dnu_qag(const GroupDe
 
 // k_m_dnu_qag's form (qag_spec).  256 histories, 73 k items: 647 us with the
 // integrand's knot walks as loops, flat accesses and the hybrid series in every
-// launch; 462 us now, three wavefronts per SIMD.
+// launch; 462 us now, three wavefronts per SIMD.  One form for the whole group:
+// with a history past kStageMax in it all read their log a through the caches,
+// which costs nothing that shows (us per solve, one history of 6200 steps and 4 k
+// beside 64 of 300 steps and 256 k: 226-230; each history in its own form by one
+// launch 225-226, by two 236-237; beside 128 of 1500 steps and 200 k 666-675,
+// 660-669 and 685-691).
 inline auto m_qag(bool staged, bool hyb)
 {
     return staged ? (hyb ? k_m_dnu_qag<true, true> : k_m_dnu_qag<true, false>)

@@ -10,9 +10,9 @@
 //    NaN smth is fatal (code 5); F *= smth.
 // MI355X design: one coalesced read+write sweep (32 B per mode, non-temporal
 // loads and stores).  The ratio table with its slopes, a table for the
-// logarithm and a uniform bucket index over logk live in LDS, so the segment
-// search is a bucket lookup plus a short forward probe instead of a binary
-// search.  All arithmetic is FP64.
+// logarithm and a uniform bucket index over logk live in LDS (res_plan), so the
+// segment search is a bucket lookup plus a short forward probe instead of a
+// binary search.  All arithmetic is FP64.
 #include <math.h>
 #include <string.h>
 
