@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <type_traits>
 
 #include "grid_pos.h"
 #include "half_log.h"
@@ -37,8 +38,8 @@ struct ResArgs {
     const double *__restrict__ gw;
 };
 
-// The ints of load_tab: buckets 0 .. nbuckets and one flag, in whole doubles.
-__host__ __device__ inline int tab_ints(int nbuckets) { return nbuckets + 2 + (nbuckets & 1); }
+// The ints of load_tab: buckets 0 .. nbuckets, in whole doubles.
+__host__ __device__ inline int tab_ints(int nbuckets) { return nbuckets + 1 + ((nbuckets + 1) & 1); }
 
 // LDS of the sweep: the logarithm's table (log_lds), the ratio table's log k,
 // ratio and slope, its ints, and the Green's factors of one axis.
@@ -53,23 +54,20 @@ struct Tab {
     const double2 *lg;           // kn_logtab
     const int *bucket;
     int nbins, nbuckets;
-    bool odd;  // a log k is not finite, or a slope overflows
     double x0, x1, inv_bw, norm, log_kunit;
 };
 
 // Ratio table, slopes, bucket index and (LOG_LDS) logarithm table into LDS (all threads of the block).
-// A table of one bin is its ratio at every k: its log k, which may be anything, is taken as 0.
 template <bool LOG_LDS>
 __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 {
     extern __shared__ double sm[];
     double *lk = sm + (LOG_LDS ? 2 * KN_LOGTAB_N : 0), *rt = lk + a.nbins, *sl = rt + a.nbins;
-    int *bucket = (int *)(sl + a.nbins), *odd = bucket + a.nbuckets + 1;
-    if (threadIdx.x == 0) *odd = 0;
+    int *bucket = (int *)(sl + a.nbins);
     if (LOG_LDS)
         for (int t = threadIdx.x; t < 2 * KN_LOGTAB_N; t += nthreads) sm[t] = kn_logtab[t];
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
-        lk[t] = a.nbins > 1 ? a.logkk[t] : 0.0;
+        lk[t] = a.logkk[t];
         rt[t] = a.ratio[t];
     }
     __syncthreads();
@@ -85,11 +83,10 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
     T.x1 = lk[a.nbins - 1];
     T.inv_bw = a.nbins > 1 ? a.nbuckets / (T.x1 - T.x0) : 0.0;
     T.norm = a.norm;
-    T.log_kunit = a.nbins > 1 ? a.log_kunit : 0.0;
+    T.log_kunit = a.log_kunit;
     for (int t = threadIdx.x; t < a.nbins; t += nthreads) {
         const double h = t + 1 < a.nbins ? lk[t + 1] - lk[t] : 0.0;
         sl[t] = h > 0.0 ? (rt[t + 1] - rt[t]) / h : 0.0;
-        if (!isfinite(lk[t]) || !isfinite(sl[t])) *odd = 1;
     }
     // bucket[q]: the GSL segment index (largest i <= n-2 with lk[i] <= x) at the bucket's left edge
     for (int q = threadIdx.x; q <= a.nbuckets; q += nthreads) {
@@ -103,7 +100,6 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
         bucket[q] = lo;
     }
     __syncthreads();
-    T.odd = __builtin_amdgcn_readfirstlane(*odd) != 0;
     return T;
 }
 
@@ -111,6 +107,11 @@ __device__ __forceinline__ Tab load_tab(const ResArgs &a, int nthreads)
 // log|k| is evaluated as log(sqrt(k2)) + log(2 pi / BoxSize): the same value as
 // the reference's log(sqrt(k2)*2*M_PI/BoxSize) to about one ulp, without the
 // sqrt and the divisions.
+// Where the stored slopes do not carry a table (a log k that is not finite, also
+// the only bin's; ratios that differ by more than the largest double times the
+// bin's width) the result is infinite or NaN; REF is the reference's own
+// expression, which needs no slope and may be finite there.
+template <bool REF>
 __device__ __forceinline__ double smth_of(int k2i, const Tab &T)
 {
     double kk = half_log(k2i, T.lg) + T.log_kunit;
@@ -120,7 +121,7 @@ __device__ __forceinline__ double smth_of(int k2i, const Tab &T)
     q = q < 0 ? 0 : (q > T.nbuckets ? T.nbuckets : q);
     int i = T.bucket[q];
     while (i < T.nbins - 2 && T.lk[i + 1] <= kk) i++;
-    if (T.odd) {  // the whole table's: the reference's expression, which needs no slope
+    if (REF) {
         const double h = T.nbins > 1 ? T.lk[i + 1] - T.lk[i] : 0.0;
         return fma(T.norm, h > 0.0 ? T.rt[i] + (kk - T.lk[i]) / h * (T.rt[i + 1] - T.rt[i]) : T.rt[i], 1.0);
     }
@@ -170,14 +171,17 @@ __global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
     constexpr int B = 64 * WAVES, T = B * U;
     const int rowlen = a.dims / 2 + 1, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    long long m = (long long)blockIdx.x * T + 64 * wave;  // the wavefront's first mode
+    const long long m0 = (long long)blockIdx.x * T + 64 * wave;  // the wavefront's first mode
     const long long n = a.modes, S = (long long)gridDim.x * T;
     double2 cur[U];
+    auto load = [&](long long m) {
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-        const long long mu = m + B * u + lane;
-        cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
-    }
+        for (int u = 0; u < U; u++) {
+            const long long mu = m + B * u + lane;
+            cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
+        }
+    };
+    load(m0);
     Tab Tb;
     const double *gw = nullptr;
     if (!GREEN || a.nbins > 0) Tb = load_tab<LOG_LDS>(a, B);
@@ -188,74 +192,86 @@ __global__ __launch_bounds__(64 * WAVES) void k_rescale(ResArgs a)
         __syncthreads();
         gw = gw_l;
     }
-    Pos p = pos_of(m, rowlen, a.dims);
-    bool saw_nan = false;
-    for (; m < n; m += S) {
-        // the wavefront's rows: z of its first mode, kx^2 + ky^2 there and in the next row (GREEN: both rows' x and y)
-        int z0[U], kxy[U][2], gx[U][2], gy[U][2];
-        if constexpr (WIDE) {
+    bool left = false, saw_nan = false;
+    auto sweep = [&](auto ref) {
+        Pos p = pos_of(m0, rowlen, a.dims);
+        for (long long m = m0; m < n; m += S) {
+            // the wavefront's rows: z of its first mode, kx^2 + ky^2 there and in the next row (GREEN: both rows' x and y)
+            int z0[U], kxy[U][2], gx[U][2], gy[U][2];
+            if constexpr (WIDE) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int x0 = a.startslab + p.i;
+                    int x1 = x0, j1 = p.j + 1;
+                    if (j1 == a.dims) {
+                        j1 = 0;
+                        x1 = x0 + 1;
+                    }
+                    const int kx0 = kval(x0, a.dims), ky0 = kval(p.j, a.dims), kx1 = kval(x1, a.dims), ky1 = kval(j1, a.dims);
+                    z0[u] = p.z;
+                    kxy[u][0] = kx0 * kx0 + ky0 * ky0;
+                    kxy[u][1] = kx1 * kx1 + ky1 * ky1;
+                    gx[u][0] = x0, gx[u][1] = x1, gy[u][0] = p.j, gy[u][1] = j1;
+                    advance(p, u + 1 < U ? a.in_tile : a.to_next, rowlen, a.dims);
+                }
+            }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const int x0 = a.startslab + p.i;
-                int x1 = x0, j1 = p.j + 1;
-                if (j1 == a.dims) {
-                    j1 = 0;
-                    x1 = x0 + 1;
+                const long long mu = m + B * u + lane;
+                int z, k2;
+                int x = 0, y = 0;
+                if constexpr (WIDE) {
+                    z = z0[u] + lane;
+                    const bool next = z >= rowlen;
+                    z -= next ? rowlen : 0;
+                    k2 = (next ? kxy[u][1] : kxy[u][0]) + __mul24(z, z);
+                    if constexpr (GREEN) {
+                        x = next ? gx[u][1] : gx[u][0];
+                        y = next ? gy[u][1] : gy[u][0];
+                    }
+                } else {
+                    const Pos q = pos_of(mu < n ? mu : 0, rowlen, a.dims);
+                    const int kx = kval(a.startslab + q.i, a.dims), ky = kval(q.j, a.dims);
+                    z = q.z;
+                    k2 = kx * kx + ky * ky + z * z;
+                    x = a.startslab + q.i;
+                    y = q.j;
                 }
-                const int kx0 = kval(x0, a.dims), ky0 = kval(p.j, a.dims), kx1 = kval(x1, a.dims), ky1 = kval(j1, a.dims);
-                z0[u] = p.z;
-                kxy[u][0] = kx0 * kx0 + ky0 * ky0;
-                kxy[u][1] = kx1 * kx1 + ky1 * ky1;
-                gx[u][0] = x0, gx[u][1] = x1, gy[u][0] = p.j, gy[u][1] = j1;
-                advance(p, u + 1 < U ? a.in_tile : a.to_next, rowlen, a.dims);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const long long mu = m + B * u + lane;
-            int z, k2;
-            int x = 0, y = 0;
-            if constexpr (WIDE) {
-                z = z0[u] + lane;
-                const bool next = z >= rowlen;
-                z -= next ? rowlen : 0;
-                k2 = (next ? kxy[u][1] : kxy[u][0]) + __mul24(z, z);
+                if (mu >= n) continue;
+                double2 f = cur[u];
+                if (k2 <= 0) {
+                    if (GREEN) kn_mem::st<true>(a.F + mu, make_double2(0.0, 0.0));
+                    continue;
+                }
+                if (!GREEN || a.nbins > 0) {
+                    double s = smth_of<false>(k2, Tb);
+                    if (isfinite(s) == decltype(ref)::value) {
+                        left = true;
+                        continue;
+                    }
+                    if constexpr (decltype(ref)::value) {
+                        s = smth_of<true>(k2, Tb);
+                        saw_nan |= isnan(s);
+                    }
+                    f.x *= s;
+                    f.y *= s;
+                }
                 if constexpr (GREEN) {
-                    x = next ? gx[u][1] : gx[u][0];
-                    y = next ? gy[u][1] : gy[u][0];
+                    const double g = green_of(k2, gw[x] * gw[y], gw[z]);
+                    f.x *= g;
+                    f.y *= g;
                 }
-            } else {
-                const Pos q = pos_of(mu < n ? mu : 0, rowlen, a.dims);
-                const int kx = kval(a.startslab + q.i, a.dims), ky = kval(q.j, a.dims);
-                z = q.z;
-                k2 = kx * kx + ky * ky + z * z;
-                x = a.startslab + q.i;
-                y = q.j;
+                kn_mem::st<true>(a.F + mu, f);
             }
-            if (mu >= n) continue;
-            double2 f = cur[u];
-            if (k2 <= 0) {
-                if (GREEN) kn_mem::st<true>(a.F + mu, make_double2(0.0, 0.0));
-                continue;
-            }
-            if (!GREEN || a.nbins > 0) {
-                const double s = smth_of(k2, Tb);
-                saw_nan |= isnan(s);
-                f.x *= s;
-                f.y *= s;
-            }
-            if constexpr (GREEN) {
-                const double g = green_of(k2, gw[x] * gw[y], gw[z]);
-                f.x *= g;
-                f.y *= g;
-            }
-            kn_mem::st<true>(a.F + mu, f);
+            load(m + S);
         }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const long long mu = m + S + B * u + lane;
-            cur[u] = mu < n ? kn_mem::ld<true>(a.F + mu) : make_double2(0.0, 0.0);
-        }
+    };
+    sweep(std::false_type{});
+    // the modes that the slopes gave no finite factor, left as they were: a second pass, which all but no table needs (a
+    // mark of such tables asked for each mode took 0.3 us of a 128^3 sweep's 9.4, the factor formed again in place 0.1)
+    if (__ballot(left)) {
+        load(m0);
+        sweep(std::true_type{});
     }
     if (saw_nan) atomicOr(a.nan_flag, 1);
 }

@@ -1,5 +1,6 @@
 """Ratio tables with values that the stored slopes cannot carry: a log k that is
 not finite, ratios whose difference over a bin's width overflows."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -50,12 +51,22 @@ TABLES = {"nan log k": (_put(BASE, 5, math.nan), RT), "nan first": (_put(BASE, 0
           "nan ratio": (BASE, _put(RT, 6, math.nan)), "close": (-8.0 + 1e-13 * np.arange(12), 1e297 * RT)}
 
 
+def _nan_flag(kn, torch):
+    """The flag that NaN factors raise, read and lowered again by the rescale that takes a host table."""
+    fn = kn.kn_rescale_from_host_table
+    dp = C.POINTER(C.c_double)
+    fn.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_double, dp, dp, C.c_int, C.c_double]
+    d, t = torch.ones((4, 4, 3), dtype=torch.complex128, device="cuda"), np.array([-9.0, -8.0])
+    return fn(d.data_ptr(), 4, 0, 4, BOX, t.ctypes.data_as(dp), t.ctypes.data_as(dp), 2, 0.1)
+
+
 @pytest.mark.parametrize("name", list(TABLES))
 @pytest.mark.parametrize("N", [12, 130])
 def test_odd_tables(kn, torch_cuda, name, N):
     """Finite where the rule is, and infinite or NaN where that is (1e-13: log k's rounding over a segment's width; the close
     table within its largest ratio)."""
     torch = torch_cuda
+    assert _nan_flag(kn, torch) == 0
     lk, rt = TABLES[name]
     print("odd table", name, N, flush=True)
     F = _rand_grid(N, 3, 1)
@@ -64,6 +75,7 @@ def test_odd_tables(kn, torch_cuda, name, N):
     n = len(lk)
     assert kn.kn_rescale_device(d.data_ptr(), N, 0, 1, BOX, tab.data_ptr(), tab.data_ptr() + 8 * n, n, NORM, None) == 0
     got = d.cpu().numpy().real[0]
+    assert _nan_flag(kn, torch) == int(np.any(np.isnan(got)))
     want = np.ones_like(got)
     for y in range(0, N, max(1, N // 16)):
         for z in range(N // 2 + 1):
