@@ -126,3 +126,20 @@ def test_returns_with_the_work_in_flight(kn, host, torch_cuda, monkeypatch):
     np.testing.assert_allclose(p, 2.0 * op[:on], rtol=1e-12)
     e = np.max(np.abs(bar.view(np.complex128).reshape(ob.shape) - 2.0 * ob))
     assert rc == 0 and e < 1e-12 * np.max(np.abs(2.0 * ob))
+
+
+def test_reports_the_mass_when_asked(kn, host, torch_cuda, monkeypatch):
+    """With KN_VERBOSE set |F(0)| is reported, as total_powerspectrum does, and the spectrum is the same."""
+    torch = torch_cuda
+    ((F, a),) = _grids(torch, 24, 1)
+    out, n = torch.zeros((2, 24), dtype=torch.float64, device="cuda"), C.c_int()
+    for i in (0, 1):
+        if i:
+            monkeypatch.setenv("KN_VERBOSE", "1")
+        else:
+            monkeypatch.delenv("KN_VERBOSE", raising=False)
+        before = host.kn_test_messages()
+        assert kn.kn_power_spectrum_device(a.data_ptr(), 24, 24, 0, 24, out[i].data_ptr(), C.byref(n), None) == 0
+        assert host.kn_test_messages() == before + i
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(out[1].cpu().numpy(), out[0].cpu().numpy(), rtol=1e-14)
